@@ -484,3 +484,55 @@ def test_small_products_around_the_16_wide_blocks(cm, rng, m, k, n, ta, tb):
     assert np.max(np.abs(c.asarray() - want) / bound) < REL
     for h in (a, b, c):
         h.free_device_memory()
+
+
+# (m, n, k) for every tile shape of k_gemm_ring (64 x 64, 64 x 32, 32 x 64, 32 x 32, 32 x 16, 16 x 32): sides at, one above and
+# one below multiples of the tile, reductions that end on a stage, one behind it and one in front of it, one to many stages
+RING_SHAPES = [(2001, 1003, 250), (640, 1280, 256), (65, 4095, 129), (1500, 300, 1001), (1472, 320, 192), (300, 1501, 333),
+               (287, 1472, 640), (814, 263, 1038), (513, 511, 511), (1024, 100, 2304), (801, 97, 1281), (100, 1025, 1300),
+               (33, 2048, 1151), (4097, 33, 255)]
+
+
+@pytest.mark.parametrize("m,n,k", RING_SHAPES)
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+def test_products_on_tiles_that_move_back_inside(cm, rng, m, n, k, ta, tb):
+    """k_gemm_ring's edges: values beyond the operands (NaN here) never reach a result, and accumulating stores every
+    output once.  fp32 sums of k terms in any order: sqrt(k) * 2^-24 of the norm expected; 16 times that allowed."""
+    def operand(a, trans):
+        stored = np.asfortranarray(a.T if trans else a)
+        rows, cols = stored.shape
+        buf = np.full((rows, cols + 2), np.nan, dtype=np.float32, order='F')
+        buf[:, 1:-1] = stored
+        whole = cm.CUDAMatrix(buf)
+        return whole, whole.slice(1, cols + 1)
+
+    A, B, C = _rand(rng, (m, k)), _rand(rng, (k, n)), _rand(rng, (m, n))
+    (wa, a), (wb, b) = operand(A, ta), operand(B, tb)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    t = cm.dot(a.T if ta else a, b.T if tb else b)
+    limit = 16 * np.sqrt(k) * 2.0 ** -24 * np.linalg.norm(want)
+    assert np.linalg.norm(t.asarray() - want) < limit
+    c = cm.CUDAMatrix(C)
+    c.add_dot(a.T if ta else a, b.T if tb else b, mult=0.5)
+    assert np.linalg.norm(c.asarray() - (C + 0.5 * want)) < limit
+    for h in (wa, wb, t, c):
+        h.free_device_memory()
+
+
+@pytest.mark.parametrize("m,n,k", [(1001, 150, 700), (700, 97, 900), (520, 300, 520)])
+def test_draws_on_tiles_that_move_back_inside(cm, rng, m, n, k):
+    """A sample drawn by the launch of k_gemm_ring is the one sample_bernoulli draws, and so is the generator's state."""
+    w, x, bias = cm.CUDAMatrix(0.1 * _rand(rng, (k, m))), cm.CUDAMatrix(_rand(rng, (k, n))), cm.CUDAMatrix(_rand(rng, (m, 1)))
+    got = []
+    for defer in (True, False):
+        cm.set_deferred_epilogues(defer)
+        try:
+            cm.CUDAMatrix.init_random(11)
+            h, s, r = cm.empty((m, n)), cm.empty((m, n)), cm.empty((m, n))
+            cm.dot(w.T, x, target=h); h.add_col_vec(bias); h.apply_sigmoid(); h.sample_bernoulli(target=s)
+            r.fill_with_rand()
+            got.append([np.array(q.asarray()) for q in (h, s, r)])
+        finally:
+            cm.set_deferred_epilogues(True)
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
