@@ -564,3 +564,55 @@ def test_a_held_back_max_pool_joins_the_response_norm_that_follows(cm, cc, rng, 
     cm.set_deferred_epilogues(True)
     for i, (w, g) in enumerate(zip(*res)):
         assert np.array_equal(w, g), "result %d differs" % i
+
+
+# k_conv_ring: tiles that hang over the last module, filter or tap, reductions around whole stages, batches in tiles
+# over several modules (multiples of 4) and in tiles of one module (others)
+RING_LAYERS = [  # N, C, H, F, k, stride, padding, groups
+    (100, 64, 7, 64, 5, 1, 2, 1),     # tiles over several modules; every module touches the padding
+    (100, 33, 6, 65, 3, 1, 0, 1),     # 65 filters (a column tile moves back 63), 297 terms
+    (36, 48, 8, 96, 3, 2, 1, 2),      # strided, 2 groups
+    (70, 40, 6, 48, 3, 1, 1, 1),      # tiles of one module, Outp on copies of 72 images
+    (33, 32, 7, 33, 3, 1, 1, 1),      # one image more than a tile; filters no multiple of 4
+    (128, 64, 6, 64, 3, 1, 2, 1),     # tiles of one pixel that leave out the taps beyond the modules
+    (64, 16, 9, 144, 5, 1, 0, 1),     # pixels with 1 to 25 taps, 16 colours
+    (20, 128, 7, 32, 3, 1, 1, 1),     # few rows
+    (8, 96, 9, 64, 7, 1, 3, 1),       # 8 images
+    (52, 36, 9, 40, 3, 1, 1, 2),      # 18 colours, 20 filters a group
+    (128, 40, 13, 188, 7, 2, 0, 1),   # more than one stage per split, many splits
+    (100, 1, 20, 96, 3, 1, 1, 1)]     # 9 terms
+
+
+@pytest.mark.parametrize("N,C,H,F,k,s,p,G", RING_LAYERS)
+def test_three_conv_passes_on_ring_tiles(cm, cc, rng, N, C, H, F, k, s, p, G):
+    test_three_conv_passes(cm, cc, rng, N, C, H, F, k, s, p, G)
+
+
+@pytest.mark.parametrize("N,C,H,F,k,s,p", [(128, 32, 6, 64, 3, 1, 1), (100, 20, 5, 48, 3, 1, 0), (67, 16, 6, 33, 3, 1, 1),
+                                           (32, 36, 5, 16, 3, 2, 1), (45, 16, 7, 20, 5, 1, 2)])
+def test_locally_connected_layers_on_ring_tiles(cm, cc, rng, N, C, H, F, k, s, p):
+    test_locally_connected_layers(cm, cc, rng, N, C, H, F, k, s, p)
+
+
+@pytest.mark.parametrize("N", [64, 50])
+def test_pixels_that_no_module_reaches_get_zero_on_ring_tiles(cm, cc, rng, N):
+    C, H, F, k, Mx = 64, 12, 64, 3, 6
+    y, w = _f(rng.standard_normal((N, F * Mx * Mx))), _f(0.1 * rng.standard_normal((F, C * k * k)))
+    down = cm.CUDAMatrix(np.full((N, C * H * H), np.nan, dtype=np.float32))
+    cc.convDown(cm.CUDAMatrix(y), cm.CUDAMatrix(w), down, Mx, 0, 1, k, H, C)
+    reach = Mx + k - 1
+    got = np.asarray(down.asarray()).reshape(N, C, H, H)
+    want = co.conv_down(y, w, C, reach, 0, 1).reshape(N, C, reach, reach)
+    assert np.linalg.norm(got[:, :, :reach, :reach] - want) < 1e-5 * np.linalg.norm(want)
+    assert not got[:, :, reach:, :].any() and not got[:, :, :, reach:].any()
+
+
+@pytest.mark.parametrize("N", [100, 70])
+def test_partial_sums_on_ring_tiles(cm, cc, rng, N):
+    C, H, F, k, s, p = 32, 6, 48, 3, 1, 1
+    Mx = co.n_modules(H, k, s, p)
+    x, y = _f(rng.standard_normal((N, C * H * H))), _f(rng.standard_normal((N, F * Mx * Mx)))
+    t = cm.empty((F, Mx * C * k * k))
+    cc.convOutp(cm.CUDAMatrix(x), cm.CUDAMatrix(y), t, Mx, p, k, s, C, partialSum=Mx)
+    want = co.conv_outp(x, y, C, Mx, k, p, s, partial_sum=Mx)
+    assert np.linalg.norm(t.asarray() - want) < 1e-5 * np.linalg.norm(want)
