@@ -254,16 +254,18 @@ __global__ void __launch_bounds__(256) k_col_softmax(const float* mat, float* ta
 }
 
 // Columns of at most 64 * 4 * NV floats stay in registers between the passes:
-// one read and one write of HBM per element.  Requires h % 4 == 0 and 16-byte
-// aligned columns.
-template <int NV>
+// one read and one write of HBM per element.  TAIL: columns of any height from 4 on at any 4-byte boundary; the last
+// group of rows moves back over its neighbour, counts what is its own and stores the neighbour's values once more.
+// (1001 x 2047: 8.5 -> 5.1 us; 10 x 128: 4.7 -> 3.2 us)
+template <int NV, bool TAIL>
 __global__ void __launch_bounds__(256) k_col_softmax_reg(const float* mat, float* target, int w, int h, SoftmaxExtras x) {
   const int col = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (col >= w) return;
   const float* c4 = mat + (size_t)col * h;
   float* t4 = target + (size_t)col * h;
-  const int n4 = h >> 2;
+  const int n4 = TAIL ? (h + 3) >> 2 : h >> 2;
+  auto first = [&](int j) { return TAIL && 4 * j + 4 > h ? h - 4 : 4 * j; };
   const bool stream = (long long)w * h >= DN_STREAM_MIN_ELEMS;
   float4 v[NV];
   float m = -FLT_MAX;
@@ -271,7 +273,7 @@ __global__ void __launch_bounds__(256) k_col_softmax_reg(const float* mat, float
   for (int k = 0; k < NV; ++k) {
     const int j = lane + k * 64;
     if (j < n4) {
-      v[k] = dn_ld4_rt(c4 + 4 * j, stream);
+      v[k] = dn_ld4_rt(c4 + first(j), stream);
       m = fmaxf(m, fmaxf(fmaxf(v[k].x, v[k].y), fmaxf(v[k].z, v[k].w)));
     }
   }
@@ -283,7 +285,12 @@ __global__ void __launch_bounds__(256) k_col_softmax_reg(const float* mat, float
     if (j < n4) {
       v[k].x = softmax_exp(v[k].x - m); v[k].y = softmax_exp(v[k].y - m);
       v[k].z = softmax_exp(v[k].z - m); v[k].w = softmax_exp(v[k].w - m);
-      s += (v[k].x + v[k].y) + (v[k].z + v[k].w);
+      if (TAIL) {
+        const int lap = 4 * j - first(j);
+        s += ((lap > 0 ? 0.f : v[k].x) + (lap > 1 ? 0.f : v[k].y)) + ((lap > 2 ? 0.f : v[k].z) + v[k].w);
+      } else {
+        s += (v[k].x + v[k].y) + (v[k].z + v[k].w);
+      }
     }
   }
   s = wave_sum(s);
@@ -293,9 +300,9 @@ __global__ void __launch_bounds__(256) k_col_softmax_reg(const float* mat, float
     const int j = lane + k * 64;
     if (j < n4) {
       const float4 pr = make_float4(v[k].x * inv, v[k].y * inv, v[k].z * inv, v[k].w * inv);
-      dn_st4_rt(t4 + 4 * j, pr, stream);
+      dn_st4_rt(t4 + first(j), pr, stream);
       if (x.labels) {
-        const int label = (int)x.labels[col], r0 = 4 * j;
+        const int label = (int)x.labels[col], r0 = first(j);
         if (x.grad)
           dn_st4_rt(x.grad + (size_t)col * h + r0,
                     make_float4(pr.x - ((label == r0) ? 1.f : 0.f), pr.y - ((label == r0 + 1) ? 1.f : 0.f),
@@ -708,7 +715,7 @@ k_rows_stage2(const float* partial, int splits, int h, float* y, float alpha, fl
   }
 }
 
-// One launch for 16-byte aligned operands: a workgroup owns 64 rows (16 lanes x 4 rows,
+// One launch for matrices of at least four rows: a workgroup owns 64 rows (16 lanes x 4 rows,
 // the 4 lane groups of a wavefront on 4 neighbouring columns: 256-byte runs) and the
 // columns [by*cps, (by+1)*cps); NW wavefronts x U loads in flight.  With more than one
 // column slice (at most ROWS_ONE_MAX_SPLITS, chosen so that about one workgroup per CU
@@ -717,6 +724,10 @@ k_rows_stage2(const float* partial, int splits, int h, float* y, float alpha, fl
 // order of arrival.  Partials travel as agent-scope atomic stores and loads (they bypass
 // the non-coherent cache levels; a release fence per wavefront was measured 5-10x slower
 // than the whole kernel), the counter returns to zero for the next launch.
+// Columns start at any 4-byte boundary (global memory serves a 16-byte request there); a height that is no
+// multiple of four moves the last group of rows back.  Before, such columns had one row per lane and mostly two launches:
+// 1001 x 2047, sum 7.1 -> 5.9 us, max 5.6 -> 5.4; the four sums of 2001 x 250 and 1003 x 250 states (one launch now)
+// 29 -> 5.6 us (under the tracer).
 #define ROWS_ONE_MAX_SPLITS 8
 
 template <int OP, int NW, int U, bool STREAM>
@@ -727,7 +738,8 @@ k_rows_one(const float* M, int ld, int h, int w, int cps, const float* x, float*
   __shared__ int s_last;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int r = lane & 15, c = lane >> 4;
-  const int row0 = (blockIdx.x * 16 + r) * 4;
+  const int own0 = (blockIdx.x * 16 + r) * 4;
+  const int row0 = own0 + 4 <= h ? own0 : h - 4;      // the last group moves back; rows that its neighbour has are that one's
   const int j0 = blockIdx.y * cps;
   const int j1 = (j0 + cps < w) ? j0 + cps : w;
   const float init = OP == ROW_MAX ? -INFINITY : 0.f;
@@ -738,7 +750,7 @@ k_rows_one(const float* M, int ld, int h, int w, int cps, const float* x, float*
     else if (OP == ROW_SUM) acc[k] += v;
     else acc[k] = fmaxf(acc[k], v);
   };
-  if (row0 < h) {
+  if (own0 < h) {
     for (int j = j0 + wv * 4 + c; j < j1; j += NW * 4 * U) {
       float4 v[U];
       float xs[U];
@@ -761,7 +773,7 @@ k_rows_one(const float* M, int ld, int h, int w, int cps, const float* x, float*
   for (int o = 16; o < 64; o <<= 1)
 #pragma unroll
     for (int k = 0; k < 4; ++k) acc[k] = row_combine<OP>(acc[k], __shfl_xor(acc[k], o, WAVE));
-  if (c == 0) *reinterpret_cast<float4*>(&sv[wv][r * 4]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  if (c == 0) rowsum_stash(&sv[wv][r * 4], acc, own0 - row0);
   __syncthreads();
   const int splits = gridDim.y;
   const int row = blockIdx.x * 64 + (int)threadIdx.x;
@@ -839,6 +851,10 @@ static void rezero_counters(unsigned* counters, int n) {
   hipGetLastError();
 }
 
+// The sums of layer states run on 256 lanes per workgroup, which start sooner than 1024 (up to 2^18 elements, or two
+// trips of the columns: four sums of 2001 x 250 and 1003 x 250 then share one launch).
+static inline bool rows_one_narrow(int h, int w) { return w <= 256 || (long long)w * h <= (1 << 18); }
+
 template <int OP>
 static int rows_reduce_one(const float* M, int ld, int h, int w, const float* x, float* y, float alpha, float beta,
                            const RowsWorkspace& ws) {
@@ -851,7 +867,7 @@ static int rows_reduce_one(const float* M, int ld, int h, int w, const float* x,
   const bool stream = (long long)w * h >= DN_STREAM_MIN_ELEMS;
   if (cps <= 64)
     hipLaunchKernelGGL((k_rows_one<OP, 4, 4, false>), grid, dim3(256), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
-  else if ((long long)w * h <= (1 << 18))   // layer states (a few hundred units x a batch): 256 lanes start sooner than 1024
+  else if (splits == 1 ? rows_one_narrow(h, w) : (long long)w * h <= (1 << 18))
     hipLaunchKernelGGL((k_rows_one<OP, 4, 8, false>), grid, dim3(256), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
   else if (stream)
     hipLaunchKernelGGL((k_rows_one<OP, 16, 8, true>), grid, dim3(1024), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
@@ -862,7 +878,7 @@ static int rows_reduce_one(const float* M, int ld, int h, int w, const float* x,
   return status;
 }
 
-static inline bool rows_one_ok(const float* M, int ld, int h) {
+static inline bool rows_aligned(const float* M, int ld, int h) {
   return dn_aligned16(M) && (ld % 4 == 0) && (h % 4 == 0);
 }
 
@@ -886,12 +902,13 @@ static int rows_workspace(int h, int w, RowsWorkspace* ws) {
 template <int OP>
 static int rows_reduce(const float* M, int ld, int h, int w, const float* x, float* y, float alpha, float beta) {
   if (h <= 0) return 0;
-  if (rows_one_ok(M, ld, h) && rows_one_splits(h, w) > 0) {
+  if (h >= 4 && rows_one_splits(h, w) > 0) {
     RowsWorkspace ws;
-    if (int e = rows_workspace(h, w, &ws)) return e;
-    return rows_reduce_one<OP>(M, ld, h, w, x, y, alpha, beta, ws);
+    const int e = rows_workspace(h, w, &ws);
+    if (e == 0) return rows_reduce_one<OP>(M, ld, h, w, x, y, alpha, beta, ws);
+    if (rows_aligned(M, ld, h)) return e;       // (other operands need no workspace below while they are small)
   }
-  const bool vec = rows_one_ok(M, ld, h) && h >= 1024;
+  const bool vec = rows_aligned(M, ld, h) && h >= 1024;
   const int rows_per_block = vec ? 256 : 64;
   const int bx = (h + rows_per_block - 1) / rows_per_block;
   int splits = (8 * dn_num_cus()) / bx;
@@ -940,14 +957,13 @@ __global__ void __launch_bounds__(256) k_rows_sum_jobs(RowSumJobs J) { rows_sum_
 
 // Whether sums along the rows of this h x w matrix run as k_rows_one<ROW_SUM, 4, ., false> with one column slice.
 bool dn_row_sum_job_ok(const float* M, int h, int w) {
-  if (h <= 0 || w <= 0 || !rows_one_ok(M, h, h) || rows_one_splits(h, w) != 1) return false;
-  return w <= 64 || (long long)w * h <= (1 << 18);
+  return h >= 4 && w > 0 && rows_one_splits(h, w) == 1 && rows_one_narrow(h, w);
 }
-// 1: as above; 2: rows that do not come in aligned groups of four, small enough for rows_reduce() to take
-// k_rows_stage1<false, ROW_SUM, 4, 4, false> with one column slice; 0: neither.
+// 1: as above; 2: fewer than four rows, which rows_reduce() gives to k_rows_stage1<false, ROW_SUM, 4, 4, false> with one
+// column slice while there are at most 2^18 elements; 0: neither.
 int dn_row_sum_job_kind(const float* M, int h, int w) {
   if (dn_row_sum_job_ok(M, h, w)) return 1;
-  if (h <= 0 || w <= 0 || rows_one_ok(M, h, h)) return 0;
+  if (h <= 0 || w <= 0 || h >= 4) return 0;
   return (long long)w * h <= (1 << 18) ? 2 : 0;
 }
 
@@ -1225,7 +1241,7 @@ int max_by_axis_noalloc(cudamat* mat, cudamat* target, int axis) {
   if (target->size[0] != h || target->size[1] != 1) return ERROR_INCOMPATIBLE_DIMENSIONS;
   if (w <= 0 || h <= 0) return 0;
   const float* M = mat->data_device;
-  if (!rows_one_ok(M, h, h) || rows_one_splits(h, w) == 0) {
+  if (!rows_aligned(M, h, h) || rows_one_splits(h, w) == 0) {
     // unaligned operand, or few rows and very many columns: the 64-row kernel over all columns,
     // one launch and no partials
     hipLaunchKernelGGL((k_rows_stage1<false, ROW_MAX, 4, 4, false>), dim3((h + 63) / 64, 1), dim3(256), 0, dn_stream(), M, h, h, w,
@@ -1435,14 +1451,17 @@ static int softmax_impl(const float* in, float* out, int w, int h, SoftmaxExtras
     else hipLaunchKernelGGL((k_col_softmax_blk<4, 4, false>), grid, block, 0, dn_stream(), in, out, w, h, x);
     return dn_launch_status();
   }
-  if (reg_ok) {
-    const int n4 = h / 4;
+  if (reg_ok || (h >= 4 && h <= 64 * 4 * 16)) {
+    const int n4 = (h + 3) / 4;
     dim3 grid((w + 3) / 4), block(256);
-    if (n4 <= 64) hipLaunchKernelGGL((k_col_softmax_reg<1>), grid, block, 0, dn_stream(), in, out, w, h, x);
-    else if (n4 <= 128) hipLaunchKernelGGL((k_col_softmax_reg<2>), grid, block, 0, dn_stream(), in, out, w, h, x);
-    else if (n4 <= 256) hipLaunchKernelGGL((k_col_softmax_reg<4>), grid, block, 0, dn_stream(), in, out, w, h, x);
-    else if (n4 <= 512) hipLaunchKernelGGL((k_col_softmax_reg<8>), grid, block, 0, dn_stream(), in, out, w, h, x);
-    else hipLaunchKernelGGL((k_col_softmax_reg<16>), grid, block, 0, dn_stream(), in, out, w, h, x);
+#define SOFTMAX_REG(NV) do { if (reg_ok) hipLaunchKernelGGL((k_col_softmax_reg<NV, false>), grid, block, 0, dn_stream(), in, out, w, h, x); \
+                             else hipLaunchKernelGGL((k_col_softmax_reg<NV, true>), grid, block, 0, dn_stream(), in, out, w, h, x); } while (0)
+    if (n4 <= 64) SOFTMAX_REG(1);
+    else if (n4 <= 128) SOFTMAX_REG(2);
+    else if (n4 <= 256) SOFTMAX_REG(4);
+    else if (n4 <= 512) SOFTMAX_REG(8);
+    else SOFTMAX_REG(16);
+#undef SOFTMAX_REG
     return dn_launch_status();
   }
   // columns of 4097 to 16384 rows still fit the registers of a workgroup (two columns or one at

@@ -22,6 +22,18 @@ __device__ __forceinline__ float rowsum_finish(float yold, float s, float alpha,
   return __fmaf_rn(alpha, s, beta == 0.f ? 0.f : __fmul_rn(beta, yold));
 }
 
+// The sums of a lane's group of four rows into the slots of its own rows, which start `lap` rows into the group (0 but
+// for a last group that moved back inside the matrix).
+__device__ __forceinline__ void rowsum_stash(float* own, const float (&acc)[4], int lap) {
+  if (lap == 0) {
+    *reinterpret_cast<float4*>(own) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  } else {
+#pragma unroll
+    for (int k = 1; k < 4; ++k)
+      if (k >= lap) own[k - lap] = acc[k];
+  }
+}
+
 // Workgroup `block` of the jobs: 64 rows of one of the vectors, on the first 256 lanes (a larger
 // workgroup's other lanes only keep the barriers company).
 __device__ __forceinline__ void rows_sum_jobs_body(const RowSumJobs& J, int block) {
@@ -33,7 +45,7 @@ __device__ __forceinline__ void rows_sum_jobs_body(const RowSumJobs& J, int bloc
   float* y = second ? J.y1 : J.y0;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int r = lane & 15, c = lane >> 4;
-  const int row0 = (bx * 16 + r) * 4;
+  const int own0 = (bx * 16 + r) * 4, row0 = own0 + 4 <= h ? own0 : h - 4;      // (as k_rows_one; h >= 4)
   const int row = bx * 64 + (int)threadIdx.x;
   const bool mine = threadIdx.x < 64 && row < h;
   float yv = mine ? y[row] : 0.f;
@@ -45,7 +57,7 @@ __device__ __forceinline__ void rows_sum_jobs_body(const RowSumJobs& J, int bloc
     const int w = job.w;
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     if (job.scalar) {
-      // matrices whose rows do not come in aligned groups of four: a lane owns one row, in the order of
+      // matrices of fewer than four rows: a lane owns one row, in the order of
       // k_rows_stage1<false, ROW_SUM, 4, 4, false> with one column slice (wavefront v the columns v, v + 4, ..,
       // four in flight; a column past the end adds a zero)
       const int srow = bx * 64 + lane;
@@ -73,7 +85,7 @@ __device__ __forceinline__ void rows_sum_jobs_body(const RowSumJobs& J, int bloc
       __syncthreads();
       continue;
     }
-    if (live && row0 < h) {
+    if (live && own0 < h) {
       for (int j = wv * 4 + c; j < w; j += NW * 4 * U) {
         float4 v[U];
 #pragma unroll
@@ -89,7 +101,7 @@ __device__ __forceinline__ void rows_sum_jobs_body(const RowSumJobs& J, int bloc
     for (int o = 16; o < 64; o <<= 1)
 #pragma unroll
       for (int k = 0; k < 4; ++k) acc[k] += __shfl_xor(acc[k], o, 64);
-    if (live && c == 0) *reinterpret_cast<float4*>(&sv[wv][r * 4]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    if (live && c == 0) rowsum_stash(&sv[wv][r * 4], acc, own0 - row0);
     __syncthreads();
     if (mine) {
       float s = sv[0][threadIdx.x];

@@ -303,3 +303,48 @@ def test_sums_leave_the_bits_of_dot_with_a_vector_of_ones(cm, rng, shape):
     ones_all = cm.CUDAMatrix(np.ones((h, w), dtype=np.float32))
     assert np.float32(a.sum()).tobytes() == np.float32(cm.vdot(a, ones_all)).tobytes()
     assert abs(a.sum() - x.astype(np.float64).sum()) <= 1e-5 * np.abs(x).astype(np.float64).sum()
+
+
+@pytest.mark.parametrize("h", [4, 5, 6, 7, 63, 65, 66, 127, 1001])
+@pytest.mark.parametrize("w", [2, 9, 250, 700, 2047])
+@pytest.mark.parametrize("skip", [0, 1])
+def test_rows_in_groups_of_four_that_move_back(cm, rng, h, w, skip):
+    """Sums and maxima along axis 1 of columns at any 4-byte boundary: every row once, nothing of the columns in front of
+    and behind the matrix (NaN).  fp32 sums of w terms in any order: at most w * 2^-24 of the sum of magnitudes."""
+    buf = np.full((h, w + 2 * skip), np.nan, dtype=np.float32, order='F')
+    x = _rand(rng, (h, w))
+    buf[:, skip:skip + w] = x
+    whole = cm.CUDAMatrix(buf)
+    a = whole.slice(skip, skip + w)
+    bound = w * 2.0 ** -24 * np.abs(x).astype(np.float64).sum(axis=1, keepdims=True) + 1e-30
+    y = cm.CUDAMatrix(np.ones((h, 1), dtype=np.float32))
+    y.add_sums(a, axis=1, mult=2.0)
+    want = x.astype(np.float64).sum(axis=1, keepdims=True)
+    assert np.all(np.abs(y.asarray() - (1.0 + 2.0 * want)) <= 2 * bound + 2.0 ** -23 * np.abs(1.0 + 2.0 * want))
+    assert np.all(np.abs(a.sum(axis=1).asarray() - want) <= bound)
+    assert np.array_equal(a.max(axis=1).asarray(), x.max(axis=1, keepdims=True))
+    whole.free_device_memory()
+
+
+@pytest.mark.parametrize("h", [4, 5, 10, 255, 257, 510, 1001, 1023, 2047, 4095])
+@pytest.mark.parametrize("skip", [0, 1])
+def test_softmax_of_columns_whose_last_group_moves_back(cm, rng, h, skip):
+    """As the double-precision value, also in place, with -inf and FLT_MAX-masked entries in the last rows."""
+    w = 37
+    x = _rand(rng, (h, w), -4.0, 4.0)
+    x[-1, ::3] = -np.inf
+    x[-2, 1::3] = -3.4028235e38
+    buf = np.full((h, w + 2 * skip), np.nan, dtype=np.float32, order='F')
+    buf[:, skip:skip + w] = x
+    whole, out = cm.CUDAMatrix(buf), cm.empty((h, w))
+    a = whole.slice(skip, skip + w)
+    e = np.exp(x.astype(np.float64) - x.max(axis=0))
+    want = e / e.sum(axis=0)
+    a.apply_softmax(target=out)
+    assert np.allclose(out.asarray(), want, rtol=REL, atol=1e-30)
+    got = out.asarray().copy()
+    a.apply_softmax()
+    assert np.array_equal(a.asarray(), got)
+    rest = np.delete(whole.asarray(), np.s_[skip:skip + w], axis=1)
+    assert np.isnan(rest).all()
+    whole.free_device_memory()
