@@ -2717,47 +2717,43 @@ static bool ring_done(const char* where) {
   return true;
 }
 
-static bool conv_up_ring(const ConvArgs& a, const char* where) {
-  const int K = a.Cg * a.kk2;
-  if (!ring_ok(a, (long long)K * (a.local ? a.M : 1))) return false;
-  // 16-byte groups must not straddle modules: a batch of any size runs in tiles of one module
-  const bool single = a.local || a.N % 4 != 0;
-  const long long rows = single ? a.N : (long long)a.M * a.N;
-  const int periods = single ? a.M : 1;
-  const ConvRingPlan plan = conv_ring_plan(CONV_UP, rows, a.Fg, (long long)periods * a.G, K, 1., false, 0.);
-  if (plan.cfg < 0 || plan.us > conv_other_us(a, CONV_UP, a.M)) return false;
-  ConvRingArgs p = ring_args(a);
-  p.a = a.img; p.b = a.flt;
-  p.a_bytes = (unsigned)((long long)a.N * a.HH * a.C * 4);
-  p.rows = (int)rows; p.cols = a.Fg; p.periods = periods; p.gz = a.G; p.K = K; p.ldc = (long long)a.N * a.M;
-  conv_ring_launch<CONV_UP>(plan, p);
-  return ring_done(where);
+// The share of a layer's taps that lie inside the image (Up) or reach a module (Down), and with it of the reduction that
+// tiles of one module or pixel have.
+static double ring_used(const ConvArgs& a, int mode) {
+  const int lines = mode == CONV_UP ? a.Mx : a.H;
+  long long taps = 0;                                                    // of a column of modules or pixels
+  for (int i = 0; i < lines; ++i) {
+    const int v = mode == CONV_UP ? i * a.s + a.pad0 : i - a.pad0;
+    const int lo = mode == CONV_UP ? -v : v - a.Mx + 1, hi = mode == CONV_UP ? a.H - v : v + 1;
+    const int n = (hi < a.k ? hi : a.k) - (lo > 0 ? lo : 0);
+    if (n > 0) taps += n;
+  }
+  const double one = (double)taps / ((double)lines * a.k);
+  return one * one;
 }
 
-static bool conv_down_ring(const ConvArgs& a, const char* where) {
+// Up and Down: tiles over any run of (module | pixel, image) groups, which needs batches of whole groups of four, or of
+// one module or pixel each, which leave out taps beyond the edge and need no masks.
+static bool conv_rows_ring(const ConvArgs& a, int mode, const char* where) {
+  const bool up = mode == CONV_UP;
   const long long bank = (long long)a.Cg * a.kk2 * (a.local ? a.M : 1);
-  if (a.s != 1 || a.Fg % 4 != 0 || !ring_ok(a, bank)) return false;     // (an entry is four filters of a tap)
-  // Tiles of one pixel where the batch asks for them or fills them: they leave out the taps that reach no module.
-  const bool single = a.local || a.N % 4 != 0 || a.N % 64 == 0;
-  const long long rows = single ? a.N : (long long)a.HH * a.N;
-  const int periods = single ? a.HH : 1, K = a.kk2 * a.Fg;
-  double used = 1.;
-  if (single) {
-    long long taps = 0;                                                  // of a column of pixels
-    for (int y = -a.pad0; y < a.H - a.pad0; ++y) {
-      const int n = (y + 1 < a.k ? y + 1 : a.k) - (y - a.Mx + 1 > 0 ? y - a.Mx + 1 : 0);
-      if (n > 0) taps += n;
-    }
-    used = (double)taps / ((double)a.H * a.k);
-    used *= used;
+  if (!ring_ok(a, bank) || (!up && (a.s != 1 || a.Fg % 4 != 0))) return false;     // (Down: an entry is four filters of a tap)
+  const int sites = up ? a.M : a.HH, cols = up ? a.Fg : a.Cg, K = a.kk2 * (up ? a.Cg : a.Fg);
+  ConvRingPlan plan = conv_ring_plan(mode, true, a.N, cols, (long long)sites * a.G, K, ring_used(a, mode), false, 0.);
+  bool single = true;
+  if (!a.local && a.N % 4 == 0) {
+    const ConvRingPlan flat = conv_ring_plan(mode, false, (long long)sites * a.N, cols, a.G, K, 1., false, 0.);
+    if (flat.cfg >= 0 && (plan.cfg < 0 || flat.us < plan.us)) { plan = flat; single = false; }
   }
-  const ConvRingPlan plan = conv_ring_plan(CONV_DOWN, rows, a.Cg, (long long)periods * a.G, K, used, false, 0.);
-  if (plan.cfg < 0 || plan.us > conv_other_us(a, CONV_DOWN, a.HH)) return false;
+  if (plan.cfg < 0 || plan.us > conv_other_us(a, mode, sites)) return false;
   ConvRingArgs p = ring_args(a);
-  p.a = a.hid; p.b = a.flt;
-  p.a_bytes = (unsigned)((long long)a.N * a.M * a.F * 4); p.b_bytes = (unsigned)(a.F * bank * 4);
-  p.rows = (int)rows; p.cols = a.Cg; p.periods = periods; p.gz = a.G; p.K = K; p.ldc = (long long)a.N * a.HH;
-  conv_ring_launch<CONV_DOWN>(plan, p);
+  p.a = up ? a.img : a.hid; p.b = a.flt;
+  p.a_bytes = (unsigned)((long long)a.N * (up ? (long long)a.HH * a.C : (long long)a.M * a.F) * 4);
+  p.b_bytes = (unsigned)(a.F * bank * 4);
+  p.rows = single ? a.N : sites * a.N; p.cols = cols; p.periods = single ? sites : 1; p.gz = a.G; p.K = K;
+  p.ldc = (long long)a.N * sites;
+  if (up) { if (single) conv_ring_launch<CONV_UP, true>(plan, p); else conv_ring_launch<CONV_UP, false>(plan, p); }
+  else { if (single) conv_ring_launch<CONV_DOWN, true>(plan, p); else conv_ring_launch<CONV_DOWN, false>(plan, p); }
   return ring_done(where);
 }
 
@@ -2775,7 +2771,7 @@ static bool conv_outp_ring(const ConvArgs& a0, cudamat* images, cudamat* hidActs
   a.N = N4;
   const int cols = a.Cg * a.kk2, K = a.m_count * a.N;
   if (!ring_ok(a, (long long)cols * a.chunks) || a.chunks > 32767) return false;
-  const ConvRingPlan plan = conv_ring_plan(CONV_OUTP, a.Fg, cols, (long long)a.G * a.chunks, K, 1., true, 2e-6 * a.chunks * a.F * cols);
+  const ConvRingPlan plan = conv_ring_plan(CONV_OUTP, false, a.Fg, cols, (long long)a.G * a.chunks, K, 1., true, 2e-6 * a.chunks * a.F * cols);
   const double maps = 1e-9 * 8. * N4 * ((double)a.M * a.F + (double)a.HH * a.C);
   // (1.12: what a layer's sums over many splits take beyond the plan's estimate)
   if (plan.cfg < 0 || 1.12 * plan.us + (N4 != a0.N ? 5. + maps / 5e-3 : 0.) > conv_other_us(a0, CONV_OUTP, a.M)) return false;
@@ -2797,7 +2793,7 @@ static bool conv_outp_ring(const ConvArgs& a0, cudamat* images, cudamat* hidActs
   p.a_bytes = (unsigned)((long long)a.N * a.M * a.F * 4); p.b_bytes = (unsigned)((long long)a.N * a.HH * a.C * 4);
   p.rows = a.Fg; p.cols = cols; p.gz = a.chunks * plan.splits * a.G; p.K = K; p.splits = plan.splits; p.split_stages = plan.split_stages;
   p.ldc = plan.splits > 1 ? a.Fg : a.F; p.out_stride = (long long)a.F * cols;
-  conv_ring_launch<CONV_OUTP>(plan, p);
+  conv_ring_launch<CONV_OUTP, false>(plan, p);
   if (plan.splits > 1) launch_outp_finish(a);
   return ring_done(where);
 }
@@ -2809,7 +2805,7 @@ void convUp(cudamat* images, cudamat* filters, cudamat* targets, int numModulesX
   conv_clear_error();
   ConvArgs a;
   if (!conv_up_args(images, filters, targets, numModulesX, paddingStart, moduleStride, numImgColors, numGroups, "convUp", false, a)) return;
-  if (conv_up_ring(a, "convUp")) return;
+  if (conv_rows_ring(a, CONV_UP, "convUp")) return;
   PaddedBatch pb(images, targets, nullptr);
   if (pb.on) {
     pb.fill(0, images);
@@ -2825,7 +2821,7 @@ void convDown(cudamat* hidActs, cudamat* filters, cudamat* targets, int imgSize,
   conv_clear_error();
   ConvArgs a;
   if (!conv_down_args(hidActs, filters, targets, imgSize, paddingStart, moduleStride, numImgColors, numGroups, "convDown", false, a)) return;
-  if (conv_down_ring(a, "convDown")) return;
+  if (conv_rows_ring(a, CONV_DOWN, "convDown")) return;
   PaddedBatch pb(hidActs, targets, nullptr);
   if (pb.on) {
     pb.fill(0, hidActs);
@@ -2866,7 +2862,7 @@ void localUp(cudamat* images, cudamat* filters, cudamat* targets, int numModules
   conv_clear_error();
   ConvArgs a;
   if (!conv_up_args(images, filters, targets, numModulesX, paddingStart, moduleStride, numImgColors, numGroups, "localUp", true, a)) return;
-  if (conv_up_ring(a, "localUp")) return;
+  if (conv_rows_ring(a, CONV_UP, "localUp")) return;
   PaddedBatch pb(images, targets, nullptr, local_batch(images->size[0]));
   if (pb.on) {
     pb.fill(0, images);
@@ -2883,7 +2879,7 @@ void localDown(cudamat* hidActs, cudamat* filters, cudamat* targets, int imgSize
   conv_clear_error();
   ConvArgs a;
   if (!conv_down_args(hidActs, filters, targets, imgSize, paddingStart, moduleStride, numImgColors, numGroups, "localDown", true, a)) return;
-  if (conv_down_ring(a, "localDown")) return;
+  if (conv_rows_ring(a, CONV_DOWN, "localDown")) return;
   PaddedBatch pb(hidActs, targets, nullptr, local_batch(hidActs->size[0]));
   if (pb.on) {
     pb.fill(0, hidActs);

@@ -34,16 +34,20 @@ struct ConvRingArgs {
 //      2: rows are colours, four filters of a tap per entry (B of Down)
 //      3: rows are filters, terms (module, image) in order of memory (A of Outp)
 //      4: rows are taps, four images of a module per entry (B of Outp)
+//   On tiles of one module or pixel every entry is an offset into each operand, or RING_FAR behind the last term:
+//      5, 6: A (x of an entry) and B (y) of Up and A of Down
+//      7: B of Down
 template <int KIND, int ROWS, int BK, int PER>
-struct ConvRingOperand : RingTile<ROWS, BK, (KIND >= 2)> {
-  using Tile = RingTile<ROWS, BK, (KIND >= 2)>;
+struct ConvRingOperand : RingTile<ROWS, BK, ((KIND >= 2 && KIND <= 4) || KIND == 7)> {
+  using Tile = RingTile<ROWS, BK, ((KIND >= 2 && KIND <= 4) || KIND == 7)>;
   using Tile::NG;
-  static constexpr bool ENT = KIND == 0;                                  // an entry per group, else one per lane and stage
+  static constexpr bool ENT = KIND == 0 || KIND == 5 || KIND == 6;        // an entry per group, else one per lane and stage
+  static constexpr bool LOOKS = KIND != 1 && KIND != 3;
   __amdgpu_buffer_rsrc_t rsrc;
   unsigned off[NG], mask[NG];
   unsigned step;                                                          // KIND 1
   int left;                                                               // KIND 3: terms behind the lane's first one
-  const uint2* tab;                                                       // KIND 0, 4
+  const uint2* tab;                                                       // KIND 0, 4 .. 7
   const unsigned* tab1;                                                   // KIND 2
   uint2 ent[ENT ? NG : 1];
   __device__ __forceinline__ void look(int t, int nst) {
@@ -54,10 +58,19 @@ struct ConvRingOperand : RingTile<ROWS, BK, (KIND >= 2)> {
     }
     if (KIND == 2) ent[0].x = tab1[at + Tile::group_k(threadIdx.x, 0) / PER];
     if (KIND == 4) ent[0] = tab[at + Tile::group_k(threadIdx.x, 0) / PER];
+    const int free = t * (BK / PER);                                      // (the table of these reaches over what is asked for)
+    if (KIND == 5 || KIND == 6) {
+#pragma unroll
+      for (int u = 0; u < NG; ++u) {
+        const uint2* e = tab + free + Tile::group_k(threadIdx.x, u) / PER;
+        ent[u].x = KIND == 5 ? e->x : e->y;
+      }
+    }
+    if (KIND == 7) ent[0].x = tab[free + Tile::group_k(threadIdx.x, 0) / PER].y;
   }
   __device__ __forceinline__ void fetch(int t, int nst, ring_f32x4 (&r)[NG]) {
     const unsigned behind = (unsigned)(nst - 1 - t) & RING_FAR;           // a stage behind the last one goes nowhere
-    if (KIND == 0 || KIND == 2 || KIND == 4) { if (t == 0) look(0, nst); }
+    if (LOOKS && t == 0) look(0, nst);
 #pragma unroll
     for (int u = 0; u < NG; ++u) {
       unsigned o;
@@ -70,13 +83,15 @@ struct ConvRingOperand : RingTile<ROWS, BK, (KIND >= 2)> {
         o = (off[u] + ent[0].x) | behind;
       } else if (KIND == 3) {
         o = t * BK < left ? off[u] + (unsigned)(t * BK * 4) : RING_FAR;
+      } else if (KIND >= 5) {
+        o = off[u] + ent[ENT ? u : 0].x;
       } else {
         const unsigned have = behind ? 0u : ent[0].y;
         o = (mask[u] & have) == mask[u] ? off[u] + ent[0].x : RING_FAR;
       }
       r[u] = __builtin_bit_cast(ring_f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)o, 0, 0));
     }
-    if (KIND == 0 || KIND == 2 || KIND == 4) look(t + 1, nst);
+    if (LOOKS) look(t + 1, nst);
   }
 };
 
@@ -87,22 +102,22 @@ struct ConvRingOperand : RingTile<ROWS, BK, (KIND >= 2)> {
 // 128 rows.  Here the rows of a tile are any run of (module | pixel, image) groups, the loads of four stages are in flight,
 // the wavefronts of a workgroup split the stage, and the offset of every 16-byte group is a lane's base plus
 // an entry of a table in LDS (what a term of the reduction adds, and a mask for the padding): five vector
-// instructions per group and stage.  Tiles of one module or pixel (locally connected layers, batches that are no
-// multiple of 4) need the batch only to be as large as the tile; convDown then leaves out taps beyond the modules.
+// instructions per group and stage.  Tiles of one module or pixel (SINGLE: locally connected layers, batches that are no
+// multiple of 4 or that the tile divides) need no masks and leave out the taps beyond the edge.
 // convOutp splits its reduction over workgroups and is summed by k_conv_outp_finish*.
 // Measured, us Up / Down / Outp, before -> now (with the copies and sums):
 //   64 -> 64 colours 5 x 5, 13 x 13, batch 100      72 / 63 / 66 -> 49 / 48 / 39      (22 each at 157 TFLOP/s)
 //   64 -> 64 colours 3 x 3, 17 x 17, batch 100      69 / 58 / 55 -> 25 / 26 / 29      (14)
 //   local 64 -> 64 colours 3 x 3, 8 x 8, batch 128  20 / 19 / 25 -> 10 / 10 / 14      (4)
 //   local 48 -> 64 colours 3 x 3, 14 x 14, 100      38 / 37 / 4570 -> 20 / 28 / 25    (7)
-//   96 -> 256 colours 5 x 5, 2 groups, 27 x 27, 128 Outp 539 -> 470; Up 540 and Down 483 on either
-// A stage takes 1.25 times its MFMAs: the offsets, and LDS reads of one value per lane for operands that are not
-// contiguous along the reduction.
-template <int MODE, int TB, int BM, int BN, int BK>
+//   96 -> 256 colours 5 x 5, 2 groups, 27 x 27, 128 Up 532 -> 492 (9 % of its taps are padding), Outp 539 -> 467; Down
+//   467 on k_conv_mfma (48 columns)
+// The MFMAs are busy for 81 to 83 % of the time there; without the masks a stage takes as long as with them.
+template <int MODE, bool SINGLE, int TB, int BM, int BN, int BK>
 __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
   constexpr int PER = MODE == CONV_UP ? 1 : 4;
-  using OA = ConvRingOperand<MODE == CONV_OUTP ? 3 : 0, BM, BK, PER>;
-  using OB = ConvRingOperand<MODE == CONV_UP ? 1 : MODE == CONV_DOWN ? 2 : 4, BN, BK, PER>;
+  using OA = ConvRingOperand<MODE == CONV_OUTP ? 3 : SINGLE ? 5 : 0, BM, BK, PER>;
+  using OB = ConvRingOperand<MODE == CONV_UP ? (SINGLE ? 6 : 1) : MODE == CONV_DOWN ? (SINGLE ? 7 : 2) : 4, BN, BK, PER>;
   using Shape = RingShape<TB, BM, BN, BK, OA, OB>;
   constexpr int EPL = Shape::EPL;
   __shared__ __attribute__((aligned(16))) float lds[Shape::LDS];
@@ -125,7 +140,54 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
   OA oa; OB ob;
   int nst, g = z;
   float* out = p.out;
-  if constexpr (MODE == CONV_UP) {
+  if constexpr (SINGLE) {
+    // One module or pixel: taps that leave the image, or reach no module, are left out.  The others are rows ky0 ..
+    // ky0 + ny - 1 and columns kx0 .. kx0 + nx - 1 of the filter.
+    const int line = div(per, MODE == CONV_UP ? p.dMx : p.dH), at = per - line * (MODE == CONV_UP ? Mx : H);
+    const int y = MODE == CONV_UP ? line * p.s + p.pad0 : line - p.pad0, x = MODE == CONV_UP ? at * p.s + p.pad0 : at - p.pad0;
+    auto range = [&](int v, int* first) {
+      const int lo = MODE == CONV_UP ? -v : v - Mx + 1, hi = MODE == CONV_UP ? H - v : v + 1;
+      *first = lo > 0 ? lo : 0;
+      return (hi < k ? hi : k) - *first;
+    };
+    int ky0, kx0;
+    int ny = range(y, &ky0), nx = range(x, &kx0);
+    if (ny <= 0 || nx <= 0) { ny = 0; nx = 1; }
+    const int area = ny * nx, K = area * (MODE == CONV_UP ? p.Cg : p.Fg);
+    nst = K > BK ? (K + BK - 1) / BK : 1;
+    // exact for dividends below 2^12 and divisors up to RING_MAX_SIDE^2
+    const unsigned inv_nx = 65536u / (unsigned)nx + 1u, inv_area = (1u << 20) / (unsigned)(area > 0 ? area : 1) + 1u;
+    const unsigned Nu = (unsigned)N, Fu = (unsigned)p.F;
+    for (int e = tid; e < (nst + RING_SETS + 3) * (BK / PER); e += RING_THREADS) {
+      uint2 t2 = make_uint2(RING_FAR, RING_FAR);
+      if (PER * e < K) {
+        const int c = MODE == CONV_UP ? (int)((unsigned)e * inv_area >> 20) : 0;
+        const int tap = MODE == CONV_UP ? e - c * area : div(4 * e, p.dFg), f = MODE == CONV_UP ? 0 : 4 * e - tap * p.Fg;
+        const int ty = (int)((unsigned)tap * inv_nx >> 16), ky = ky0 + ty, kx = kx0 + tap - ty * nx;
+        if (MODE == CONV_UP) {
+          const int bank = p.local ? per : 0;
+          t2.x = 4u * Nu * (unsigned)((g * p.Cg + c) * p.HH + (y + ky) * H + x + kx);
+          t2.y = 4u * Fu * (unsigned)((bank * p.Cg + c) * p.kk2 + ky * k + kx);
+        } else {
+          const int m = (y - ky) * Mx + x - kx;
+          t2.x = 4u * Nu * (unsigned)(p.M * (g * p.Fg + f) + m);
+          t2.y = 4u * ((unsigned)f + Fu * (unsigned)(ky * k + kx + p.Cg * p.kk2 * (p.local ? m : 0)));
+        }
+      }
+      table[e] = t2;
+    }
+    oa.tab = ob.tab = table;
+    const int n = m0 + OA::group_row(tid, 0);
+#pragma unroll
+    for (int u = 0; u < OA::NG; ++u) oa.off[u] = 4u * (unsigned)(n + (PER == 4 ? N * p.M * (OA::group_k(tid, u) % 4) : 0));
+#pragma unroll
+    for (int u = 0; u < OB::NG; ++u) {
+      const int col = n0 + OB::group_row(tid, u);
+      ob.off[u] = 4u * (unsigned)(g * p.Fg + (MODE == CONV_UP ? col : p.F * p.kk2 * col));
+    }
+    ob.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p.b, 0, (int)p.b_bytes, 0x00020000);
+    out += (long long)g * p.cols * p.ldc + (long long)per * p.rows;
+  } else if constexpr (MODE == CONV_UP) {
     const int K = p.Cg * p.kk2;
     nst = (K + BK - 1) / BK;
     for (int e = tid; e < nst * BK; e += RING_THREADS) {
@@ -133,7 +195,7 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
       table[e] = e < K ? make_uint2(4u * (unsigned)N * (unsigned)(c * p.HH + ky * H + kx), 1u << ky | 1u << (RING_MAX_SIDE + kx))
                        : make_uint2(0u, RING_FAR);
     }
-    const int r = per * p.rows + m0 + OA::group_row(tid, 0);
+    const int r = m0 + OA::group_row(tid, 0);
     const int m = div(r, p.dN), n = r - m * N, my = div(m, p.dMx), mx = m - my * Mx;
     const int y = my * p.s + p.pad0, x = mx * p.s + p.pad0;
 #pragma unroll
@@ -142,36 +204,23 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
       oa.mask[u] = ring_bits(-y, H - y < k ? H - y : k) | ring_bits(-x, H - x < k ? H - x : k) << RING_MAX_SIDE;
     }
     oa.tab = table;
-    const int bank = p.local ? per : 0;
-    const unsigned bank_bytes = 4u * (unsigned)K * (unsigned)p.F;
-    ob.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(p.b + (size_t)bank * K * p.F), 0, (int)bank_bytes, 0x00020000);
+    ob.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p.b, 0, (int)(4u * (unsigned)K * (unsigned)p.F), 0x00020000);
     ob.step = 4u * BK * (unsigned)p.F;
 #pragma unroll
     for (int u = 0; u < OB::NG; ++u)
       ob.off[u] = 4u * (unsigned)(OB::group_k(tid, u) * p.F + g * p.Fg + n0 + OB::group_row(tid, u));
-    out += (long long)g * p.Fg * p.ldc + (long long)per * p.rows;
+    out += (long long)g * p.Fg * p.ldc;
   } else if constexpr (MODE == CONV_DOWN) {
-    // a tile on one pixel leaves out the taps that reach no module: they are the rows and columns ky0.. and kx0.. of the filter
-    int ky0 = 0, kx0 = 0, ny = k, nx = k;
-    const int prow = div(per, p.dH), py = prow - p.pad0, px = per - prow * H - p.pad0;
-    if (p.periods > 1) {
-      ky0 = py - Mx + 1 > 0 ? py - Mx + 1 : 0; ny = (py + 1 < k ? py + 1 : k) - ky0;
-      kx0 = px - Mx + 1 > 0 ? px - Mx + 1 : 0; nx = (px + 1 < k ? px + 1 : k) - kx0;
-      if (ny <= 0 || nx <= 0) ny = 0, nx = 1;
-    }
-    const int K = ny * nx * p.Fg;
+    const int K = p.kk2 * p.Fg;
     nst = (K + BK - 1) / BK;
-    if (nst < 1) nst = 1;
-    const int inv_nx = 65536 / nx + 1;      // exact for tap < RING_MAX_SIDE^2
     unsigned* tab1 = reinterpret_cast<unsigned*>(table + nst * (BK / 4));
     for (int e = tid; e < nst * (BK / 4); e += RING_THREADS) {
-      const int tap = div(4 * e, p.dFg), f = 4 * e - tap * p.Fg, ty = tap * inv_nx >> 16, ky = ky0 + ty, kx = kx0 + tap - ty * nx;
-      const int bank = p.local ? (py - ky) * Mx + px - kx : 0;
+      const int tap = div(4 * e, p.dFg), f = 4 * e - tap * p.Fg, ky = div(tap, p.dk), kx = tap - ky * k;
       const bool in = 4 * e < K;
       table[e] = make_uint2(4u * (unsigned)N * (unsigned)(p.M * f - ky * Mx - kx), in ? 1u << ky | 1u << (RING_MAX_SIDE + kx) : RING_FAR);
-      tab1[e] = in ? 4u * (unsigned)(f + p.F * (ky * k + kx + p.Cg * p.kk2 * bank)) : RING_FAR;
+      tab1[e] = in ? 4u * (unsigned)(f + p.F * tap) : RING_FAR;
     }
-    const int r = per * p.rows + m0 + OA::group_row(tid, 0);
+    const int r = m0 + OA::group_row(tid, 0);
     const int pix = div(r, p.dN), n = r - pix * N, yy = div(pix, p.dH), y = yy - p.pad0, x = pix - yy * H - p.pad0;
 #pragma unroll
     for (int u = 0; u < OA::NG; ++u) {
@@ -183,7 +232,7 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
     ob.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p.b, 0, (int)p.b_bytes, 0x00020000);
 #pragma unroll
     for (int u = 0; u < OB::NG; ++u) ob.off[u] = 4u * (unsigned)(g * p.Fg + p.F * p.kk2 * (n0 + OB::group_row(tid, u)));
-    out += (long long)g * p.Cg * p.ldc + (long long)per * p.rows;
+    out += (long long)g * p.Cg * p.ldc;
   } else {
     const int cz = div(z, p.dG), chunk = div(cz, p.dsplits), k_beg = (cz - chunk * p.splits) * p.split_stages * BK;
     g = z - cz * p.G;
@@ -226,20 +275,25 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
   }
 }
 
-// The tiles and what they cost: us per stage and per tile of a round (a tile on every CU).  Fitted to 233 measured
-// passes (rms 3 to 5 %); behind a product's 0.43 us a stage are the lanes' offsets, and what a tile costs besides its
-// stages is its table and its first trip to memory.
+// The tiles and what they cost: us per stage and per tile of a round (a tile on every CU).  Fitted to 500 measured
+// passes (rms 4 to 8 %; masks or none, no difference); what a tile costs besides its stages is its table and its first
+// trip to memory.
 static const struct { int bm, bn, bk; double stage, tile; } g_conv_ring_cfgs[] = {
-    {64, 64, 32, 0.53, 1.62}, {64, 32, 64, 0.60, 1.61}, {32, 64, 64, 0.59, 1.55},
-    {32, 32, 64, 0.344, 1.21}, {32, 16, 128, 0.414, 1.27}, {16, 32, 128, 0.41, 1.25}};
+    {64, 64, 32, 0.545, 1.45}, {64, 32, 64, 0.574, 1.46}, {32, 64, 64, 0.58, 1.45},
+    {32, 32, 64, 0.322, 1.0}, {32, 16, 128, 0.372, 1.2}, {16, 32, 128, 0.372, 1.17}};
 #define RING_TABLE_BYTES 26624      // what a workgroup's LDS holds besides the tiles (64 KB in all)
 
 struct ConvRingPlan { int cfg, splits, split_stages; double us; };
 
+static int conv_ring_entry(int mode, bool single, int bk) {      // table bytes per stage
+  return mode == CONV_UP ? 8 * bk : mode == CONV_DOWN && !single ? 3 * bk : 2 * bk;
+}
+
 // The tile that is expected to be fastest, cfg < 0: none fits.  rows x cols outputs per period, `jobs` periods x groups x
 // chunks, K terms each, of which a tile has the share `used` on average; split_us: what adding up one more
 // partial output costs (Outp).
-static ConvRingPlan conv_ring_plan(int mode, long long rows, int cols, long long jobs, int K, double used, bool can_split, double split_us) {
+static ConvRingPlan conv_ring_plan(int mode, bool single, long long rows, int cols, long long jobs, int K, double used, bool can_split,
+                                   double split_us) {
   ConvRingPlan best = {-1, 1, 0, 0.};
   const int cus = dn_num_cus();
   for (int c = 0; c < 6; ++c) {
@@ -247,8 +301,7 @@ static ConvRingPlan conv_ring_plan(int mode, long long rows, int cols, long long
     if (rows < f.bm || cols < f.bn) continue;
     const long long tiles = (rows + f.bm - 1) / f.bm * ((cols + f.bn - 1) / f.bn) * jobs;
     const int nst = (K + f.bk - 1) / f.bk;
-    const int entry = mode == CONV_UP ? 8 * f.bk : mode == CONV_DOWN ? 3 * f.bk : 2 * f.bk;   // table bytes per stage
-    const int most = RING_TABLE_BYTES / entry;
+    const int most = RING_TABLE_BYTES / conv_ring_entry(mode, single, f.bk) - (single ? RING_SETS + 3 : 0);
     const int lo = (nst + most - 1) / most, hi = can_split ? (nst / 4 < 512 ? nst / 4 : 512) : 1;
     if (lo > 1 && (!can_split || lo > hi)) continue;
     // the fewest splits, and the most that fill 1 .. 8 rounds of the CUs
@@ -260,14 +313,14 @@ static ConvRingPlan conv_ring_plan(int mode, long long rows, int cols, long long
       const long long all = tiles * real;
       if (all >= 1ll << 28) continue;
       const double rounds = all <= 4 * cus ? (double)((all + cus - 1) / cus) : 0.5 + (double)all / cus;
-      const double us = 2.7 + rounds * (used * per * f.stage + f.tile) + (real > 1 ? 2.5 + real * split_us : 0.);
+      const double us = 3. + rounds * (used * per * f.stage + f.tile) + (real > 1 ? 2.5 + real * split_us : 0.);
       if (best.cfg < 0 || us < best.us) best = {c, real, per, us};
     }
   }
   return best;
 }
 
-template <int MODE>
+template <int MODE, bool SINGLE>
 static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
   const auto& f = g_conv_ring_cfgs[plan.cfg];
   p.gx = (p.rows + f.bm - 1) / f.bm; p.gy = (p.cols + f.bn - 1) / f.bn;
@@ -277,8 +330,8 @@ static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
   p.dN = make_fastdiv(p.N); p.dMx = make_fastdiv(p.Mx); p.dk = make_fastdiv(p.k); p.dkk2 = make_fastdiv(p.kk2); p.dH = make_fastdiv(p.H);
   p.dFg = make_fastdiv(p.Fg); p.dgx = make_fastdiv(p.gx); p.dgy = make_fastdiv(p.gy); p.dper = make_fastdiv(p.periods);
   p.dsplits = make_fastdiv(p.splits); p.dG = make_fastdiv(p.G);
-  const size_t tab = (size_t)(stages < 1 ? 1 : stages) * f.bk * (MODE == CONV_UP ? 8 : MODE == CONV_DOWN ? 3 : 2);
-#define CONV_RING(TB, BM, BN, BK) hipLaunchKernelGGL((k_conv_ring<MODE, TB, BM, BN, BK>), grid, dim3(RING_THREADS), tab, dn_stream(), p)
+  const size_t tab = (size_t)((stages < 1 ? 1 : stages) + (SINGLE ? RING_SETS + 3 : 0)) * conv_ring_entry(MODE, SINGLE, f.bk);
+#define CONV_RING(TB, BM, BN, BK) hipLaunchKernelGGL((k_conv_ring<MODE, SINGLE, TB, BM, BN, BK>), grid, dim3(RING_THREADS), tab, dn_stream(), p)
   switch (plan.cfg) {
     case 0: CONV_RING(32, 64, 64, 32); break;
     case 1: CONV_RING(32, 64, 32, 64); break;
