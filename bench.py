@@ -281,7 +281,7 @@ class MLP(object):
 def net_mlp(cm, sizes=(784, 1024, 1024, 10), B=128, seed=3, fused=False):
     """The MLP of config 3 as a deepnet net: Layer / Edge / NeuralNet objects of this package
     driven by TrainOneBatch, i.e. the reference's own control flow (neuralnet.py:138-337) with
-    its per-step loss read-backs (two blocking sums per step in SoftmaxLayer.GetLoss)."""
+    its per-step loss read-backs (two sums per step, read by the host at its end)."""
     from deepnet_amd import layer as dl, neuralnet as dnn, parameter as dp
     rng = np.random.default_rng(seed)
     sgd = dict(base_epsilon=0.01, initial_momentum=0.9, final_momentum=0.9)
@@ -716,7 +716,7 @@ def main():
         t = time_loop(cm, lambda: net.TrainOneBatch(0), 100, 10)
         secondary['mlp_through_neuralnet_classes'] = {
             'steps_per_sec': round(1.0 / t, 1), 'us_per_step': round(t * 1e6, 1),
-            'note': 'same net as Layer / Edge / NeuralNet objects, TrainOneBatch with its two blocking loss read-backs per step'}
+            'note': 'same net as Layer / Edge / NeuralNet objects, TrainOneBatch, which reads its two losses per step on the host'}
         for obj in net.layer + net.edge:
             obj.fused = True
         t = time_loop(cm, lambda: net.TrainOneBatch(0), 100, 10)

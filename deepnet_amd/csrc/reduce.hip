@@ -1126,63 +1126,83 @@ k_dot_one(const float* a, const float* b, long long n, double* partial, unsigned
   }
 }
 
-// The host's side of the result word: pinned memory that the kernel writes directly, so a
+// The host's side of the result words: pinned memory that the kernel writes directly, so a
 // scalar result costs no copy call.  The host polls the word for this call's tag for a
 // while (a result of a short kernel arrives within microseconds) and otherwise waits for
-// the stream.
+// the stream.  Word 0 belongs to the calls that wait for their result, the others to those
+// that read it later (read_later, read_now).
+#define RESULT_WORDS 64
 static unsigned long long* g_result_host = nullptr;
 static unsigned long long* g_result_dev = nullptr;
 static unsigned g_result_tag = 0;
+struct DotTicket { unsigned tag; int word, n_counters; unsigned* counter; hipStream_t stream; };
+static DotTicket g_late[RESULT_WORDS];
 
-static bool result_word() {
+static bool result_words() {
   if (g_result_host) return true;
   void* h = nullptr;
   void* d = nullptr;
-  if (hipHostMalloc(&h, 64, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess) { hipGetLastError(); return false; }
+  if (hipHostMalloc(&h, RESULT_WORDS * 8, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess) { hipGetLastError(); return false; }
   if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) { hipGetLastError(); hipHostFree(h); return false; }
   g_result_host = (unsigned long long*)h;
   g_result_dev = (unsigned long long*)d;
-  *g_result_host = 0ull;
+  memset(h, 0, RESULT_WORDS * 8);
   return true;
 }
 
-#define DOT_POLLS (1 << 16)
-static int flat_dot(const float* a, const float* b, long long n, int take_sqrt, float* result) {
-  *result = 0.f;
+// Launches the sum of n > 0 products; its result arrives in a word of its own when `late`, else in word 0.
+static int flat_dot_launch(const float* a, const float* b, long long n, int take_sqrt, bool late, DotTicket* out) {
   if (dn_capturing()) return ERROR_UNSUPPORTED;        // the result is read back: nothing to record
-  if (n <= 0) return 0;
   const bool vec = dn_aligned16(a) && (!b || dn_aligned16(b)) && n >= 1024;   // b == nullptr: a vector of ones
   long long nb = (n + (vec ? 4095 : 1023)) / (vec ? 4096 : 1024);
   const long long cap = (long long)dn_num_cus() * 2;   // (more workgroups: more arrivals; 4 per CU cost 2 us at 4096 x 4096)
   if (nb > cap) nb = cap;
   double* partial = (double*)dn_scratch((size_t)nb * sizeof(double));
-  unsigned* counter = dn_zero_words(DOT_COUNTER_PITCH * (1 + (int)((nb + DOT_GROUP - 1) / DOT_GROUP)));
-  if (!partial || !counter || !result_word()) return CUDA_ERROR;
-  const unsigned tag = ++g_result_tag ? g_result_tag : ++g_result_tag;   // never 0, the word's first content
+  DotTicket t;
+  t.n_counters = DOT_COUNTER_PITCH * (1 + (int)((nb + DOT_GROUP - 1) / DOT_GROUP));
+  t.counter = dn_zero_words(t.n_counters);
+  if (!partial || !t.counter || !result_words()) return CUDA_ERROR;
+  t.tag = ++g_result_tag ? g_result_tag : ++g_result_tag;   // never 0, the words' first content
+  t.word = late ? 1 + (int)(t.tag % (RESULT_WORDS - 1)) : 0;
+  t.stream = dn_stream();
+  unsigned long long* result = g_result_dev + t.word;
   const dim3 grid((unsigned)nb), block(256);
 #define DOT_GO(VEC, STREAM, MODE) \
-  hipLaunchKernelGGL((k_dot_one<VEC, STREAM, MODE>), grid, block, 0, dn_stream(), a, b, n, partial, counter, g_result_dev, tag, take_sqrt)
+  hipLaunchKernelGGL((k_dot_one<VEC, STREAM, MODE>), grid, block, 0, t.stream, a, b, n, partial, t.counter, result, t.tag, take_sqrt)
 #define DOT_SAME(VEC, STREAM) do { if (a == b) DOT_GO(VEC, STREAM, 1); else if (!b) DOT_GO(VEC, STREAM, 2); else DOT_GO(VEC, STREAM, 0); } while (0)
   if (vec && n >= DN_STREAM_MIN_ELEMS) DOT_SAME(true, true);
   else if (vec) DOT_SAME(true, false);
   else DOT_SAME(false, false);
 #undef DOT_SAME
 #undef DOT_GO
-  const int n_counters = DOT_COUNTER_PITCH * (1 + (int)((nb + DOT_GROUP - 1) / DOT_GROUP));
-  if (hipGetLastError() != hipSuccess) { rezero_counters(counter, n_counters); return CUDA_ERROR; }
+  if (hipGetLastError() != hipSuccess) { rezero_counters(t.counter, t.n_counters); return CUDA_ERROR; }
+  *out = t;
+  return 0;
+}
+
+#define DOT_POLLS (1 << 16)
+static int flat_dot_wait(const DotTicket& t, float* result) {
   unsigned long long word = 0;
   for (int i = 0; i < DOT_POLLS; ++i) {
-    word = __atomic_load_n(g_result_host, __ATOMIC_ACQUIRE);
-    if ((unsigned)(word >> 32) == tag) break;
+    word = __atomic_load_n(g_result_host + t.word, __ATOMIC_ACQUIRE);
+    if ((unsigned)(word >> 32) == t.tag) break;
   }
-  if ((unsigned)(word >> 32) != tag) {
-    if (hipStreamSynchronize(dn_stream()) != hipSuccess) { rezero_counters(counter, n_counters); return CUDA_ERROR; }
-    word = __atomic_load_n(g_result_host, __ATOMIC_ACQUIRE);
-    if ((unsigned)(word >> 32) != tag) { rezero_counters(counter, n_counters); return CUDA_ERROR; }
+  if ((unsigned)(word >> 32) != t.tag) {
+    if (hipStreamSynchronize(t.stream) != hipSuccess) { rezero_counters(t.counter, t.n_counters); return CUDA_ERROR; }
+    word = __atomic_load_n(g_result_host + t.word, __ATOMIC_ACQUIRE);
+    if ((unsigned)(word >> 32) != t.tag) { rezero_counters(t.counter, t.n_counters); return CUDA_ERROR; }
   }
   const unsigned bits = (unsigned)word;
   memcpy(result, &bits, sizeof(float));
   return 0;
+}
+
+static int flat_dot(const float* a, const float* b, long long n, int take_sqrt, float* result) {
+  *result = 0.f;
+  if (n <= 0) return dn_capturing() ? ERROR_UNSUPPORTED : 0;
+  DotTicket t;
+  if (int e = flat_dot_launch(a, b, n, take_sqrt, false, &t)) return e;
+  return flat_dot_wait(t, result);
 }
 
 // ------------------------------------------------------------------ C ABI
@@ -1661,6 +1681,29 @@ float euclid_norm(cudamat* mat, int* err_code) {
   const int e = flat_dot(mat->data_device, mat->data_device, dn_len(mat), 1, &res);
   *err_code = e;
   return e ? -1.f : res;
+}
+
+// sum_all (norm == 0) or euclid_norm of mat as it is now, to be read by read_now(*ticket): the kernel is launched and
+// nothing waits.  The value is kept until RESULT_WORDS - 1 more have been asked for (read_now then fails).
+int read_later(cudamat* mat, int norm, unsigned* ticket) {
+  *ticket = 0;
+  if (!mat->on_device) return ERROR_NOT_ON_DEVICE;
+  if (dn_capturing()) return ERROR_UNSUPPORTED;
+  if (dn_len(mat) <= 0) return 0;                      // (ticket 0 reads as zero)
+  DotTicket t;
+  if (int e = flat_dot_launch(mat->data_device, norm ? mat->data_device : nullptr, dn_len(mat), norm ? 1 : 0, true, &t)) return e;
+  g_late[t.word] = t;
+  *ticket = t.tag;
+  return 0;
+}
+
+float read_now(unsigned ticket, int* err_code) {
+  *err_code = 0;
+  if (ticket == 0) return 0.f;
+  const DotTicket& t = g_late[1 + (int)(ticket % (RESULT_WORDS - 1))];
+  float res = 0.f;
+  *err_code = t.tag == ticket ? flat_dot_wait(t, &res) : ERROR_GENERIC;
+  return *err_code ? -1.f : res;
 }
 
 }  // extern "C"

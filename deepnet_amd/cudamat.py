@@ -128,6 +128,7 @@ _SIGNATURES = {
     'free_device_memory_sparse': (_i, [_S]),
     'sparse_dot': (_i, [_S, _M, _M, _f, _f]),
     'vdot': (_f, [_M, _M, ct.POINTER(_i)]), 'euclid_norm': (_f, [_M, ct.POINTER(_i)]), 'sum_all': (_f, [_M, ct.POINTER(_i)]),
+    'read_later': (_i, [_M, _i, ct.POINTER(_u)]), 'read_now': (_f, [_u, ct.POINTER(_i)]),
     'add_mult': (_i, [_M, _M, _f]), 'add_mult_sign': (_i, [_M, _M, _f]),
     'assign_scalar': (_i, [_M, _f]),
     'selectRows': (_i, [_M, _M, _M]), 'setSelectedRows': (_i, [_M, _M, _M]),
@@ -404,6 +405,19 @@ class CUDAMatrix(object):
             _check(err_code.value)
             return res
         return sum(self, axis, target)
+
+    def read_later(self, norm=False):
+        """sum() of this matrix as it is now (or its euclid_norm()) as a function that waits for the value: the kernel is
+        queued, the program goes on.  At most 63 such values may be outstanding."""
+        ticket = ct.c_uint(0)
+        _check(_cudamat.read_later(self.p_mat, int(norm), ct.byref(ticket)))
+
+        def value():
+            err_code = ct.c_int(0)
+            res = _cudamat.read_now(ticket, ct.byref(err_code))
+            _check(err_code.value)
+            return res
+        return value
 
     def add_sums(self, mat, axis, mult=1.):
         """self += mult * (sums of mat along axis)."""

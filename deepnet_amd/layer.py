@@ -152,11 +152,22 @@ class Layer(Parameter):
     def GetLoss(self, get_deriv=False, **kwargs):
         pass
 
+    # Loss values that are read when the step has been queued (NeuralNet.TrainOneBatch): a list of
+    # (record, field, function that waits for the value, whether to square it); None: read at once.
+    pending = None
+
+    def _report(self, perf, field, mat, norm=False):
+        """perf.field = sum of ``mat``, or its squared norm."""
+        if self.pending is None or len(self.pending) >= 32:
+            setattr(perf, field, mat.euclid_norm() ** 2 if norm else mat.sum())
+        else:
+            self.pending.append((perf, field, mat.read_later(norm), norm))
+
     def _squared_loss(self, perf, get_deriv, acc_deriv):
         """The SQUARED_LOSS branch shared by logistic and ReLU units (logistic_layer.py:50-60)."""
         target = self.statesize
         self.state.subtract(self.data, target=target)
-        perf.error = target.euclid_norm() ** 2
+        self._report(perf, 'error', target, norm=True)
         if acc_deriv:
             # (the reference passes the weight as `alpha=`, a keyword cudamat.py:1114 does not have)
             self.deriv.add_mult(target, mult=self.loss_weight)
@@ -183,7 +194,7 @@ class LinearLayer(Layer):
             raise Exception('Unknown loss function for linear units.')
         target = self.deriv if get_deriv else self.statesize
         self.state.subtract(self.data, target=target)
-        perf.error = target.euclid_norm() ** 2
+        self._report(perf, 'error', target, norm=True)
         if get_deriv:
             self.ComputeDeriv()
         return perf
@@ -214,9 +225,9 @@ class LogisticLayer(Layer):
         if self.loss_function == P.CROSS_ENTROPY:
             temp1 = self.statesize
             cm.cross_entropy_bernoulli(self.data, self.state, target=temp1, tiny=self.tiny)
-            perf.cross_entropy = temp1.sum()
+            self._report(perf, 'cross_entropy', temp1)
             cm.correct_preds(self.data, self.state, target=temp1, cutoff=0.5)
-            perf.correct_preds = temp1.sum()
+            self._report(perf, 'correct_preds', temp1)
             if get_deriv:
                 self.state.subtract(self.data, target=self.deriv)
         elif self.loss_function == P.SQUARED_LOSS:
@@ -249,7 +260,7 @@ class TanhLayer(Layer):
         if self.loss_function != P.SQUARED_LOSS:
             raise Exception('Unknown loss function for tanh units.')
         self.state.subtract(self.data, target=self.deriv)
-        perf.error = self.deriv.euclid_norm() ** 2
+        self._report(perf, 'error', self.deriv, norm=True)
         if get_deriv:
             self.ComputeDeriv()
         return perf
@@ -319,15 +330,16 @@ class SoftmaxLayer(Layer):
         self.deriv.reshape((numlabels, dimensions * batchsize))
         try:
             if self.loss_function == P.CROSS_ENTROPY:
-                state.get_softmax_correct(data, target=temp)
-                perf.correct_preds = temp.sum()
+                # (loss and gradient first: where the softmax is held back they join its launch)
                 state.get_softmax_cross_entropy(data, target=temp, tiny=self.tiny)
-                perf.cross_entropy = temp.sum()
                 if get_deriv:
                     state.apply_softmax_grad(data, target=self.deriv)
+                self._report(perf, 'cross_entropy', temp)
+                state.get_softmax_correct(data, target=temp)
+                self._report(perf, 'correct_preds', temp)
             elif self.loss_function == P.SQUARED_LOSS:
                 state.apply_softmax_grad(data, target=self.deriv)
-                perf.error = self.deriv.euclid_norm() ** 2
+                self._report(perf, 'error', self.deriv, norm=True)
             else:
                 raise Exception('Unknown loss function for Softmax units.')
         finally:

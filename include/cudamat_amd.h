@@ -163,6 +163,10 @@ int add_sum_by_axis(cudamat* mat, cudamat* target, int axis, float mult);
  * as long as the matrix).  vdot's kernel without the vector, same bits; the error code comes back
  * the way vdot and euclid_norm hand it back. */
 float sum_all(cudamat* mat, int* err_code);
+/* sum_all (norm 0) or euclid_norm (norm 1) without the wait: read_later launches the kernel and hands out a ticket,
+ * read_now waits for the ticket's value.  The last 63 tickets can be read. */
+int read_later(cudamat* mat, int norm, unsigned* ticket);
+float read_now(unsigned ticket, int* err_code);
 int sqsum_by_axis(cudamat* mat, cudamat* target, int axis, float mult, float p);
 int normlimit_by_axis(cudamat* mat, cudamat* target, int axis, float norm);
 

@@ -348,3 +348,25 @@ def test_softmax_of_columns_whose_last_group_moves_back(cm, rng, h, skip):
     rest = np.delete(whole.asarray(), np.s_[skip:skip + w], axis=1)
     assert np.isnan(rest).all()
     whole.free_device_memory()
+
+
+def test_scalars_that_are_read_later(cm, rng):
+    """read_later() is the value at the time of the call, with the bits of sum() and euclid_norm(), in any order of reading;
+    a value that 63 others have followed is refused."""
+    a = cm.CUDAMatrix(_rand(rng, (300, 70)))
+    want, got = [], []
+    for i in range(20):
+        a.mult(0.75)
+        got.append(a.read_later(norm=i % 2 == 1))
+        want.append(a.sum() if i % 2 == 0 else a.euclid_norm())
+    for i in reversed(range(20)):
+        assert got[i]() == want[i]
+        assert got[i]() == want[i]
+    for _ in range(43):
+        a.read_later()
+    assert got[-1]() == want[-1]
+    for _ in range(63):
+        last = a.read_later()
+    with pytest.raises(cm.CUDAMatException):
+        got[-1]()
+    assert last() == a.sum()
