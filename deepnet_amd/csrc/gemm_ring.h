@@ -4,7 +4,8 @@
 
 // Stage t of an operand as this lane's 16-byte groups; a stage behind the last one is an out-of-range offset, which the
 // buffer hardware answers with zeros without going to memory (every trip of the loop issues the same requests, so
-// the compiler can count them).
+// the compiler can count them).  The bit that puts it out of range stands in the lanes' offset: the scalar one takes
+// no part in the range check.
 template <int ROWS, int BK, bool KC>
 struct RingOperand : RingTile<ROWS, BK, KC> {
   using Tile = RingTile<ROWS, BK, KC>;
@@ -25,10 +26,10 @@ struct RingOperand : RingTile<ROWS, BK, KC> {
   }
   __device__ __forceinline__ void fetch(int t, int nst, f32x4 (&r)[NG]) const {
     const unsigned at = (unsigned)t * step;                       // (without a branch: the loop stays one block)
-    const unsigned so = (at < last ? at : last) | ((unsigned)(nst - 1 - t) & 0x80000000u);
+    const unsigned so = at < last ? at : last, behind = (unsigned)(nst - 1 - t) & 0x80000000u;
 #pragma unroll
     for (int u = 0; u < NG; ++u)
-      r[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)voff[u], (int)so, 0));
+      r[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(voff[u] | behind), (int)so, 0));
   }
 };
 
