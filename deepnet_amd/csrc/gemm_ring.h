@@ -4,17 +4,18 @@
 
 // Stage t of an operand as this lane's 16-byte groups; a stage behind the last one is an out-of-range offset, which the
 // buffer hardware answers with zeros without going to memory (every trip of the loop issues the same requests, so
-// the compiler can count them).  The bit that puts it out of range stands in the lanes' offset: the scalar one takes
-// no part in the range check.
+// the compiler can count them).  The scalar offset takes no part in the range check, so such a stage has a buffer of no
+// bytes instead; a bit in the lanes' offsets is a vector instruction per request (dense 1001 x 1500 x 300, three
+// products: 46.4 against 49.0 us).
 template <int ROWS, int BK, bool KC>
 struct RingOperand : RingTile<ROWS, BK, KC> {
   using Tile = RingTile<ROWS, BK, KC>;
   using Tile::NG;
-  __amdgpu_buffer_rsrc_t rsrc;
+  const float* P0;
   unsigned voff[NG];
-  unsigned step, last;
+  unsigned n_bytes, step, last;
   __device__ __forceinline__ void init(const float* P, unsigned bytes, int ld, int row0, int K, int tid) {
-    rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)P, 0, (int)bytes, 0x00020000);
+    P0 = P; n_bytes = bytes;
 #pragma unroll
     for (int u = 0; u < NG; ++u) {
       const unsigned row = (unsigned)(row0 + Tile::group_row(tid, u)), k = (unsigned)Tile::group_k(tid, u);
@@ -26,10 +27,11 @@ struct RingOperand : RingTile<ROWS, BK, KC> {
   }
   __device__ __forceinline__ void fetch(int t, int nst, f32x4 (&r)[NG]) const {
     const unsigned at = (unsigned)t * step;                       // (without a branch: the loop stays one block)
-    const unsigned so = at < last ? at : last, behind = (unsigned)(nst - 1 - t) & 0x80000000u;
+    const unsigned in = ~(unsigned)((nst - 1 - t) >> 31), so = (at < last ? at : last) & in;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)P0, 0, (int)(n_bytes & in), 0x00020000);
 #pragma unroll
     for (int u = 0; u < NG; ++u)
-      r[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(voff[u] | behind), (int)so, 0));
+      r[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)voff[u], (int)so, 0));
   }
 };
 
