@@ -902,7 +902,8 @@ static int rows_workspace(int h, int w, RowsWorkspace* ws) {
 template <int OP>
 static int rows_reduce(const float* M, int ld, int h, int w, const float* x, float* y, float alpha, float beta) {
   if (h <= 0) return 0;
-  if (h >= 4 && rows_one_splits(h, w) > 0) {
+  // (no columns: no slices to divide them into; the two-stage kernels below write the empty sums)
+  if (h >= 4 && w > 0 && rows_one_splits(h, w) > 0) {
     RowsWorkspace ws;
     const int e = rows_workspace(h, w, &ws);
     if (e == 0) return rows_reduce_one<OP>(M, ld, h, w, x, y, alpha, beta, ws);

@@ -132,3 +132,27 @@ def test_sparse_struct_layout_and_host_side_init():
     assert sp.mat.data_host.indptr[2] == 3 and sp.mat.data_host.data[1] == 2.0
     with pytest.raises(ValueError):
         cm.SparseCUDAMatrix([1.0], [0], [0, 1], (2, 3), copy_to_device=False)
+
+
+@pytest.mark.parametrize("call", ["sum_by_axis", "add_sum_by_axis", "sqsum_by_axis", "max_by_axis"])
+@pytest.mark.parametrize("h", [1, 3, 4, 5, 8, 1025])
+def test_reductions_over_no_columns_come_back(call, h):
+    """The host side of a reduction along the rows of an h x 0 matrix returns (here with a launch error at most: the device
+    is hidden) instead of dividing by the number of columns."""
+    import subprocess
+    import sys
+    code = """if True:
+        import ctypes as ct, numpy as np
+        from deepnet_amd import cudamat as cm
+        buf = np.zeros(%d, dtype=np.float32)
+        def mat(cols):
+            m = cm.cudamat()
+            m.data_device = buf.ctypes.data_as(type(m.data_device))
+            m.on_device, m.size[0], m.size[1] = 1, %d, cols
+            return ct.byref(m)
+        args = dict(sum_by_axis=(1,), add_sum_by_axis=(1, 2.0), sqsum_by_axis=(1, 1.0, 0.0), max_by_axis=(1,))['%s']
+        print('code', cm._cudamat.%s(mat(0), mat(1), *args))
+    """ % (h, h, call, call)
+    env = dict(os.environ, HIP_VISIBLE_DEVICES='-1')
+    r = subprocess.run([sys.executable, '-c', code], cwd=ROOT, env=env, capture_output=True, text=True)
+    assert r.returncode == 0 and r.stdout.startswith('code'), (r.returncode, r.stderr)

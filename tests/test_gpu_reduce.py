@@ -370,3 +370,20 @@ def test_scalars_that_are_read_later(cm, rng):
     with pytest.raises(cm.CUDAMatException):
         got[-1]()
     assert last() == a.sum()
+
+
+@pytest.mark.parametrize("h", [1, 4, 5, 8, 1025, 2048])
+def test_reductions_along_rows_of_no_columns(cm, rng, h):
+    """Sums over no columns are zero, and what is added to is kept."""
+    whole, before = cm.CUDAMatrix(_rand(rng, (h, 1))), _rand(rng, (h, 1))
+    none = whole.slice(0, 1)
+    none.mat.size[1] = 0
+    y = cm.CUDAMatrix(before)
+    none.sum(axis=1, target=y)
+    assert not y.asarray().any()
+    y = cm.CUDAMatrix(before)
+    y.add_sums(none, axis=1, mult=2.0)
+    assert np.array_equal(y.asarray(), before)
+    none.sqsum(axis=1, target=y)
+    assert not y.asarray().any()
+    whole.free_device_memory()
