@@ -1137,7 +1137,11 @@ static unsigned long long* g_result_host = nullptr;
 static unsigned long long* g_result_dev = nullptr;
 static unsigned g_result_tag = 0;
 struct DotTicket { unsigned tag; int word, n_counters; unsigned* counter; hipStream_t stream; };
-static DotTicket g_late[RESULT_WORDS];
+// The values to be read later have a count of their own (a ticket), so that calls that wait for theirs use up no words.
+struct LateValue { unsigned ticket; DotTicket t; };
+static LateValue g_late[RESULT_WORDS];
+static unsigned g_late_ticket = 0;
+static inline int late_word(unsigned ticket) { return 1 + (int)(ticket % (RESULT_WORDS - 1)); }
 
 static bool result_words() {
   if (g_result_host) return true;
@@ -1151,8 +1155,8 @@ static bool result_words() {
   return true;
 }
 
-// Launches the sum of n > 0 products; its result arrives in a word of its own when `late`, else in word 0.
-static int flat_dot_launch(const float* a, const float* b, long long n, int take_sqrt, bool late, DotTicket* out) {
+// Launches the sum of n > 0 products, whose result arrives in result word `word`.
+static int flat_dot_launch(const float* a, const float* b, long long n, int take_sqrt, int word, DotTicket* out) {
   if (dn_capturing()) return ERROR_UNSUPPORTED;        // the result is read back: nothing to record
   const bool vec = dn_aligned16(a) && (!b || dn_aligned16(b)) && n >= 1024;   // b == nullptr: a vector of ones
   long long nb = (n + (vec ? 4095 : 1023)) / (vec ? 4096 : 1024);
@@ -1164,7 +1168,7 @@ static int flat_dot_launch(const float* a, const float* b, long long n, int take
   t.counter = dn_zero_words(t.n_counters);
   if (!partial || !t.counter || !result_words()) return CUDA_ERROR;
   t.tag = ++g_result_tag ? g_result_tag : ++g_result_tag;   // never 0, the words' first content
-  t.word = late ? 1 + (int)(t.tag % (RESULT_WORDS - 1)) : 0;
+  t.word = word;
   t.stream = dn_stream();
   unsigned long long* result = g_result_dev + t.word;
   const dim3 grid((unsigned)nb), block(256);
@@ -1202,7 +1206,7 @@ static int flat_dot(const float* a, const float* b, long long n, int take_sqrt, 
   *result = 0.f;
   if (n <= 0) return dn_capturing() ? ERROR_UNSUPPORTED : 0;
   DotTicket t;
-  if (int e = flat_dot_launch(a, b, n, take_sqrt, false, &t)) return e;
+  if (int e = flat_dot_launch(a, b, n, take_sqrt, 0, &t)) return e;
   return flat_dot_wait(t, result);
 }
 
@@ -1691,19 +1695,21 @@ int read_later(cudamat* mat, int norm, unsigned* ticket) {
   if (!mat->on_device) return ERROR_NOT_ON_DEVICE;
   if (dn_capturing()) return ERROR_UNSUPPORTED;
   if (dn_len(mat) <= 0) return 0;                      // (ticket 0 reads as zero)
+  // 1 .. a multiple of the words there are, so that they are taken in turn; never 0
+  const unsigned next = g_late_ticket % ((RESULT_WORDS - 1u) << 26) + 1u;
   DotTicket t;
-  if (int e = flat_dot_launch(mat->data_device, norm ? mat->data_device : nullptr, dn_len(mat), norm ? 1 : 0, true, &t)) return e;
-  g_late[t.word] = t;
-  *ticket = t.tag;
+  if (int e = flat_dot_launch(mat->data_device, norm ? mat->data_device : nullptr, dn_len(mat), norm ? 1 : 0, late_word(next), &t)) return e;
+  g_late[t.word] = LateValue{next, t};
+  *ticket = g_late_ticket = next;
   return 0;
 }
 
 float read_now(unsigned ticket, int* err_code) {
   *err_code = 0;
   if (ticket == 0) return 0.f;
-  const DotTicket& t = g_late[1 + (int)(ticket % (RESULT_WORDS - 1))];
+  const LateValue& v = g_late[late_word(ticket)];
   float res = 0.f;
-  *err_code = t.tag == ticket ? flat_dot_wait(t, &res) : ERROR_GENERIC;
+  *err_code = v.ticket == ticket ? flat_dot_wait(v.t, &res) : ERROR_GENERIC;
   return *err_code ? -1.f : res;
 }
 
