@@ -20,9 +20,48 @@ def _zeros(shape):
     return cm.CUDAMatrix(np.zeros(shape, dtype=np.float32, order='F'))
 
 
+class LossRecord(types.SimpleNamespace):
+    """A record whose fields may still be on their way from the GPU.  Whoever looks at it (reads, assigns, lists or prints
+    a field) waits for them first, so that nobody sees the value that a field had before."""
+
+    __slots__ = ('_late',)          # field -> function that waits for its value; not set: nothing on its way
+
+    def late(self, field, value):
+        try:
+            self._late[field] = value
+        except AttributeError:
+            self._late = {field: value}
+
+    def settle(self):
+        """Waits for the fields that are on their way."""
+        try:
+            late = self._late
+        except AttributeError:
+            return
+        while late:
+            field = next(iter(late))
+            super(LossRecord, self).__setattr__(field, late[field]())
+            del late[field]
+
+    def __getattribute__(self, name):
+        get = super(LossRecord, self).__getattribute__
+        if name not in ('_late', 'late', 'settle'):
+            get('settle')()
+        return get(name)
+
+    def __setattr__(self, name, value):
+        if name != '_late':
+            self.settle()
+        super(LossRecord, self).__setattr__(name, value)
+
+    def __repr__(self):
+        self.settle()
+        return super(LossRecord, self).__repr__()
+
+
 def _metrics(count):
     """The fields of deepnet.proto's Metrics that the losses below fill."""
-    return types.SimpleNamespace(count=count, cross_entropy=0.0, correct_preds=0.0, error=0.0)
+    return LossRecord(count=count, cross_entropy=0.0, correct_preds=0.0, error=0.0)
 
 
 class Layer(Parameter):
@@ -152,8 +191,8 @@ class Layer(Parameter):
     def GetLoss(self, get_deriv=False, **kwargs):
         pass
 
-    # Loss values that are read when the step has been queued (NeuralNet.TrainOneBatch): a list of
-    # (record, field, function that waits for the value, whether to square it); None: read at once.
+    # The records with values that are read when the step has been queued (NeuralNet.TrainOneBatch), one entry per
+    # value; None: read at once.
     pending = None
 
     def _report(self, perf, field, mat, norm=False):
@@ -161,7 +200,9 @@ class Layer(Parameter):
         if self.pending is None or len(self.pending) >= 32:
             setattr(perf, field, mat.euclid_norm() ** 2 if norm else mat.sum())
         else:
-            self.pending.append((perf, field, mat.read_later(norm), norm))
+            value = mat.read_later(norm)
+            perf.late(field, (lambda: value() ** 2) if norm else value)
+            self.pending.append(perf)
 
     def _squared_loss(self, perf, get_deriv, acc_deriv):
         """The SQUARED_LOSS branch shared by logistic and ReLU units (logistic_layer.py:50-60)."""

@@ -255,8 +255,8 @@ class NeuralNet(object):
         finally:
             for layer in outputs:
                 layer.pending = None
-        for perf, field, value, square in pending:
-            setattr(perf, field, value() ** 2 if square else value())
+        for perf in pending:
+            perf.settle()
         return losses
 
     def EvaluateOneBatch(self):

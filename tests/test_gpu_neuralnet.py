@@ -220,3 +220,30 @@ def test_sin_and_cos_hidden_units(cm, dn):
     assert type(net.layer[1]).__name__ == 'SinLayer' and type(net.layer[2]).__name__ == 'CosLayer'
     batches = [(3.0 * rng.standard_normal((24, B)), rng.integers(0, 6, (1, B)).astype(np.float64)) for _ in range(3)]
     _train_and_compare(cm, net, onet, batches)
+
+
+@pytest.mark.parametrize("act", ['LINEAR', 'SOFTMAX', 'LOGISTIC'])
+def test_losses_can_be_used_inside_the_step(cm, dn, act):
+    """A layer that looks at its base class's record during TrainOneBatch finds the values that the step returns."""
+    rng, B, seen = np.random.default_rng(4), 20, []
+    base = {'LINEAR': dn.layer.LinearLayer, 'SOFTMAX': dn.layer.SoftmaxLayer, 'LOGISTIC': dn.layer.LogisticLayer}[act]
+
+    class Watched(base):
+        def GetLoss(self, *args, **kwargs):
+            perf = base.GetLoss(self, *args, **kwargs)
+            seen.append((perf.error, perf.cross_entropy, perf.correct_preds))
+            return perf
+
+    hyp = lambda **kw: dn.P.Hyperparams(base_epsilon=0.01, initial_momentum=0.9, final_momentum=0.9, **kw)
+    loss = dn.P.SQUARED_LOSS if act == 'LINEAR' else dn.P.CROSS_ENTROPY
+    x = dn.layer.LinearLayer('input', 30, B, hyperparams=dn.P.Hyperparams(), is_input=True)
+    out = Watched('output', 1 if act == 'SOFTMAX' else 7, B, hyperparams=hyp(activation=getattr(dn.P, act)),
+                  numlabels=7 if act == 'SOFTMAX' else 1, is_output=True, loss_function=loss)
+    net = dn.nn.NeuralNet([x, out], [dn.nn.Edge(x, out, _f(0.1 * rng.standard_normal((30, 7))), hyperparams=hyp())])
+    x.data.assign(cm.CUDAMatrix(_f(rng.standard_normal((30, B)))))
+    out.data.assign(cm.CUDAMatrix(_f(rng.integers(0, 7, (1, B)) if act == 'SOFTMAX' else rng.random((7, B)))))
+    for step in range(3):
+        got, = net.TrainOneBatch(step)
+        assert seen[-1] == (got.error, got.cross_entropy, got.correct_preds)
+        assert seen[-1][0 if act == 'LINEAR' else 1] != 0.0
+    assert len(seen) == 3

@@ -1,0 +1,51 @@
+"""The loss records of a training step, whose values arrive when the step has been queued (CPU only)."""
+import copy
+import pickle
+import types
+
+import pytest
+
+from deepnet_amd.layer import _metrics
+from deepnet_amd.neuralnet import Accumulate
+
+
+def _late(asked):
+    perf = _metrics(10)
+
+    def value():
+        asked.append(1)
+        return 2.5
+    perf.late('error', value)
+    return perf
+
+
+@pytest.mark.parametrize("look", [lambda p: p.error, lambda p: vars(p)['error'], lambda p: p.__dict__['error'],
+                                  lambda p: getattr(p, 'error'), lambda p: copy.copy(p).error, lambda p: pickle.loads(pickle.dumps(p)).error,
+                                  lambda p: Accumulate([], [p])[0].error, lambda p: Accumulate([_metrics(3)], [p])[0].error,
+                                  lambda p: eval(repr(p), {'LossRecord': types.SimpleNamespace, 'namespace': types.SimpleNamespace}).error])
+def test_whoever_looks_at_a_record_gets_the_value(look):
+    asked = []
+    perf = _late(asked)
+    assert look(perf) == 2.5 and perf.error == 2.5 and len(asked) == 1
+    assert vars(perf) == dict(count=10, cross_entropy=0.0, correct_preds=0.0, error=2.5)
+
+
+def test_an_assigned_field_keeps_what_was_assigned():
+    perf = _late([])
+    perf.error = 7.0
+    perf.settle()
+    assert perf.error == 7.0
+    perf = _late([])
+    perf.error *= 2
+    assert perf.error == 5.0
+
+
+def test_a_value_that_cannot_be_had_is_not_zero():
+    perf = _metrics(10)
+
+    def value():
+        raise RuntimeError('lost')
+    perf.late('error', value)
+    for _ in range(2):
+        with pytest.raises(RuntimeError):
+            perf.error
