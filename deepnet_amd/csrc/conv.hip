@@ -42,15 +42,12 @@
 #include <type_traits>
 
 #include "../../include/cudamat_conv_amd.h"
+#include "conv_ring_plan.h"
 #include <math.h>
 #include <stdio.h>
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// CONV_DOWNM: convDown for strided layers with few colours, all stride*stride pixel
-// phases merged into the columns of one product (uniform-row kernels only).
-enum { CONV_UP = 0, CONV_DOWN = 1, CONV_OUTP = 2, CONV_DOWNM = 3 };
 
 struct ConvArgs {
   const float* img;   // images: input of Up/Outp
@@ -2482,14 +2479,6 @@ extern "C" const char* conv_last_error(void) { return g_conv_failed ? g_conv_err
 // images add nothing to a weight gradient and their outputs are dropped, so results are the
 // padded pass's exactly.  (64 -> 64 filters of 5 x 5 on 13 x 13 maps at batch 100: convUp
 // 977 us on the one-lane-per-output kernel.)
-static int padded_batch(int N) {
-  if (N <= 16 || N % 16 == 0) return N;
-  const int n128 = (N + 127) / 128 * 128;
-  return (n128 - N) * 10 <= 3 * N ? n128 : (N + 31) / 32 * 32;
-}
-
-// The batch of a locally connected layer, whose uniform-row kernels need a multiple of 128.
-static int local_batch(int N) { return N >= 32 ? (N + 127) / 128 * 128 : N <= 16 || N % 16 == 0 ? N : 32; }
 
 // dst (Np x cols) = src (N x cols) with zero rows N .. Np-1, or back (rows 0 .. N-1 only).
 // One lane per group of four rows when VEC (both batch sizes are then multiples of 4); the
@@ -2563,9 +2552,6 @@ struct PaddedBatch {
 // modules) layout, so that is one contiguous copy and a zero tail), and the pass runs on the
 // copies; the extra outputs of convUp and the extra rows of a weight gradient are dropped.
 // (20 -> 50 filters of 5 x 5 at batch 128: convOutp 390 us on the one-lane-per-output kernel.)
-static int padded_filters(int F, int numGroups) {
-  return numGroups == 1 && F > 0 && F % 16 != 0 ? (F + 15) / 16 * 16 : F;
-}
 
 // Filter-major arrays (f + F*q): dst (Fp x Q) = src (F x Q) with zero rows F .. Fp-1, or back.
 __global__ void __launch_bounds__(256) k_pad_filters(const float* src, float* dst, int F, int Fp, long long Q, int unpad) {
@@ -2666,44 +2652,6 @@ static void conv_outp_filters(cudamat* images, cudamat* hidActs, cudamat* target
 }
 
 // ------------------------------------------------------------------ the passes on ring tiles
-// Every pass first asks what the fastest ring tile would take (conv_ring_plan) and what the other kernels would
-// (conv_other_us), and runs on the ring when that is less.  Both estimates were held against 360 passes over
-// random layers: the pass so chosen was 1.65 times as fast as before on average, none more than 9 us slower.
-
-// What all three passes need: offsets of 31 bits, masks of RING_MAX_SIDE filter rows.
-static bool ring_ok(const ConvArgs& a, long long bank_cols) {
-  return a.k <= RING_MAX_SIDE && (long long)a.N * a.M * a.F * 4 < (1ll << 31) &&
-         (long long)a.N * a.HH * a.C * 4 < (1ll << 31) && (long long)a.F * bank_cols * 4 < (1ll << 31);
-}
-
-// What a pass takes, in us, on the other matrix-core kernels: operations on whole blocks at the rate that these reach,
-// and the copies of a batch or filter count that they do not take; or on the one-lane-per-output kernels.
-// rows: positions of the output per image (Up: modules, Down: pixels).
-static double conv_other_us(const ConvArgs& a, int mode, long long rows) {
-  const int Np = !a.local ? padded_batch(a.N) : mode != CONV_OUTP ? local_batch(a.N) : a.N;
-  const int Fp = padded_filters(a.F, a.G), Fg = Fp / a.G, K = a.Cg * a.kk2;
-  const bool copy_n = Np != a.N, copy_f = Fp != a.F;
-  const bool aligned = (copy_n || (dn_aligned16(a.img ? a.img : a.hid) && dn_aligned16(a.hid) && dn_aligned16(a.out))) && dn_aligned16(a.flt);
-  if (Np % 16 != 0 || Fg % 16 != 0 || !aligned || (a.local && (copy_f || (mode != CONV_OUTP && Np % 128 != 0))))
-    return 5. + 2e-6 * a.N * rows * a.F * K;                            // (1 TFLOP/s)
-  auto up = [](long long v, int b) { return (double)((v + b - 1) / b * b); };
-  double flops, rate;                                                    // GFLOP, TFLOP/s
-  if (mode == CONV_UP) {
-    flops = 2e-9 * Np * rows * up(Fg, Fg <= 96 ? 32 : 64) * a.G * up(K, 16);
-    rate = a.local ? 45. : Np % 128 == 0 && K >= 256 && (Fg <= 64 || Fg > 96) ? 105. : 85.;
-  } else if (mode == CONV_DOWN) {
-    flops = 2e-9 * Np * rows * up(a.Cg, a.Cg > 32 && a.Cg <= 48 ? 16 : 32) * a.G * a.kk2 * Fg;
-    rate = a.local ? 70. : Np % 128 == 0 && a.kk2 * Fg >= 256 && (a.Cg <= 64 || a.Cg > 96) ? 115. : 65.;
-  } else {
-    const int BMs = Fg <= 32 ? 32 : Fg <= 64 ? 64 : Fg <= 96 || (Fg > 128 && (Fg + 95) / 96 * 96 < (Fg + 127) / 128 * 128) ? 96 : 128;
-    flops = 2e-9 * Np * rows * up(Fg, BMs) * a.G * up(K, K <= 80 && Fg <= 64 ? 16 : 128);
-    rate = a.local ? 45. : 110.;
-  }
-  const double maps = 1e-9 * 8. * Np * ((double)a.M * a.F + (double)a.HH * a.C), hid = 1e-9 * 8. * Np * a.M * Fp;   // GB of a copy
-  // (a long reduction may be split, and is summed by another launch)
-  return (mode == CONV_OUTP || K >= 256 ? 9. : 5.) + flops / rate * 1e3 + (copy_n ? 5. + maps / 5e-3 : 0.) + (copy_f ? 5. + hid / 5e-3 : 0.);
-}
-
 static ConvRingArgs ring_args(const ConvArgs& a) {
   ConvRingArgs p = {};
   p.N = a.N; p.H = a.H; p.HH = a.HH; p.Mx = a.Mx; p.M = a.M; p.k = a.k; p.kk2 = a.kk2; p.s = a.s; p.pad0 = a.pad0;
@@ -2717,35 +2665,18 @@ static bool ring_done(const char* where) {
   return true;
 }
 
-// The share of a layer's taps that lie inside the image (Up) or reach a module (Down), and with it of the reduction that
-// tiles of one module or pixel have.
-static double ring_used(const ConvArgs& a, int mode) {
-  const int lines = mode == CONV_UP ? a.Mx : a.H;
-  long long taps = 0;                                                    // of a column of modules or pixels
-  for (int i = 0; i < lines; ++i) {
-    const int v = mode == CONV_UP ? i * a.s + a.pad0 : i - a.pad0;
-    const int lo = mode == CONV_UP ? -v : v - a.Mx + 1, hi = mode == CONV_UP ? a.H - v : v + 1;
-    const int n = (hi < a.k ? hi : a.k) - (lo > 0 ? lo : 0);
-    if (n > 0) taps += n;
-  }
-  const double one = (double)taps / ((double)lines * a.k);
-  return one * one;
+static bool ring_maps16(const ConvArgs& a) {
+  return dn_aligned16(a.img ? a.img : a.hid) && dn_aligned16(a.hid) && dn_aligned16(a.out);
 }
 
-// Up and Down: tiles over any run of (module | pixel, image) groups, which needs batches of whole groups of four, or of
-// one module or pixel each, which leave out taps beyond the edge and need no masks.
+// Up and Down on ring tiles; false: not a pass for them.
 static bool conv_rows_ring(const ConvArgs& a, int mode, const char* where) {
   const bool up = mode == CONV_UP;
-  const long long bank = (long long)a.Cg * a.kk2 * (a.local ? a.M : 1);
-  if (!ring_ok(a, bank) || (!up && (a.s != 1 || a.Fg % 4 != 0))) return false;     // (Down: an entry is four filters of a tap)
+  const ConvRingPlan plan = conv_rows_plan(a, mode, ring_maps16(a), dn_aligned16(a.flt), dn_num_cus());
+  if (plan.cfg < 0) return false;
+  const bool single = plan.single;
   const int sites = up ? a.M : a.HH, cols = up ? a.Fg : a.Cg, K = a.kk2 * (up ? a.Cg : a.Fg);
-  ConvRingPlan plan = conv_ring_plan(mode, true, a.N, cols, (long long)sites * a.G, K, ring_used(a, mode), false, 0.);
-  bool single = true;
-  if (!a.local && a.N % 4 == 0) {
-    const ConvRingPlan flat = conv_ring_plan(mode, false, (long long)sites * a.N, cols, a.G, K, 1., false, 0.);
-    if (flat.cfg >= 0 && (plan.cfg < 0 || flat.us < plan.us)) { plan = flat; single = false; }
-  }
-  if (plan.cfg < 0 || plan.us > conv_other_us(a, mode, sites)) return false;
+  const long long bank = (long long)a.Cg * a.kk2 * (a.local ? a.M : 1);
   ConvRingArgs p = ring_args(a);
   p.a = up ? a.img : a.hid; p.b = a.flt;
   p.a_bytes = (unsigned)((long long)a.N * (up ? (long long)a.HH * a.C : (long long)a.M * a.F) * 4);
@@ -2765,16 +2696,11 @@ static void launch_outp_finish(const ConvArgs& a) {
 }
 
 static bool conv_outp_ring(const ConvArgs& a0, cudamat* images, cudamat* hidActs, const char* where) {
+  const ConvRingPlan plan = conv_outp_plan(a0, ring_maps16(a0), dn_aligned16(a0.flt), dn_num_cus());
+  if (plan.cfg < 0) return false;
   ConvArgs a = a0;
-  // whole groups of four images: other batches are copied with up to three images of zeros behind them
-  const int N4 = (a.N + 3) / 4 * 4;
+  const int N4 = (a.N + 3) / 4 * 4, cols = a.Cg * a.kk2, K = a.m_count * N4;
   a.N = N4;
-  const int cols = a.Cg * a.kk2, K = a.m_count * a.N;
-  if (!ring_ok(a, (long long)cols * a.chunks) || a.chunks > 32767) return false;
-  const ConvRingPlan plan = conv_ring_plan(CONV_OUTP, false, a.Fg, cols, (long long)a.G * a.chunks, K, 1., true, 2e-6 * a.chunks * a.F * cols);
-  const double maps = 1e-9 * 8. * N4 * ((double)a.M * a.F + (double)a.HH * a.C);
-  // (1.12: what a layer's sums over many splits take beyond the plan's estimate)
-  if (plan.cfg < 0 || 1.12 * plan.us + (N4 != a0.N ? 5. + maps / 5e-3 : 0.) > conv_other_us(a0, CONV_OUTP, a.M)) return false;
   ConvRingArgs p = ring_args(a);
   if (plan.splits > 1) {
     a.splits = plan.splits;

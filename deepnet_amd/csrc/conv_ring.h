@@ -1,13 +1,14 @@
 // Convolution passes on the tile loop of ring_tile.h: see k_conv_ring.  Included by conv.hip (ConvArgs).
 #pragma once
 #include "ring_tile.h"
+#include "conv_ring_plan.h"
 
 // A term of the reduction, as the workgroup keeps it in LDS for its reduction (one entry per term for Up, per four
 // for Down and Outp): the byte offset that it adds to a lane's, and which filter rows (bits 0-14) and columns (15-29)
 // have to be inside (Up, Down: `mask` of the entry has to be part of the lane's) or are inside (Outp: the other way
 // round).  RING_FAR stands in no lane's mask: such a term reads as zero.
 #define RING_FAR 0x80000000u
-#define RING_MAX_SIDE 15
+static_assert(RING_AHEAD >= RING_SETS + 3, "fetch() looks one stage ahead, the loop RING_SETS + 2");
 __device__ __forceinline__ unsigned ring_bits(int lo, int hi) {      // bits lo .. hi - 1
   lo = lo < 0 ? 0 : lo;
   hi = hi < lo ? lo : hi;
@@ -158,7 +159,7 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
     // exact for dividends below 2^12 and divisors up to RING_MAX_SIDE^2
     const unsigned inv_nx = 65536u / (unsigned)nx + 1u, inv_area = (1u << 20) / (unsigned)(area > 0 ? area : 1) + 1u;
     const unsigned Nu = (unsigned)N, Fu = (unsigned)p.F;
-    for (int e = tid; e < (nst + RING_SETS + 3) * (BK / PER); e += RING_THREADS) {
+    for (int e = tid; e < (nst + RING_AHEAD) * (BK / PER); e += RING_THREADS) {
       uint2 t2 = make_uint2(RING_FAR, RING_FAR);
       if (PER * e < K) {
         const int c = MODE == CONV_UP ? (int)((unsigned)e * inv_area >> 20) : 0;
@@ -275,51 +276,6 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
   }
 }
 
-// The tiles and what they cost: us per stage and per tile of a round (a tile on every CU).  Fitted to 500 measured
-// passes (rms 4 to 8 %; masks or none, no difference); what a tile costs besides its stages is its table and its first
-// trip to memory.
-static const struct { int bm, bn, bk; double stage, tile; } g_conv_ring_cfgs[] = {
-    {64, 64, 32, 0.545, 1.45}, {64, 32, 64, 0.574, 1.46}, {32, 64, 64, 0.58, 1.45},
-    {32, 32, 64, 0.322, 1.0}, {32, 16, 128, 0.372, 1.2}, {16, 32, 128, 0.372, 1.17}};
-#define RING_TABLE_BYTES 26624      // what a workgroup's LDS holds besides the tiles (64 KB in all)
-
-struct ConvRingPlan { int cfg, splits, split_stages; double us; };
-
-static int conv_ring_entry(int mode, bool single, int bk) {      // table bytes per stage
-  return mode == CONV_UP ? 8 * bk : mode == CONV_DOWN && !single ? 3 * bk : 2 * bk;
-}
-
-// The tile that is expected to be fastest, cfg < 0: none fits.  rows x cols outputs per period, `jobs` periods x groups x
-// chunks, K terms each, of which a tile has the share `used` on average; split_us: what adding up one more
-// partial output costs (Outp).
-static ConvRingPlan conv_ring_plan(int mode, bool single, long long rows, int cols, long long jobs, int K, double used, bool can_split,
-                                   double split_us) {
-  ConvRingPlan best = {-1, 1, 0, 0.};
-  const int cus = dn_num_cus();
-  for (int c = 0; c < 6; ++c) {
-    const auto& f = g_conv_ring_cfgs[c];
-    if (rows < f.bm || cols < f.bn) continue;
-    const long long tiles = (rows + f.bm - 1) / f.bm * ((cols + f.bn - 1) / f.bn) * jobs;
-    const int nst = (K + f.bk - 1) / f.bk;
-    const int most = RING_TABLE_BYTES / conv_ring_entry(mode, single, f.bk) - (single ? RING_SETS + 3 : 0);
-    const int lo = (nst + most - 1) / most, hi = can_split ? (nst / 4 < 512 ? nst / 4 : 512) : 1;
-    if (lo > 1 && (!can_split || lo > hi)) continue;
-    // the fewest splits, and the most that fill 1 .. 8 rounds of the CUs
-    for (int r = 0; r <= (can_split ? 8 : 0); ++r) {
-      int s = r == 0 ? lo : (int)((long long)r * cus / tiles);
-      if (s > hi) s = hi;
-      if (s < lo || s < 1) s = lo;
-      const int per = (nst + s - 1) / s, real = (nst + per - 1) / per;
-      const long long all = tiles * real;
-      if (all >= 1ll << 28) continue;
-      const double rounds = all <= 4 * cus ? (double)((all + cus - 1) / cus) : 0.5 + (double)all / cus;
-      const double us = 3. + rounds * (used * per * f.stage + f.tile) + (real > 1 ? 2.5 + real * split_us : 0.);
-      if (best.cfg < 0 || us < best.us) best = {c, real, per, us};
-    }
-  }
-  return best;
-}
-
 template <int MODE, bool SINGLE>
 static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
   const auto& f = g_conv_ring_cfgs[plan.cfg];
@@ -330,7 +286,7 @@ static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
   p.dN = make_fastdiv(p.N); p.dMx = make_fastdiv(p.Mx); p.dk = make_fastdiv(p.k); p.dkk2 = make_fastdiv(p.kk2); p.dH = make_fastdiv(p.H);
   p.dFg = make_fastdiv(p.Fg); p.dgx = make_fastdiv(p.gx); p.dgy = make_fastdiv(p.gy); p.dper = make_fastdiv(p.periods);
   p.dsplits = make_fastdiv(p.splits); p.dG = make_fastdiv(p.G);
-  const size_t tab = (size_t)((stages < 1 ? 1 : stages) + (SINGLE ? RING_SETS + 3 : 0)) * conv_ring_entry(MODE, SINGLE, f.bk);
+  const size_t tab = (size_t)conv_ring_table(MODE, SINGLE, f.bk, stages);
 #define CONV_RING(TB, BM, BN, BK) hipLaunchKernelGGL((k_conv_ring<MODE, SINGLE, TB, BM, BN, BK>), grid, dim3(RING_THREADS), tab, dn_stream(), p)
   switch (plan.cfg) {
     case 0: CONV_RING(32, 64, 64, 32); break;

@@ -1,0 +1,161 @@
+// Which convolution passes run on k_conv_ring, and on which of its tiles (host code without HIP; the tests build it by
+// itself).  Args: ConvArgs or anything with its sizes.
+#pragma once
+
+// CONV_DOWNM: convDown for strided layers with few colours, all stride*stride pixel
+// phases merged into the columns of one product (uniform-row kernels only).
+enum { CONV_UP = 0, CONV_DOWN = 1, CONV_OUTP = 2, CONV_DOWNM = 3 };
+
+#define RING_MAX_SIDE 15   // filter rows and columns that a mask has room for
+#define RING_AHEAD 7       // stages that the table of a tile of one module or pixel reaches beyond its last one
+
+// The batch that a pass is copied to when it is no multiple of 16 images (see PaddedBatch).
+static inline int padded_batch(int N) {
+  if (N <= 16 || N % 16 == 0) return N;
+  const int n128 = (N + 127) / 128 * 128;
+  return (n128 - N) * 10 <= 3 * N ? n128 : (N + 31) / 32 * 32;
+}
+
+// The batch of a locally connected layer, whose uniform-row kernels need a multiple of 128.
+static inline int local_batch(int N) { return N >= 32 ? (N + 127) / 128 * 128 : N <= 16 || N % 16 == 0 ? N : 32; }
+
+// The filter count that a bank is copied to (see conv_up_filters).
+static inline int padded_filters(int F, int numGroups) {
+  return numGroups == 1 && F > 0 && F % 16 != 0 ? (F + 15) / 16 * 16 : F;
+}
+
+// The tiles and what they cost: us per stage and per tile of a round (a tile on every CU).  Fitted to 500 measured
+// passes (rms 4 to 8 %; masks or none, no difference); what a tile costs besides its stages is its table and its first
+// trip to memory.
+static const struct { int bm, bn, bk; double stage, tile; } g_conv_ring_cfgs[] = {
+    {64, 64, 32, 0.545, 1.45}, {64, 32, 64, 0.574, 1.46}, {32, 64, 64, 0.58, 1.45},
+    {32, 32, 64, 0.322, 1.0}, {32, 16, 128, 0.372, 1.2}, {16, 32, 128, 0.372, 1.17}};
+#define RING_TABLE_BYTES 26624      // what a workgroup's LDS holds besides the tiles (64 KB in all)
+
+struct ConvRingPlan { int cfg, splits, split_stages; bool single; double us; };
+
+static inline int conv_ring_entry(int mode, bool single, int bk) {      // table bytes per stage
+  return mode == CONV_UP ? 8 * bk : mode == CONV_DOWN && !single ? 3 * bk : 2 * bk;
+}
+static inline int conv_ring_table(int mode, bool single, int bk, int stages) {      // table bytes of a workgroup
+  return ((stages < 1 ? 1 : stages) + (single ? RING_AHEAD : 0)) * conv_ring_entry(mode, single, bk);
+}
+
+// The tile that is expected to be fastest, cfg < 0: none fits.  rows x cols outputs per period, `jobs` periods x groups x
+// chunks, K terms each, of which a tile has the share `used` on average; split_us: what adding up one more
+// partial output costs (Outp).
+static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows, int cols, long long jobs, int K, double used,
+                                          bool can_split, double split_us, int cus) {
+  ConvRingPlan best = {-1, 1, 0, false, 0.};
+  for (int c = 0; c < 6; ++c) {
+    const auto& f = g_conv_ring_cfgs[c];
+    if (rows < f.bm || cols < f.bn) continue;
+    const long long tiles = (rows + f.bm - 1) / f.bm * ((cols + f.bn - 1) / f.bn) * jobs;
+    const int nst = (K + f.bk - 1) / f.bk;
+    const int most = RING_TABLE_BYTES / conv_ring_entry(mode, single, f.bk) - (single ? RING_AHEAD : 0);
+    const int lo = (nst + most - 1) / most, hi = can_split ? (nst / 4 < 512 ? nst / 4 : 512) : 1;
+    if (lo > 1 && (!can_split || lo > hi)) continue;
+    // the fewest splits, and the most that fill 1 .. 8 rounds of the CUs
+    for (int r = 0; r <= (can_split ? 8 : 0); ++r) {
+      int s = r == 0 ? lo : (int)((long long)r * cus / tiles);
+      if (s > hi) s = hi;
+      if (s < lo || s < 1) s = lo;
+      const int per = (nst + s - 1) / s, real = (nst + per - 1) / per;
+      const long long all = tiles * real;
+      if (all >= 1ll << 28) continue;
+      const double rounds = all <= 4 * cus ? (double)((all + cus - 1) / cus) : 0.5 + (double)all / cus;
+      const double us = 3. + rounds * (used * per * f.stage + f.tile) + (real > 1 ? 2.5 + real * split_us : 0.);
+      if (best.cfg < 0 || us < best.us) best = {c, real, per, single, us};
+    }
+  }
+  return best;
+}
+
+// Every pass first asks what the fastest ring tile would take (conv_ring_plan) and what the other kernels would
+// (conv_other_us), and runs on the ring when that is less.  Both estimates were held against 360 passes over
+// random layers: the pass so chosen was 1.65 times as fast as before on average, none more than 9 us slower.
+
+// What all three passes need: offsets of 31 bits, masks of RING_MAX_SIDE filter rows.
+template <class Args>
+static inline bool ring_ok(const Args& a, long long bank_cols) {
+  return a.k <= RING_MAX_SIDE && (long long)a.N * a.M * a.F * 4 < (1ll << 31) &&
+         (long long)a.N * a.HH * a.C * 4 < (1ll << 31) && (long long)a.F * bank_cols * 4 < (1ll << 31);
+}
+
+// What a pass takes, in us, on the other matrix-core kernels: operations on whole blocks at the rate that these reach,
+// and the copies of a batch or filter count that they do not take; or on the one-lane-per-output kernels.
+// rows: positions of the output per image (Up: modules, Down: pixels); maps16, filters16: 16-byte aligned.
+template <class Args>
+static inline double conv_other_us(const Args& a, int mode, long long rows, bool maps16, bool filters16) {
+  const int Np = !a.local ? padded_batch(a.N) : mode != CONV_OUTP ? local_batch(a.N) : a.N;
+  const int Fp = padded_filters(a.F, a.G), Fg = Fp / a.G, K = a.Cg * a.kk2;
+  const bool copy_n = Np != a.N, copy_f = Fp != a.F;
+  const bool aligned = (copy_n || maps16) && filters16;
+  if (Np % 16 != 0 || Fg % 16 != 0 || !aligned || (a.local && (copy_f || (mode != CONV_OUTP && Np % 128 != 0))))
+    return 5. + 2e-6 * a.N * rows * a.F * K;                            // (1 TFLOP/s)
+  auto up = [](long long v, int b) { return (double)((v + b - 1) / b * b); };
+  double flops, rate;                                                    // GFLOP, TFLOP/s
+  if (mode == CONV_UP) {
+    flops = 2e-9 * Np * rows * up(Fg, Fg <= 96 ? 32 : 64) * a.G * up(K, 16);
+    rate = a.local ? 45. : Np % 128 == 0 && K >= 256 && (Fg <= 64 || Fg > 96) ? 105. : 85.;
+  } else if (mode == CONV_DOWN) {
+    flops = 2e-9 * Np * rows * up(a.Cg, a.Cg > 32 && a.Cg <= 48 ? 16 : 32) * a.G * a.kk2 * Fg;
+    rate = a.local ? 70. : Np % 128 == 0 && a.kk2 * Fg >= 256 && (a.Cg <= 64 || a.Cg > 96) ? 115. : 65.;
+  } else {
+    const int BMs = Fg <= 32 ? 32 : Fg <= 64 ? 64 : Fg <= 96 || (Fg > 128 && (Fg + 95) / 96 * 96 < (Fg + 127) / 128 * 128) ? 96 : 128;
+    flops = 2e-9 * Np * rows * up(Fg, BMs) * a.G * up(K, K <= 80 && Fg <= 64 ? 16 : 128);
+    rate = a.local ? 45. : 110.;
+  }
+  const double maps = 1e-9 * 8. * Np * ((double)a.M * a.F + (double)a.HH * a.C), hid = 1e-9 * 8. * Np * a.M * Fp;   // GB of a copy
+  // (a long reduction may be split, and is summed by another launch)
+  return (mode == CONV_OUTP || K >= 256 ? 9. : 5.) + flops / rate * 1e3 + (copy_n ? 5. + maps / 5e-3 : 0.) + (copy_f ? 5. + hid / 5e-3 : 0.);
+}
+
+// The share of a layer's taps that lie inside the image (Up) or reach a module (Down), and with it of the reduction that
+// tiles of one module or pixel have.
+template <class Args>
+static inline double ring_used(const Args& a, int mode) {
+  const int lines = mode == CONV_UP ? a.Mx : a.H;
+  long long taps = 0;                                                    // of a column of modules or pixels
+  for (int i = 0; i < lines; ++i) {
+    const int v = mode == CONV_UP ? i * a.s + a.pad0 : i - a.pad0;
+    const int lo = mode == CONV_UP ? -v : v - a.Mx + 1, hi = mode == CONV_UP ? a.H - v : v + 1;
+    const int n = (hi < a.k ? hi : a.k) - (lo > 0 ? lo : 0);
+    if (n > 0) taps += n;
+  }
+  const double one = (double)taps / ((double)lines * a.k);
+  return one * one;
+}
+
+static inline ConvRingPlan conv_no_ring() { return {-1, 1, 0, false, 0.}; }
+
+// Up and Down: tiles over any run of (module | pixel, image) groups, which needs batches of whole groups of four, or of
+// one module or pixel each, which leave out taps beyond the edge and need no masks.  cfg < 0: another kernel.
+template <class Args>
+static inline ConvRingPlan conv_rows_plan(const Args& a, int mode, bool maps16, bool filters16, int cus) {
+  const bool up = mode == CONV_UP;
+  if (!ring_ok(a, (long long)a.Cg * a.kk2 * (a.local ? a.M : 1)) || (!up && (a.s != 1 || a.Fg % 4 != 0)))
+    return conv_no_ring();                                               // (Down: an entry is four filters of a tap)
+  const int sites = up ? a.M : a.HH, cols = up ? a.Fg : a.Cg, K = a.kk2 * (up ? a.Cg : a.Fg);
+  ConvRingPlan plan = conv_ring_plan(mode, true, a.N, cols, (long long)sites * a.G, K, ring_used(a, mode), false, 0., cus);
+  if (!a.local && a.N % 4 == 0) {
+    const ConvRingPlan flat = conv_ring_plan(mode, false, (long long)sites * a.N, cols, a.G, K, 1., false, 0., cus);
+    if (flat.cfg >= 0 && (plan.cfg < 0 || flat.us < plan.us)) plan = flat;
+  }
+  return plan.cfg < 0 || plan.us > conv_other_us(a, mode, sites, maps16, filters16) ? conv_no_ring() : plan;
+}
+
+// Outp of `a`, whose batch the ring takes in whole groups of four images: others are copied with up to three images of zeros.
+template <class Args>
+static inline ConvRingPlan conv_outp_plan(const Args& a, bool maps16, bool filters16, int cus) {
+  Args r = a;
+  r.N = (a.N + 3) / 4 * 4;
+  const int cols = a.Cg * a.kk2;
+  if (!ring_ok(r, (long long)cols * a.chunks) || a.chunks > 32767) return conv_no_ring();
+  const ConvRingPlan plan = conv_ring_plan(CONV_OUTP, false, a.Fg, cols, (long long)a.G * a.chunks, a.m_count * r.N, 1., true,
+                                           2e-6 * a.chunks * a.F * cols, cus);
+  const double maps = 1e-9 * 8. * r.N * ((double)a.M * a.F + (double)a.HH * a.C);
+  // (1.12: what a layer's sums over many splits take beyond the plan's estimate)
+  return plan.cfg < 0 || 1.12 * plan.us + (r.N != a.N ? 5. + maps / 5e-3 : 0.) > conv_other_us(a, CONV_OUTP, a.M, maps16, filters16)
+             ? conv_no_ring() : plan;
+}

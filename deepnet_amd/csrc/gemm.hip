@@ -1221,20 +1221,10 @@ static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, co
     if (fused) *fused = true;
     return dn_launch_status();
   }
-  // Reductions of more than 128 terms: k_gemm_ring, unless another kernel is expected to be faster.  The alternatives, as
-  // measured: 16 x 16 blocks take 2.9 us + 2.8 us per 1024 terms and round of the CUs (500 x 100 x 784 4.7 us against 5.6,
-  // 300 x 300 x 300 4.0 against 4.5; two rounds of 500 terms, 784 x 100 x 500, 5.5 against 5.1); slices of K with a second
-  // kernel what `heavy` says (few outputs over very long reductions); 128 x 128 tiles reach the same rate per output
-  // as 64 x 64 ones here (2000 x 2000 x 2000 130 us both) and win where their count fills the CUs as evenly.
+  // Reductions of more than 128 terms: k_gemm_ring, unless another kernel is expected to be faster (gemm_ring_plan).
   const size_t a_bytes = (size_t)lda * (a_kc ? M : K) * sizeof(float), b_bytes = (size_t)ldb * (b_kc ? N : K) * sizeof(float);
-  const RingPlan ring = K > BOX_K ? ring_plan(M, N, K, a_bytes, b_bytes, cus) : RingPlan{-1, 0.};
-  auto rounds_of = [&](long long t) { return (t + cus - 1) / cus; };
-  const double t16_us = 2.9 + 2.8 * (double)rounds_of(tiles16) * K / 1024.0;
-  const long long tiles128 = (long long)((M + 127) / 128) * ((N + 127) / 128);
-  const double sliced_us = 12.0 + 1.5e-8 * (double)M * (double)N * (double)K;
-  const bool use_ring = ring.cfg >= 0 && (tiles16 > 2ll * cus || ring.us < t16_us) && ring.us < sliced_us &&
-                        !(tiles128 >= cus && 4 * rounds_of(tiles128) <= rounds_of(tiles64));
-  if (use_ring) {
+  const RingPlan ring = K > BOX_K ? gemm_ring_plan(M, N, K, a_bytes, b_bytes, cus) : RingPlan{-1, 0.};
+  if (ring.cfg >= 0) {
     const RingArgs g = {A, B, C, (unsigned)a_bytes, (unsigned)b_bytes, lda, ldb, ldc, M, N, K, 0, 0, alpha, beta};
     ring_launch(ring.cfg, a_kc, b_kc, g, epi);
     if (fused) *fused = true;

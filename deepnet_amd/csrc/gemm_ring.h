@@ -1,6 +1,7 @@
 // Mid-sized products: see k_gemm_ring.  Included by gemm.hip (GemmEpilogue, f32x16).
 #pragma once
 #include "ring_tile.h"
+#include "gemm_ring_plan.h"
 
 // Stage t of an operand as this lane's 16-byte groups; a stage behind the last one is an out-of-range offset, which the
 // buffer hardware answers with zeros without going to memory (every trip of the loop issues the same requests, so
@@ -115,27 +116,6 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_gemm_ring(RingArgs g, GemmE
     }
   }
   if (t == 0) gemm_draw_idle_streams(tid, RING_THREADS, epi);
-}
-
-// The tile that is expected to be fastest, with its time in us; cfg < 0: none fits (a tile has to lie inside the
-// matrices and a stage inside the reduction; offsets are 31 bits).
-struct RingPlan { int cfg; double us; };
-static const struct { int bm, bn, bk; double stage; } g_ring_cfgs[] = {
-    // us per stage, measured with one tile on every CU
-    {64, 64, 32, 0.43}, {64, 32, 64, 0.52}, {32, 64, 64, 0.52}, {32, 32, 64, 0.25}, {32, 16, 128, 0.31}, {16, 32, 128, 0.33}};
-static RingPlan ring_plan(int M, int N, int K, size_t a_bytes, size_t b_bytes, int cus) {
-  RingPlan best = {-1, 0.};
-  if (a_bytes >= (1ull << 31) || b_bytes >= (1ull << 31)) return best;
-  for (int c = 0; c < (int)(sizeof(g_ring_cfgs) / sizeof(g_ring_cfgs[0])); ++c) {
-    const auto& f = g_ring_cfgs[c];
-    if (M < f.bm || N < f.bn || K < f.bk) continue;
-    const long long tiles = (long long)((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn);
-    const double rounds = (double)((tiles + cus - 1) / cus);
-    // a CU holds two workgroups; from the third on a tile's first trip to memory is not hidden
-    const double us = 4.2 + rounds * ((K + f.bk - 1) / f.bk) * f.stage + (rounds > 2 ? 1.3 * (rounds - 2) : 0.);
-    if (best.cfg < 0 || us < best.us) best = {c, us};
-  }
-  return best;
 }
 
 template <int TB, int BM, int BN, int BK>

@@ -1,0 +1,42 @@
+// Which products run on k_gemm_ring, and on which of its tiles (host code without HIP; the tests build it by itself).
+#pragma once
+#include <stddef.h>
+
+// The tile that is expected to be fastest, with its time in us; cfg < 0: none fits (a tile has to lie inside the
+// matrices and a stage inside the reduction; offsets are 31 bits).
+struct RingPlan { int cfg; double us; };
+static const struct { int bm, bn, bk; double stage; } g_ring_cfgs[] = {
+    // us per stage, measured with one tile on every CU
+    {64, 64, 32, 0.43}, {64, 32, 64, 0.52}, {32, 64, 64, 0.52}, {32, 32, 64, 0.25}, {32, 16, 128, 0.31}, {16, 32, 128, 0.33}};
+static inline RingPlan ring_plan(int M, int N, int K, size_t a_bytes, size_t b_bytes, int cus) {
+  RingPlan best = {-1, 0.};
+  if (a_bytes >= (1ull << 31) || b_bytes >= (1ull << 31)) return best;
+  for (int c = 0; c < (int)(sizeof(g_ring_cfgs) / sizeof(g_ring_cfgs[0])); ++c) {
+    const auto& f = g_ring_cfgs[c];
+    if (M < f.bm || N < f.bn || K < f.bk) continue;
+    const long long tiles = (long long)((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn);
+    const double rounds = (double)((tiles + cus - 1) / cus);
+    // a CU holds two workgroups; from the third on a tile's first trip to memory is not hidden
+    const double us = 4.2 + rounds * ((K + f.bk - 1) / f.bk) * f.stage + (rounds > 2 ? 1.3 * (rounds - 2) : 0.);
+    if (best.cfg < 0 || us < best.us) best = {c, us};
+  }
+  return best;
+}
+
+// The same for products that k_gemm_ring is to take; cfg < 0: another kernel is expected to be faster.  The alternatives, as
+// measured: 16 x 16 blocks take 2.9 us + 2.8 us per 1024 terms and round of the CUs (500 x 100 x 784 4.7 us against 5.6,
+// 300 x 300 x 300 4.0 against 4.5; two rounds of 500 terms, 784 x 100 x 500, 5.5 against 5.1); slices of K with a second
+// kernel 12 us + 1.5 us per 1e8 multiply-adds (few outputs over very long reductions); 128 x 128 tiles reach the same rate
+// per output as 64 x 64 ones here (2000 x 2000 x 2000 130 us both) and win where their count fills the CUs as evenly.
+static inline RingPlan gemm_ring_plan(int M, int N, int K, size_t a_bytes, size_t b_bytes, int cus) {
+  const RingPlan none = {-1, 0.}, ring = ring_plan(M, N, K, a_bytes, b_bytes, cus);
+  if (ring.cfg < 0) return none;
+  auto tiles = [&](int side) { return (long long)((M + side - 1) / side) * ((N + side - 1) / side); };
+  auto rounds = [&](long long t) { return (t + cus - 1) / cus; };
+  const double t16_us = 2.9 + 2.8 * (double)rounds(tiles(16)) * K / 1024.0;
+  const double sliced_us = 12.0 + 1.5e-8 * (double)M * (double)N * (double)K;
+  if (tiles(16) <= 2ll * cus && ring.us >= t16_us) return none;
+  if (ring.us >= sliced_us) return none;
+  if (tiles(128) >= cus && 4 * rounds(tiles(128)) <= rounds(tiles(64))) return none;
+  return ring;
+}

@@ -579,8 +579,20 @@ RING_LAYERS = [  # N, C, H, F, k, stride, padding, groups
     (20, 128, 7, 32, 3, 1, 1, 1),     # few rows
     (8, 96, 9, 64, 7, 1, 3, 1),       # 8 images
     (52, 36, 9, 40, 3, 1, 1, 2),      # 18 colours, 20 filters a group
-    (128, 40, 13, 188, 7, 2, 0, 1),   # more than one stage per split, many splits
-    (100, 1, 20, 96, 3, 1, 1, 1)]     # 9 terms
+    (128, 40, 13, 188, 7, 2, 0, 1),   # 1960 taps and 188 filters: Outp in one piece, 100 stages
+    (100, 1, 20, 96, 3, 1, 1, 1),     # 9 terms
+    (100, 1, 34, 32, 7, 2, 0, 1),     # Outp in more than 40 pieces
+    (28, 8, 13, 144, 3, 2, 1, 2),     # the tiles that the layers above leave out (tests/test_ring_plans.py): Up over several
+    (4, 3, 9, 45, 7, 2, 1, 1),        # modules on 32 x 64 and 16 x 32,
+    (100, 144, 6, 8, 5, 1, 1, 2),     # Down over several pixels on 64 x 64,
+    (60, 79, 10, 8, 3, 1, 1, 1),
+    (20, 68, 11, 16, 3, 1, 1, 2),     # 64 x 32,
+    (16, 164, 13, 16, 3, 1, 1, 1),    # 32 x 64,
+    (28, 87, 7, 8, 3, 1, 1, 1),       # 32 x 32
+    (16, 25, 5, 16, 7, 1, 1, 1),      # and 32 x 16,
+    (80, 108, 5, 8, 7, 1, 1, 1),      # and of one pixel on 32 x 64,
+    (1, 50, 21, 240, 5, 1, 1, 1),     # Outp on 64 x 64
+    (100, 75, 7, 35, 3, 1, 1, 1)]     # and 32 x 64
 
 
 @pytest.mark.parametrize("N,C,H,F,k,s,p,G", RING_LAYERS)
@@ -588,8 +600,11 @@ def test_three_conv_passes_on_ring_tiles(cm, cc, rng, N, C, H, F, k, s, p, G):
     test_three_conv_passes(cm, cc, rng, N, C, H, F, k, s, p, G)
 
 
-@pytest.mark.parametrize("N,C,H,F,k,s,p", [(128, 32, 6, 64, 3, 1, 1), (100, 20, 5, 48, 3, 1, 0), (67, 16, 6, 33, 3, 1, 1),
-                                           (32, 36, 5, 16, 3, 2, 1), (45, 16, 7, 20, 5, 1, 2)])
+RING_LOCAL = [(128, 32, 6, 64, 3, 1, 1), (100, 20, 5, 48, 3, 1, 0), (67, 16, 6, 33, 3, 1, 1), (32, 36, 5, 16, 3, 2, 1),
+              (45, 16, 7, 20, 5, 1, 2)]
+
+
+@pytest.mark.parametrize("N,C,H,F,k,s,p", RING_LOCAL)
 def test_locally_connected_layers_on_ring_tiles(cm, cc, rng, N, C, H, F, k, s, p):
     test_locally_connected_layers(cm, cc, rng, N, C, H, F, k, s, p)
 

@@ -486,11 +486,14 @@ def test_small_products_around_the_16_wide_blocks(cm, rng, m, k, n, ta, tb):
         h.free_device_memory()
 
 
-# (m, n, k) for every tile shape of k_gemm_ring (64 x 64, 64 x 32, 32 x 64, 32 x 32, 32 x 16, 16 x 32): sides at, one above and
-# one below multiples of the tile, reductions that end on a stage, one behind it and one in front of it, one to many stages
+# (m, n, k) for every tile shape of k_gemm_ring (64 x 64, 64 x 32, 32 x 64, 32 x 32, 32 x 16, 16 x 32; which of them a product
+# runs on is checked in tests/test_ring_plans.py): sides at, one above and one below multiples of the tile, reductions that
+# end on a stage, one behind it and one in front of it, one to many stages
 RING_SHAPES = [(2001, 1003, 250), (640, 1280, 256), (65, 4095, 129), (1500, 300, 1001), (1472, 320, 192), (300, 1501, 333),
                (287, 1472, 640), (814, 263, 1038), (513, 511, 511), (1024, 100, 2304), (801, 97, 1281), (100, 1025, 1300),
-               (33, 2048, 1151), (4097, 33, 255)]
+               (33, 2048, 1151), (4097, 33, 255),
+              (2859, 333, 154), (2048, 449, 897), (1983, 712, 832),       # 64 x 32
+              (333, 2859, 193), (449, 2048, 960), (726, 2749, 1091)]      # 32 x 64
 
 
 @pytest.mark.parametrize("m,n,k", RING_SHAPES)

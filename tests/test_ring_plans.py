@@ -1,0 +1,65 @@
+"""Which products and convolution passes the host gives to the ring kernels, and on which of their tiles (CPU only): the
+layers and products that the GPU tests run reach every tile, on a chip of 256 CUs."""
+import ctypes as ct
+import os
+import subprocess
+
+import pytest
+
+import test_gpu_conv as conv
+import test_gpu_dot as dot
+from oracle import conv_oracle as co
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CUS = 256
+UP, DOWN, OUTP = 0, 1, 2
+TILES = [(64, 64), (64, 32), (32, 64), (32, 32), (32, 16), (16, 32)]
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("plans") / "ring_plans.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", os.path.join(HERE, "ring_plans.cpp"), "-o", lib],
+                   check=True)
+    return ct.CDLL(lib)
+
+
+def gemm_tile(plans, m, n, k):
+    """Tile of a product; None: another kernel."""
+    t = plans.gemm_tile(m, n, k, CUS)
+    return TILES[t] if t >= 0 else None
+
+
+def conv_tile(plans, mode, N, C, H, F, k, s, p, G=1, local=False, partial_sum=0):
+    """(tile, whether it lies in one module or pixel, splits, table bytes) of a pass; None: another kernel."""
+    out = (ct.c_int * 4)()
+    plans.conv_tile(mode, N, C, H, F, k, co.n_modules(H, k, s, p), s, -p, G, int(local), 1 if local and mode == OUTP else partial_sum, CUS, out)
+    return (TILES[out[0]], bool(out[1]), out[2], out[3]) if out[0] >= 0 else None
+
+
+def test_the_products_of_the_gpu_tests_reach_every_tile(plans):
+    got = [gemm_tile(plans, *shape) for shape in dot.RING_SHAPES]
+    assert None not in got
+    for tile in TILES:
+        edges = [(m % tile[0] != 0) + (n % tile[1] != 0) for (m, n, k), t in zip(dot.RING_SHAPES, got) if t == tile]
+        assert edges and max(edges) == 2, tile           # one of them hangs over both edges
+
+
+def test_the_layers_of_the_gpu_tests_reach_every_tile(plans):
+    reached = set()
+    for mode in (UP, DOWN, OUTP):
+        for layer in conv.CASES + conv.RING_LAYERS:
+            t = conv_tile(plans, mode, *layer)
+            if t:
+                reached.add((mode, t[1], t[0]))
+    want = {(mode, single, tile) for mode in (UP, DOWN, OUTP) for single in (False, True) for tile in TILES if not (mode == OUTP and single)}
+    assert reached == want, sorted(want - reached)
+
+
+def test_layers_are_planned_as_their_comments_say(plans):
+    t = conv_tile(plans, OUTP, 128, 40, 13, 188, 7, 2, 0)
+    assert t[2] == 1
+    t = conv_tile(plans, OUTP, 100, 1, 34, 32, 7, 2, 0)
+    assert t[2] > 40
+    for layer in conv.RING_LOCAL:
+        assert any(conv_tile(plans, mode, *layer, local=True) for mode in (UP, DOWN, OUTP))
