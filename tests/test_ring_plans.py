@@ -63,3 +63,9 @@ def test_layers_are_planned_as_their_comments_say(plans):
     assert t[2] > 40
     for layer in conv.RING_LOCAL:
         assert any(conv_tile(plans, mode, *layer, local=True) for mode in (UP, DOWN, OUTP))
+
+
+@pytest.mark.parametrize("m,n,k", [(5899, 21, 312), (23, 4407, 250), (4585, 22, 381), (28, 4655, 180), (6641, 17, 198), (31, 8192, 139)])
+def test_strips_that_a_16_wide_tile_halves_stay_on_32_wide_blocks(plans, m, n, k):
+    assert gemm_tile(plans, m, n, k) is None
+    assert gemm_tile(plans, m + 16 if m < 32 else m, n + 16 if n < 32 else n, k) is not None
