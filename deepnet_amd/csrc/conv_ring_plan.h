@@ -94,10 +94,17 @@ static inline double conv_other_us(const Args& a, int mode, long long rows, bool
   if (Np % 16 != 0 || Fg % 16 != 0 || !aligned || (a.local && (copy_f || (mode != CONV_OUTP && Np % 128 != 0))))
     return 5. + 2e-6 * a.N * rows * a.F * K;                            // (1 TFLOP/s)
   auto up = [](long long v, int b) { return (double)((v + b - 1) / b * b); };
-  double flops, rate;                                                    // GFLOP, TFLOP/s
+  const double maps = 1e-9 * 8. * Np * ((double)a.M * a.F + (double)a.HH * a.C), hid = 1e-9 * 8. * Np * a.M * Fp;   // GB of a copy
+  double flops, rate, copy = 5e-3;                                       // GFLOP, TFLOP/s, GB per us
   if (mode == CONV_UP) {
     flops = 2e-9 * Np * rows * up(Fg, Fg <= 96 ? 32 : 64) * a.G * up(K, 16);
     rate = a.local ? 45. : Np % 128 == 0 && K >= 256 && (Fg <= 64 || Fg > 96) ? 105. : 85.;
+    // (few colours: the register-resident bank or 256-row tiles, and maps whose copies mostly stay in the caches)
+    if (!a.local && copy_n && K < 256 && Fg <= 64 && a.Cg <= 4) { rate = Fg > 32 && a.pad0 == 0 ? 100. : 90.; copy = 6e-3; }
+  } else if (mode == CONV_DOWN && !a.local && a.s == 1 && a.Cg <= 16) {
+    // the patch matrix, written by a product and read by a gather
+    const double patch = 1e-9 * 8. * Np * a.M * a.Cg * a.kk2 * a.G;       // GB
+    return 9. + (2e-9 * Np * a.M * Fp * K / 105. + patch / 5.) * 1e3 + (copy_n ? 5. + maps / copy : 0.) + (copy_f ? 5. + hid / copy : 0.);
   } else if (mode == CONV_DOWN) {
     flops = 2e-9 * Np * rows * up(a.Cg, a.Cg > 32 && a.Cg <= 48 ? 16 : 32) * a.G * a.kk2 * Fg;
     rate = a.local ? 70. : Np % 128 == 0 && a.kk2 * Fg >= 256 && (a.Cg <= 64 || a.Cg > 96) ? 115. : 65.;
@@ -106,9 +113,8 @@ static inline double conv_other_us(const Args& a, int mode, long long rows, bool
     flops = 2e-9 * Np * rows * up(Fg, BMs) * a.G * up(K, K <= 80 && Fg <= 64 ? 16 : 128);
     rate = a.local ? 45. : 110.;
   }
-  const double maps = 1e-9 * 8. * Np * ((double)a.M * a.F + (double)a.HH * a.C), hid = 1e-9 * 8. * Np * a.M * Fp;   // GB of a copy
   // (a long reduction may be split, and is summed by another launch)
-  return (mode == CONV_OUTP || K >= 256 ? 9. : 5.) + flops / rate * 1e3 + (copy_n ? 5. + maps / 5e-3 : 0.) + (copy_f ? 5. + hid / 5e-3 : 0.);
+  return (mode == CONV_OUTP || K >= 256 ? 9. : 5.) + flops / rate * 1e3 + (copy_n ? 5. + maps / copy : 0.) + (copy_f ? 5. + hid / copy : 0.);
 }
 
 // The share of a layer's taps that lie inside the image (Up) or reach a module (Down), and with it of the reduction that
@@ -127,6 +133,25 @@ static inline double ring_used(const Args& a, int mode) {
   return one * one;
 }
 
+// How much more of the taps than the average the busiest XCD has: every XCD gets a contiguous eighth of the pixels (one
+// group), and the lines in the middle of a map reach more modules than those at its edge.
+template <class Args>
+static inline double ring_crowd(const Args& a) {
+  double all = 0., most = 0.;
+  for (int x = 0; x < 8; ++x) {
+    double sum = 0.;
+    for (int i = x * a.H / 8; i < (x + 1) * a.H / 8 || i == x * a.H / 8; ++i) {
+      const int v = i - a.pad0, lo = v - a.Mx + 1 > 0 ? v - a.Mx + 1 : 0, hi = v + 1 < a.k ? v + 1 : a.k;
+      sum += hi > lo ? hi - lo : 0;
+    }
+    const int lines = (x + 1) * a.H / 8 - x * a.H / 8;
+    sum /= lines > 0 ? lines : 1;
+    all += sum / 8.;
+    most = sum > most ? sum : most;
+  }
+  return all > 0. ? most / all : 1.;
+}
+
 static inline ConvRingPlan conv_no_ring() { return {-1, 1, 0, false, 0.}; }
 
 // Up and Down: tiles over any run of (module | pixel, image) groups, which needs batches of whole groups of four, or of
@@ -142,7 +167,10 @@ static inline ConvRingPlan conv_rows_plan(const Args& a, int mode, bool maps16, 
     const ConvRingPlan flat = conv_ring_plan(mode, false, (long long)sites * a.N, cols, a.G, K, 1., false, 0., cus);
     if (flat.cfg >= 0 && (plan.cfg < 0 || flat.us < plan.us)) plan = flat;
   }
-  return plan.cfg < 0 || plan.us > conv_other_us(a, mode, sites, maps16, filters16) ? conv_no_ring() : plan;
+  // (the patch form of few colours does all pixels at once: there the busiest XCD counts, elsewhere the estimates do not
+  // differ by as little)
+  const double crowd = !up && plan.single && !a.local && a.Cg <= 16 ? ring_crowd(a) : 1.;
+  return plan.cfg < 0 || crowd * plan.us > conv_other_us(a, mode, sites, maps16, filters16) ? conv_no_ring() : plan;
 }
 
 // Outp of `a`, whose batch the ring takes in whole groups of four images: others are copied with up to three images of zeros.

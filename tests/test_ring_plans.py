@@ -69,3 +69,15 @@ def test_layers_are_planned_as_their_comments_say(plans):
 def test_strips_that_a_16_wide_tile_halves_stay_on_32_wide_blocks(plans, m, n, k):
     assert gemm_tile(plans, m, n, k) is None
     assert gemm_tile(plans, m + 16 if m < 32 else m, n + 16 if n < 32 else n, k) is not None
+
+
+@pytest.mark.parametrize("mode,layer", [(DOWN, (100, 16, 30, 208, 7, 1, 0)), (DOWN, (80, 16, 19, 172, 5, 1, 0)), (UP, (100, 3, 64, 48, 7, 1, 0)),
+                                        (UP, (100, 3, 161, 48, 7, 2, 0)), (UP, (100, 1, 90, 32, 7, 1, 3)), (UP, (234, 1, 79, 40, 7, 1, 3))])
+def test_layers_of_few_colours_that_other_kernels_are_faster_on(plans, mode, layer):
+    assert conv_tile(plans, mode, *layer) is None
+
+
+@pytest.mark.parametrize("mode,layer", [(DOWN, (100, 16, 28, 208, 7, 1, 3)), (DOWN, (117, 16, 25, 64, 7, 1, 3)), (DOWN, (202, 16, 8, 224, 5, 1, 0)),
+                                        (UP, (100, 3, 74, 64, 5, 1, 0)), (UP, (100, 1, 54, 32, 7, 2, 0))])
+def test_layers_of_few_colours_that_ring_tiles_are_faster_on(plans, mode, layer):
+    assert conv_tile(plans, mode, *layer) is not None
