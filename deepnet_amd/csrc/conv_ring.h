@@ -9,11 +9,6 @@
 // round).  RING_FAR stands in no lane's mask: such a term reads as zero.
 #define RING_FAR 0x80000000u
 static_assert(RING_AHEAD >= RING_SETS + 3, "fetch() looks one stage ahead, the loop RING_SETS + 2");
-__device__ __forceinline__ unsigned ring_bits(int lo, int hi) {      // bits lo .. hi - 1
-  lo = lo < 0 ? 0 : lo;
-  hi = hi < lo ? lo : hi;
-  return ((1u << hi) - 1u) & ~((1u << lo) - 1u);
-}
 
 struct ConvRingArgs {
   const float* a; const float* b;

@@ -9,6 +9,14 @@ enum { CONV_UP = 0, CONV_DOWN = 1, CONV_OUTP = 2, CONV_DOWNM = 3 };
 #define RING_MAX_SIDE 15   // filter rows and columns that a mask has room for
 #define RING_AHEAD 7       // stages that the table of a tile of one module or pixel reaches beyond its last one
 
+// Bits lo .. hi - 1 of a mask, hi <= RING_MAX_SIDE.  lo grows with the padding, and with the image beyond the modules' reach
+// (host and device).
+static constexpr unsigned ring_bits(int lo, int hi) {
+  lo = lo < 0 ? 0 : lo > RING_MAX_SIDE ? RING_MAX_SIDE : lo;
+  hi = hi < lo ? lo : hi;
+  return ((1u << hi) - 1u) & ~((1u << lo) - 1u);
+}
+
 // The batch that a pass is copied to when it is no multiple of 16 images (see PaddedBatch).
 static inline int padded_batch(int N) {
   if (N <= 16 || N % 16 == 0) return N;

@@ -2,6 +2,10 @@
 #include "../deepnet_amd/csrc/gemm_ring_plan.h"
 #include "../deepnet_amd/csrc/conv_ring_plan.h"
 
+// (a shift by 32 or more does not compile here)
+static_assert(ring_bits(2, 5) == 0x1c && ring_bits(-3, 4) == 0xf && ring_bits(0, RING_MAX_SIDE) == 0x7fff && ring_bits(4, 4) == 0, "");
+static_assert(ring_bits(5, 3) == 0 && ring_bits(14, -2) == 0 && ring_bits(33, 7) == 0 && ring_bits(400, 15) == 0, "");
+
 struct Sizes { int N, C, Cg, H, HH, F, Fg, k, kk2, Mx, M, s, pad0, G, local, m_count, chunks; };
 
 extern "C" {

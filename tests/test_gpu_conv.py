@@ -592,7 +592,8 @@ RING_LAYERS = [  # N, C, H, F, k, stride, padding, groups
     (16, 25, 5, 16, 7, 1, 1, 1),      # and 32 x 16,
     (80, 108, 5, 8, 7, 1, 1, 1),      # and of one pixel on 32 x 64,
     (1, 50, 21, 240, 5, 1, 1, 1),     # Outp on 64 x 64
-    (100, 75, 7, 35, 3, 1, 1, 1)]     # and 32 x 64
+    (100, 75, 7, 35, 3, 1, 1, 1),     # and 32 x 64
+    (4, 16, 6, 32, 5, 1, 40, 1)]      # padding of more rows than a mask has bits
 
 
 @pytest.mark.parametrize("N,C,H,F,k,s,p,G", RING_LAYERS)
@@ -609,9 +610,9 @@ def test_locally_connected_layers_on_ring_tiles(cm, cc, rng, N, C, H, F, k, s, p
     test_locally_connected_layers(cm, cc, rng, N, C, H, F, k, s, p)
 
 
-@pytest.mark.parametrize("N", [64, 50])
-def test_pixels_that_no_module_reaches_get_zero_on_ring_tiles(cm, cc, rng, N):
-    C, H, F, k, Mx = 64, 12, 64, 3, 6
+@pytest.mark.parametrize("N,H", [(64, 12), (50, 12), (4, 50), (20, 50)])
+def test_pixels_that_no_module_reaches_get_zero_on_ring_tiles(cm, cc, rng, N, H):
+    C, F, k, Mx = 64, 64, 3, 6
     y, w = _f(rng.standard_normal((N, F * Mx * Mx))), _f(0.1 * rng.standard_normal((F, C * k * k)))
     down = cm.CUDAMatrix(np.full((N, C * H * H), np.nan, dtype=np.float32))
     cc.convDown(cm.CUDAMatrix(y), cm.CUDAMatrix(w), down, Mx, 0, 1, k, H, C)
