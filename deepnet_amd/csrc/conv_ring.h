@@ -116,6 +116,7 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
   using OB = ConvRingOperand<MODE == CONV_UP ? (SINGLE ? 6 : 1) : MODE == CONV_DOWN ? (SINGLE ? 7 : 2) : 4, BN, BK, PER>;
   using Shape = RingShape<TB, BM, BN, BK, OA, OB>;
   constexpr int EPL = Shape::EPL;
+  static_assert(Shape::LDS * 4 == conv_ring_lds(MODE, BM, BN, BK) && Shape::LDS * 4 + RING_TABLE_BYTES <= RING_CU_LDS, "as planned");
   __shared__ __attribute__((aligned(16))) float lds[Shape::LDS];
   extern __shared__ uint2 table[];
   const int tid = threadIdx.x;

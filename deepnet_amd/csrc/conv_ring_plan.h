@@ -38,7 +38,16 @@ static inline int padded_filters(int F, int numGroups) {
 static const struct { int bm, bn, bk; double stage, tile; } g_conv_ring_cfgs[] = {
     {64, 64, 32, 0.545, 1.45}, {64, 32, 64, 0.574, 1.46}, {32, 64, 64, 0.58, 1.45},
     {32, 32, 64, 0.322, 1.0}, {32, 16, 128, 0.372, 1.2}, {16, 32, 128, 0.372, 1.17}};
-#define RING_TABLE_BYTES 26624      // what a workgroup's LDS holds besides the tiles (64 KB in all)
+// What a workgroup's LDS holds besides the two stages of its tile, which take 36 to 57 KB.  Two workgroups share a CU while
+// they take half of its 160 KB each; with a full table convUp on 32 x 16 and 16 x 32 tiles takes 82 KB and is alone.
+#define RING_TABLE_BYTES 26624
+#define RING_CU_LDS (160 << 10)
+
+// LDS of the two stages of a tile in bytes (k_conv_ring checks that it is what its tile loop takes).
+static constexpr int conv_ring_lds(int mode, int bm, int bn, int bk) {
+  const int a = mode == CONV_OUTP ? bm * (bk + 4) : bk * (bm + 4), b = mode == CONV_UP ? bk * (bn + 4) : bn * (bk + 4);
+  return 8 * (a + b);
+}
 
 struct ConvRingPlan { int cfg, splits, split_stages; bool single; double us; };
 
@@ -71,7 +80,9 @@ static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows,
       const int per = (nst + s - 1) / s, real = (nst + per - 1) / per;
       const long long all = tiles * real;
       if (all >= 1ll << 28) continue;
-      const double rounds = all <= 4 * cus ? (double)((all + cus - 1) / cus) : 0.5 + (double)all / cus;
+      double rounds = all <= 4 * cus ? (double)((all + cus - 1) / cus) : 0.5 + (double)all / cus;
+      // alone on its CU a workgroup shows its waits (122 -> 126 colours of 5 x 5 on 16 filters, 24 x 24, batch 100: 66 -> 77 us)
+      if (rounds > 1. && 2 * (conv_ring_lds(mode, f.bm, f.bn, f.bk) + conv_ring_table(mode, single, f.bk, per)) > RING_CU_LDS) rounds *= 1.16;
       const double us = 3. + rounds * (used * per * f.stage + f.tile) + (real > 1 ? 2.5 + real * split_us : 0.);
       if (best.cfg < 0 || us < best.us) best = {c, real, per, single, us};
     }

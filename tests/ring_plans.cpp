@@ -15,15 +15,17 @@ int gemm_tile(int M, int N, int K, int cus) {
   return K > 128 ? gemm_ring_plan(M, N, K, (size_t)M * K * 4, (size_t)N * K * 4, cus).cfg : -1;
 }
 
-// out = {tile number or -1, one module or pixel per tile, splits, table bytes}
-void conv_tile(int mode, int N, int C, int H, int F, int k, int Mx, int s, int pad0, int G, int local, int partial_sum, int cus, int* out) {
+// out = {tile number or -1, one module or pixel per tile, splits, LDS bytes of a workgroup, us}
+void conv_tile(int mode, int N, int C, int H, int F, int k, int Mx, int s, int pad0, int G, int local, int partial_sum, int cus, double* out) {
   const int m = partial_sum ? partial_sum : Mx * Mx;
   const Sizes a = {N, C, C / G, H, H * H, F, F / G, k, k * k, Mx, Mx * Mx, s, pad0, G, local, m, Mx * Mx / m};
   const ConvRingPlan p = mode == CONV_OUTP ? conv_outp_plan(a, N % 4 == 0, true, cus) : conv_rows_plan(a, mode, N % 4 == 0, true, cus);
   out[0] = p.cfg; out[1] = p.single; out[2] = p.splits;
   const int K = mode == CONV_OUTP ? 0 : a.kk2 * (mode == CONV_UP ? a.Cg : a.Fg);
-  const int bk = p.cfg < 0 ? 1 : g_conv_ring_cfgs[p.cfg].bk, stages = mode == CONV_OUTP ? p.split_stages : (K + bk - 1) / bk;
-  out[3] = p.cfg < 0 ? 0 : conv_ring_table(mode, p.single, bk, stages);
+  if (p.cfg < 0) return;
+  const auto& f = g_conv_ring_cfgs[p.cfg];
+  out[3] = conv_ring_lds(mode, f.bm, f.bn, f.bk) + conv_ring_table(mode, p.single, f.bk, mode == CONV_OUTP ? p.split_stages : (K + f.bk - 1) / f.bk);
+  out[4] = p.us;
 }
 
 }  // extern "C"

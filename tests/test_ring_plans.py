@@ -31,10 +31,10 @@ def gemm_tile(plans, m, n, k):
 
 
 def conv_tile(plans, mode, N, C, H, F, k, s, p, G=1, local=False, partial_sum=0):
-    """(tile, whether it lies in one module or pixel, splits, table bytes) of a pass; None: another kernel."""
-    out = (ct.c_int * 4)()
+    """(tile, whether it lies in one module or pixel, splits, LDS bytes, us) of a pass; None: another kernel."""
+    out = (ct.c_double * 5)()
     plans.conv_tile(mode, N, C, H, F, k, co.n_modules(H, k, s, p), s, -p, G, int(local), 1 if local and mode == OUTP else partial_sum, CUS, out)
-    return (TILES[out[0]], bool(out[1]), out[2], out[3]) if out[0] >= 0 else None
+    return (TILES[int(out[0])], bool(out[1]), out[2], out[3], out[4]) if out[0] >= 0 else None
 
 
 def test_the_products_of_the_gpu_tests_reach_every_tile(plans):
@@ -54,6 +54,13 @@ def test_the_layers_of_the_gpu_tests_reach_every_tile(plans):
                 reached.add((mode, t[1], t[0]))
     want = {(mode, single, tile) for mode in (UP, DOWN, OUTP) for single in (False, True) for tile in TILES if not (mode == OUTP and single)}
     assert reached == want, sorted(want - reached)
+
+
+def test_a_workgroup_that_is_alone_on_its_cu_costs_more(plans):
+    """convUp on 32 x 16 tiles: with 24 stages of table two workgroups fit the 160 KB of a CU, with 25 one."""
+    two, one = (conv_tile(plans, UP, 100, colors, 24, 16, 5, 1, 0) for colors in (122, 126))
+    assert two[0] == one[0] == (32, 16) and two[3] <= 80 << 10 < one[3]
+    assert one[4] > 1.15 * two[4]
 
 
 def test_layers_are_planned_as_their_comments_say(plans):
