@@ -350,6 +350,22 @@ def test_softmax_of_columns_whose_last_group_moves_back(cm, rng, h, skip):
     whole.free_device_memory()
 
 
+@pytest.mark.parametrize("h,w", [(8192, 128), (8195, 129), (4096, 256), (4100, 256), (4099, 255), (65536, 256), (65537, 256), (2047, 257)])
+def test_rows_of_tall_matrices_around_one_trip_of_the_columns(cm, rng, h, w):
+    """256, 512 and 1024 lanes a workgroup: sums as a double-precision one (at most w * 2^-24 of the magnitudes), maxima exactly."""
+    x = _rand(rng, (h, w))
+    a = cm.CUDAMatrix(x)
+    want, bound = x.astype(np.float64).sum(axis=1, keepdims=True), w * 2.0 ** -24 * np.abs(x).astype(np.float64).sum(axis=1, keepdims=True)
+    assert np.all(np.abs(a.sum(axis=1).asarray() - want) <= bound)
+    assert np.array_equal(a.max(axis=1).asarray(), x.max(axis=1, keepdims=True))
+    sq = (x.astype(np.float64) ** 2).sum(axis=1, keepdims=True)
+    assert np.all(np.abs(a.sqsum(axis=1).asarray() - sq) <= (w + 1) * 2.0 ** -24 * sq)
+    y = cm.CUDAMatrix(np.ones((h, 1), dtype=np.float32))
+    y.add_sums(a, axis=1, mult=0.5)
+    assert np.all(np.abs(y.asarray() - (1.0 + 0.5 * want)) <= bound + 2.0 ** -23 * np.abs(1.0 + 0.5 * want))
+    a.free_device_memory()
+
+
 def test_scalars_that_are_read_later(cm, rng):
     """read_later() is the value at the time of the call, with the bits of sum() and euclid_norm(), in any order of reading;
     a value that 63 others have followed is refused."""
