@@ -2,8 +2,9 @@
 against the float64 restatement: 1e-4 relative for the convolutions (error measured
 against the sum of magnitudes, as for dot), exact for pooling, 2e-6 relative for the
 normalisation's denominators and 1e-5 for its outputs (x^-p through the hardware log2 / exp2,
-as the reference's __powf).  Shapes with a batch that is not a multiple of 16 run the
-one-lane-per-output kernels; the others the matrix-core kernel."""
+as the reference's __powf).  Which kernel a convolution runs on follows from its sizes: most of the
+small layers here run on ring tiles (tests/test_ring_plans.py), OTHER_LAYERS and OTHER_LOCAL on every
+form of the kernels that larger ones have."""
 import numpy as np
 import pytest
 
@@ -13,6 +14,7 @@ pytestmark = pytest.mark.gpu
 
 REL = 1e-4
 
+# (the comments say what is special about a layer; the kernels that they name have it at larger sizes)
 CASES = [  # N, C, H, F, k, stride, padding, groups
     (2, 3, 6, 16, 3, 1, 1, 1),       # direct kernels (batch 2)
     (3, 4, 7, 8, 3, 2, 1, 2),
@@ -632,3 +634,103 @@ def test_partial_sums_on_ring_tiles(cm, cc, rng, N):
     cc.convOutp(cm.CUDAMatrix(x), cm.CUDAMatrix(y), t, Mx, p, k, s, C, partialSum=Mx)
     want = co.conv_outp(x, y, C, Mx, k, p, s, partial_sum=Mx)
     assert np.linalg.norm(t.asarray() - want) < 1e-5 * np.linalg.norm(want)
+
+
+# Layers that k_conv_ring does not take, for every form of the other kernels: layer -> the passes (tests/test_ring_plans.py
+# checks that they are not on ring tiles), and which form each is there for
+OTHER_LAYERS = {  # N, C, H, F, k, stride, padding, groups
+    (64, 1, 5, 10, 3, 3, 0, 1): "up",               # Up taps<1,1,3>
+    (64, 1, 6, 9, 5, 4, 1, 1): "up",                # Up taps<1,1,5>
+    (16, 1, 5, 112, 2, 2, 1, 1): "outp",            # Outp 128-row tiles
+    (100, 16, 4, 12, 4, 2, 0, 1): "down outp up",   # Down merged phases, 64 columns; Outp 32-row tiles, inside; Up uniform rows, 16 columns split
+    (64, 48, 4, 9, 4, 1, 0, 1): "down",             # Down 128-row tiles, 64 columns split
+    (100, 62, 4, 9, 4, 1, 0, 1): "down",            # Down uniform rows, 64 columns split
+    (256, 9, 5, 11, 3, 3, 1, 1): "down outp",       # Down merged phases, 96 columns; Outp small<1,3>
+    (144, 1, 15, 32, 7, 4, 1, 1): "outp",           # Outp registers<2,4>
+    (20, 97, 6, 36, 6, 3, 0, 1): "down up",         # Down 128-row tiles, 128 columns; Up 128-row tiles, 64 columns split
+    (176, 4, 5, 48, 3, 1, 0, 1): "outp",            # Outp registers<3,3>
+    (176, 1, 6, 80, 2, 1, 1, 1): "up",              # Up 128-row tiles, 96 columns
+    (144, 1, 12, 64, 6, 3, 1, 1): "outp",           # Outp registers<4,3>
+    (144, 1, 13, 48, 7, 3, 0, 1): "outp",           # Outp registers<3,4>
+    (256, 1, 17, 48, 3, 3, 1, 1): "up",             # Up taps<2,1,3>
+    (192, 1, 11, 208, 2, 2, 0, 1): "outp up",       # Outp 128-row tiles, inside; Up 128-row tiles, 128 columns
+    (144, 1, 9, 64, 7, 4, 3, 1): "outp",            # Outp registers<4,4>
+    (20, 68, 7, 90, 7, 3, 0, 1): "down up",         # Down 128-row tiles, 96 columns; Up 128-row tiles, 96 columns split
+    (128, 143, 5, 21, 5, 1, 0, 1): "down up",       # Down uniform rows, 64 of more split; Up uniform rows, 32 columns split
+    (64, 1, 34, 48, 5, 3, 2, 1): "up",              # Up taps<2,1,5>
+    (176, 1, 41, 10, 2, 1, 0, 1): "up",             # Up 256-row tiles, 32 columns, inside
+    (256, 3, 17, 48, 3, 3, 1, 1): "up",             # Up taps<2,3,3>
+    (20, 136, 6, 125, 6, 1, 0, 1): "down up",       # Down 128-row tiles, 128 columns split; Up 128-row tiles, 128 columns split
+    (144, 1, 32, 33, 2, 1, 0, 1): "up",             # Up 256-row tiles, 64 columns
+    (100, 144, 5, 9, 6, 1, 1, 1): "down",           # Down uniform rows, 128 columns split
+    (128, 64, 9, 48, 7, 3, 0, 1): "down up",        # Down uniform rows, 64 columns; Up uniform rows, 48 columns split
+    (100, 20, 33, 10, 3, 3, 1, 1): "down",          # Down 256-row tiles, 32 columns
+    (100, 114, 4, 64, 6, 3, 1, 1): "down up",       # Down uniform rows, 64 of more; Up uniform rows, 64 columns split
+    (144, 2, 48, 96, 2, 2, 0, 2): "up",             # Up 256-row tiles, 64 columns, inside
+    (100, 102, 11, 27, 11, 3, 1, 1): "down",        # Down uniform rows, 128 columns
+    (160, 1, 30, 71, 2, 1, 0, 1): "up",             # Up 256-row tiles, 96 columns
+    (100, 32, 9, 112, 11, 2, 1, 1): "down up",      # Down uniform rows, 32 columns; Up uniform rows, 64 of more split
+    (80, 1, 45, 9, 7, 1, 1, 1): "outp up",          # Outp registers<1,4>; Up 256-row tiles, 32 columns
+    (37, 92, 47, 11, 4, 4, 0, 1): "down",           # Down 256-row tiles, 96 columns
+    (100, 33, 36, 9, 4, 2, 0, 1): "down up",        # Down 256-row tiles, 64 columns; Up uniform rows, 16 columns
+    (96, 4, 18, 96, 6, 1, 1, 2): "outp",            # Outp registers<3,5>
+    (16, 68, 19, 48, 11, 2, 0, 1): "outp",          # Outp 64-row tiles, inside
+    (128, 24, 12, 64, 6, 3, 3, 1): "outp",          # Outp 64-row tiles
+    (128, 20, 17, 17, 4, 1, 1, 1): "up",            # Up uniform rows, 32 columns
+    (256, 28, 18, 112, 3, 3, 0, 1): "up",           # Up uniform rows, 128 columns split
+    (39, 68, 44, 10, 5, 2, 1, 1): "up",             # Up 256-row tiles, 32 columns split
+    (20, 29, 45, 10, 6, 1, 0, 1): "up",             # Up 256-row tiles, 32 columns, inside split
+    (256, 2, 22, 48, 11, 1, 0, 1): "up",            # Up uniform rows, 48 columns
+    (256, 2, 20, 64, 11, 1, 1, 1): "up",            # Up uniform rows, 64 columns
+    (128, 16, 48, 208, 4, 4, 0, 1): "up",           # Up uniform rows, 64 of more
+}
+OTHER_LOCAL = {   # the same of locally connected layers
+    (32, 2, 6, 16, 5, 4, 1, 1): "down",             # Down merged phases, 32 columns
+    (64, 3, 6, 16, 4, 4, 0, 1): "down",             # Down merged phases, 48 columns
+    (64, 4, 7, 16, 4, 4, 0, 1): "down",             # Down merged phases, 64 columns
+    (64, 1, 5, 128, 3, 3, 0, 1): "outp",            # Outp 128-row tiles, inside
+    (100, 5, 7, 16, 4, 4, 0, 1): "down",            # Down merged phases, 96 columns
+    (16, 1, 8, 80, 2, 2, 1, 1): "outp",             # Outp 96-row tiles
+    (32, 16, 4, 16, 4, 3, 0, 1): "down",            # Down merged phases, 128 columns
+    (128, 4, 5, 32, 2, 1, 1, 2): "down outp up",    # Down uniform rows, 16 columns; Outp 32-row tiles; Up uniform rows, 16 columns
+    (256, 1, 5, 48, 2, 1, 1, 1): "outp up",         # Outp 64-row tiles; Up uniform rows, 48 columns
+    (48, 80, 5, 16, 6, 2, 1, 1): "down up",         # Down uniform rows, 64 of more; Up uniform rows, 16 columns split
+    (256, 1, 9, 32, 2, 1, 1, 1): "up",              # Up uniform rows, 32 columns
+    (128, 2, 5, 256, 2, 1, 1, 2): "outp up",        # Outp 128-row tiles; Up uniform rows, 64 of more
+    (256, 1, 11, 64, 2, 1, 0, 1): "outp up",        # Outp 64-row tiles, inside; Up uniform rows, 64 columns
+    (128, 2, 10, 160, 2, 1, 0, 2): "outp up",       # Outp 96-row tiles, inside; Up uniform rows, 128 columns
+    (128, 52, 5, 32, 7, 3, 1, 1): "down up",        # Down uniform rows, 64 columns; Up uniform rows, 32 columns split
+    (64, 78, 10, 48, 7, 4, 0, 1): "down up",        # Down uniform rows, 128 columns; Up uniform rows, 48 columns split
+    (128, 54, 8, 64, 7, 4, 1, 1): "up",             # Up uniform rows, 64 columns split
+    (64, 38, 4, 80, 11, 4, 5, 1): "down up",        # Down uniform rows, 48 columns; Up uniform rows, 64 of more split
+    (76, 29, 11, 112, 11, 1, 0, 1): "down",         # Down uniform rows, 32 columns split
+    (128, 36, 6, 80, 2, 1, 1, 1): "down",           # Down uniform rows, 48 columns split
+    (48, 89, 6, 96, 6, 2, 3, 1): "up",              # Up uniform rows, 128 columns split
+    (64, 63, 11, 160, 11, 1, 1, 1): "down",         # Down uniform rows, 64 columns split
+}
+
+
+@pytest.mark.parametrize("N,C,H,F,k,s,p,G", list(OTHER_LAYERS))
+def test_three_conv_passes_on_the_other_kernels(cm, cc, rng, N, C, H, F, k, s, p, G):
+    test_three_conv_passes(cm, cc, rng, N, C, H, F, k, s, p, G)
+
+
+@pytest.mark.parametrize("N,C,H,F,k,s,p,G", list(OTHER_LOCAL))
+def test_locally_connected_layers_on_the_other_kernels(cm, cc, rng, N, C, H, F, k, s, p, G):
+    Mx = co.n_modules(H, k, s, p)
+    M, Cg, Fg, HH = Mx * Mx, C // G, F // G, H * H
+    x, w, y = _f(rng.standard_normal((N, C * HH))), _f(0.1 * rng.standard_normal((F, M * Cg * k * k))), _f(rng.standard_normal((N, F * M)))
+    X, W, Y = cm.CUDAMatrix(x), cm.CUDAMatrix(w), cm.CUDAMatrix(y)
+    up, down, outp = (cm.CUDAMatrix(np.full(shape, np.nan, dtype=np.float32)) for shape in ((N, F * M), (N, C * HH), (F, M * Cg * k * k)))
+    cc.localUp(X, W, up, Mx, p, s, C, G)
+    cc.localDown(Y, W, down, Mx, p, s, k, H, C, numGroups=G)
+    cc.localOutp(X, Y, outp, Mx, p, k, s, C, numGroups=G)
+    for g in range(G):
+        maps, units, rows = slice(g * Cg * HH, (g + 1) * Cg * HH), slice(g * Fg * M, (g + 1) * Fg * M), slice(g * Fg, (g + 1) * Fg)
+        a, b, c = x[:, maps], w[rows], y[:, units]
+        for got, f in ((up.asarray()[:, units], lambda x, w, y: co.local_up(x, w, Cg, Mx, p, s)),
+                       (down.asarray()[:, maps], lambda x, w, y: co.local_down(y, w, Cg, H, p, s)),
+                       (outp.asarray()[rows], lambda x, w, y: co.local_outp(x, y, Cg, Mx, k, p, s))):
+            assert _relerr(got, f(a, b, c), f(np.abs(a), np.abs(b), np.abs(c)) + 1e-6) < REL
+    for m in (X, W, Y, up, down, outp):
+        m.free_device_memory()

@@ -123,10 +123,12 @@ def test_large_square_products(cm, rng, n):
 
 
 @pytest.mark.parametrize("m,k,n", [(1000, 1001, 1000), (1001, 1000, 1000), (1000, 1000, 1001), (1003, 999, 1005), (1088, 50, 1088),
-                                   (1100, 48, 1000), (1100, 47, 1000), (2000, 130, 1300), (1004, 1030, 996)])
+                                   (1100, 48, 1000), (1100, 47, 1000), (2000, 130, 1300), (1004, 1030, 996), (2040, 333, 2047),
+                                   (2046, 129, 2041)])
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True)])
 def test_products_on_the_tile_loop_with_any_alignment(cm, rng, m, k, n, ta, tb):
-    """More 64 x 64 tiles than the single-launch kernels take: the loop over 16-deep slabs whose
+    """More 64 x 64 tiles than the single-launch kernels take: with up to 128 terms, or a number of tiles that fills the
+    CUs evenly (the last two; k_gemm_ring has the others), the loop over 16-deep slabs whose
     loads are unconditional 16-byte requests.  Leading dimensions that are not multiples of four
     floats, operands that start at an odd float of a parent buffer, tiles that hang over the edge,
     reductions of exactly three slabs (the shortest that enter the loop) and of one float less."""
@@ -223,8 +225,9 @@ def test_dot_bias_act_is_bit_identical_to_the_three_calls(cm, rng, m, n, k, ta, 
     (500, 100, 784, True, 'sigmoid'),      # the RBM's up-pass: 16 x 16 blocks, 5 draws per stream
     (37, 19, 50, False, 'sigmoid'),        # fewer outputs than streams: the idle streams keep their words
     (1024, 128, 784, True, 'sigmoid'),     # 16 x 16 blocks on 512 workgroups, 11 draws per stream
-    (768, 192, 300, True, 'sigmoid'),      # 32 x 32 blocks (144 of them), 12 draws per stream
-    (1024, 128, 512, True, 'relu'),        # 32 x 32 blocks: both operands K-contiguous, rows 2 KiB apart
+    (768, 192, 300, True, 'sigmoid'),      # 32 x 32 ring tiles (144 of them), 12 draws per stream
+    (1024, 128, 512, True, 'relu'),        # 32 x 16 ring tiles: both operands K-contiguous, rows 2 KiB apart
+    (4608, 27, 300, True, 'sigmoid'),      # 32 x 32 blocks (144 of them)
     (96, 128, 64, False, 'tanh'),          # exactly 12288 outputs
     (1024, 200, 300, True, 'sigmoid'),     # more than 16 draws per stream: separate kernels
     (2048, 2048, 64, False, 'sigmoid'),    # a product on the big tiles: separate sample kernel
@@ -496,10 +499,16 @@ RING_SHAPES = [(2001, 1003, 250), (640, 1280, 256), (65, 4095, 129), (1500, 300,
               (333, 2859, 193), (449, 2048, 960), (726, 2749, 1091)]      # 32 x 64
 
 
-@pytest.mark.parametrize("m,n,k", RING_SHAPES)
+# products of more than 128 terms that k_gemm_ring does not take (tests/test_ring_plans.py): strips and 32 x 32 blocks over
+# eight wavefronts, 64 x 64 tiles in whole rounds of the CUs, slices of long reductions, 128 x 128 tiles
+OTHER_SHAPES = [(5899, 21, 312), (23, 4407, 250), (4100, 31, 300), (4097, 17, 129), (2040, 2047, 333), (2048, 2048, 300),
+                (1023, 1041, 2100), (130, 129, 9000), (2041, 2046, 1060)]
+
+
+@pytest.mark.parametrize("m,n,k", RING_SHAPES + OTHER_SHAPES)
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
 def test_products_on_tiles_that_move_back_inside(cm, rng, m, n, k, ta, tb):
-    """k_gemm_ring's edges: values beyond the operands (NaN here) never reach a result, and accumulating stores every
+    """The edges of k_gemm_ring, and of the kernels beside it: values beyond the operands (NaN here) never reach a result, and accumulating stores every
     output once.  fp32 sums of k terms in any order: sqrt(k) * 2^-24 of the norm expected; 16 times that allowed."""
     def operand(a, trans):
         stored = np.asfortranarray(a.T if trans else a)
@@ -522,9 +531,10 @@ def test_products_on_tiles_that_move_back_inside(cm, rng, m, n, k, ta, tb):
         h.free_device_memory()
 
 
-@pytest.mark.parametrize("m,n,k", [(1001, 150, 700), (700, 97, 900), (520, 300, 520)])
+# (the last two: 32 x 32 blocks)
+@pytest.mark.parametrize("m,n,k", [(1001, 150, 700), (700, 97, 900), (520, 300, 520), (4585, 22, 381), (4100, 31, 260)])
 def test_draws_on_tiles_that_move_back_inside(cm, rng, m, n, k):
-    """A sample drawn by the launch of k_gemm_ring is the one sample_bernoulli draws, and so is the generator's state."""
+    """A sample drawn by the product's launch is the one sample_bernoulli draws, and so is the generator's state."""
     w, x, bias = cm.CUDAMatrix(0.1 * _rand(rng, (k, m))), cm.CUDAMatrix(_rand(rng, (k, n))), cm.CUDAMatrix(_rand(rng, (m, 1)))
     got = []
     for defer in (True, False):

@@ -45,6 +45,10 @@ def test_the_products_of_the_gpu_tests_reach_every_tile(plans):
         assert edges and max(edges) == 2, tile           # one of them hangs over both edges
 
 
+def test_the_products_of_the_other_kernels_are_not_on_ring_tiles(plans):
+    assert [shape for shape in dot.OTHER_SHAPES if gemm_tile(plans, *shape)] == []
+
+
 def test_the_layers_of_the_gpu_tests_reach_every_tile(plans):
     reached = set()
     for mode in (UP, DOWN, OUTP):
@@ -88,3 +92,11 @@ def test_layers_of_few_colours_that_other_kernels_are_faster_on(plans, mode, lay
                                         (UP, (100, 3, 74, 64, 5, 1, 0)), (UP, (100, 1, 54, 32, 7, 2, 0))])
 def test_layers_of_few_colours_that_ring_tiles_are_faster_on(plans, mode, layer):
     assert conv_tile(plans, mode, *layer) is not None
+
+
+def test_the_layers_of_the_other_kernels_are_not_on_ring_tiles(plans):
+    """Most layers of the tests are small, and small layers go to ring tiles: these are there for the other kernels."""
+    for layers, local in ((conv.OTHER_LAYERS, False), (conv.OTHER_LOCAL, True)):
+        for layer, passes in layers.items():
+            for name in passes.split():
+                assert conv_tile(plans, dict(up=UP, down=DOWN, outp=OUTP)[name], *layer, local=local) is None, (layer, name)
