@@ -39,9 +39,11 @@ static inline RingPlan gemm_ring_plan(int M, int N, int K, size_t a_bytes, size_
   if (ring.us >= sliced_us) return none;
   // Strips of 17 to 31 rows or columns: the second 16-wide tile is nearly empty, a 32 x 32 block is not, and while those
   // fit one round of the CUs they take 3.8 us + 5 us per 1024 terms (operands from memory, us, ring -> blocks: 5899 x 21 x
-  // 312 8.3 -> 7.3, 23 x 4407 x 250 6.2 -> 5.4, 4585 x 22 x 381 8.1 -> 7.2, 28 x 4655 x 180 5.9 -> 5.2).
+  // 312 8.3 -> 7.3, 23 x 4407 x 250 6.2 -> 5.4, 4585 x 22 x 381 8.1 -> 7.2, 28 x 4655 x 180 5.9 -> 5.2).  Longer ones wait
+  // for what a CU can pull in and win on the ring (from the caches, 6434 x 20 x 1675 16.2 against 21.9, 7038 x 19 x 743 9.3
+  // against 11.6).
   const int thin = M < N ? M : N;
-  if (thin > 16 && thin < 32 && tiles(32) <= cus && ring.us >= 3.8 + 5.0 * K / 1024.0) return none;
+  if (thin > 16 && thin < 32 && K <= 512 && tiles(32) <= cus && ring.us >= 3.8 + 5.0 * K / 1024.0) return none;
   if (tiles(128) >= cus && 4 * rounds(tiles(128)) <= rounds(tiles(64))) return none;
   return ring;
 }

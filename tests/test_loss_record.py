@@ -5,8 +5,17 @@ import types
 
 import pytest
 
-from deepnet_amd.layer import _metrics
-from deepnet_amd.neuralnet import Accumulate
+
+# (the package is imported when a test runs, not when it is collected: it loads the HIP runtime, and in a process that
+# imports torch as well torch's has to come first)
+def _metrics(count):
+    from deepnet_amd.layer import _metrics
+    return _metrics(count)
+
+
+def Accumulate(stats, losses):
+    from deepnet_amd.neuralnet import Accumulate
+    return Accumulate(stats, losses)
 
 
 def _late(asked):

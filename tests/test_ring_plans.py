@@ -80,6 +80,7 @@ def test_layers_are_planned_as_their_comments_say(plans):
 def test_strips_that_a_16_wide_tile_halves_stay_on_32_wide_blocks(plans, m, n, k):
     assert gemm_tile(plans, m, n, k) is None
     assert gemm_tile(plans, m + 16 if m < 32 else m, n + 16 if n < 32 else n, k) is not None
+    assert gemm_tile(plans, m, n, 4 * k + 400) is not None
 
 
 @pytest.mark.parametrize("mode,layer", [(DOWN, (100, 16, 30, 208, 7, 1, 0)), (DOWN, (80, 16, 19, 172, 5, 1, 0)), (UP, (100, 3, 64, 48, 7, 1, 0)),
