@@ -853,9 +853,11 @@ static void rezero_counters(unsigned* counters, int n) {
 
 // The sums of layer states run on 256 lanes per workgroup, which start sooner than 1024: up to 2^18 elements, one trip of the
 // columns (128) whatever the height (50176 x 128 from memory 7.6 -> 6.9 us, from the caches 5.9 -> 3.4), or two trips up to
-// 2^20 elements (four sums of 2001 x 250 and 1003 x 250 then share one launch).
+// 2^24 elements, where several sums share one launch (four of 2001 x 250 and 1003 x 250 states; add_sums of 10560 x 208 2.3 us
+// a call, 3.3 alone).  By itself a sum of 129 to 256 columns gains where they were written a moment ago (32768 x 192 from the
+// caches 5.4 -> 3.8 us) and loses where they come from memory (6.3 -> 6.4; 16384 x 256 5.0 -> 5.3).
 static inline bool rows_one_narrow(int h, int w) {
-  return w <= 128 || (w <= 256 && (long long)w * h <= (1 << 20)) || (long long)w * h <= (1 << 18);
+  return w <= 128 || (w <= 256 && (long long)w * h < (1 << 24)) || (long long)w * h <= (1 << 18);
 }
 
 template <int OP>
@@ -872,14 +874,10 @@ static int rows_reduce_one(const float* M, int ld, int h, int w, const float* x,
     hipLaunchKernelGGL((k_rows_one<OP, 4, 4, false>), grid, dim3(256), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
   else if (splits == 1 ? rows_one_narrow(h, w) : (long long)w * h <= (1 << 18))
     hipLaunchKernelGGL((k_rows_one<OP, 4, 8, false>), grid, dim3(256), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
-  // Taller ones of 129 to 256 columns on 512 lanes, which take all columns in one trip (us from memory, 256 lanes / 1024 /
-  // 512: 16384 x 160 4.4 / 4.0 / 3.9, 16384 x 256 5.3 / 5.0 / 5.0; from the caches, where these were written a moment
-  // ago: 32768 x 192 3.7 / 4.4 / 3.4, 32768 x 256 3.9 / 5.4 / 3.7, from memory 7.9 / 7.6 / 8.2).  From 2^24 elements on
-  // they are streams (65536 x 256 14.1 / 13.2 / 12.8, 131072 x 192 21.7 / 20.5 / 18.4).
-  else if (splits == 1 && w <= 256 && (long long)w * h >= (1 << 24))
-    hipLaunchKernelGGL((k_rows_one<OP, 8, 8, true>), grid, dim3(512), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
+  // Larger ones of 129 to 256 columns are streams, all columns in one trip (from memory, us, 256 lanes / 1024 / 512: 65536 x
+  // 256 14.1 / 13.2 / 12.8, 131072 x 129 15.3 / 15.4 / 12.8, 131072 x 192 21.6 / 20.3 / 18.3).
   else if (splits == 1 && w <= 256)
-    hipLaunchKernelGGL((k_rows_one<OP, 8, 8, false>), grid, dim3(512), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
+    hipLaunchKernelGGL((k_rows_one<OP, 8, 8, true>), grid, dim3(512), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
   else if (stream)
     hipLaunchKernelGGL((k_rows_one<OP, 16, 8, true>), grid, dim3(1024), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
   else
