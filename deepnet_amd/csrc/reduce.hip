@@ -860,6 +860,10 @@ static inline bool rows_one_narrow(int h, int w) {
   return w <= 128 || (w <= 256 && (long long)w * h < (1 << 24)) || (long long)w * h <= (1 << 18);
 }
 
+static inline bool rows_aligned(const float* M, int ld, int h) {
+  return dn_aligned16(M) && (ld % 4 == 0) && (h % 4 == 0);
+}
+
 template <int OP>
 static int rows_reduce_one(const float* M, int ld, int h, int w, const float* x, float* y, float alpha, float beta,
                            const RowsWorkspace& ws) {
@@ -869,14 +873,16 @@ static int rows_reduce_one(const float* M, int ld, int h, int w, const float* x,
   const int cps = (w + splits - 1) / splits;
   splits = (w + cps - 1) / cps;
   dim3 grid(bx, splits);
-  const bool stream = (long long)w * h >= DN_STREAM_MIN_ELEMS;
+  // (runs at any other alignment share cache lines with their neighbours, which loads that leave no copy fetch twice:
+  // 19407 x 2144 from memory 40.2 -> 36.9 us, 30001 x 1000 28.4 -> 27.0)
+  const bool stream = (long long)w * h >= DN_STREAM_MIN_ELEMS && rows_aligned(M, ld, h);
   if (cps <= 64)
     hipLaunchKernelGGL((k_rows_one<OP, 4, 4, false>), grid, dim3(256), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
   else if (splits == 1 ? rows_one_narrow(h, w) : (long long)w * h <= (1 << 18))
     hipLaunchKernelGGL((k_rows_one<OP, 4, 8, false>), grid, dim3(256), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
   // Larger ones of 129 to 256 columns are streams, all columns in one trip (from memory, us, 256 lanes / 1024 / 512: 65536 x
   // 256 14.1 / 13.2 / 12.8, 131072 x 129 15.3 / 15.4 / 12.8, 131072 x 192 21.6 / 20.3 / 18.3).
-  else if (splits == 1 && w <= 256)
+  else if (stream && splits == 1 && w <= 256)
     hipLaunchKernelGGL((k_rows_one<OP, 8, 8, true>), grid, dim3(512), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
   else if (stream)
     hipLaunchKernelGGL((k_rows_one<OP, 16, 8, true>), grid, dim3(1024), 0, dn_stream(), M, ld, h, w, cps, x, y, ws.partial, ws.counters, alpha, beta);
@@ -885,10 +891,6 @@ static int rows_reduce_one(const float* M, int ld, int h, int w, const float* x,
   const int status = dn_launch_status();
   if (status && splits > 1) rezero_counters(ws.counters, bx);
   return status;
-}
-
-static inline bool rows_aligned(const float* M, int ld, int h) {
-  return dn_aligned16(M) && (ld % 4 == 0) && (h % 4 == 0);
 }
 
 // The library's own workspace: arrival counters for 16384 row blocks (matrices with more rows
