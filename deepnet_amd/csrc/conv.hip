@@ -2519,8 +2519,7 @@ struct PaddedBatch {
   cudamat m[3];
   int N, Np;
   bool on;
-  // to: the batch to round up to; 0 for padded_batch's, 128 f images on (locally connected
-  // layers, whose matrix-core kernels need that)
+  // to: the batch to round up to, 0 for padded_batch()'s
   PaddedBatch(cudamat* a, cudamat* b, cudamat* c, int to = 0)
       : N(a->size[0]), Np(to), on(false) {
     cudamat* src[3] = {a, b, c};

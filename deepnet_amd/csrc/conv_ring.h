@@ -101,14 +101,15 @@ struct ConvRingOperand : RingTile<ROWS, BK, ((KIND >= 2 && KIND <= 4) || KIND ==
 // instructions per group and stage.  Tiles of one module or pixel (SINGLE: locally connected layers, batches that are no
 // multiple of 4 or that the tile divides) need no masks and leave out the taps beyond the edge.
 // convOutp splits its reduction over workgroups and is summed by k_conv_outp_finish*.
-// Measured, us Up / Down / Outp, before -> now (with the copies and sums):
-//   64 -> 64 colours 5 x 5, 13 x 13, batch 100      72 / 63 / 66 -> 49 / 48 / 39      (22 each at 157 TFLOP/s)
-//   64 -> 64 colours 3 x 3, 17 x 17, batch 100      69 / 58 / 55 -> 25 / 26 / 29      (14)
-//   local 64 -> 64 colours 3 x 3, 8 x 8, batch 128  20 / 19 / 25 -> 10 / 10 / 14      (4)
-//   local 48 -> 64 colours 3 x 3, 14 x 14, 100      38 / 37 / 4570 -> 20 / 28 / 25    (7)
-//   96 -> 256 colours 5 x 5, 2 groups, 27 x 27, 128 Up 532 -> 492 (9 % of its taps are padding), Outp 539 -> 467; Down
-//   467 on k_conv_mfma (48 columns)
-// The MFMAs are busy for 81 to 83 % of the time there; without the masks a stage takes as long as with them.
+// Measured, us Up / Down / Outp, operands from memory, before -> now (with the copies and sums):
+//   64 -> 64 colours 5 x 5, 13 x 13, batch 100      70 / 62 / 65 -> 46 / 45 / 39      (22 each at 157 TFLOP/s)
+//   64 -> 64 colours 3 x 3, 17 x 17, batch 100      69 / 57 / 55 -> 27 / 27 / 32      (14)
+//   local 64 -> 64 colours 3 x 3, 8 x 8, batch 128  21 / 20 / 26 -> 11 / 10 / 14      (4)
+//   local 48 -> 64 colours 3 x 3, 14 x 14, 100      39 / 37 / 4630 -> 21 / 31 / 27    (7)
+//   96 -> 256 colours 5 x 5, 2 groups, 27 x 27, 128 Up 500 -> 412 (9 % of its taps are padding), Outp 532 -> 446; Down
+//   449 on k_conv_mfma (48 columns)
+// The MFMAs are busy for 81 (Up) and 83 % (Outp) of the time of the last layer, without bank conflicts; without the masks a
+// stage takes as long as with them.
 template <int MODE, bool SINGLE, int TB, int BM, int BN, int BK>
 __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
   constexpr int PER = MODE == CONV_UP ? 1 : 4;

@@ -40,6 +40,8 @@ static const struct { int bm, bn, bk; double stage, tile; } g_conv_ring_cfgs[] =
     {32, 32, 64, 0.322, 1.0}, {32, 16, 128, 0.372, 1.2}, {16, 32, 128, 0.372, 1.17}};
 // What a workgroup's LDS holds besides the two stages of its tile, which take 36 to 57 KB.  Two workgroups share a CU while
 // they take half of its 160 KB each; with a full table convUp on 32 x 16 and 16 x 32 tiles takes 82 KB and is alone.
+// The table also bounds the reduction of a convUp, with 8 bytes a term: 3328 terms on tiles over several modules, 3104 to
+// 2432 on those of one.  Longer ones (7 x 7 filters on 68 colours or more) stay on the other kernels.
 #define RING_TABLE_BYTES 26624
 #define RING_CU_LDS (160 << 10)
 

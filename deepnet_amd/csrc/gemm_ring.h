@@ -3,11 +3,11 @@
 #include "ring_tile.h"
 #include "gemm_ring_plan.h"
 
-// Stage t of an operand as this lane's 16-byte groups; a stage behind the last one is an out-of-range offset, which the
-// buffer hardware answers with zeros without going to memory (every trip of the loop issues the same requests, so
-// the compiler can count them).  The scalar offset takes no part in the range check, so such a stage has a buffer of no
-// bytes instead; a bit in the lanes' offsets is a vector instruction per request (dense 1001 x 1500 x 300, three
-// products: 46.4 against 49.0 us).
+// Stage t of an operand as this lane's 16-byte groups.  Every trip of the loop issues the same requests, so that the
+// compiler can count them; those of a stage behind the last one go to a buffer of no bytes, which answers with zeros
+// and does not go to memory.  An offset beyond the buffer would do as well, the lanes' or the scalar one (both take part in
+// the range check: measured on buffers inside a larger allocation, loads and stores); a bit in the lanes' offsets is
+// a vector instruction per request (dense 1001 x 1500 x 300, three products: 46.4 against 49.0 us).
 template <int ROWS, int BK, bool KC>
 struct RingOperand : RingTile<ROWS, BK, KC> {
   using Tile = RingTile<ROWS, BK, KC>;
@@ -54,14 +54,18 @@ struct RingOperand : RingTile<ROWS, BK, KC> {
 // for the order of terms that `frag` reads (pitch 4 mod 8).
 // Tiles are numbered so that each XCD gets a contiguous run of them, along the shorter side first (shared panels
 // meet in its L2).
-// Measured (us, before -> now; before: the best of the other kernels), first operand transposed / neither / second:
-//   1500 x 300 x 1001   22.1 -> 13.6  24.1 -> 13.6  26.0 -> 13.6      64 x 32 tiles (floor at 157 TFLOP/s: 5.7)
-//   2001 x 1003 x 250   16.1 -> 13.9  20.3 -> 14.5  20.3 -> 14.6      64 x 64
-//   1024 x 100 x 2304   16.1 -> 9.3   14.2 -> 10.0  14.9 -> 11.2      32 x 16
-//   814 x 263 x 1038    11.1 -> 8.0   13.6 -> 8.5   14.9 -> 8.7       32 x 32
-//   1000 x 1000 x 1000  26.9 -> 21.3  23.5 -> 19.9  23.8 -> 20.2      64 x 64
+// Measured (us, operands from memory, before -> now; before: the best of the other kernels), first operand transposed /
+// neither / second:
+//   1500 x 300 x 1001   23.3 -> 15.7  24.5 -> 16.5  27.0 -> 17.1      32 x 32 tiles (floor at 157 TFLOP/s: 5.7)
+//   2001 x 1003 x 250   17.4 -> 17.0  20.5 -> 17.1  21.6 -> 17.0      64 x 64
+//   1024 x 100 x 2304   17.2 -> 10.8  16.6 -> 13.3  17.8 -> 15.7      32 x 16
+//   814 x 263 x 1038    11.7 -> 8.7   13.7 -> 9.0   15.2 -> 9.4       32 x 32
+//   1000 x 1000 x 1000  26.9 -> 21.2  27.0 -> 21.4  26.7 -> 21.6      64 x 64
+//   2074 x 464 x 912    34.4 -> 22.0                                  64 x 32
+//   726 x 2749 x 1091                 81.1 -> 51.6                    32 x 64
 // What is left above the MFMAs' time at 64 x 64 is 4.3 us: launch 2.4, the first trip to memory, the sum over the
-// wavefronts and the stores.  The smaller tiles run at what the L2s give (20 TB/s over the chip).
+// wavefronts and the stores.  The smaller tiles run at what the L2s give: a stage of a 32 x 16 tile is 24.6 KB in 0.31 us on
+// every CU, 20 TB/s over the chip.
 struct RingArgs {
   const float* A; const float* B;
   float* C;
