@@ -21,42 +21,46 @@ def _zeros(shape):
 
 
 class LossRecord(types.SimpleNamespace):
-    """A record whose fields may still be on their way from the GPU.  Whoever looks at it (reads, assigns, lists or prints
-    a field) waits for them first, so that nobody sees the value that a field had before."""
+    """A loss record.  While fields of it are on their way from the GPU it is a _LateRecord: whoever looks at it (reads,
+    assigns, lists or prints a field) waits for them first, so that nobody sees the value that a field had before."""
 
-    __slots__ = ('_late',)          # field -> function that waits for its value; not set: nothing on its way
+    __slots__ = ('_late',)          # field -> function that waits for its value
 
-    def late(self, field, value):
-        try:
-            self._late[field] = value
-        except AttributeError:
-            self._late = {field: value}
 
-    def settle(self):
-        """Waits for the fields that are on their way."""
-        try:
-            late = self._late
-        except AttributeError:
-            return
-        while late:
-            field = next(iter(late))
-            super(LossRecord, self).__setattr__(field, late[field]())
-            del late[field]
+class _LateRecord(LossRecord):
+    __slots__ = ()
 
     def __getattribute__(self, name):
-        get = super(LossRecord, self).__getattribute__
-        if name not in ('_late', 'late', 'settle'):
-            get('settle')()
-        return get(name)
+        settle(self)
+        return getattr(self, name)
 
     def __setattr__(self, name, value):
-        if name != '_late':
-            self.settle()
-        super(LossRecord, self).__setattr__(name, value)
+        settle(self)
+        setattr(self, name, value)
 
     def __repr__(self):
-        self.settle()
-        return super(LossRecord, self).__repr__()
+        settle(self)
+        return repr(self)
+
+
+_waiting = LossRecord._late.__get__            # (past _LateRecord's own access)
+
+
+def late(record, field, value):
+    """``record.field`` becomes ``value()``, when somebody asks for it."""
+    if type(record) is _LateRecord:
+        _waiting(record)[field] = value
+    else:
+        record._late = {field: value}
+        record.__class__ = _LateRecord
+
+
+def settle(record):
+    """Waits for the fields that are on their way."""
+    if type(record) is _LateRecord:
+        values = {field: value() for field, value in _waiting(record).items()}     # (all of them, or it stays as it is)
+        object.__setattr__(record, '__class__', LossRecord)
+        vars(record).update(values)
 
 
 def _metrics(count):
@@ -201,7 +205,7 @@ class Layer(Parameter):
             setattr(perf, field, mat.euclid_norm() ** 2 if norm else mat.sum())
         else:
             value = mat.read_later(norm)
-            perf.late(field, (lambda: value() ** 2) if norm else value)
+            late(perf, field, (lambda: value() ** 2) if norm else value)
             self.pending.append(perf)
 
     def _squared_loss(self, perf, get_deriv, acc_deriv):

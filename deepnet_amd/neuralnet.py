@@ -17,6 +17,7 @@ import numpy as np
 from .choose_matrix_library import cm
 from .convolutions import ConvolveUp, AccumulateConvDeriv, ConvOuter, AddConvolveUp, ConvEdge
 from . import parameter as P
+from .layer import settle
 from .parameter import Parameter, Hyperparams
 
 
@@ -256,7 +257,7 @@ class NeuralNet(object):
             for layer in outputs:
                 layer.pending = None
         for perf in pending:
-            perf.settle()
+            settle(perf)
         return losses
 
     def EvaluateOneBatch(self):

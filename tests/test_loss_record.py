@@ -18,13 +18,23 @@ def Accumulate(stats, losses):
     return Accumulate(stats, losses)
 
 
+def late(*args):
+    from deepnet_amd.layer import late
+    late(*args)
+
+
+def settle(record):
+    from deepnet_amd.layer import settle
+    settle(record)
+
+
 def _late(asked):
     perf = _metrics(10)
 
     def value():
         asked.append(1)
         return 2.5
-    perf.late('error', value)
+    late(perf, 'error', value)
     return perf
 
 
@@ -39,10 +49,20 @@ def test_whoever_looks_at_a_record_gets_the_value(look):
     assert vars(perf) == dict(count=10, cross_entropy=0.0, correct_preds=0.0, error=2.5)
 
 
+def test_several_fields_may_be_on_their_way():
+    perf = _late([])
+    late(perf, 'cross_entropy', lambda: 1.5)
+    assert (perf.cross_entropy, perf.error, perf.count) == (1.5, 2.5, 10)
+    late(perf, 'error', lambda: 3.5)
+    settle(perf)
+    settle(perf)
+    assert vars(perf) == dict(count=10, cross_entropy=1.5, correct_preds=0.0, error=3.5)
+
+
 def test_an_assigned_field_keeps_what_was_assigned():
     perf = _late([])
     perf.error = 7.0
-    perf.settle()
+    settle(perf)
     assert perf.error == 7.0
     perf = _late([])
     perf.error *= 2
@@ -54,7 +74,7 @@ def test_a_value_that_cannot_be_had_is_not_zero():
 
     def value():
         raise RuntimeError('lost')
-    perf.late('error', value)
+    late(perf, 'error', value)
     for _ in range(2):
         with pytest.raises(RuntimeError):
             perf.error
