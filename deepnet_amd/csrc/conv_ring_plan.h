@@ -112,8 +112,12 @@ static inline double conv_other_us(const Args& a, int mode, long long rows, bool
   const int Fp = padded_filters(a.F, a.G), Fg = Fp / a.G, K = a.Cg * a.kk2;
   const bool copy_n = Np != a.N, copy_f = Fp != a.F;
   const bool aligned = (copy_n || maps16) && filters16;
-  if (Np % 16 != 0 || Fg % 16 != 0 || !aligned || (a.local && (copy_f || (mode != CONV_OUTP && Np % 128 != 0))))
-    return 5. + 2e-6 * a.N * rows * a.F * K;                            // (1 TFLOP/s)
+  if (Np % 16 != 0 || Fg % 16 != 0 || !aligned || (a.local && (copy_f || (mode != CONV_OUTP && Np % 128 != 0)))) {
+    // one lane per output: 1 TFLOP/s, convUp 3, but a chain of K loads (2 groups of 2 -> 24 colours 3 x 3, 38 x 38, batch 128:
+    // 101 us against 134 on ring tiles)
+    const double all = 2e-6 * a.N * rows * a.F * K;
+    return 5. + (mode == CONV_UP && !a.local ? (all / 3. > 0.25 * K ? all / 3. : 0.25 * K) : all);
+  }
   auto up = [](long long v, int b) { return (double)((v + b - 1) / b * b); };
   const double maps = 1e-9 * 8. * Np * ((double)a.M * a.F + (double)a.HH * a.C), hid = 1e-9 * 8. * Np * a.M * Fp;   // GB of a copy
   double flops, rate, copy = 5e-3;                                       // GFLOP, TFLOP/s, GB per us
