@@ -44,6 +44,11 @@ static inline RingPlan gemm_ring_plan(int M, int N, int K, size_t a_bytes, size_
   // against 11.6).
   const int thin = M < N ? M : N;
   if (thin > 16 && thin < 32 && K <= 512 && tiles(32) <= cus && ring.us >= 3.8 + 5.0 * K / 1024.0) return none;
+  // Of 33 to 63 the 64-wide tile does not fit and the second 32-wide one mostly repeats the first.  From one and a half
+  // 64 x 64 tiles per CU on the slab loop, whose tiles may hang over, is at least as fast (operands from memory, us, ring ->
+  // slab loop: 57 x 25160 x 149 17.2 -> 12.7, 44 x 38103 x 167 21.4 -> 17.6, 26761 x 44 x 168 17.9 -> 15.4, 27552 x 55 x 239
+  // 20.9 -> 21.2; fewer, 19399 x 49 x 252, 17.1 against 21.3).
+  if (thin > 32 && thin < 64 && 20 * tiles(64) >= 29ll * cus) return none;
   if (tiles(128) >= cus && 4 * rounds(tiles(128)) <= rounds(tiles(64))) return none;
   return ring;
 }

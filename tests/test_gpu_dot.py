@@ -502,7 +502,7 @@ RING_SHAPES = [(2001, 1003, 250), (640, 1280, 256), (65, 4095, 129), (1500, 300,
 # products of more than 128 terms that k_gemm_ring does not take (tests/test_ring_plans.py): strips and 32 x 32 blocks over
 # eight wavefronts, 64 x 64 tiles in whole rounds of the CUs, slices of long reductions, 128 x 128 tiles
 OTHER_SHAPES = [(5899, 21, 312), (23, 4407, 250), (4100, 31, 300), (4097, 17, 129), (2040, 2047, 333), (2048, 2048, 300),
-                (1023, 1041, 2100), (130, 129, 9000), (2041, 2046, 1060)]
+                (1023, 1041, 2100), (130, 129, 9000), (2041, 2046, 1060), (57, 25161, 149)]
 
 
 @pytest.mark.parametrize("m,n,k", RING_SHAPES + OTHER_SHAPES)

@@ -101,3 +101,10 @@ def test_the_layers_of_the_other_kernels_are_not_on_ring_tiles(plans):
         for layer, passes in layers.items():
             for name in passes.split():
                 assert conv_tile(plans, dict(up=UP, down=DOWN, outp=OUTP)[name], *layer, local=local) is None, (layer, name)
+
+
+def test_long_strips_of_33_to_63_are_not_on_ring_tiles(plans):
+    for m, n, k in ((57, 25160, 149), (44, 38103, 167), (26761, 44, 168)):
+        assert gemm_tile(plans, m, n, k) is None
+    for m, n, k in ((19399, 49, 252), (57, 17393, 163), (26761, 64, 168), (32, 26761, 168)):
+        assert gemm_tile(plans, m, n, k) is not None
