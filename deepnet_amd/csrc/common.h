@@ -55,7 +55,7 @@ int dn_rng_bernoulli_keep(rnd_struct* rnd, float* uni, float* probs, size_t n);
 struct DnRowSumJob { const float* M; float* y; int h, w; float alpha, beta; int scalar; };   // scalar: dn_row_sum_job_kind() == 2
 bool dn_defer_row_sum(const float* M, float* y, int h, int w, float alpha, float beta, int* err);
 bool dn_row_sum_job_ok(const float* M, int h, int w);     // kind 1
-int dn_row_sum_job_kind(const float* M, int h, int w);    // 0: not as a job, 1: 16-byte loads of four rows, 2: fewer than four rows
+int dn_row_sum_job_kind(const float* M, int h, int w);    // 0: not as a job, 1: 16-byte loads of four rows, 2: one row per lane
 int dn_row_sum_jobs(const DnRowSumJob* jobs, int n);
 int dn_gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, const float* A, int lda, const float* B, int ldb,
             float beta, float* C, int ldc);

@@ -971,11 +971,12 @@ __global__ void __launch_bounds__(256) k_rows_sum_jobs(RowSumJobs J) { rows_sum_
 bool dn_row_sum_job_ok(const float* M, int h, int w) {
   return h >= 4 && w > 0 && rows_one_splits(h, w) == 1 && rows_one_narrow(h, w);
 }
-// 1: as above; 2: fewer than four rows, which rows_reduce() gives to k_rows_stage1<false, ROW_SUM, 4, 4, false> with one
-// column slice while there are at most 2^18 elements; 0: neither.
+// 1: as above; 2: what rows_reduce() gives to k_rows_stage1<false, ROW_SUM, 4, 4, false> with one column slice, fewer than
+// four rows or so few rows of so many columns that k_rows_one has too few slices, up to 2^18 elements of any alignment but
+// 16 bytes (two add_sums of 13 x 2367 69 us in one launch, 75 in two); 0: neither.
 int dn_row_sum_job_kind(const float* M, int h, int w) {
   if (dn_row_sum_job_ok(M, h, w)) return 1;
-  if (h <= 0 || w <= 0 || h >= 4) return 0;
+  if (h <= 0 || w <= 0 || rows_aligned(M, h, h) || (h >= 4 && rows_one_splits(h, w) > 0)) return 0;
   return (long long)w * h <= (1 << 18) ? 2 : 0;
 }
 
@@ -1258,7 +1259,8 @@ int max_by_axis(cudamat* mat, cudamat* target, int axis) {
 }
 
 // max_by_axis without any allocation (no counterpart in cudamat.cu; for callers that cannot
-// allocate device memory).  Same kernels and the same results as max_by_axis; the slice
+// allocate device memory).  The same results as max_by_axis, and its kernels but for columns that are not 16-byte
+// aligned or of a height that is no multiple of four (64 rows a workgroup over all columns here); the slice
 // partials and arrival counters of the axis-1 kernel live in this library's fixed workspace
 // instead of the grow-only scratch.  Returns ERROR_UNSUPPORTED when a call would need more
 // than NOALLOC_PARTIAL_FLOATS partials or NOALLOC_COUNTERS row blocks of 64 rows with

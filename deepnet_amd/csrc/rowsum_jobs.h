@@ -57,7 +57,7 @@ __device__ __forceinline__ void rows_sum_jobs_body(const RowSumJobs& J, int bloc
     const int w = job.w;
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     if (job.scalar) {
-      // matrices of fewer than four rows: a lane owns one row, in the order of
+      // fewer than four rows, or few rows of very many columns: a lane owns one row, in the order of
       // k_rows_stage1<false, ROW_SUM, 4, 4, false> with one column slice (wavefront v the columns v, v + 4, ..,
       // four in flight; a column past the end adds a zero)
       const int srow = bx * 64 + lane;

@@ -366,6 +366,24 @@ def test_rows_of_tall_matrices_around_one_trip_of_the_columns(cm, rng, h, w):
     a.free_device_memory()
 
 
+@pytest.mark.parametrize("h,w", [(3, 500), (5, 3303), (13, 2367), (50, 3109), (8, 3000), (13, 700), (250, 230)])
+def test_sums_that_share_a_launch_have_the_bits_of_separate_ones(cm, rng, h, w):
+    x = [cm.CUDAMatrix(_rand(rng, (h, w))) for _ in range(2)]
+    got = []
+    for defer in (True, False):
+        cm.set_deferred_epilogues(defer)
+        try:
+            y = cm.CUDAMatrix(np.ones((h, 1), dtype=np.float32))
+            for i in range(5):
+                y.add_sums(x[i % 2], axis=1, mult=0.5 - i)
+            got.append(y.asarray().copy())
+        finally:
+            cm.set_deferred_epilogues(True)
+    assert np.array_equal(*got)
+    want = 1.0 + sum((0.5 - i) * x[i % 2].numpy_array.astype(np.float64).sum(axis=1, keepdims=True) for i in range(5))
+    assert np.allclose(got[0], want, rtol=1e-4, atol=1e-2)
+
+
 def test_scalars_that_are_read_later(cm, rng):
     """read_later() is the value at the time of the call, with the bits of sum() and euclid_norm(), in any order of reading;
     a value that 63 others have followed is refused."""
