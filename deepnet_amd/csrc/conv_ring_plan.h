@@ -107,7 +107,7 @@ static inline bool ring_ok(const Args& a, long long bank_cols) {
 // and the copies of a batch or filter count that they do not take; or on the one-lane-per-output kernels.
 // rows: positions of the output per image (Up: modules, Down: pixels); maps16, filters16: 16-byte aligned.
 template <class Args>
-static inline double conv_other_us(const Args& a, int mode, long long rows, bool maps16, bool filters16) {
+static inline double conv_other_us(const Args& a, int mode, long long rows, bool maps16, bool filters16, int cus) {
   const int Np = !a.local ? padded_batch(a.N) : mode != CONV_OUTP ? local_batch(a.N) : a.N;
   const int Fp = padded_filters(a.F, a.G), Fg = Fp / a.G, K = a.Cg * a.kk2;
   const bool copy_n = Np != a.N, copy_f = Fp != a.F;
@@ -131,8 +131,10 @@ static inline double conv_other_us(const Args& a, int mode, long long rows, bool
     const double patch = 1e-9 * 8. * Np * a.M * a.Cg * a.kk2 * a.G;       // GB
     return 9. + (2e-9 * Np * a.M * Fp * K / 105. + patch / 5.) * 1e3 + (copy_n ? 5. + maps / copy : 0.) + (copy_f ? 5. + hid / copy : 0.);
   } else if (mode == CONV_DOWN) {
-    flops = 2e-9 * Np * rows * up(a.Cg, a.Cg > 32 && a.Cg <= 48 ? 16 : 32) * a.G * a.kk2 * Fg;
-    rate = a.local ? 70. : Np % 128 == 0 && a.kk2 * Fg >= 256 && (a.Cg <= 64 || a.Cg > 96) ? 115. : 65.;
+    // (uniform rows: 16-wide blocks for 33 to 48 colours; others: 85 where every CU has two tiles)
+    const bool uniform = a.local || (Np % 128 == 0 && a.kk2 * Fg >= 256 && (a.Cg <= 64 || a.Cg > 96));
+    flops = 2e-9 * Np * rows * up(a.Cg, uniform && a.Cg > 32 && a.Cg <= 48 ? 16 : 32) * a.G * a.kk2 * Fg;
+    rate = a.local ? 70. : uniform ? 115. : a.Cg > 32 && rows * Np * a.G >= 2ll * 128 * cus ? 85. : 65.;
   } else {
     const int BMs = Fg <= 32 ? 32 : Fg <= 64 ? 64 : Fg <= 96 || (Fg > 128 && (Fg + 95) / 96 * 96 < (Fg + 127) / 128 * 128) ? 96 : 128;
     flops = 2e-9 * Np * rows * up(Fg, BMs) * a.G * up(K, K <= 80 && Fg <= 64 ? 16 : 128);
@@ -195,7 +197,7 @@ static inline ConvRingPlan conv_rows_plan(const Args& a, int mode, bool maps16, 
   // (the patch form of few colours does all pixels at once: there the busiest XCD counts, elsewhere the estimates do not
   // differ by as little)
   const double crowd = !up && plan.single && !a.local && a.Cg <= 16 ? ring_crowd(a) : 1.;
-  return plan.cfg < 0 || crowd * plan.us > conv_other_us(a, mode, sites, maps16, filters16) ? conv_no_ring() : plan;
+  return plan.cfg < 0 || crowd * plan.us > conv_other_us(a, mode, sites, maps16, filters16, cus) ? conv_no_ring() : plan;
 }
 
 // Outp of `a`, whose batch the ring takes in whole groups of four images: others are copied with up to three images of zeros.
@@ -209,6 +211,6 @@ static inline ConvRingPlan conv_outp_plan(const Args& a, bool maps16, bool filte
                                            2e-6 * a.chunks * a.F * cols, cus);
   const double maps = 1e-9 * 8. * r.N * ((double)a.M * a.F + (double)a.HH * a.C);
   // (1.12: what a layer's sums over many splits take beyond the plan's estimate)
-  return plan.cfg < 0 || 1.12 * plan.us + (r.N != a.N ? 5. + maps / 5e-3 : 0.) > conv_other_us(a, CONV_OUTP, a.M, maps16, filters16)
+  return plan.cfg < 0 || 1.12 * plan.us + (r.N != a.N ? 5. + maps / 5e-3 : 0.) > conv_other_us(a, CONV_OUTP, a.M, maps16, filters16, cus)
              ? conv_no_ring() : plan;
 }
