@@ -409,12 +409,12 @@ class CUDAMatrix(object):
     def read_later(self, norm=False):
         """sum() of this matrix as it is now (or its euclid_norm()) as a function that waits for the value: the kernel is
         queued, the program goes on.  At most 63 such values may be outstanding."""
-        ticket = ct.c_uint(0)
-        _check(_cudamat.read_later(self.p_mat, int(norm), ct.byref(ticket)))
+        ticket = ct.c_uint(0)                   # (handed over as it is: the signatures make pointers of these)
+        _check(_cudamat.read_later(self.p_mat, int(norm), ticket))
 
         def value():
             err_code = ct.c_int(0)
-            res = _cudamat.read_now(ticket, ct.byref(err_code))
+            res = _cudamat.read_now(ticket, err_code)
             _check(err_code.value)
             return res
         return value

@@ -24,7 +24,7 @@ class LossRecord(types.SimpleNamespace):
     """A loss record.  While fields of it are on their way from the GPU it is a _LateRecord: whoever looks at it (reads,
     assigns, lists or prints a field) waits for them first, so that nobody sees the value that a field had before."""
 
-    __slots__ = ('_late',)          # field -> function that waits for its value
+    __slots__ = ('_late',)          # the fields, and field -> function that waits for its value
 
 
 class _LateRecord(LossRecord):
@@ -43,24 +43,25 @@ class _LateRecord(LossRecord):
         return repr(self)
 
 
-_waiting = LossRecord._late.__get__            # (past _LateRecord's own access)
+_waiting, _set = LossRecord._late.__get__, object.__setattr__            # (past _LateRecord's own access)
 
 
 def late(record, field, value):
     """``record.field`` becomes ``value()``, when somebody asks for it."""
     if type(record) is _LateRecord:
-        _waiting(record)[field] = value
+        _waiting(record)[1][field] = value
     else:
-        record._late = {field: value}
+        record._late = record.__dict__, {field: value}
         record.__class__ = _LateRecord
 
 
 def settle(record):
-    """Waits for the fields that are on their way."""
+    """Waits for the fields that are on their way (all of them, or it stays as it is)."""
     if type(record) is _LateRecord:
-        values = {field: value() for field, value in _waiting(record).items()}     # (all of them, or it stays as it is)
-        object.__setattr__(record, '__class__', LossRecord)
-        vars(record).update(values)
+        fields, waiting = _waiting(record)
+        for field, value in waiting.items():
+            fields[field] = value()
+        _set(record, '__class__', LossRecord)
 
 
 def _metrics(count):

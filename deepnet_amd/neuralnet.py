@@ -247,14 +247,13 @@ class NeuralNet(object):
         # The losses are read when the whole step has been queued: waiting for them in the middle leaves the GPU idle
         # while the rest is queued (784-1024-1024-10, batch 128: 142 -> 129 us; deepnet's convnet at batch 100: 384 -> 340).
         pending = []
-        outputs = [layer for layer in self.layer if layer.is_output]
-        for layer in outputs:
+        for layer in self.output_datalayer:
             layer.pending = pending
         try:
             losses = self.ForwardPropagate(train=True)
             losses.extend(self.BackwardPropagate(step))
         finally:
-            for layer in outputs:
+            for layer in self.output_datalayer:
                 layer.pending = None
         for perf in pending:
             settle(perf)
