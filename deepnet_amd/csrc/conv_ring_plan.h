@@ -93,8 +93,9 @@ static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows,
 }
 
 // Every pass first asks what the fastest ring tile would take (conv_ring_plan) and what the other kernels would
-// (conv_other_us), and runs on the ring when that is less.  Both estimates were held against 360 passes over
-// random layers: the pass so chosen was 1.65 times as fast as before on average, none more than 9 us slower.
+// (conv_other_us), and runs on the ring when that is less.  Both estimates are held against passes over random layers: of
+// 1260, those so chosen were 1.4 (any), 2.0 (at most 24 images) and 4 times (two groups; locally connected) as fast on
+// average as before the ring, and four more than 5 % slower, 42 -> 44 us the longest of them.
 
 // What all three passes need: offsets of 31 bits, masks of RING_MAX_SIDE filter rows.
 template <class Args>
@@ -137,7 +138,8 @@ static inline double conv_other_us(const Args& a, int mode, long long rows, bool
     rate = a.local ? 70. : uniform ? 115. : a.Cg > 32 && rows * Np * a.G >= 2ll * 128 * cus ? 85. : 65.;
   } else {
     const int BMs = Fg <= 32 ? 32 : Fg <= 64 ? 64 : Fg <= 96 || (Fg > 128 && (Fg + 95) / 96 * 96 < (Fg + 127) / 128 * 128) ? 96 : 128;
-    flops = 2e-9 * Np * rows * up(Fg, BMs) * a.G * up(K, K <= 80 && Fg <= 64 ? 16 : 128);
+    const bool regs = K <= 80 && Fg <= 64;                               // 16 x 16 blocks in registers
+    flops = 2e-9 * Np * rows * up(Fg, regs && !a.local && Fg > 32 ? 16 : BMs) * a.G * up(K, regs ? 16 : 128);
     rate = a.local ? 45. : 110.;
   }
   // (a long reduction may be split, and is summed by another launch)

@@ -83,7 +83,8 @@ def test_strips_that_a_16_wide_tile_halves_stay_on_32_wide_blocks(plans, m, n, k
     assert gemm_tile(plans, m, n, 4 * k + 400) is not None
 
 
-@pytest.mark.parametrize("mode,layer", [(DOWN, (100, 16, 30, 208, 7, 1, 0)), (DOWN, (80, 16, 19, 172, 5, 1, 0)), (UP, (100, 3, 64, 48, 7, 1, 0)),
+@pytest.mark.parametrize("mode,layer", [(OUTP, (160, 1, 97, 48, 7, 2, 0)), (OUTP, (128, 1, 38, 48, 7, 1, 0)), (DOWN, (100, 16, 30, 208, 7, 1, 0)),
+                                        (DOWN, (80, 16, 19, 172, 5, 1, 0)), (UP, (100, 3, 64, 48, 7, 1, 0)),
                                         (UP, (100, 3, 161, 48, 7, 2, 0)), (UP, (128, 4, 38, 48, 3, 1, 0, 2)), (UP, (100, 1, 90, 32, 7, 1, 3)), (UP, (234, 1, 79, 40, 7, 1, 3))])
 def test_layers_of_few_colours_that_other_kernels_are_faster_on(plans, mode, layer):
     assert conv_tile(plans, mode, *layer) is None
