@@ -22,7 +22,8 @@ def _zeros(shape):
 
 class LossRecord(types.SimpleNamespace):
     """A loss record.  While fields of it are on their way from the GPU it is a _LateRecord: whoever looks at it (reads,
-    assigns, lists or prints a field) waits for them first, so that nobody sees the value that a field had before."""
+    assigns, deletes, lists or prints a field, or compares records) waits for them first, so that nobody sees the value that
+    a field had before."""
 
     __slots__ = ('_late',)          # the fields, and field -> function that waits for its value
 
@@ -37,6 +38,21 @@ class _LateRecord(LossRecord):
     def __setattr__(self, name, value):
         settle(self)
         setattr(self, name, value)
+
+    def __delattr__(self, name):
+        settle(self)
+        delattr(self, name)
+
+    def __eq__(self, other):
+        settle(self)
+        if isinstance(other, LossRecord):
+            settle(other)
+        return self == other
+
+    def __ne__(self, other):
+        return not self == other
+
+    __hash__ = None
 
     def __repr__(self):
         settle(self)

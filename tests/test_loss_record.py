@@ -49,6 +49,22 @@ def test_whoever_looks_at_a_record_gets_the_value(look):
     assert vars(perf) == dict(count=10, cross_entropy=0.0, correct_preds=0.0, error=2.5)
 
 
+def test_records_are_compared_by_the_values_on_their_way():
+    same = _metrics(10)
+    same.error = 2.5
+    assert _late([]) == same and same == _late([]) and _late([]) == _late([])
+    assert _late([]) != _metrics(10) and _metrics(10) != _late([])
+    assert _late([]) == types.SimpleNamespace(**vars(same)) and types.SimpleNamespace(**vars(same)) == _late([])
+    assert _late([]) != 3
+
+
+def test_a_deleted_field_stays_deleted():
+    perf = _late([])
+    del perf.error
+    settle(perf)
+    assert not hasattr(perf, 'error')
+
+
 def test_several_fields_may_be_on_their_way():
     perf = _late([])
     late(perf, 'cross_entropy', lambda: 1.5)
