@@ -1223,7 +1223,7 @@ static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, co
   }
   // Reductions of more than 128 terms: k_gemm_ring, unless another kernel is expected to be faster (gemm_ring_plan).
   const size_t a_bytes = (size_t)lda * (a_kc ? M : K) * sizeof(float), b_bytes = (size_t)ldb * (b_kc ? N : K) * sizeof(float);
-  const RingPlan ring = K > BOX_K ? gemm_ring_plan(M, N, K, a_bytes, b_bytes, cus) : RingPlan{-1, 0.};
+  const RingPlan ring = K > BOX_K ? gemm_ring_plan(M, N, K, a_bytes, b_bytes, cus, a_vec && b_vec && !(a_kc && b_kc)) : RingPlan{-1, 0.};
   if (ring.cfg >= 0) {
     const RingArgs g = {A, B, C, (unsigned)a_bytes, (unsigned)b_bytes, lda, ldb, ldc, M, N, K, 0, 0, alpha, beta};
     ring_launch(ring.cfg, a_kc, b_kc, g, epi);

@@ -28,7 +28,9 @@ static inline RingPlan ring_plan(int M, int N, int K, size_t a_bytes, size_t b_b
 // 300 x 300 x 300 4.0 against 4.5; two rounds of 500 terms, 784 x 100 x 500, 5.5 against 5.1); slices of K with a second
 // kernel 12 us + 1.5 us per 1e8 multiply-adds (few outputs over very long reductions); 128 x 128 tiles reach the same rate
 // per output as 64 x 64 ones here (2000 x 2000 x 2000 130 us both) and win where their count fills the CUs as evenly.
-static inline RingPlan gemm_ring_plan(int M, int N, int K, size_t a_bytes, size_t b_bytes, int cus) {
+// vec: the columns of both operands start at 16-byte boundaries, and one of them or both have the product's rows or columns
+// along theirs.  The other kernels read those in 16-byte groups (the ring any), and short reductions are faster there.
+static inline RingPlan gemm_ring_plan(int M, int N, int K, size_t a_bytes, size_t b_bytes, int cus, bool vec) {
   const RingPlan none = {-1, 0.}, ring = ring_plan(M, N, K, a_bytes, b_bytes, cus);
   if (ring.cfg < 0) return none;
   auto tiles = [&](int side) { return (long long)((M + side - 1) / side) * ((N + side - 1) / side); };
@@ -49,6 +51,24 @@ static inline RingPlan gemm_ring_plan(int M, int N, int K, size_t a_bytes, size_
   // slab loop: 57 x 25160 x 149 17.2 -> 12.7, 44 x 38103 x 167 21.4 -> 17.6, 26761 x 44 x 168 17.9 -> 15.4, 27552 x 55 x 239
   // 20.9 -> 21.2; fewer, 19399 x 49 x 252, 17.1 against 21.3).
   if (thin > 32 && thin < 64 && 20 * tiles(64) >= 29ll * cus) return none;
+  // So does the second 64-wide tile of 65 to 85, more than two tiles per CU, as long as the reduction is short (23636 x 81 x
+  // 243 25.3 -> 22.0, 17144 x 80 x 135 16.2 -> 14.5; longer ones, 77 x 21204 x 262, 24.9 against 28.8).
+  if (thin > 64 && thin < 86 && tiles(64) > 2ll * cus && K <= 256) return none;
+  // Strips of 17 to 31: one 64 x 64 tile per CU takes 5.9 us + 1.15 us per 100 terms, two 6.5 us + 3 us (12800 x 18 x 288
+  // 11.2 -> 8.9, 15488 x 25 x 160 9.9 -> 7.9, 24200 x 25 x 144 13.7 -> 10.8; 20000 x 25 x 256 11.7 against 14.2).
+  if (thin > 16 && thin < 32 && K <= 400 && 2 * tiles(64) <= 3ll * cus &&
+      ring.us >= (tiles(64) <= cus ? 5.9 + 0.0115 * K : 6.5 + 0.03 * K)) return none;
+  if (vec) {
+    // More than two 64 x 64 tiles per CU: five workgroups of the slab loop share one and hide each other's waits (16384 x 147 x
+    // 160 20.6 -> 16.0, 12800 x 200 x 208 25.7 -> 20.6, 10368 x 196 x 240 23.7 -> 19.4, 128 x 18880 x 240 24.3 -> 20.4;
+    // of 546 the geometric means are, on the ring / there, 1.08 up to 256 terms, 1.01 up to 400, and 0.95 from 513 on).
+    if (ring.cfg < 3 && tiles(64) > 2ll * cus && K <= (ring.cfg == 0 ? 400 : 256)) return none;
+    // Strips of 33 to 63 from half a 64 x 64 tile per CU on (18432 x 49 x 208 15.7 -> 13.5, 10000 x 50 x 208 11.0 -> 9.3).
+    if (thin > 32 && thin < 64 && K <= 256 && 2 * tiles(64) > cus) return none;
+    // One round of 32 x 32 blocks of four stages at most: the blocks over eight wavefronts take the whole reduction at once
+    // (1648 x 96 x 224 5.4 -> 4.6, 176 x 912 x 256 5.4 -> 4.8).
+    if (ring.cfg == 3 && tiles(32) <= cus && K > 192 && K <= 256) return none;
+  }
   if (tiles(128) >= cus && 4 * rounds(tiles(128)) <= rounds(tiles(64))) return none;
   return ring;
 }

@@ -10,9 +10,9 @@ struct Sizes { int N, C, Cg, H, HH, F, Fg, k, kk2, Mx, M, s, pad0, G, local, m_c
 
 extern "C" {
 
-// Tile number (the order of g_ring_cfgs) of an M x N x K product of whole matrices; -1: not on k_gemm_ring.
-int gemm_tile(int M, int N, int K, int cus) {
-  return K > 128 ? gemm_ring_plan(M, N, K, (size_t)M * K * 4, (size_t)N * K * 4, cus).cfg : -1;
+// Tile number (the order of g_ring_cfgs) of an M x N x K product of whole matrices; -1: not on k_gemm_ring.  vec: as there.
+int gemm_tile(int M, int N, int K, int cus, int vec) {
+  return K > 128 ? gemm_ring_plan(M, N, K, (size_t)M * K * 4, (size_t)N * K * 4, cus, vec != 0).cfg : -1;
 }
 
 // out = {tile number or -1, one module or pixel per tile, splits, LDS bytes of a workgroup, us}

@@ -502,10 +502,14 @@ RING_SHAPES = [(2001, 1003, 250), (640, 1280, 256), (65, 4095, 129), (1500, 300,
 # products of more than 128 terms that k_gemm_ring does not take (tests/test_ring_plans.py): strips and 32 x 32 blocks over
 # eight wavefronts, 64 x 64 tiles in whole rounds of the CUs, slices of long reductions, 128 x 128 tiles
 OTHER_SHAPES = [(5899, 21, 312), (23, 4407, 250), (4100, 31, 300), (4097, 17, 129), (2040, 2047, 333), (2048, 2048, 300),
-                (1023, 1041, 2100), (130, 129, 9000), (2041, 2046, 1060), (57, 25161, 149)]
+                (1023, 1041, 2100), (130, 129, 9000), (2041, 2046, 1060), (57, 25161, 149), (17145, 81, 135),
+                (12803, 20, 288), (29, 20740, 192)]
+# the same of operands whose columns are all 16-byte aligned and not both along the reduction, which k_gemm_ring takes of others:
+# more than two 64 x 64 tiles per CU, strips of 33 to 63, one round of 32 x 32 blocks
+VEC_SHAPES = [(16388, 148, 160), (36, 9804, 204), (1652, 92, 224)]
 
 
-@pytest.mark.parametrize("m,n,k", RING_SHAPES + OTHER_SHAPES)
+@pytest.mark.parametrize("m,n,k", RING_SHAPES + OTHER_SHAPES + VEC_SHAPES)
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
 def test_products_on_tiles_that_move_back_inside(cm, rng, m, n, k, ta, tb):
     """The edges of k_gemm_ring, and of the kernels beside it: values beyond the operands (NaN here) never reach a result, and accumulating stores every

@@ -24,9 +24,9 @@ def plans(tmp_path_factory):
     return ct.CDLL(lib)
 
 
-def gemm_tile(plans, m, n, k):
-    """Tile of a product; None: another kernel."""
-    t = plans.gemm_tile(m, n, k, CUS)
+def gemm_tile(plans, m, n, k, vec=False):
+    """Tile of a product; None: another kernel.  vec: of operands that the other kernels read in 16-byte groups."""
+    t = plans.gemm_tile(m, n, k, CUS, vec)
     return TILES[t] if t >= 0 else None
 
 
@@ -47,6 +47,8 @@ def test_the_products_of_the_gpu_tests_reach_every_tile(plans):
 
 def test_the_products_of_the_other_kernels_are_not_on_ring_tiles(plans):
     assert [shape for shape in dot.OTHER_SHAPES if gemm_tile(plans, *shape)] == []
+    assert [shape for shape in dot.VEC_SHAPES if gemm_tile(plans, *shape, vec=True) or not gemm_tile(plans, *shape)] == []
+    assert [shape for shape in dot.RING_SHAPES if gemm_tile(plans, *shape, vec=True) != gemm_tile(plans, *shape)] == []
 
 
 def test_the_layers_of_the_gpu_tests_reach_every_tile(plans):
@@ -109,6 +111,20 @@ def test_the_layers_of_the_other_kernels_are_not_on_ring_tiles(plans):
         for layer, passes in layers.items():
             for name in passes.split():
                 assert conv_tile(plans, dict(up=UP, down=DOWN, outp=OUTP)[name], *layer, local=local) is None, (layer, name)
+
+
+def test_aligned_operands_take_the_ring_for_long_reductions_only(plans):
+    for m, n, k in ((16384, 147, 160), (128, 18880, 240), (10368, 196, 400), (18432, 49, 208), (1648, 96, 224)):
+        assert gemm_tile(plans, m, n, k, vec=True) is None
+    for m, n, k in ((16384, 147, 416), (8192, 256, 400), (18432, 49, 272), (7000, 49, 208), (1648, 96, 160), (1648, 96, 272)):
+        assert gemm_tile(plans, m, n, k, vec=True) is not None
+
+
+def test_strips_of_one_or_two_tiles_per_cu(plans):
+    for m, n, k in ((12800, 18, 288), (24200, 25, 144), (27, 15300, 160), (23636, 81, 243), (80, 17144, 135)):
+        assert gemm_tile(plans, m, n, k) is None
+    for m, n, k in ((20000, 25, 256), (27, 15300, 416), (23636, 81, 272), (23636, 92, 243)):
+        assert gemm_tile(plans, m, n, k) is not None
 
 
 def test_long_strips_of_33_to_63_are_not_on_ring_tiles(plans):
