@@ -132,10 +132,11 @@ static inline double conv_other_us(const Args& a, int mode, long long rows, bool
     const double patch = 1e-9 * 8. * Np * a.M * a.Cg * a.kk2 * a.G;       // GB
     return 9. + (2e-9 * Np * a.M * Fp * K / 105. + patch / 5.) * 1e3 + (copy_n ? 5. + maps / copy : 0.) + (copy_f ? 5. + hid / copy : 0.);
   } else if (mode == CONV_DOWN) {
-    // (uniform rows: 16-wide blocks for 33 to 48 colours; others: 85 where every CU has two tiles)
+    // (uniform rows: 16-wide blocks for 33 to 48 colours; others: 85 where every CU has two tiles, 97 with reductions of 400
+    // terms and more: 96 colours from 48 filters of 3 x 3, 32 x 32, batch 128 128 us on ring tiles, 112 there)
     const bool uniform = a.local || (Np % 128 == 0 && a.kk2 * Fg >= 256 && (a.Cg <= 64 || a.Cg > 96));
     flops = 2e-9 * Np * rows * up(a.Cg, uniform && a.Cg > 32 && a.Cg <= 48 ? 16 : 32) * a.G * a.kk2 * Fg;
-    rate = a.local ? 70. : uniform ? 115. : a.Cg > 32 && rows * Np * a.G >= 2ll * 128 * cus ? 85. : 65.;
+    rate = a.local ? 70. : uniform ? 115. : a.Cg > 32 && rows * Np * a.G >= 2ll * 128 * cus ? (a.kk2 * Fg >= 400 ? 97. : 85.) : 65.;
   } else {
     const int BMs = Fg <= 32 ? 32 : Fg <= 64 ? 64 : Fg <= 96 || (Fg > 128 && (Fg + 95) / 96 * 96 < (Fg + 127) / 128 * 128) ? 96 : 128;
     const bool regs = K <= 80 && Fg <= 64;                               // 16 x 16 blocks in registers
