@@ -94,8 +94,8 @@ static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows,
 
 // Every pass first asks what the fastest ring tile would take (conv_ring_plan) and what the other kernels would
 // (conv_other_us), and runs on the ring when that is less.  Both estimates are held against passes over random layers: of
-// 1260, those so chosen were 1.4 (any), 2.0 (at most 24 images) and 4 times (two groups; locally connected) as fast on
-// average as before the ring, and four more than 5 % slower, 42 -> 44 us the longest of them.
+// 3900, those so chosen were 1.4 to 1.5 (any), 2.0 (at most 24 images) and 4 times (two groups; locally connected) as fast on
+// average as before the ring, and about one in a hundred more than 5 % slower, by 14 % at most.
 
 // What all three passes need: offsets of 31 bits, masks of RING_MAX_SIDE filter rows.
 template <class Args>
