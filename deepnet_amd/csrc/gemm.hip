@@ -1078,6 +1078,7 @@ k_gemm_box_sums(const float* __restrict__ A, int lda, const float* __restrict__ 
 }
 
 #include "gemm_ring.h"
+#include "gemm_split.h"
 
 __global__ void k_gemm_splitk_finish(const float* partial, int splits, float* C, int ldc, int M, int N, float alpha,
                                      float beta) {
@@ -1224,9 +1225,14 @@ static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, co
   // Reductions of more than 128 terms: k_gemm_ring, unless another kernel is expected to be faster (gemm_ring_plan).
   const size_t a_bytes = (size_t)lda * (a_kc ? M : K) * sizeof(float), b_bytes = (size_t)ldb * (b_kc ? N : K) * sizeof(float);
   const RingPlan ring = K > BOX_K ? gemm_ring_plan(M, N, K, a_bytes, b_bytes, cus, a_vec && b_vec && !(a_kc && b_kc)) : RingPlan{-1, 0.};
+  const RingArgs rargs = {A, B, C, (unsigned)a_bytes, (unsigned)b_bytes, lda, ldb, ldc, M, N, K, 0, 0, alpha, beta};
+  if (!epi.sample && gemm_split_wins(M, N, K, beta != 0.f, a_bytes, b_bytes, ring, cus)) {   // (samples are of fewer outputs)
+    split_launch(a_kc, b_kc, rargs, epi);
+    if (fused) *fused = true;
+    return dn_launch_status();
+  }
   if (ring.cfg >= 0) {
-    const RingArgs g = {A, B, C, (unsigned)a_bytes, (unsigned)b_bytes, lda, ldb, ldc, M, N, K, 0, 0, alpha, beta};
-    ring_launch(ring.cfg, a_kc, b_kc, g, epi);
+    ring_launch(ring.cfg, a_kc, b_kc, rargs, epi);
     if (fused) *fused = true;
     if (sampled) *sampled = epi.sample != nullptr;
     return dn_launch_status();
@@ -1309,19 +1315,7 @@ static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, co
     if (sampled) *sampled = epi.sample != nullptr;
     return dn_launch_status();
   }
-  const long long tiles_big = (long long)((M + 127) / 128) * ((N + 127) / 128);
-  // 128 x 128 tiles (two workgroups per CU) against 64 x 64 tiles (five), as measured:
-  // short reductions are mostly prologue and epilogue, which more resident workgroups hide
-  // (4096 x 4096 x 128, beta = 1: 71 us against 60 us; up to K = 512 when C is also read, K = 256 otherwise); and
-  // a tile count that leaves the last round of a CU half empty costs more than the smaller
-  // tile's lower matrix-core rate of about 0.92 (3072 x 3072 x 2048: 404 us against 336 us).
-  // (with the present main loop: 4096 x 4096 x 256 84 us on 64 x 64 tiles against 88 us, x 512 even, x 1024 268 us
-  // against 254 us; fewer than two big tiles per CU leave the CU to one or two workgroups, and the small
-  // tiles win up to K = 1024: 2048 x 2048 x 256 24.2 us against 30.3 us, x 512 39.6 against 46.7, x 1024 71.4
-  // against 75.5)
-  const int kmax64 = tiles_big < 2ll * cus ? 1024 : beta != 0.f ? 512 : 256;
-  auto fill = [&](long long t) { return (double)t / (double)(((t + cus - 1) / cus) * cus); };
-  const bool big = tiles_big >= cus && K > kmax64 && fill(tiles_big) >= 0.92 * fill(tiles64);
+  const bool big = gemm_slab_big(M, N, K, beta != 0.f, cus);
   const int BM = big ? 128 : 64, BN = big ? 128 : 64;
   const int gx = (M + BM - 1) / BM, gy = (N + BN - 1) / BN;
   int splits = 1;

@@ -8,10 +8,11 @@
 // and does not go to memory.  An offset beyond the buffer would do as well, the lanes' or the scalar one (both take part in
 // the range check: measured on buffers inside a larger allocation, loads and stores); a bit in the lanes' offsets is
 // a vector instruction per request (dense 1001 x 1500 x 300, three products: 46.4 against 49.0 us).
-template <int ROWS, int BK, bool KC>
-struct RingOperand : RingTile<ROWS, BK, KC> {
-  using Tile = RingTile<ROWS, BK, KC>;
+template <class Tile>
+struct RingOperand : Tile {
   using Tile::NG;
+  static constexpr int BK = Tile::BK;
+  static constexpr bool KC = Tile::KC;
   const float* P0;
   unsigned voff[NG];
   unsigned n_bytes, step, last;
@@ -79,8 +80,8 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_gemm_ring(RingArgs g, GemmE
   float* C = g.C;
   const int ldc = g.ldc, M = g.M, N = g.N, K = g.K, gx = g.gx, gy = g.gy;
   const float alpha = g.alpha, beta = g.beta;
-  using OA = RingOperand<BM, BK, A_KC>;
-  using OB = RingOperand<BN, BK, B_KC>;
+  using OA = RingOperand<RingTile<BM, BK, A_KC>>;
+  using OB = RingOperand<RingTile<BN, BK, B_KC>>;
   using Shape = RingShape<TB, BM, BN, BK, OA, OB>;
   constexpr int EPL = Shape::EPL;
   __shared__ __attribute__((aligned(16))) float lds[Shape::LDS];

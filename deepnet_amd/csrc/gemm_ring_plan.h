@@ -1,4 +1,5 @@
-// Which products run on k_gemm_ring, and on which of its tiles (host code without HIP; the tests build it by itself).
+// Which products run on k_gemm_ring, and on which of its tiles, and which on k_gemm_split (host code without HIP; the tests
+// build it by itself).
 #pragma once
 #include <stddef.h>
 
@@ -71,4 +72,59 @@ static inline RingPlan gemm_ring_plan(int M, int N, int K, size_t a_bytes, size_
   }
   if (tiles(128) >= cus && 4 * rounds(tiles(128)) <= rounds(tiles(64))) return none;
   return ring;
+}
+
+// Whether k_gemm runs a product on 128 x 128 tiles (see gemm()), else on 64 x 64.
+static inline bool gemm_slab_big(int M, int N, int K, bool beta, int cus) {
+  auto tiles = [&](int side) { return (long long)((M + side - 1) / side) * ((N + side - 1) / side); };
+  auto fill = [&](long long t) { return (double)t / (double)(((t + cus - 1) / cus) * cus); };
+  // 128 x 128 tiles (two workgroups per CU) against 64 x 64 tiles (five), as measured:
+  // short reductions are mostly prologue and epilogue, which more resident workgroups hide
+  // (4096 x 4096 x 128, beta = 1: 71 us against 60 us; up to K = 512 when C is also read, K = 256 otherwise); and
+  // a tile count that leaves the last round of a CU half empty costs more than the smaller
+  // tile's lower matrix-core rate of about 0.92 (3072 x 3072 x 2048: 404 us against 336 us).
+  // (with the present main loop: 4096 x 4096 x 256 84 us on 64 x 64 tiles against 88 us, x 512 even, x 1024 268 us
+  // against 254 us; fewer than two big tiles per CU leave the CU to one or two workgroups, and the small
+  // tiles win up to K = 1024: 2048 x 2048 x 256 24.2 us against 30.3 us, x 512 39.6 against 46.7, x 1024 71.4
+  // against 75.5)
+  const int kmax64 = tiles(128) < 2ll * cus ? 1024 : beta ? 512 : 256;
+  return tiles(128) >= cus && K > kmax64 && fill(tiles(128)) >= 0.92 * fill(tiles(64));
+}
+
+#define SPLIT_BM 128       // k_gemm_split's tile, and its stage of the reduction
+#define SPLIT_BK 32
+
+// What a product takes on k_gemm_split, in us: fitted to 462 measured products of 128 to 90000 per side and 32 to 5000 terms
+// (rms 8 %).  A workgroup is alone on its CU, so what a tile costs besides its stages (first trip to memory, sums to
+// memory) is not hidden; from the third round on the clock is what the matrix cores' power leaves.  < 0: no tile fits.
+static inline double split_us(int M, int N, int K, size_t a_bytes, size_t b_bytes, int cus) {
+  if (M < SPLIT_BM || N < SPLIT_BM || K < SPLIT_BK || a_bytes >= (1ull << 31) || b_bytes >= (1ull << 31)) return -1.;
+  const long long tiles = (long long)((M + SPLIT_BM - 1) / SPLIT_BM) * ((N + SPLIT_BM - 1) / SPLIT_BM);
+  const double rounds = tiles <= 3 * cus ? (double)((tiles + cus - 1) / cus) : 0.5 + (double)tiles / cus;
+  return 4. + rounds * (1.05 * ((K + SPLIT_BK - 1) / SPLIT_BK) + 8.) * (rounds > 2. ? 1.18 : 1.);
+}
+
+// Whether k_gemm_split is expected to be faster than `ring` or, where that is none, than k_gemm (fitted to the same
+// products).  Of the 462 it takes 99, which were 1.31 times as fast on average (4096 x 4096 x 4096 950 -> 670 us, 2048 x
+// 2048 x 2048 140 -> 90, 3904 x 800 x 1568 112 -> 70, 3278 x 3637 x 1110 279 -> 170); the best choice for each would have
+// gained 1 % more over all.  Strips of 129 to 191, whose second tile is mostly a repeat, have to win by more (169 x 54443 x
+// 552 117 -> 137).
+static inline bool gemm_split_wins(int M, int N, int K, bool beta, size_t a_bytes, size_t b_bytes, const RingPlan& ring, int cus) {
+  auto tiles = [&](int side) { return (long long)((M + side - 1) / side) * ((N + side - 1) / side); };
+  const double us = split_us(M, N, K, a_bytes, b_bytes, cus);
+  if (us < 0. || K < 200) return false;               // (short ones are mostly first trip and stores: 4349 x 2436 x 86 36 -> 43)
+  const int slabs = (K + 15) / 16;
+  double other;
+  if (ring.cfg >= 0) {
+    other = 1.12 * ring.us;
+  } else if (tiles(32) <= 2ll * cus) {
+    return false;                                     // small products, or few outputs over a long reduction
+  } else if (gemm_slab_big(M, N, K, beta, cus)) {
+    const long long t = tiles(128);
+    other = 8. + (t <= 3 * cus ? (double)((t + cus - 1) / cus) : 0.5 + (double)t / cus) * (1.16 * slabs + 3.);
+  } else {
+    other = 9. + 0.38 * slabs * (double)tiles(64) / cus;
+  }
+  const int thin = M < N ? M : N;
+  return us * (thin > SPLIT_BM && 2 * thin < 3 * SPLIT_BM ? 1.3 : 1.05) < other;
 }

@@ -10,8 +10,10 @@ typedef float ring_f32x4 __attribute__((ext_vector_type(4)));
 
 // One operand of a stage in LDS: [row][BK + 4] when it is K-contiguous in memory (KC), [k][rows + 4] otherwise, both free
 // of bank conflicts for the order of terms that `frag` reads (pitch 4 mod 8).  A stage is NG 16-byte groups per lane.
-template <int ROWS, int BK, bool KC>
+template <int ROWS, int BK_, bool KC_>
 struct RingTile {
+  static constexpr int BK = BK_;
+  static constexpr bool KC = KC_;
   static constexpr int NG = ROWS * BK / 4 / RING_THREADS;
   static_assert(NG * RING_THREADS * 4 == ROWS * BK, "whole groups per lane");
   static constexpr int PITCH = KC ? BK + 4 : ROWS + 4;

@@ -15,6 +15,12 @@ int gemm_tile(int M, int N, int K, int cus, int vec) {
   return K > 128 ? gemm_ring_plan(M, N, K, (size_t)M * K * 4, (size_t)N * K * 4, cus, vec != 0).cfg : -1;
 }
 
+// Whether the product is k_gemm_split's (of a target that is not read).
+int gemm_split(int M, int N, int K, int cus, int vec) {
+  const size_t a = (size_t)M * K * 4, b = (size_t)N * K * 4;
+  return gemm_split_wins(M, N, K, false, a, b, K > 128 ? gemm_ring_plan(M, N, K, a, b, cus, vec != 0) : RingPlan{-1, 0.}, cus);
+}
+
 // out = {tile number or -1, one module or pixel per tile, splits, LDS bytes of a workgroup, us}
 void conv_tile(int mode, int N, int C, int H, int F, int k, int Mx, int s, int pad0, int G, int local, int partial_sum, int cus, double* out) {
   const int m = partial_sum ? partial_sum : Mx * Mx;

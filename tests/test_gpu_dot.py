@@ -509,7 +509,12 @@ OTHER_SHAPES = [(5899, 21, 312), (23, 4407, 250), (4100, 31, 300), (4097, 17, 12
 VEC_SHAPES = [(16388, 148, 160), (36, 9804, 204), (1652, 92, 224)]
 
 
-@pytest.mark.parametrize("m,n,k", RING_SHAPES + OTHER_SHAPES + VEC_SHAPES)
+# products that the host gives to k_gemm_split (tests/test_ring_plans.py): whole tiles, edges on both sides, a last stage of one
+# term and of all but one, two and more rounds of the CUs
+SPLIT_SHAPES = [(2048, 2048, 224), (1409, 1537, 705), (2049, 2047, 1001), (513, 4095, 703), (255, 16001, 200), (2048, 4095, 223), (3070, 2700, 400)]
+
+
+@pytest.mark.parametrize("m,n,k", RING_SHAPES + OTHER_SHAPES + VEC_SHAPES + SPLIT_SHAPES)
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
 def test_products_on_tiles_that_move_back_inside(cm, rng, m, n, k, ta, tb):
     """The edges of k_gemm_ring, and of the kernels beside it: values beyond the operands (NaN here) never reach a result, and accumulating stores every
@@ -553,3 +558,43 @@ def test_draws_on_tiles_that_move_back_inside(cm, rng, m, n, k):
             cm.set_deferred_epilogues(True)
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+def test_split_products_are_nearer_than_fp32_sums(cm, rng, ta, tb):
+    """k_gemm_split against 64 bits.  A sum of k terms in fp32, one rounding (2^-25 of the partial sum, rms) per two terms, is
+    off by 2^-25 sqrt(k / 4) of its rms; measured 0.35 of that, 0.6 allowed.  So are operands near the ends of the range,
+    whose parts would be denormal or beyond bf16 if they were not scaled."""
+    m, n, k = 1409, 1537, 705
+    A, B = _rand(rng, (m, k)), _rand(rng, (k, n))
+    for fa, fb in ((1.0, 1.0), (2.0 ** -120, 1.0), (1.0, 2.0 ** -130), (2.0 ** 90, 2.0 ** -60), (2.0 ** -60, 2.0 ** -60)):
+        a, b = (A * np.float32(fa)).astype(np.float32), (B * np.float32(fb)).astype(np.float32)
+        ga = cm.CUDAMatrix(np.asfortranarray(a.T if ta else a)); gb = cm.CUDAMatrix(np.asfortranarray(b.T if tb else b))
+        t = cm.dot(ga.T if ta else ga, gb.T if tb else gb)
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        # (results below the normal range are rounded to multiples of 2^-149)
+        limit = 0.6 * 2.0 ** -25 * np.sqrt(k / 4.0) * np.linalg.norm(want) + 2.0 ** -149 * np.sqrt(m * n)
+        assert np.linalg.norm(t.asarray().astype(np.float64) - want) < limit, (fa, fb)
+        for h in (ga, gb, t):
+            h.free_device_memory()
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+def test_split_products_keep_infinities_and_overflows(cm, rng, ta, tb):
+    """A tile with sums that are not finite is computed on the fp32 instructions: infinities, NaN and overflows stand where
+    fp32 sums have them, and every other output (in tiles with and without them) is right."""
+    m, n, k = 1409, 1537, 705
+    A, B = _rand(rng, (m, k)), _rand(rng, (k, n))
+    A[3, 5] = np.inf; A[200, 704] = -np.inf; A[700, 0] = np.nan; A[1408, 7] = 3e38
+    B[9, 40] = 1e36; B[703, 1536] = np.inf; B[5, 60] = 0.0
+    a = cm.CUDAMatrix(np.asfortranarray(A.T if ta else A)); b = cm.CUDAMatrix(np.asfortranarray(B.T if tb else B))
+    got = cm.dot(a.T if ta else a, b.T if tb else b).asarray().astype(np.float64)
+    with np.errstate(invalid='ignore', over='ignore'):
+        want = A.astype(np.float64) @ B.astype(np.float64)
+    size = np.abs(np.nan_to_num(A, posinf=0, neginf=0)).astype(np.float64) @ np.abs(np.nan_to_num(B, posinf=0, neginf=0)).astype(np.float64)
+    over = np.abs(want) > 3.5e38
+    near = (size > 1e38) & ~over                       # (partial sums may overflow or not)
+    assert np.array_equal(np.isnan(got[~near]), np.isnan(want[~near]))
+    assert np.array_equal(got[over], np.sign(want[over]) * np.inf)
+    ok = np.isfinite(want) & ~near & ~over
+    assert ok.sum() > 0.98 * m * n and np.all(np.abs(got[ok] - want[ok]) <= 16 * np.sqrt(k) * 2.0 ** -24 * size[ok])

@@ -51,6 +51,13 @@ def test_the_products_of_the_other_kernels_are_not_on_ring_tiles(plans):
     assert [shape for shape in dot.RING_SHAPES if gemm_tile(plans, *shape, vec=True) != gemm_tile(plans, *shape)] == []
 
 
+def test_the_split_products_of_the_gpu_tests_are_k_gemm_split_s(plans):
+    assert [shape for shape in dot.SPLIT_SHAPES + [(1409, 1537, 705)] for vec in (0, 1) if not plans.gemm_split(*shape, CUS, vec)] == []
+    # tiles have to lie inside the product, and offsets in 31 bits
+    assert [shape for shape in ((127, 30000, 4000), (30000, 127, 4000), (65536, 256, 8192), (256, 65536, 8192), (4096, 4096, 199))
+            if plans.gemm_split(*shape, CUS, 0)] == []
+
+
 def test_the_layers_of_the_gpu_tests_reach_every_tile(plans):
     reached = set()
     for mode in (UP, DOWN, OUTP):
