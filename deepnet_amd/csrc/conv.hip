@@ -2671,7 +2671,7 @@ static bool ring_maps16(const ConvArgs& a) {
 // Up and Down on ring tiles; false: not a pass for them.
 static bool conv_rows_ring(const ConvArgs& a, int mode, const char* where) {
   const bool up = mode == CONV_UP;
-  const ConvRingPlan plan = conv_rows_plan(a, mode, ring_maps16(a), dn_aligned16(a.flt), dn_num_cus());
+  const ConvRingPlan plan = conv_rows_choice(a, mode, ring_maps16(a), dn_aligned16(a.flt), dn_num_cus());
   if (plan.cfg < 0) return false;
   const bool single = plan.single;
   const int sites = up ? a.M : a.HH, cols = up ? a.Fg : a.Cg, K = a.kk2 * (up ? a.Cg : a.Fg);
@@ -2695,7 +2695,7 @@ static void launch_outp_finish(const ConvArgs& a) {
 }
 
 static bool conv_outp_ring(const ConvArgs& a0, cudamat* images, cudamat* hidActs, const char* where) {
-  const ConvRingPlan plan = conv_outp_plan(a0, ring_maps16(a0), dn_aligned16(a0.flt), dn_num_cus());
+  const ConvRingPlan plan = conv_outp_choice(a0, ring_maps16(a0), dn_aligned16(a0.flt), dn_num_cus());
   if (plan.cfg < 0) return false;
   ConvArgs a = a0;
   const int N4 = (a.N + 3) / 4 * 4, cols = a.Cg * a.kk2, K = a.m_count * N4;

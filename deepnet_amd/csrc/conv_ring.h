@@ -1,6 +1,6 @@
 // Convolution passes on the tile loop of ring_tile.h: see k_conv_ring.  Included by conv.hip (ConvArgs).
 #pragma once
-#include "ring_tile.h"
+#include "split_tile.h"
 #include "conv_ring_plan.h"
 
 // A term of the reduction, as the workgroup keeps it in LDS for its reduction (one entry per term for Up, per four
@@ -33,11 +33,13 @@ struct ConvRingArgs {
 //   On tiles of one module or pixel every entry is an offset into each operand, or RING_FAR behind the last term:
 //      5, 6: A (x of an entry) and B (y) of Up and A of Down
 //      7: B of Down
-template <int KIND, int ROWS, int BK, int PER>
-struct ConvRingOperand : RingTile<ROWS, BK, ((KIND >= 2 && KIND <= 4) || KIND == 7)> {
-  using Tile = RingTile<ROWS, BK, ((KIND >= 2 && KIND <= 4) || KIND == 7)>;
+template <int KIND, class Tile, int PER>
+struct ConvRingOperand : Tile {
+  static_assert(Tile::KC == ((KIND >= 2 && KIND <= 4) || KIND == 7), "terms or rows in order of memory");
   using Tile::NG;
-  static constexpr bool ENT = KIND == 0 || KIND == 5 || KIND == 6;        // an entry per group, else one per lane and stage
+  static constexpr int BK = Tile::BK;
+  // an entry per group, else one per lane and stage
+  static constexpr bool ENT = (KIND == 0 || KIND == 5 || KIND == 6) && !(Tile::KPACK >= NG && NG <= PER);
   static constexpr bool LOOKS = KIND != 1 && KIND != 3;
   __amdgpu_buffer_rsrc_t rsrc;
   unsigned off[NG], mask[NG];
@@ -50,14 +52,14 @@ struct ConvRingOperand : RingTile<ROWS, BK, ((KIND >= 2 && KIND <= 4) || KIND ==
     const int at = (t < nst ? t : nst - 1) * (BK / PER);
     if (KIND == 0) {
 #pragma unroll
-      for (int u = 0; u < NG; ++u) ent[u] = tab[at + Tile::group_k(threadIdx.x, u) / PER];
+      for (int u = 0; u < (ENT ? NG : 1); ++u) ent[u] = tab[at + Tile::group_k(threadIdx.x, u) / PER];
     }
     if (KIND == 2) ent[0].x = tab1[at + Tile::group_k(threadIdx.x, 0) / PER];
     if (KIND == 4) ent[0] = tab[at + Tile::group_k(threadIdx.x, 0) / PER];
     const int free = t * (BK / PER);                                      // (the table of these reaches over what is asked for)
     if (KIND == 5 || KIND == 6) {
 #pragma unroll
-      for (int u = 0; u < NG; ++u) {
+      for (int u = 0; u < (ENT ? NG : 1); ++u) {
         const uint2* e = tab + free + Tile::group_k(threadIdx.x, u) / PER;
         ent[u].x = KIND == 5 ? e->x : e->y;
       }
@@ -71,8 +73,9 @@ struct ConvRingOperand : RingTile<ROWS, BK, ((KIND >= 2 && KIND <= 4) || KIND ==
     for (int u = 0; u < NG; ++u) {
       unsigned o;
       if (KIND == 0) {
-        const unsigned need = ent[u].y | behind;
-        o = (mask[u] & need) == need ? off[u] + ent[u].x : RING_FAR;
+        const uint2 e = ent[ENT ? u : 0];
+        const unsigned need = e.y | behind;
+        o = (mask[u] & need) == need ? off[u] + e.x : RING_FAR;
       } else if (KIND == 1) {
         o = off[u] + (unsigned)t * step;                                  // (beyond the last term: beyond the buffer)
       } else if (KIND == 2) {
@@ -110,15 +113,39 @@ struct ConvRingOperand : RingTile<ROWS, BK, ((KIND >= 2 && KIND <= 4) || KIND ==
 //   449 on k_conv_mfma (48 columns)
 // The MFMAs are busy for 81 (Up) and 83 % (Outp) of the time of the last layer, without bank conflicts; without the masks a
 // stage takes as long as with them.
-template <int MODE, bool SINGLE, int TB, int BM, int BN, int BK>
-__global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
-  constexpr int PER = MODE == CONV_UP ? 1 : 4;
-  using OA = ConvRingOperand<MODE == CONV_OUTP ? 3 : SINGLE ? 5 : 0, BM, BK, PER>;
-  using OB = ConvRingOperand<MODE == CONV_UP ? (SINGLE ? 6 : 1) : MODE == CONV_DOWN ? (SINGLE ? 7 : 2) : 4, BN, BK, PER>;
-  using Shape = RingShape<TB, BM, BN, BK, OA, OB>;
-  constexpr int EPL = Shape::EPL;
-  static_assert(Shape::LDS * 4 == conv_ring_lds(MODE, BM, BN, BK) && Shape::LDS * 4 + RING_TABLE_BYTES <= RING_CU_LDS, "as planned");
-  __shared__ __attribute__((aligned(16))) float lds[Shape::LDS];
+// Layers with enough outputs for tiles of 128 x 48 to 128 x 128 (64 x 64 in a few cases) run on the bf16 matrix cores
+// (ConvSplitCfg, split_tile.h), where taking the operands apart is as much work as the MFMAs: a number of a map is used by
+// as many columns as the tile is wide.  Measured as above, fp32 tile or other kernel -> now:
+//   96 -> 256 colours 5 x 5, 2 groups, 27 x 27, 128   Up 413 -> 290 (128 x 128), Down 457 -> 415 (128 x 48), Outp 450 -> 306
+//   3 -> 96 colours 11 x 11, stride 4, 224 x 224, 128 Up 260 -> 217 (128 x 96), Outp 237 -> 170 (96 x 128)
+//   32 -> 128 colours 3 x 3, 32 x 32, 128             Up 95 -> 68, Outp 91 -> 75
+//   64 -> 64 colours 5 x 5, 24 x 24, 128              Outp 128 -> 107 (64 x 128), Up and Down 124 and 118 -> 117 and 117: stay
+template <int TB, int BM_, int BN_, int BK_>
+struct ConvRingCfg {
+  static constexpr int BM = BM_, BN = BN_, BK = BK_, THREADS = RING_THREADS, WAVES = 4;
+  static constexpr bool SPLIT = false;
+  template <int ROWS, bool KC> using Tile = RingTile<ROWS, BK, KC>;
+  template <class OA, class OB> using Shape = RingShape<TB, BM, BN, BK, OA, OB>;
+};
+// (on the bf16 matrix cores: see split_tile.h)
+template <int BM_, int BN_, int BK_, int WM, int WN, int KS, int SETS, int WAVES_>
+struct ConvSplitCfg {
+  static constexpr int BM = BM_, BN = BN_, BK = BK_, THREADS = 64 * WM * WN * KS, WAVES = WAVES_;
+  static constexpr bool SPLIT = true;
+  template <int ROWS, bool KC> using Tile = SplitTile<ROWS, BK, KC, THREADS>;
+  template <class OA, class OB> using Shape = SplitShape<BM, BN, BK, WM, WN, KS, SETS, OA, OB>;
+};
+template <int MODE, bool SINGLE, class Cfg>
+__global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRingArgs p) {
+  constexpr int PER = MODE == CONV_UP ? 1 : 4, BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, THREADS = Cfg::THREADS;
+  using OA = ConvRingOperand<MODE == CONV_OUTP ? 3 : SINGLE ? 5 : 0, typename Cfg::template Tile<BM, MODE == CONV_OUTP>, PER>;
+  using OB = ConvRingOperand<MODE == CONV_UP ? (SINGLE ? 6 : 1) : MODE == CONV_DOWN ? (SINGLE ? 7 : 2) : 4,
+                             typename Cfg::template Tile<BN, MODE != CONV_UP>, PER>;
+  using Shape = typename Cfg::template Shape<OA, OB>;
+  constexpr int EPL = Shape::EPL, LDS = Cfg::SPLIT ? Shape::LDS : 4 * Shape::LDS;
+  static_assert(LDS == (Cfg::SPLIT ? conv_split_lds(BM, BN, BK) : conv_ring_lds(MODE, BM, BN, BK)) && LDS + RING_TABLE_BYTES <= RING_CU_LDS,
+                "as planned");
+  __shared__ __attribute__((aligned(16))) char lds[LDS];
   extern __shared__ uint2 table[];
   const int tid = threadIdx.x;
   const int N = p.N, H = p.H, Mx = p.Mx, k = p.k;
@@ -156,7 +183,7 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
     // exact for dividends below 2^12 and divisors up to RING_MAX_SIDE^2
     const unsigned inv_nx = 65536u / (unsigned)nx + 1u, inv_area = (1u << 20) / (unsigned)(area > 0 ? area : 1) + 1u;
     const unsigned Nu = (unsigned)N, Fu = (unsigned)p.F;
-    for (int e = tid; e < (nst + RING_AHEAD) * (BK / PER); e += RING_THREADS) {
+    for (int e = tid; e < (nst + RING_AHEAD) * (BK / PER); e += THREADS) {
       uint2 t2 = make_uint2(RING_FAR, RING_FAR);
       if (PER * e < K) {
         const int c = MODE == CONV_UP ? (int)((unsigned)e * inv_area >> 20) : 0;
@@ -188,7 +215,7 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
   } else if constexpr (MODE == CONV_UP) {
     const int K = p.Cg * p.kk2;
     nst = (K + BK - 1) / BK;
-    for (int e = tid; e < nst * BK; e += RING_THREADS) {
+    for (int e = tid; e < nst * BK; e += THREADS) {
       const int c = div(e, p.dkk2), tap = e - c * p.kk2, ky = div(tap, p.dk), kx = tap - ky * k;
       table[e] = e < K ? make_uint2(4u * (unsigned)N * (unsigned)(c * p.HH + ky * H + kx), 1u << ky | 1u << (RING_MAX_SIDE + kx))
                        : make_uint2(0u, RING_FAR);
@@ -212,7 +239,7 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
     const int K = p.kk2 * p.Fg;
     nst = (K + BK - 1) / BK;
     unsigned* tab1 = reinterpret_cast<unsigned*>(table + nst * (BK / 4));
-    for (int e = tid; e < nst * (BK / 4); e += RING_THREADS) {
+    for (int e = tid; e < nst * (BK / 4); e += THREADS) {
       const int tap = div(4 * e, p.dFg), f = 4 * e - tap * p.Fg, ky = div(tap, p.dk), kx = tap - ky * k;
       const bool in = 4 * e < K;
       table[e] = make_uint2(4u * (unsigned)N * (unsigned)(p.M * f - ky * Mx - kx), in ? 1u << ky | 1u << (RING_MAX_SIDE + kx) : RING_FAR);
@@ -236,7 +263,7 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
     g = z - cz * p.G;
     const int count = p.K - k_beg < p.split_stages * BK ? p.K - k_beg : p.split_stages * BK, first = chunk * p.m_count * N + k_beg;
     nst = (count + BK - 1) / BK;
-    for (int e = tid; e < nst * (BK / 4); e += RING_THREADS) {
+    for (int e = tid; e < nst * (BK / 4); e += THREADS) {
       const int r = first + 4 * e, m = div(r, p.dN), n = r - m * N, my = div(m, p.dMx), mx = m - my * Mx;
       const int y = my * p.s + p.pad0, x = mx * p.s + p.pad0;
       table[e] = 4 * e < count ? make_uint2(4u * (unsigned)(n + N * (y * H + x)),
@@ -261,21 +288,28 @@ __global__ void __launch_bounds__(RING_THREADS, 4) k_conv_ring(ConvRingArgs p) {
   oa.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, (int)p.a_bytes, 0x00020000);
   __syncthreads();
 
-  float sum[EPL];
-  Shape::template run<false>(lds, oa, ob, nst, 0, sum, [] {});
-  const int em = m0 + tid % BM, en0 = n0 + tid / BM;
+  if constexpr (Cfg::SPLIT) {
+    Shape::template run<false>(lds, oa, ob, nst, 0, [] {});
 #pragma unroll
-  for (int u = 0; u < EPL; ++u) {
-    const int en = en0 + u * (RING_THREADS / BM);
-    if (em >= m_lo && en >= n_lo) {
-      out[(long long)en * p.ldc + em] = sum[u];
+    for (int u = 0; u < EPL; ++u) {
+      const int e = tid + THREADS * u, em = m0 + e % BM, en = n0 + e / BM;
+      if (em >= m_lo && en >= n_lo) out[(long long)en * p.ldc + em] = Shape::sum(lds, tid, u);
+    }
+  } else {
+    float sum[EPL];
+    Shape::template run<false>(reinterpret_cast<float*>(lds), oa, ob, nst, 0, sum, [] {});
+    const int em = m0 + tid % BM, en0 = n0 + tid / BM;
+#pragma unroll
+    for (int u = 0; u < EPL; ++u) {
+      const int en = en0 + u * (THREADS / BM);
+      if (em >= m_lo && en >= n_lo) out[(long long)en * p.ldc + em] = sum[u];
     }
   }
 }
 
 template <int MODE, bool SINGLE>
 static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
-  const auto& f = g_conv_ring_cfgs[plan.cfg];
+  const ConvRingTile f = conv_ring_cfg(MODE, plan.cfg);
   p.gx = (p.rows + f.bm - 1) / f.bm; p.gy = (p.cols + f.bn - 1) / f.bn;
   const long long tiles = (long long)p.periods * p.gx * p.gy * p.gz;
   const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)));
@@ -284,14 +318,19 @@ static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
   p.dFg = make_fastdiv(p.Fg); p.dgx = make_fastdiv(p.gx); p.dgy = make_fastdiv(p.gy); p.dper = make_fastdiv(p.periods);
   p.dsplits = make_fastdiv(p.splits); p.dG = make_fastdiv(p.G);
   const size_t tab = (size_t)conv_ring_table(MODE, SINGLE, f.bk, stages);
-#define CONV_RING(TB, BM, BN, BK) hipLaunchKernelGGL((k_conv_ring<MODE, SINGLE, TB, BM, BN, BK>), grid, dim3(RING_THREADS), tab, dn_stream(), p)
+#define CONV_RING(...) hipLaunchKernelGGL((k_conv_ring<MODE, SINGLE, __VA_ARGS__>), grid, dim3(__VA_ARGS__::THREADS), tab, dn_stream(), p)
   switch (plan.cfg) {
-    case 0: CONV_RING(32, 64, 64, 32); break;
-    case 1: CONV_RING(32, 64, 32, 64); break;
-    case 2: CONV_RING(32, 32, 64, 64); break;
-    case 3: CONV_RING(16, 32, 32, 64); break;
-    case 4: CONV_RING(16, 32, 16, 128); break;
-    default: CONV_RING(16, 16, 32, 128); break;
+    case 0: CONV_RING(ConvRingCfg<32, 64, 64, 32>); break;
+    case 1: CONV_RING(ConvRingCfg<32, 64, 32, 64>); break;
+    case 2: CONV_RING(ConvRingCfg<32, 32, 64, 64>); break;
+    case 3: CONV_RING(ConvRingCfg<16, 32, 32, 64>); break;
+    case 4: CONV_RING(ConvRingCfg<16, 32, 16, 128>); break;
+    case 5: CONV_RING(ConvRingCfg<16, 16, 32, 128>); break;
+    case 6: CONV_RING(ConvSplitCfg<128, 128, 32, 2, 4, 1, 2, 2>); break;
+    case 7: if constexpr (MODE == CONV_OUTP) CONV_RING(ConvSplitCfg<96, 128, 32, 2, 4, 1, 2, 2>); else CONV_RING(ConvSplitCfg<128, 96, 32, 4, 2, 1, 2, 2>); break;
+    case 8: if constexpr (MODE == CONV_OUTP) CONV_RING(ConvSplitCfg<64, 128, 32, 2, 4, 1, 2, 2>); else CONV_RING(ConvSplitCfg<128, 64, 32, 4, 2, 1, 2, 2>); break;
+    case 9: CONV_RING(ConvSplitCfg<64, 64, 32, 2, 2, 1, 2, 3>); break;
+    default: if constexpr (MODE == CONV_DOWN) CONV_RING(ConvSplitCfg<128, 48, 64, 4, 1, 2, 2, 2>); break;
   }
 #undef CONV_RING
 }

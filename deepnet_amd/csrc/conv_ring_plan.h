@@ -35,9 +35,21 @@ static inline int padded_filters(int F, int numGroups) {
 // The tiles and what they cost: us per stage and per tile of a round (a tile on every CU).  Fitted to 500 measured
 // passes (rms 4 to 8 %; masks or none, no difference); what a tile costs besides its stages is its table and its first
 // trip to memory.
-static const struct { int bm, bn, bk; double stage, tile; } g_conv_ring_cfgs[] = {
+struct ConvRingTile { int bm, bn, bk; double stage, tile; };
+#define CONV_RING_CFGS 6                 // the fp32 tiles
+#define CONV_CFGS 11
+static const ConvRingTile g_conv_ring_cfgs[CONV_CFGS] = {
     {64, 64, 32, 0.545, 1.45}, {64, 32, 64, 0.574, 1.46}, {32, 64, 64, 0.58, 1.45},
-    {32, 32, 64, 0.322, 1.0}, {32, 16, 128, 0.372, 1.2}, {16, 32, 128, 0.372, 1.17}};
+    {32, 32, 64, 0.322, 1.0}, {32, 16, 128, 0.372, 1.2}, {16, 32, 128, 0.372, 1.17},
+    // on the bf16 matrix cores (split_tile.h), fitted to 280 passes (rms 11 to 24 %)
+    {128, 128, 32, 1.12, 5.}, {128, 96, 32, 1.08, 4.5}, {128, 64, 32, 0.8, 3.5}, {64, 64, 32, 0.53, 1.}, {128, 48, 64, 1.2, 4.}};
+// (of Outp the rows are the filters, and there is no tile of 48)
+static inline ConvRingTile conv_ring_cfg(int mode, int c) {
+  ConvRingTile f = g_conv_ring_cfgs[c];
+  if (mode == CONV_OUTP && (c == 7 || c == 8)) { f.bm = f.bn; f.bn = 128; }
+  if (c == 10 && mode != CONV_DOWN) f.bm = 0;
+  return f;
+}
 // What a workgroup's LDS holds besides the two stages of its tile, which take 36 to 57 KB.  Two workgroups share a CU while
 // they take half of its 160 KB each; with a full table convUp on 32 x 16 and 16 x 32 tiles takes 82 KB and is alone.
 // The table also bounds the reduction of a convUp, with 8 bytes a term: 3328 terms on tiles over several modules, 3104 to
@@ -51,6 +63,15 @@ static constexpr int conv_ring_lds(int mode, int bm, int bn, int bk) {
   return 8 * (a + b);
 }
 
+// The same on the bf16 matrix cores: two stages of three planes each, or the sums.
+static constexpr int conv_split_lds(int bm, int bn, int bk) {
+  return 12 * bk * (bm + bn) > 4 * bm * bn ? 12 * bk * (bm + bn) : 4 * bm * bn;
+}
+static inline int conv_tile_lds(int mode, int c) {
+  const ConvRingTile f = conv_ring_cfg(mode, c);
+  return c < CONV_RING_CFGS ? conv_ring_lds(mode, f.bm, f.bn, f.bk) : conv_split_lds(f.bm, f.bn, f.bk);
+}
+
 struct ConvRingPlan { int cfg, splits, split_stages; bool single; double us; };
 
 static inline int conv_ring_entry(int mode, bool single, int bk) {      // table bytes per stage
@@ -60,15 +81,15 @@ static inline int conv_ring_table(int mode, bool single, int bk, int stages) {  
   return ((stages < 1 ? 1 : stages) + (single ? RING_AHEAD : 0)) * conv_ring_entry(mode, single, bk);
 }
 
-// The tile that is expected to be fastest, cfg < 0: none fits.  rows x cols outputs per period, `jobs` periods x groups x
+// The tile (of the fp32 ones, or of those on the bf16 matrix cores) that is expected to be fastest, cfg < 0: none fits.  rows x cols outputs per period, `jobs` periods x groups x
 // chunks, K terms each, of which a tile has the share `used` on average; split_us: what adding up one more
 // partial output costs (Outp).
 static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows, int cols, long long jobs, int K, double used,
-                                          bool can_split, double split_us, int cus) {
+                                          bool can_split, double split_us, int cus, bool bf16 = false) {
   ConvRingPlan best = {-1, 1, 0, false, 0.};
-  for (int c = 0; c < 6; ++c) {
-    const auto& f = g_conv_ring_cfgs[c];
-    if (rows < f.bm || cols < f.bn) continue;
+  for (int c = bf16 ? CONV_RING_CFGS : 0; c < (bf16 ? CONV_CFGS : CONV_RING_CFGS); ++c) {
+    const ConvRingTile f = conv_ring_cfg(mode, c);
+    if (f.bm == 0 || rows < f.bm || cols < f.bn) continue;
     const long long tiles = (rows + f.bm - 1) / f.bm * ((cols + f.bn - 1) / f.bn) * jobs;
     const int nst = (K + f.bk - 1) / f.bk;
     const int most = RING_TABLE_BYTES / conv_ring_entry(mode, single, f.bk) - (single ? RING_AHEAD : 0);
@@ -84,8 +105,16 @@ static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows,
       if (all >= 1ll << 28) continue;
       double rounds = all <= 4 * cus ? (double)((all + cus - 1) / cus) : 0.5 + (double)all / cus;
       // alone on its CU a workgroup shows its waits (122 -> 126 colours of 5 x 5 on 16 filters, 24 x 24, batch 100: 66 -> 77 us)
-      if (rounds > 1. && 2 * (conv_ring_lds(mode, f.bm, f.bn, f.bk) + conv_ring_table(mode, single, f.bk, per)) > RING_CU_LDS) rounds *= 1.16;
-      const double us = 3. + rounds * (used * per * f.stage + f.tile) + (real > 1 ? 2.5 + real * split_us : 0.);
+      if (rounds > 1. && c < CONV_RING_CFGS && 2 * (conv_tile_lds(mode, c) + conv_ring_table(mode, single, f.bk, per)) > RING_CU_LDS) rounds *= 1.16;
+      double share = used;
+      if (c >= CONV_RING_CFGS) {
+        // these have few rounds, and the tiles in the middle of a map, which have all taps, end the last one
+        share += (1. - used) / (rounds > 1. ? rounds : 1.);
+        // (several of the smallest share a CU, and one alone shows its waits)
+        if (f.bm == 64 && f.bn == 64 && rounds <= 1.) rounds = 1.2;
+        rounds *= 1.08;                               // (what the estimates miss: they are to win by that much)
+      }
+      const double us = 3. + rounds * (share * per * f.stage + f.tile) + (real > 1 ? 2.5 + real * split_us : 0.);
       if (best.cfg < 0 || us < best.us) best = {c, real, per, single, us};
     }
   }
@@ -185,35 +214,63 @@ static inline double ring_crowd(const Args& a) {
 static inline ConvRingPlan conv_no_ring() { return {-1, 1, 0, false, 0.}; }
 
 // Up and Down: tiles over any run of (module | pixel, image) groups, which needs batches of whole groups of four, or of
-// one module or pixel each, which leave out taps beyond the edge and need no masks.  cfg < 0: another kernel.
+// one module or pixel each, which leave out taps beyond the edge and need no masks.  cfg < 0: none fits.
 template <class Args>
-static inline ConvRingPlan conv_rows_plan(const Args& a, int mode, bool maps16, bool filters16, int cus) {
+static inline ConvRingPlan conv_rows_best(const Args& a, int mode, int cus, bool bf16) {
   const bool up = mode == CONV_UP;
   if (!ring_ok(a, (long long)a.Cg * a.kk2 * (a.local ? a.M : 1)) || (!up && (a.s != 1 || a.Fg % 4 != 0)))
     return conv_no_ring();                                               // (Down: an entry is four filters of a tap)
   const int sites = up ? a.M : a.HH, cols = up ? a.Fg : a.Cg, K = a.kk2 * (up ? a.Cg : a.Fg);
-  ConvRingPlan plan = conv_ring_plan(mode, true, a.N, cols, (long long)sites * a.G, K, ring_used(a, mode), false, 0., cus);
+  if (bf16 && K < 9) return conv_no_ring();                              // (a stage of 32 terms is mostly empty)
+  ConvRingPlan plan = conv_ring_plan(mode, true, a.N, cols, (long long)sites * a.G, K, ring_used(a, mode), false, 0., cus, bf16);
   if (!a.local && a.N % 4 == 0) {
-    const ConvRingPlan flat = conv_ring_plan(mode, false, (long long)sites * a.N, cols, a.G, K, 1., false, 0., cus);
+    const ConvRingPlan flat = conv_ring_plan(mode, false, (long long)sites * a.N, cols, a.G, K, 1., false, 0., cus, bf16);
     if (flat.cfg >= 0 && (plan.cfg < 0 || flat.us < plan.us)) plan = flat;
   }
+  return plan;
+}
+
+// The fp32 tile for Up and Down, cfg < 0: another kernel.
+template <class Args>
+static inline ConvRingPlan conv_rows_plan(const Args& a, int mode, bool maps16, bool filters16, int cus) {
+  const ConvRingPlan plan = conv_rows_best(a, mode, cus, false);
+  const bool up = mode == CONV_UP;
   // (the patch form of few colours does all pixels at once: there the busiest XCD counts, elsewhere the estimates do not
   // differ by as little)
   const double crowd = !up && plan.single && !a.local && a.Cg <= 16 ? ring_crowd(a) : 1.;
-  return plan.cfg < 0 || crowd * plan.us > conv_other_us(a, mode, sites, maps16, filters16, cus) ? conv_no_ring() : plan;
+  return plan.cfg < 0 || crowd * plan.us > conv_other_us(a, mode, up ? a.M : a.HH, maps16, filters16, cus) ? conv_no_ring() : plan;
+}
+
+// The tile for Up and Down, on the bf16 matrix cores where that is expected to be faster.
+template <class Args>
+static inline ConvRingPlan conv_rows_choice(const Args& a, int mode, bool maps16, bool filters16, int cus) {
+  const ConvRingPlan ring = conv_rows_plan(a, mode, maps16, filters16, cus), split = conv_rows_best(a, mode, cus, true);
+  const double other = ring.cfg >= 0 ? ring.us : conv_other_us(a, mode, mode == CONV_UP ? a.M : a.HH, maps16, filters16, cus);
+  return split.cfg >= 0 && split.us < other ? split : ring;
 }
 
 // Outp of `a`, whose batch the ring takes in whole groups of four images: others are copied with up to three images of zeros.
 template <class Args>
-static inline ConvRingPlan conv_outp_plan(const Args& a, bool maps16, bool filters16, int cus) {
+static inline ConvRingPlan conv_outp_best(const Args& a, int cus, bool bf16) {
   Args r = a;
   r.N = (a.N + 3) / 4 * 4;
   const int cols = a.Cg * a.kk2;
   if (!ring_ok(r, (long long)cols * a.chunks) || a.chunks > 32767) return conv_no_ring();
-  const ConvRingPlan plan = conv_ring_plan(CONV_OUTP, false, a.Fg, cols, (long long)a.G * a.chunks, a.m_count * r.N, 1., true,
-                                           2e-6 * a.chunks * a.F * cols, cus);
+  ConvRingPlan plan = conv_ring_plan(CONV_OUTP, false, a.Fg, cols, (long long)a.G * a.chunks, a.m_count * r.N, 1., true,
+                                     2e-6 * a.chunks * a.F * cols, cus, bf16);
   const double maps = 1e-9 * 8. * r.N * ((double)a.M * a.F + (double)a.HH * a.C);
   // (1.12: what a layer's sums over many splits take beyond the plan's estimate)
-  return plan.cfg < 0 || 1.12 * plan.us + (r.N != a.N ? 5. + maps / 5e-3 : 0.) > conv_other_us(a, CONV_OUTP, a.M, maps16, filters16, cus)
-             ? conv_no_ring() : plan;
+  plan.us = 1.12 * plan.us + (r.N != a.N ? 5. + maps / 5e-3 : 0.);
+  return plan;
+}
+template <class Args>
+static inline ConvRingPlan conv_outp_plan(const Args& a, bool maps16, bool filters16, int cus) {
+  const ConvRingPlan plan = conv_outp_best(a, cus, false);
+  return plan.cfg < 0 || plan.us > conv_other_us(a, CONV_OUTP, a.M, maps16, filters16, cus) ? conv_no_ring() : plan;
+}
+template <class Args>
+static inline ConvRingPlan conv_outp_choice(const Args& a, bool maps16, bool filters16, int cus) {
+  const ConvRingPlan ring = conv_outp_plan(a, maps16, filters16, cus), split = conv_outp_best(a, cus, true);
+  const double other = ring.cfg >= 0 ? ring.us : conv_other_us(a, CONV_OUTP, a.M, maps16, filters16, cus);
+  return split.cfg >= 0 && split.us < other ? split : ring;
 }

@@ -46,12 +46,13 @@ template <int ROWS_, int BK_, bool KC_, int NT_>
 struct SplitTile {
   static constexpr int ROWS = ROWS_, BK = BK_, NT = NT_;
   static constexpr bool KC = KC_;
-  static constexpr int GROUPS = ROWS * BK / 4, NG = (GROUPS + NT - 1) / NT, PACKS = KC ? 2 : 8 / NG;
+  static constexpr int GROUPS = ROWS * BK / 4, NGS = (GROUPS + NT - 1) / NT, NG = KC || NGS > 1 ? NGS : 2, PACKS = KC ? 2 : 8 / NG;
+  static constexpr int KPACK = KC ? 4 : NG;                // consecutive terms of a lane's groups
   static_assert(GROUPS % 64 == 0 && ROWS % 16 == 0 && BK % 32 == 0 && NT % (BK / 4) == 0, "whole wavefronts and blocks");
-  static_assert(KC || (GROUPS == NG * NT && (NG == 2 || NG == 4) && ROWS % 32 == 0), "whole packs of terms");
+  static_assert(KC || ((NG == 2 || NG == 4) && ROWS % 32 == 0 && GROUPS / NG % 64 == 0), "whole packs of terms");
   static constexpr int Q = ROWS % 64 == 0 ? 16 : 8;
   static constexpr int PLANE = BK * ROWS * 2, BYTES = 3 * PLANE;
-  // group u of lane `tid`: its (first) term of the stage and its (first) row
+  // group u of lane `tid`: its (first) term of the stage and its (first) row (beyond the stage for lanes that are left over)
   __device__ __forceinline__ static int group_k(int tid, int u) {
     return KC ? 4 * (tid % (BK / 4)) : 8 * (tid / (8 * PACKS * (ROWS / 32))) + NG * (tid / 8 % PACKS) + u;
   }
@@ -88,7 +89,7 @@ struct SplitTile {
             *reinterpret_cast<split_u32x2*>(D + p * PLANE + (group_row(tid, u) ^ swap(kg)) * 16) = split_u32x2{a[p], b[p]};
         }
       }
-    } else {
+    } else if (GROUPS == NG * NT || tid < GROUPS / NG) {
       const int slot = slot_of(group_row(tid, 0)) ^ swap(kg);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -113,7 +114,7 @@ struct SplitTile {
   __device__ __forceinline__ static void stash32(float* S, int tid, const ring_f32x4 (&r)[NG], int kmin) {
 #pragma unroll
     for (int u = 0; u < NG; ++u) {
-      if (!KC || GROUPS == NG * NT || tid + u * NT < GROUPS) {
+      if (GROUPS == NG * NT || (KC ? tid + u * NT < GROUPS : tid < GROUPS / NG)) {
         const int k = group_k(tid, u), row = group_row(tid, u);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -143,8 +144,8 @@ struct SplitShape {
   static constexpr int STAGE = OA::BYTES + OB::BYTES, RED = 4 * KS * BM * BN;
   static constexpr int LDS = 2 * STAGE > RED ? 2 * STAGE : RED;
   static_assert(LDS >= 4 * BK * (BM + BN), "a stage in fp32");
-  static constexpr int EPL = BM * BN / NT;                 // outputs per lane: (tid % BM, tid / BM + u * NT / BM)
-  static_assert(NT % BM == 0 && EPL * NT == BM * BN, "whole columns");
+  static constexpr int EPL = BM * BN / NT;                 // outputs per lane: e = tid + u * NT is (e % BM, e / BM)
+  static_assert(EPL * NT == BM * BN, "whole tiles");
 
   struct Acc { ring_f32x4 main[TN][TM], small[TN][TM]; };
   struct Frags { split_bf16x8 a[TM], b[TN]; };             // of one plane
@@ -257,7 +258,14 @@ struct SplitShape {
           bad |= !(__builtin_fabsf(x) < __builtin_inff());
           acc.main[j][i][v] = x * SPLIT_OUT;
         }
-    if (__syncthreads_or(bad)) {
+    int* vote = reinterpret_cast<int*>(lds);
+    if (tid == 0) *vote = 0;
+    __syncthreads();
+    if (bad) *vote = 1;
+    __syncthreads();
+    bad = *vote;
+    __syncthreads();
+    if (bad) {
       float *SA = reinterpret_cast<float*>(lds), *SB = SA + BK * BM;
 #pragma unroll
       for (int j = 0; j < TN; ++j)

@@ -21,16 +21,20 @@ int gemm_split(int M, int N, int K, int cus, int vec) {
   return gemm_split_wins(M, N, K, false, a, b, K > 128 ? gemm_ring_plan(M, N, K, a, b, cus, vec != 0) : RingPlan{-1, 0.}, cus);
 }
 
-// out = {tile number or -1, one module or pixel per tile, splits, LDS bytes of a workgroup, us}
+// The fp32 tile of a pass, or with mode + 4 the tile of all: out = {tile number or -1, one module or pixel per tile, splits, LDS bytes of a workgroup, us}
 void conv_tile(int mode, int N, int C, int H, int F, int k, int Mx, int s, int pad0, int G, int local, int partial_sum, int cus, double* out) {
   const int m = partial_sum ? partial_sum : Mx * Mx;
   const Sizes a = {N, C, C / G, H, H * H, F, F / G, k, k * k, Mx, Mx * Mx, s, pad0, G, local, m, Mx * Mx / m};
-  const ConvRingPlan p = mode == CONV_OUTP ? conv_outp_plan(a, N % 4 == 0, true, cus) : conv_rows_plan(a, mode, N % 4 == 0, true, cus);
+  const bool all = mode >= 4;          // 4 + mode: of all tiles
+  mode &= 3;
+  const bool maps16 = N % 4 == 0;
+  const ConvRingPlan p = mode == CONV_OUTP ? (all ? conv_outp_choice(a, maps16, true, cus) : conv_outp_plan(a, maps16, true, cus))
+                                           : (all ? conv_rows_choice(a, mode, maps16, true, cus) : conv_rows_plan(a, mode, maps16, true, cus));
   out[0] = p.cfg; out[1] = p.single; out[2] = p.splits;
   const int K = mode == CONV_OUTP ? 0 : a.kk2 * (mode == CONV_UP ? a.Cg : a.Fg);
   if (p.cfg < 0) return;
-  const auto& f = g_conv_ring_cfgs[p.cfg];
-  out[3] = conv_ring_lds(mode, f.bm, f.bn, f.bk) + conv_ring_table(mode, p.single, f.bk, mode == CONV_OUTP ? p.split_stages : (K + f.bk - 1) / f.bk);
+  const ConvRingTile f = conv_ring_cfg(mode, p.cfg);
+  out[3] = conv_tile_lds(mode, p.cfg) + conv_ring_table(mode, p.single, f.bk, mode == CONV_OUTP ? p.split_stages : (K + f.bk - 1) / f.bk);
   out[4] = p.us;
 }
 

@@ -603,6 +603,62 @@ def test_three_conv_passes_on_ring_tiles(cm, cc, rng, N, C, H, F, k, s, p, G):
     test_three_conv_passes(cm, cc, rng, N, C, H, F, k, s, p, G)
 
 
+# Layers with a pass on each tile of the bf16 matrix cores (tests/test_ring_plans.py): batches and filters that the tiles do
+# not divide, last stages of a few terms, one module or pixel per tile and runs of them, two groups, Outp in pieces.
+SPLIT_LAYERS = [  # N, C, H, F, k, stride, padding, groups
+    (100, 4, 11, 194, 2, 1, 1, 1),    # Up: 128 x 128 over several modules,
+    (251, 8, 20, 128, 3, 2, 1, 1),    # of one,
+    (132, 8, 10, 192, 2, 1, 1, 2),    # 128 x 96 over several (16 terms),
+    (130, 8, 10, 141, 3, 1, 0, 1),    # of one,
+    (80, 4, 12, 65, 7, 1, 3, 1),      # 128 x 64 over several,
+    (130, 20, 18, 100, 3, 2, 0, 1),   # of one,
+    (132, 4, 15, 65, 2, 2, 0, 1),     # 64 x 64 over several,
+    (65, 8, 4, 272, 2, 1, 0, 2),      # of one
+    (96, 256, 11, 96, 2, 1, 0, 2),    # Down, in the same order, and 128 x 48
+    (130, 128, 11, 48, 2, 1, 1, 1),
+    (132, 96, 12, 48, 2, 1, 0, 1),
+    (130, 130, 8, 48, 2, 1, 1, 1),
+    (132, 100, 10, 48, 2, 1, 0, 1),
+    (130, 64, 11, 48, 2, 1, 1, 1),
+    (96, 65, 16, 48, 2, 1, 0, 1),
+    (65, 64, 15, 48, 2, 1, 0, 1),
+    (144, 130, 7, 96, 2, 1, 0, 2),
+    (130, 48, 11, 48, 2, 1, 0, 1),
+    (130, 50, 19, 199, 3, 2, 0, 1),   # Outp: 128, 96 and 64 filters by 128 taps, 64 by 64
+    (67, 256, 7, 260, 7, 2, 0, 2),
+    (256, 256, 7, 144, 7, 1, 0, 2),
+    (65, 130, 7, 176, 7, 1, 0, 1)]
+SPLIT_LOCAL = [(64, 16, 8, 65, 3, 1, 1), (70, 33, 8, 96, 3, 1, 1), (164, 33, 6, 65, 3, 1, 1), (129, 4, 8, 96, 3, 1, 1)]
+
+
+@pytest.mark.parametrize("N,C,H,F,k,s,p,G", SPLIT_LAYERS)
+def test_three_conv_passes_on_the_bf16_matrix_cores(cm, cc, rng, N, C, H, F, k, s, p, G):
+    test_three_conv_passes(cm, cc, rng, N, C, H, F, k, s, p, G)
+
+
+@pytest.mark.parametrize("N,C,H,F,k,s,p", SPLIT_LOCAL)
+def test_locally_connected_layers_on_the_bf16_matrix_cores(cm, cc, rng, N, C, H, F, k, s, p):
+    test_locally_connected_layers(cm, cc, rng, N, C, H, F, k, s, p)
+
+
+def test_infinities_on_the_bf16_matrix_cores(cm, cc, rng):
+    """A tile whose sums are not finite is computed on the fp32 instructions: infinities and NaN are where they belong, every
+    other output is as without them."""
+    N, C, H, F, k, s, p = 130, 20, 18, 100, 3, 2, 0
+    Mx = co.n_modules(H, k, s, p)
+    x, w = _f(rng.standard_normal((N, C * H * H))), _f(0.1 * rng.standard_normal((F, C * k * k)))
+    want = co.conv_up(x, w, C, Mx, p, s)
+    x[7, 5] = np.inf; x[100, 2000] = np.nan
+    up = cm.CUDAMatrix(np.full((N, F * Mx * Mx), np.nan, dtype=np.float32))
+    cc.convUp(cm.CUDAMatrix(x), cm.CUDAMatrix(w), up, Mx, p, s, C)
+    got = up.asarray()
+    with np.errstate(invalid='ignore'):
+        odd = co.conv_up(x, w, C, Mx, p, s)
+    assert np.array_equal(np.isnan(got), np.isnan(odd)) and np.array_equal(np.isinf(got), np.isinf(odd))
+    ok = np.isfinite(odd)
+    assert 0 < (~ok).sum() < 2000 and np.linalg.norm(got[ok] - want[ok]) < 1e-5 * np.linalg.norm(want)
+
+
 RING_LOCAL = [(128, 32, 6, 64, 3, 1, 1), (100, 20, 5, 48, 3, 1, 0), (67, 16, 6, 33, 3, 1, 1), (32, 36, 5, 16, 3, 2, 1),
               (45, 16, 7, 20, 5, 1, 2)]
 
@@ -682,7 +738,8 @@ OTHER_LAYERS = {  # N, C, H, F, k, stride, padding, groups
     (20, 29, 45, 10, 6, 1, 0, 1): "up",             # Up 256-row tiles, 32 columns, inside split
     (256, 2, 22, 48, 11, 1, 0, 1): "up",            # Up uniform rows, 48 columns
     (256, 2, 20, 64, 11, 1, 1, 1): "up",            # Up uniform rows, 64 columns
-    (128, 16, 48, 208, 4, 4, 0, 1): "up",           # Up uniform rows, 64 of more
+    (128, 16, 48, 208, 4, 4, 0, 1): "up",           # (bf16 matrix cores)
+    (128, 24, 16, 176, 3, 3, 0, 1): "up",           # Up uniform rows, 64 of more
 }
 OTHER_LOCAL = {   # the same of locally connected layers
     (32, 2, 6, 16, 5, 4, 1, 1): "down",             # Down merged phases, 32 columns

@@ -69,6 +69,23 @@ def test_the_layers_of_the_gpu_tests_reach_every_tile(plans):
     assert reached == want, sorted(want - reached)
 
 
+def test_the_layers_of_the_gpu_tests_reach_every_tile_of_the_bf16_matrix_cores(plans):
+    def tile(mode, N, C, H, F, k, s, p, G=1, local=False):
+        out = (ct.c_double * 5)()
+        partial = 1 if local and mode == OUTP else 0
+        plans.conv_tile(4 + mode, N, C, H, F, k, co.n_modules(H, k, s, p), s, -p, G, int(local), partial, CUS, out)
+        assert out[0] < 6 or out[3] <= 160 << 10                     # (tile and table are a workgroup's LDS)
+        return (mode, bool(out[1]), int(out[0])) if out[0] >= 6 else None
+
+    modes = (UP, DOWN, OUTP)
+    reached = {tile(mode, *layer) for mode in modes for layer in conv.SPLIT_LAYERS} - {None}
+    want = {(mode, single, t) for mode in (UP, DOWN) for single in (False, True) for t in range(6, 11)} - {(UP, False, 10), (UP, True, 10)}
+    assert reached == want | {(OUTP, False, t) for t in range(6, 10)}, sorted(want - reached)
+    assert all(any(tile(mode, *layer, local=True) for mode in modes) for layer in conv.SPLIT_LOCAL)
+    moved = [layer for layer, passes in conv.OTHER_LAYERS.items() if any(tile(dict(up=UP, down=DOWN, outp=OUTP)[n], *layer) for n in passes.split())]
+    assert moved == [(128, 16, 48, 208, 4, 4, 0, 1)]
+
+
 def test_a_workgroup_that_is_alone_on_its_cu_costs_more(plans):
     """convUp on 32 x 16 tiles: with 24 stages of table two workgroups fit the 160 KB of a CU, with 25 one."""
     two, one = (conv_tile(plans, UP, 100, colors, 24, 16, 5, 1, 0) for colors in (122, 126))
