@@ -837,3 +837,70 @@ def test_random_sequences_keep_their_bits(cm, shape, seed):
     assert len(res[0]) == len(res[1])
     for i, (w, gt) in enumerate(zip(*res)):
         assert np.array_equal(gt, w), "result %d differs" % i
+
+
+# ---- elementwise calls that wait for each other and run as one pass
+
+def _ew_call(cm, kind, x, y, t, vecs, s):
+    col, row = vecs
+    calls = {'mult': lambda: x.mult(y, target=t), 'add': lambda: x.add(y, target=t), 'subtract': lambda: x.subtract(y, target=t),
+             'divide': lambda: x.divide(y, target=t), 'sigmoid': lambda: x.apply_sigmoid(target=t), 'tanh': lambda: cm.tanh(x, target=t),
+             'exp': lambda: cm.exp(x, target=t), 'add_mult': lambda: t.add_mult(y, s), 'scale': lambda: x.mult(s, target=t),
+             'shift': lambda: x.add(s, target=t), 'gate': lambda: x.apply_rectified_linear_deriv(y, target=t),
+             'lower': lambda: x.lower_bound(s, target=t), 'col': lambda: x.mult_by_col(col, target=t), 'row': lambda: x.add_row_vec(row, target=t),
+             'add_col': lambda: x.add_col_vec(col, target=t), 'col_mult': lambda: x.add_col_mult(col, s, target=t),
+             'sum': lambda: x.sum(axis=0, target=row), 'assign': lambda: t.assign(x)}
+    calls[kind]()
+
+
+@pytest.mark.parametrize("h,w", [(1, 1), (3, 1), (1, 7), (64, 33), (65, 33), (130, 127), (1001, 37), (2052, 2049)])
+@pytest.mark.parametrize("seed", range(4))
+def test_elementwise_calls_that_wait_keep_their_bits(cm, h, w, seed):
+    """Random programs over few matrices (in place, reading what the call before wrote, through column views that overlap
+    and start at any 4-byte boundary) give the bits of the calls one by one."""
+    kinds = ['mult', 'add', 'subtract', 'divide', 'sigmoid', 'tanh', 'exp', 'add_mult', 'scale', 'shift', 'gate', 'lower', 'col', 'row',
+             'add_col', 'col_mult', 'sum', 'assign']
+    rng = np.random.default_rng([seed, h, w])
+    start = [np.asarray(rng.standard_normal((h, w + 2)), dtype=np.float32, order='F') for _ in range(5)]
+    vec = [np.asarray(rng.standard_normal(shape), dtype=np.float32, order='F') for shape in ((h, 1), (1, w))]
+    # in half of the programs the calls fit together: sources from one half of the matrices, targets in the other
+    apart = seed % 2 == 0
+    program = []
+    for _ in range(40):
+        src = rng.integers(0, 2 if apart and rng.random() < 0.8 else 5, 2)
+        dst = rng.integers(2, 5) if apart else rng.integers(0, 5)
+        offs = rng.integers(0, 3, 3) if rng.random() < 0.3 else [1, 1, 1]
+        program.append((kinds[rng.integers(0, len(kinds))], src, dst, offs, float(np.float32(rng.standard_normal()))))
+    got = []
+    for defer in (True, False):
+        cm.set_deferred_epilogues(defer)
+        try:
+            mats = [cm.CUDAMatrix(a) for a in start]
+            vecs = [cm.CUDAMatrix(v) for v in vec]
+            for kind, src, dst, offs, s in program:
+                x, y, t = (mats[i].slice(int(o), int(o) + w) for i, o in zip((src[0], src[1], dst), offs))
+                # (views of one matrix that overlap in part are not defined: such a call takes its input in place)
+                x, y = ((t if (i == dst and o != offs[2]) else v) for v, i, o in ((x, src[0], offs[0]), (y, src[1], offs[1])))
+                _ew_call(cm, kind, x, y, t, vecs, s)
+            got.append([np.array(m.asarray()) for m in mats + vecs])
+        finally:
+            cm.set_deferred_epilogues(True)
+    for a, b in zip(*got):
+        assert np.array_equal(a, b, equal_nan=True)
+
+
+def test_a_waiting_elementwise_call_is_seen_by_what_follows(cm, rng):
+    a = cm.CUDAMatrix(np.asarray(rng.standard_normal((130, 70)), dtype=np.float32, order='F'))
+    want = a.asarray() * 2
+    t = cm.empty((130, 70))
+    a.mult(2.0, target=t)
+    assert np.array_equal(t.asarray(), want)                     # a copy to the host
+    t2, s = cm.empty((130, 70)), cm.empty((1, 70))
+    a.mult(2.0, target=t2)
+    a.add(1.0, target=t)
+    t2.sum(axis=0, target=s)                                     # a reduction
+    assert np.allclose(s.asarray(), want.sum(axis=0, keepdims=True), atol=1e-4)
+    b = cm.empty((130, 70))
+    a.mult(2.0, target=b)
+    a.free_device_memory()                                       # the operand's memory goes away
+    assert np.array_equal(b.asarray(), want)
