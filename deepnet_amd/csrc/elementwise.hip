@@ -766,7 +766,7 @@ static bool ew_hold(const EwCall& c) {
   if (c.a != c.t && overlap(c.a, c.len, c.t, c.len)) return false;
   if (c.b && !(c.b == c.t && !c.bcast) && overlap(c.b, nb, c.t, c.len)) return false;
   bool joins = g_ewn > 0 && g_ewn < EW_MANY && g_ew[0].len == c.len && head_of(g_ew[0].t) == head && !g_pend.active && !g_acc.active &&
-               g_nsums == 0 && g_drop.stage == 0 && queued_calls() == 0 && batched_updates() == 0 && !dn_softmax_held();
+               g_nsums == 0 && g_drop.stage == 0 && queued_calls() == 0 && batched_updates() == 0 && !dn_softmax_held() && !dn_reductions_held();
   const float* in[EW_INPUTS + 2];
   int inputs = 0;
   auto input = [&](const float* p) {
@@ -808,6 +808,7 @@ static void flush_pending() {
   if (g_acc.active || g_nsums > 0) run_stats();
   if (g_drop.stage) run_drop(nullptr);
   dn_softmax_flush();
+  dn_reductions_flush();                           // (nothing else waits with these)
   g_flushing = false;
   refresh_pending();
 }
@@ -1117,7 +1118,7 @@ static bool update_ready() { return g_eqn > 0 && g_eq_ready; }
 static int batched_updates() { return g_ubn; }
 // anything held back besides complete updates that wait for more of their kind
 static bool held_besides_updates() {
-  return g_pend.active || g_eqn > 0 || g_acc.active || g_nsums > 0 || g_drop.stage != 0 || g_ewn > 0 || dn_softmax_held();
+  return g_pend.active || g_eqn > 0 || g_acc.active || g_nsums > 0 || g_drop.stage != 0 || g_ewn > 0 || dn_softmax_held() || dn_reductions_held();
 }
 static void refresh_pending() { dn_set_pending(held_besides_updates() || g_ubn > 0); }
 void dn_refresh_pending() { refresh_pending(); }

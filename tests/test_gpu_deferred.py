@@ -904,3 +904,65 @@ def test_a_waiting_elementwise_call_is_seen_by_what_follows(cm, rng):
     a.mult(2.0, target=b)
     a.free_device_memory()                                       # the operand's memory goes away
     assert np.array_equal(b.asarray(), want)
+
+
+# ---- sums and maxima of one matrix that wait for each other
+
+# k_col_sum_max on a wavefront and on a workgroup per column; k_colblock on 2 and 4 columns, streams and not; k_rows_one with one
+# slice (of 64, 128, 256 and more columns, streams and not) and with several; few rows, whose row sums and maxima do not wait
+RED_SHAPES = [(1, 1), (3, 5), (4, 3), (5, 130), (67, 1), (130, 70), (1001, 2047), (4097, 33), (1024, 2048), (1028, 1030), (2052, 1500), (16384, 200),
+              (16390, 260), (1024, 16640), (4100, 4100), (65540, 260), (7, 9000)]
+
+
+@pytest.mark.parametrize("h,w", RED_SHAPES)
+def test_sums_and_maxima_that_wait_keep_their_bits(cm, h, w):
+    rng = np.random.default_rng([h, w])
+    a = np.asarray(rng.standard_normal((h, w), dtype=np.float32), order='F')
+    a[rng.integers(0, h), rng.integers(0, w)] = np.inf
+    a[rng.integers(0, h), rng.integers(0, w)] = -np.inf
+    a[rng.integers(0, h), :] = -np.finfo(np.float32).max
+    a[rng.integers(0, h), rng.integers(0, w)] = np.nan
+    m = cm.CUDAMatrix(a)
+    got = []
+    for order in ('sSmM', 'MmSs', 'sm', 'MS'):
+        for defer in (True, False):
+            cm.set_deferred_epilogues(defer)
+            try:
+                out = {'s': cm.empty((1, w)), 'S': cm.empty((h, 1)), 'm': cm.empty((1, w)), 'M': cm.empty((h, 1))}
+                for k in order:
+                    (m.sum if k in 'sS' else m.max)(axis=int(k in 'SM'), target=out[k])
+                got.append({k: np.array(out[k].asarray()) for k in order})
+            finally:
+                cm.set_deferred_epilogues(True)
+        for k in order:
+            assert np.array_equal(got[-2][k], got[-1][k], equal_nan=True), (order, k)
+    # (comparisons that NaN fails, from the lowest finite value along a column and from -infinity along a row)
+    assert np.array_equal(got[0]['m'], np.fmax.reduce(a, axis=0, keepdims=True, initial=-np.finfo(np.float32).max))
+    assert np.array_equal(got[0]['M'], np.fmax.reduce(a, axis=1, keepdims=True, initial=-np.inf))
+
+
+def test_sums_and_maxima_that_do_not_go_together(cm, rng):
+    """One result twice, results that share memory with the matrix or with each other, other matrices and what reads a result."""
+    a, b = (np.asarray(rng.standard_normal((64, 48)), dtype=np.float32, order='F') for _ in range(2))
+    x, y = cm.CUDAMatrix(a), cm.CUDAMatrix(b)
+    row = cm.empty((1, 48))
+    x.sum(axis=0, target=row)
+    x.max(axis=0, target=row)                                    # over the sum
+    assert np.array_equal(row.asarray(), a.max(axis=0, keepdims=True))
+    r1, r2, col = cm.empty((1, 48)), cm.empty((1, 48)), cm.empty((64, 1))
+    x.max(axis=0, target=r1)
+    x.max(axis=0, target=r2)                                     # again, elsewhere
+    y.max(axis=1, target=col)
+    x.sum(axis=1, target=x.slice(0, 1))                          # into the matrix's first column
+    x.max(axis=0, target=row)
+    want = a.copy()
+    want[:, 0] = a.astype(np.float64).sum(axis=1)
+    assert np.array_equal(r1.asarray(), a.max(axis=0, keepdims=True)) and np.array_equal(r2.asarray(), r1.asarray())
+    assert np.array_equal(col.asarray(), b.max(axis=1, keepdims=True))
+    # (48 terms of about 1: rounding of each of the 48 additions, sums below 32)
+    assert np.allclose(row.asarray(), want.max(axis=0, keepdims=True), rtol=0, atol=48 * 32 * 2.0 ** -24)
+    x.max(axis=1, target=col)
+    x.mult(2.0)                                                  # the matrix changes behind a maximum that waits
+    y.sum(axis=1, target=col)
+    y.add_col_vec(col)                                           # reads what waits
+    assert np.allclose(y.asarray(), b + b.astype(np.float64).sum(axis=1, keepdims=True), rtol=0, atol=48 * 32 * 2.0 ** -24)
