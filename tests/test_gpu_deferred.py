@@ -662,7 +662,35 @@ def upd_reset_of_another_gradient(cm, P):
     P[0][1].mult(0.9); P[0][1].add_mult(P[0][2]); P[0][0].add_mult(P[0][1], -0.01); P[1][2].assign(0); _upd(*P[1])
 
 
-UPDS = [upd_six_in_a_row, upd_without_resets, upd_mixed_decays_and_resets, upd_eleven, upd_tied, upd_gradient_is_another_delta,
+def upd_sums_between(cm, P):
+    # a layer's weights, its biases behind a sum of their gradient (twice: the sums and the updates of a net in turn)
+    _upd(*P[0]); P[1][2].add_sums(P[2][2], axis=1, mult=0.01); _upd(*P[1])
+    P[3][2].add_sums(P[2][1], axis=1, mult=0.02); P[3][2].add_sums(P[2][2], axis=1, mult=0.5); _upd(*P[3]); _upd(*P[4], l2=0.001)
+
+
+def upd_sums_of_what_waits(cm, P):
+    _upd(*P[2]); P[1][2].add_sums(P[2][0], axis=1, mult=0.01); _upd(*P[1])           # reads the weights
+    _upd(*P[2], reset=False); P[3][2].add_sums(P[2][2], axis=1, mult=0.01); _upd(*P[3])          # reads the gradient
+    _upd(*P[2]); P[1][0].add_sums(P[2][1], axis=1, mult=0.01); _upd(*P[1])           # reads the step
+
+
+def upd_sums_into_what_waits(cm, P):
+    for i in range(3):
+        _upd(*P[1], reset=i != 1); P[1][i].add_sums(P[2][0], axis=1, mult=0.01); _upd(*P[2])
+
+
+def upd_sums_that_join_and_do_not(cm, P):
+    _upd(*P[1]); P[3][2].add_sums(P[2][0], axis=1); P[1][0].add_sums(P[2][0], axis=1); _upd(*P[3])
+    _upd(*P[0]); P[1][2].add_sums(P[2][0], axis=1); P[1][2].add_sums(P[2][1], axis=1); P[3][2].add_sums(P[2][2], axis=1)
+    P[3][2].add_sums(P[2][1], axis=1); _upd(*P[3]); _upd(*P[2])                     # four sums are launched at once
+
+
+def upd_sum_then_read(cm, P):
+    _upd(*P[0]); P[1][2].add_sums(P[2][2], axis=1, mult=0.01)
+    return P[0][0].asarray().view(np.uint32).copy()
+
+
+UPDS = [upd_sums_between, upd_sums_of_what_waits, upd_sums_into_what_waits, upd_sums_that_join_and_do_not, upd_sum_then_read, upd_six_in_a_row, upd_without_resets, upd_mixed_decays_and_resets, upd_eleven, upd_tied, upd_gradient_is_another_delta,
         upd_then_scale_that_is_no_update, upd_then_read, upd_interleaved_with_a_product, upd_reset_of_another_gradient]
 
 
