@@ -137,7 +137,7 @@ EW_CODE(FLowerS, EW_LOWERS)
 template <class F> static auto ew_scalar(const F& f, int) -> decltype(f.s) { return f.s; }
 template <class F> static float ew_scalar(const F&, long) { return 0.f; }
 // One call: t = f(a, b) over len elements, b a matrix (bcast 0, or null), a column vector (1) or a row vector (2) of an h-row one.
-struct EwCall { int code, bcast, h; const float *a, *b; float* t; float s; long long len; };
+struct EwCall { int code, bcast, h; const float *a, *b; float* t; float s; long long len; int chain = 0; };   // chain: see EwMany
 static bool ew_hold(const EwCall& c);
 
 template <int NIN, class F>
@@ -590,7 +590,8 @@ static int run_drop(cudamat* state) {
 // ---- elementwise calls on matrices of one shape wait for each other and run as one pass over their inputs: a step of a net
 // and the sequences of a program in numpy's manner apply one call after the other to the same matrix, each a read of it
 // and a launch.  A call joins when it reads nothing that a waiting one writes and writes nothing that one reads or writes
-// (another than its own input in place), so that the order of the calls within the pass does not matter; every element
+// (another than its own input in place), so that the order of the calls within the pass does not matter, or when it goes on
+// in place with the result of the last one (x.add_col_vec(b); x.lower_bound(0)), which is then written once.  Every element
 // goes through the functor of its call: the bits of the separate launches.
 #define EW_MANY 8
 #define EW_INPUTS 4
@@ -599,7 +600,7 @@ struct EwMany {
   long long len, n4;
   FastDiv fd;
   const float* in[EW_INPUTS];
-  struct { int code, bcast, a, b; const float* vec; float* t; float s; } op[EW_MANY];
+  struct { int code, bcast, a, b, chain, store; const float* vec; float* t; float s; } op[EW_MANY];   // chain: on the last result
 };
 
 template <class F> __device__ __forceinline__ float4 ew4(const F& f, float4 x, float4 y) {
@@ -632,8 +633,10 @@ __device__ __forceinline__ float4 ew_pick(int i, float4 a, float4 b, float4 c, f
 
 // Bound by memory: every input is read once and every target written once.  4096 x 4096, six calls on three inputs (add_mult,
 // mult, sigmoid, exp, mult_by_col, add_row_vec): 164 us one by one, 110 so (36 bytes an element instead of 56, 5.5 TB/s);
-// 1001 x 2047: 10 us less.  Calls are picked by uniform branches, inputs by selects.
-template <bool STREAM>
+// 1001 x 2047: 10 us less.  Calls are picked by uniform branches, inputs by selects.  CHAINS: some go on with the last result;
+// add_col_vec and lower_bound of one matrix 6.8 -> 4.4 us at 10816 x 100, 43 -> 29 at 4096 x 4096 (28 x 28 convnet, batch 100,
+// which has two such pairs: 330 -> 327 us a step).
+template <bool STREAM, bool CHAINS>
 __global__ void __launch_bounds__(EW_THREADS) k_ew_many(EwMany m) {
   const long long tid = (long long)blockIdx.x * EW_THREADS + threadIdx.x;
   if (tid < m.n4) {
@@ -648,10 +651,11 @@ __global__ void __launch_bounds__(EW_THREADS) k_ew_many(EwMany m) {
     if (m.inputs > 3) in3 = dn_ld4<STREAM>(m.in[3] + e);
     uint32_t q = 0, r = 0;
     if (m.bcast) { q = fd_div((uint32_t)e, m.fd); r = (uint32_t)e - q * m.fd.d; }
+    float4 res = none;
 #pragma unroll 1
     for (int i = 0; i < m.n; ++i) {
       const auto& o = m.op[i];
-      const float4 x = ew_pick(o.a, in0, in1, in2, in3);
+      const float4 x = CHAINS && o.chain ? res : ew_pick(o.a, in0, in1, in2, in3);
       float4 y;
       if (o.bcast) {
         uint32_t qq = q, rr = r;
@@ -665,7 +669,8 @@ __global__ void __launch_bounds__(EW_THREADS) k_ew_many(EwMany m) {
       } else {
         y = ew_pick(o.b, in0, in1, in2, in3);
       }
-      dn_st4<STREAM>(o.t + e, ew_apply(o.code, o.s, x, y));
+      res = ew_apply(o.code, o.s, x, y);
+      if (!CHAINS || o.store) dn_st4<STREAM>(o.t + e, res);
     }
   }
   // the up to three elements in front and behind
@@ -675,11 +680,13 @@ __global__ void __launch_bounds__(EW_THREADS) k_ew_many(EwMany m) {
   else if (tid - m.head < m.len - tail0) e = tail0 + (tid - m.head);
   if (e >= 0) {
     const uint32_t q = m.bcast ? fd_div((uint32_t)e, m.fd) : 0, r = m.bcast ? (uint32_t)e - q * m.fd.d : 0;
+    float res = 0.f;
 #pragma unroll 1
     for (int i = 0; i < m.n; ++i) {
       const auto& o = m.op[i];
-      const float x = m.in[o.a][e], y = o.bcast ? o.vec[o.bcast == 1 ? r : q] : m.in[o.b][e];
-      o.t[e] = ew_apply(o.code, o.s, make_float4(x, x, x, x), make_float4(y, y, y, y)).x;
+      const float x = CHAINS && o.chain ? res : m.in[o.a][e], y = o.bcast ? o.vec[o.bcast == 1 ? r : q] : m.in[o.b][e];
+      res = ew_apply(o.code, o.s, make_float4(x, x, x, x), make_float4(y, y, y, y)).x;
+      if (!CHAINS || o.store) o.t[e] = res;
     }
   }
 }
@@ -732,6 +739,7 @@ static int run_ew() {
     m.head = (int)(ht < m.len ? ht : m.len);
     m.n4 = (m.len - m.head) / 4;
     m.fd = make_fastdiv(1);
+    bool chains = false;
     auto input = [&](const float* p) {
       int i = 0;
       while (i < m.inputs && m.in[i] != p) ++i;
@@ -742,15 +750,20 @@ static int run_ew() {
       const EwCall& c = q[i];
       auto& o = m.op[i];
       o.code = c.code; o.bcast = c.bcast; o.t = c.t; o.s = c.s;
-      o.a = input(c.a);
+      chains |= c.chain != 0;
+      o.chain = c.chain; o.store = !(i + 1 < n && q[i + 1].chain);
+      o.a = c.chain ? 0 : input(c.a);
       o.b = !c.bcast && c.b ? input(c.b) : o.a;
       o.vec = c.bcast ? c.b : nullptr;
       if (c.bcast) { m.bcast = 1; m.fd = make_fastdiv((uint32_t)c.h); }
     }
     long long blocks = (m.n4 + EW_THREADS - 1) / EW_THREADS;
     if (blocks < 1) blocks = 1;
-    if (m.len >= DN_STREAM_MIN_ELEMS) hipLaunchKernelGGL((k_ew_many<true>), dim3((unsigned)blocks), dim3(EW_THREADS), 0, dn_stream(), m);
-    else hipLaunchKernelGGL((k_ew_many<false>), dim3((unsigned)blocks), dim3(EW_THREADS), 0, dn_stream(), m);
+#define EW_RUN(...) hipLaunchKernelGGL((k_ew_many<__VA_ARGS__>), dim3((unsigned)blocks), dim3(EW_THREADS), 0, dn_stream(), m)
+    if (m.len >= DN_STREAM_MIN_ELEMS) { if (chains) EW_RUN(true, true); else EW_RUN(true, false); }
+    else if (chains) EW_RUN(false, true);
+    else EW_RUN(false, false);
+#undef EW_RUN
     e = dn_launch_status();
   }
   g_no_defer = saved;
@@ -775,22 +788,26 @@ static bool ew_hold(const EwCall& c) {
       if (in[i] == p) return;
     if (inputs < EW_INPUTS + 2) in[inputs++] = p;
   };
+  const bool chain = joins && c.a == c.t && c.t == g_ew[g_ewn - 1].t && c.b != c.t;
   for (int i = 0; i < g_ewn && joins; ++i) {
     const EwCall& w = g_ew[i];
     const long long wb = w.bcast == 1 ? w.h : w.bcast == 2 ? w.len / w.h : w.len;
-    joins = !overlap(c.t, c.len, w.t, w.len) && !overlap(c.t, c.len, w.a, w.len) && !(w.b && overlap(c.t, c.len, w.b, wb)) &&
-            !overlap(c.a, c.len, w.t, w.len) && !(c.b && overlap(c.b, nb, w.t, w.len)) && !(c.bcast && w.bcast && c.h != w.h);
-    input(w.a);
+    if (!w.chain) input(w.a);
     if (!w.bcast && w.b) input(w.b);
     if (inputs > EW_INPUTS) joins = false;
+    if (c.bcast && w.bcast && c.h != w.h) joins = false;
+    if (w.t == c.t && chain) continue;             // (the last one, or one that it goes on with)
+    joins = joins && !overlap(c.t, c.len, w.t, w.len) && !overlap(c.t, c.len, w.a, w.len) && !(w.b && overlap(c.t, c.len, w.b, wb)) &&
+            !overlap(c.a, c.len, w.t, w.len) && !(c.b && overlap(c.b, nb, w.t, w.len));
   }
   if (joins) {
-    input(c.a);
+    if (!chain) input(c.a);
     if (!c.bcast && c.b) input(c.b);
     joins = inputs <= EW_INPUTS;
   }
   if (!joins) dn_flush();             // (everything that is held back is older)
-  g_ew[g_ewn++] = c;
+  g_ew[g_ewn] = c;
+  g_ew[g_ewn++].chain = joins && chain;
   dn_set_pending(true);
   return true;
 }

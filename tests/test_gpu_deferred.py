@@ -917,6 +917,36 @@ def test_elementwise_calls_that_wait_keep_their_bits(cm, h, w, seed):
         assert np.array_equal(a, b, equal_nan=True)
 
 
+@pytest.mark.parametrize("h,w", [(1, 1), (3, 1), (65, 33), (1001, 37), (2052, 2049)])
+@pytest.mark.parametrize("seed", range(4))
+def test_elementwise_calls_that_go_on_in_place_keep_their_bits(cm, h, w, seed):
+    """Chains of calls on one matrix, with others between them and with the matrix itself as the other operand."""
+    kinds = ['mult', 'add', 'subtract', 'sigmoid', 'tanh', 'add_mult', 'scale', 'shift', 'gate', 'lower', 'col', 'row', 'add_col', 'col_mult']
+    rng = np.random.default_rng([seed, h, w, 1])
+    start = [np.asarray(rng.standard_normal((h, w + 1)), dtype=np.float32, order='F') for _ in range(5)]
+    vec = [np.asarray(rng.standard_normal(shape), dtype=np.float32, order='F') for shape in ((h, 1), (1, w))]
+    program, at = [], 0
+    for _ in range(40):
+        if rng.random() < 0.3:
+            at = int(rng.integers(0, 5))
+        x, y = (at, int(rng.integers(0, 5))) if rng.random() < 0.8 else rng.integers(0, 5, 2)
+        program.append((kinds[rng.integers(0, len(kinds))], int(x), int(y), at, float(np.float32(rng.standard_normal()))))
+    got = []
+    for defer in (True, False):
+        cm.set_deferred_epilogues(defer)
+        try:
+            mats = [cm.CUDAMatrix(a) for a in start]
+            views = [m.slice(seed % 2, seed % 2 + w) for m in mats]
+            vecs = [cm.CUDAMatrix(v) for v in vec]
+            for kind, x, y, t, s in program:
+                _ew_call(cm, kind, views[x], views[y], views[t], vecs, s)
+            got.append([np.array(m.asarray()) for m in mats + vecs])
+        finally:
+            cm.set_deferred_epilogues(True)
+    for a, b in zip(*got):
+        assert np.array_equal(a, b, equal_nan=True)
+
+
 def test_a_waiting_elementwise_call_is_seen_by_what_follows(cm, rng):
     a = cm.CUDAMatrix(np.asarray(rng.standard_normal((130, 70)), dtype=np.float32, order='F'))
     want = a.asarray() * 2
