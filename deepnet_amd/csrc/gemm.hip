@@ -7,7 +7,9 @@
 // prefetched into registers while the current one is multiplied) and each of
 // its 4 wavefronts accumulates WM x WN blocks of 32 x 32.  Vector-shaped
 // products (a single row or column on either side, which is how sum(axis) and
-// add_sums arrive) go to the streaming matrix-vector kernels instead.
+// add_sums arrive) go to the streaming matrix-vector kernels instead.  Large
+// products run on the bf16 matrix cores without loss (gemm_split.h), mid-sized
+// ones on smaller tiles (gemm_ring.h).
 #include "common.h"
 #include "rowsum_jobs.h"
 #include "rng.h"
