@@ -110,8 +110,10 @@ static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows,
       if (c >= CONV_RING_CFGS) {
         // these have few rounds, and the tiles in the middle of a map, which have all taps, end the last one
         share += (1. - used) / (rounds > 1. ? rounds : 1.);
-        // (several of the smallest share a CU, and one alone shows its waits)
-        if (f.bm == 64 && f.bn == 64 && rounds <= 1.) rounds = 1.2;
+        // Few of the smallest per CU show their waits.  Measured on two cards, against the fp32 tiles: convUp and convDown take
+        // 1.10 and 1.08 times as long with one, 1.02 and 0.97 with two, 0.84 and 0.80 with more; Outp, of short reductions,
+        // 1.05 and 1.01 with one or two, 0.95 and 0.90 with three or four, 0.88 and 0.83 with more.
+        if (f.bm == 64 && f.bn == 64 && all <= (mode == CONV_OUTP ? 2 : 1) * cus) continue;
         rounds *= 1.08;                               // (what the estimates miss: they are to win by that much)
       }
       const double us = 3. + rounds * (share * per * f.stage + f.tile) + (real > 1 ? 2.5 + real * split_us : 0.);

@@ -612,8 +612,8 @@ SPLIT_LAYERS = [  # N, C, H, F, k, stride, padding, groups
     (130, 8, 10, 141, 3, 1, 0, 1),    # of one,
     (80, 4, 12, 65, 7, 1, 3, 1),      # 128 x 64 over several,
     (130, 20, 18, 100, 3, 2, 0, 1),   # of one,
-    (132, 4, 15, 65, 2, 2, 0, 1),     # 64 x 64 over several,
-    (65, 8, 4, 272, 2, 1, 0, 2),      # of one
+    (100, 4, 12, 70, 3, 1, 1, 1),     # 64 x 64 over several,
+    (87, 9, 11, 70, 2, 1, 0, 1),      # of one
     (96, 256, 11, 96, 2, 1, 0, 2),    # Down, in the same order, and 128 x 48
     (130, 128, 11, 48, 2, 1, 1, 1),
     (132, 96, 12, 48, 2, 1, 0, 1),
@@ -624,19 +624,22 @@ SPLIT_LAYERS = [  # N, C, H, F, k, stride, padding, groups
     (65, 64, 15, 48, 2, 1, 0, 1),
     (144, 130, 7, 96, 2, 1, 0, 2),
     (130, 48, 11, 48, 2, 1, 0, 1),
-    (130, 50, 19, 199, 3, 2, 0, 1),   # Outp: 128, 96 and 64 filters by 128 taps, 64 by 64
+    (130, 50, 19, 199, 3, 2, 0, 1),   # Outp: 128, 96 and 64 filters by 128 taps (64 by 64 in SPLIT_LOCAL)
     (67, 256, 7, 260, 7, 2, 0, 2),
-    (256, 256, 7, 144, 7, 1, 0, 2),
-    (65, 130, 7, 176, 7, 1, 0, 1)]
-SPLIT_LOCAL = [(64, 16, 8, 65, 3, 1, 1), (70, 33, 8, 96, 3, 1, 1), (164, 33, 6, 65, 3, 1, 1), (129, 4, 8, 96, 3, 1, 1)]
+    (256, 256, 7, 144, 7, 1, 0, 2)]
+SPLIT_LOCAL = [(70, 33, 8, 96, 3, 1, 1), (164, 33, 6, 65, 3, 1, 1), (129, 4, 8, 96, 3, 1, 1), (31, 9, 14, 65, 3, 1, 0)]
+# passes that few of the smallest tiles would make, which are slower than fp32 tiles (a wider tile for Outp of the last layer)
+FEW_SMALL_TILES = [('up', (32, 1, 17, 68, 3, 1, 0, 1)), ('up', (100, 1, 16, 176, 5, 2, 0, 1)), ('up', (80, 1, 20, 128, 5, 2, 2, 1)),
+                   ('up', (132, 4, 15, 65, 2, 2, 0, 1)), ('up', (65, 8, 4, 272, 2, 1, 0, 2)), ('outp', (65, 130, 7, 176, 7, 1, 0, 1))]
+FEW_SMALL_TILES_LOCAL = [('outp', (30, 84, 5, 64, 3, 1, 0)), ('outp', (64, 16, 8, 65, 3, 1, 1)), ('outp', (128, 68, 7, 64, 3, 1, 1))]
 
 
-@pytest.mark.parametrize("N,C,H,F,k,s,p,G", SPLIT_LAYERS)
+@pytest.mark.parametrize("N,C,H,F,k,s,p,G", SPLIT_LAYERS + [layer for _, layer in FEW_SMALL_TILES])
 def test_three_conv_passes_on_the_bf16_matrix_cores(cm, cc, rng, N, C, H, F, k, s, p, G):
     test_three_conv_passes(cm, cc, rng, N, C, H, F, k, s, p, G)
 
 
-@pytest.mark.parametrize("N,C,H,F,k,s,p", SPLIT_LOCAL)
+@pytest.mark.parametrize("N,C,H,F,k,s,p", SPLIT_LOCAL + [layer for _, layer in FEW_SMALL_TILES_LOCAL])
 def test_locally_connected_layers_on_the_bf16_matrix_cores(cm, cc, rng, N, C, H, F, k, s, p):
     test_locally_connected_layers(cm, cc, rng, N, C, H, F, k, s, p)
 

@@ -80,9 +80,13 @@ def test_the_layers_of_the_gpu_tests_reach_every_tile_of_the_bf16_matrix_cores(p
     modes = (UP, DOWN, OUTP)
     reached = {tile(mode, *layer) for mode in modes for layer in conv.SPLIT_LAYERS} - {None}
     want = {(mode, single, t) for mode in (UP, DOWN) for single in (False, True) for t in range(6, 11)} - {(UP, False, 10), (UP, True, 10)}
-    assert reached == want | {(OUTP, False, t) for t in range(6, 10)}, sorted(want - reached)
-    assert all(any(tile(mode, *layer, local=True) for mode in modes) for layer in conv.SPLIT_LOCAL)
-    moved = [layer for layer, passes in conv.OTHER_LAYERS.items() if any(tile(dict(up=UP, down=DOWN, outp=OUTP)[n], *layer) for n in passes.split())]
+    assert reached == want | {(OUTP, False, t) for t in range(6, 9)}, sorted(want - reached)
+    local = [{tile(mode, *layer, local=True) for mode in modes} - {None} for layer in conv.SPLIT_LOCAL]
+    assert all(local) and (OUTP, False, 9) in set.union(*local)
+    number = dict(up=UP, down=DOWN, outp=OUTP)
+    assert [layer for mode, layer in conv.FEW_SMALL_TILES if tile(number[mode], *layer)] == []
+    assert [tile(number[mode], *layer, local=True) for mode, layer in conv.FEW_SMALL_TILES_LOCAL] == [None, None, (OUTP, False, 8)]
+    moved = [layer for layer, passes in conv.OTHER_LAYERS.items() if any(tile(number[n], *layer) for n in passes.split())]
     assert moved == [(128, 16, 48, 208, 4, 4, 0, 1)]
 
 
