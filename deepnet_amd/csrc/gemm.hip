@@ -1081,6 +1081,7 @@ k_gemm_box_sums(const float* __restrict__ A, int lda, const float* __restrict__ 
 
 #include "gemm_ring.h"
 #include "gemm_split.h"
+static_assert(GEMM_SAMPLE_OUTPUTS == GEMM_SAMPLE_MAX_DRAWS * NUM_RND_STREAMS, "the plan knows which products may draw");
 
 __global__ void k_gemm_splitk_finish(const float* partial, int splits, float* C, int ldc, int M, int N, float alpha,
                                      float beta) {
@@ -1228,7 +1229,7 @@ static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, co
   const size_t a_bytes = (size_t)lda * (a_kc ? M : K) * sizeof(float), b_bytes = (size_t)ldb * (b_kc ? N : K) * sizeof(float);
   const RingPlan ring = K > BOX_K ? gemm_ring_plan(M, N, K, a_bytes, b_bytes, cus, a_vec && b_vec && !(a_kc && b_kc)) : RingPlan{-1, 0.};
   const RingArgs rargs = {A, B, C, (unsigned)a_bytes, (unsigned)b_bytes, lda, ldb, ldc, M, N, K, 0, 0, alpha, beta};
-  if (!epi.sample && gemm_split_wins(M, N, K, beta != 0.f, a_bytes, b_bytes, ring, cus)) {   // (samples are of fewer outputs)
+  if (gemm_split_wins(M, N, K, beta != 0.f, a_bytes, b_bytes, ring, cus)) {   // (no product that draws a sample)
     split_launch(a_kc, b_kc, rargs, epi);
     if (fused) *fused = true;
     return dn_launch_status();

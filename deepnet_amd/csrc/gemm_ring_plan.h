@@ -93,6 +93,7 @@ static inline bool gemm_slab_big(int M, int N, int K, bool beta, int cus) {
 
 #define SPLIT_BM 128       // k_gemm_split's tile, and its stage of the reduction
 #define SPLIT_BK 32
+#define GEMM_SAMPLE_OUTPUTS (16 * 96 * 128)      // most outputs of a product that draws a sample of them (gemm.hip)
 
 // What a product takes on k_gemm_split, in us: fitted to 462 measured products of 128 to 90000 per side and 32 to 5000 terms
 // (rms 8 %).  A workgroup is alone on its CU, so what a tile costs besides its stages (first trip to memory, sums to
@@ -113,6 +114,9 @@ static inline bool gemm_split_wins(int M, int N, int K, bool beta, size_t a_byte
   auto tiles = [&](int side) { return (long long)((M + side - 1) / side) * ((N + side - 1) / side); };
   const double us = split_us(M, N, K, a_bytes, b_bytes, cus);
   if (us < 0. || K < 200) return false;               // (short ones are mostly first trip and stores: 4349 x 2436 x 86 36 -> 43)
+  // A product that may draw a sample stays on the kernels that can, with and without one: the bits are those of the
+  // calls one by one.  (On 256 CUs the estimates never differ on these; on 32 they would, 435 x 429 x 2008.)
+  if ((long long)M * N <= GEMM_SAMPLE_OUTPUTS) return false;
   const int slabs = (K + 15) / 16;
   double other;
   if (ring.cfg >= 0) {

@@ -58,6 +58,16 @@ def test_the_split_products_of_the_gpu_tests_are_k_gemm_split_s(plans):
             if plans.gemm_split(*shape, CUS, 0)] == []
 
 
+@pytest.mark.parametrize("cus", [16, 32, 64, 128, 256, 304])
+def test_products_that_may_draw_a_sample_do_not_change_their_kernel_for_it(plans, cus):
+    """k_gemm_split draws no samples: it takes no product that is small enough for one, however few CUs there are."""
+    limit = 16 * 96 * 128
+    sides = [(128, n) for n in (128, 700, 1536)] + [(m, limit // m) for m in (129, 200, 298, 384, 435, 443)]
+    shapes = [s + (k,) for m, n in sides for s in ((m, n), (n, m)) for k in (200, 640, 2008, 5000)]
+    assert [s for s in shapes for vec in (0, 1) if plans.gemm_split(*s, cus, vec)] == []
+    assert cus > 32 or plans.gemm_split(444, 444, 2008, cus, 0)                  # 197136 outputs
+
+
 def test_the_layers_of_the_gpu_tests_reach_every_tile(plans):
     reached = set()
     for mode in (UP, DOWN, OUTP):
