@@ -21,7 +21,8 @@ def _bits(m):
 
 
 SHAPES = [(500, 784, 100, True), (784, 500, 100, False), (1024, 784, 128, True), (10, 1024, 128, True), (33, 17, 5, False),
-          (2048, 128, 2048, True), (64, 4096, 64, True), (3, 2, 2, False)]       # m, k, n, first operand transposed
+          (2048, 128, 2048, True), (64, 4096, 64, True), (3, 2, 2, False),       # m, k, n, first operand transposed
+          (1409, 705, 1537, True)]                                               # (k_gemm_split: tests/test_ring_plans.py)
 
 
 def _run(cm, deferred, seq, shape, seed):

@@ -183,7 +183,9 @@ def test_split_k_products(cm, rng, ta, tb):
     (10, 128, 1024, True, False),      # MLP output layer (fewer rows than a tile)
     (300, 700, 96, False, True),       # mid-sized: the single-launch kernel
     (1024, 1024, 2304, True, False),   # one 64 x 64 tile per CU and a long K: split-K, falls back to separate launches
-    (2048, 2048, 64, False, False),    # big tiles, fused epilogue
+    (2048, 2048, 64, False, False),    # many 64 x 64 tiles, fused epilogue
+    (1409, 1537, 705, True, False),    # k_gemm_split: edges on both sides,
+    (2048, 2048, 224, False, True),    # whole tiles
     (37, 1, 50, False, False),         # one output column: matrix-vector kernel
 ])
 @pytest.mark.parametrize("act", [None, 'sigmoid', 'relu', 'tanh'])

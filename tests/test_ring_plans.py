@@ -7,6 +7,7 @@ import subprocess
 import pytest
 
 import test_gpu_conv as conv
+import test_gpu_deferred as deferred
 import test_gpu_dot as dot
 from oracle import conv_oracle as co
 
@@ -53,6 +54,7 @@ def test_the_products_of_the_other_kernels_are_not_on_ring_tiles(plans):
 
 def test_the_split_products_of_the_gpu_tests_are_k_gemm_split_s(plans):
     assert [shape for shape in dot.SPLIT_SHAPES + [(1409, 1537, 705)] for vec in (0, 1) if not plans.gemm_split(*shape, CUS, vec)] == []
+    assert [s for s in deferred.SHAPES if plans.gemm_split(s[0], s[2], s[1], CUS, 0)] == deferred.SHAPES[-1:]
     # tiles have to lie inside the product, and offsets in 31 bits
     assert [shape for shape in ((127, 30000, 4000), (30000, 127, 4000), (65536, 256, 8192), (256, 65536, 8192), (4096, 4096, 199))
             if plans.gemm_split(*shape, CUS, 0)] == []
