@@ -21,6 +21,13 @@ int gemm_split(int M, int N, int K, int cus, int vec) {
   return gemm_split_wins(M, N, K, false, a, b, K > 128 ? gemm_ring_plan(M, N, K, a, b, cus, vec != 0) : RingPlan{-1, 0.}, cus);
 }
 
+// The side of k_gemm's tiles, 128 or 64, for a product of more than 128 terms; 0: another kernel's.
+int gemm_slab(int M, int N, int K, int cus, int vec) {
+  const long long tiles32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
+  if (gemm_tile(M, N, K, cus, vec) >= 0 || gemm_split(M, N, K, cus, vec) || tiles32 <= 2ll * cus) return 0;
+  return gemm_slab_big(M, N, K, false, cus) ? 128 : 64;
+}
+
 // The fp32 tile of a pass, or with mode + 4 the tile of all: out = {tile number or -1, one module or pixel per tile, splits, LDS bytes of a workgroup, us}
 void conv_tile(int mode, int N, int C, int H, int F, int k, int Mx, int s, int pad0, int G, int local, int partial_sum, int cus, double* out) {
   const int m = partial_sum ? partial_sum : Mx * Mx;

@@ -124,11 +124,11 @@ def test_large_square_products(cm, rng, n):
 
 @pytest.mark.parametrize("m,k,n", [(1000, 1001, 1000), (1001, 1000, 1000), (1000, 1000, 1001), (1003, 999, 1005), (1088, 50, 1088),
                                    (1100, 48, 1000), (1100, 47, 1000), (2000, 130, 1300), (1004, 1030, 996), (2040, 333, 2047),
-                                   (2046, 129, 2041)])
+                                   (2040, 180, 2047), (2046, 129, 2041)])
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True)])
 def test_products_on_the_tile_loop_with_any_alignment(cm, rng, m, k, n, ta, tb):
     """More 64 x 64 tiles than the single-launch kernels take: with up to 128 terms, or a number of tiles that fills the
-    CUs evenly (the last two; k_gemm_ring has the others), the loop over 16-deep slabs whose
+    CUs evenly (the last two; k_gemm_ring and k_gemm_split have the others), the loop over 16-deep slabs whose
     loads are unconditional 16-byte requests.  Leading dimensions that are not multiples of four
     floats, operands that start at an odd float of a parent buffer, tiles that hang over the edge,
     reductions of exactly three slabs (the shortest that enter the loop) and of one float less."""
@@ -501,11 +501,14 @@ RING_SHAPES = [(2001, 1003, 250), (640, 1280, 256), (65, 4095, 129), (1500, 300,
               (333, 2859, 193), (449, 2048, 960), (726, 2749, 1091)]      # 32 x 64
 
 
-# products of more than 128 terms that k_gemm_ring does not take (tests/test_ring_plans.py): strips and 32 x 32 blocks over
-# eight wavefronts, 64 x 64 tiles in whole rounds of the CUs, slices of long reductions, 128 x 128 tiles
-OTHER_SHAPES = [(5899, 21, 312), (23, 4407, 250), (4100, 31, 300), (4097, 17, 129), (2040, 2047, 333), (2048, 2048, 300),
-                (1023, 1041, 2100), (130, 129, 9000), (2041, 2046, 1060), (57, 25161, 149), (17145, 81, 135),
+# products of more than 128 terms that neither k_gemm_ring nor k_gemm_split takes (tests/test_ring_plans.py): strips and 32 x 32
+# blocks over eight wavefronts, slices of long reductions, strips of 33 to 127 on 64 x 64 tiles
+OTHER_SHAPES = [(5899, 21, 312), (23, 4407, 250), (4100, 31, 300), (4097, 17, 129),
+                (1023, 1041, 2100), (130, 129, 9000), (57, 25161, 149), (17145, 81, 135),
                 (12803, 20, 288), (29, 20740, 192)]
+# ... 64 x 64 tiles in whole rounds of the CUs (of aligned operands and others), and long strips on 128 x 128 tiles
+SLAB64_SHAPES = [(2041, 2046, 199), (2048, 2048, 160), (2040, 2047, 131)]
+SLAB128_SHAPES = [(47177, 131, 258), (172, 47119, 288), (67, 65472, 514), (65529, 36, 514)]   # (the last two with beta too)
 # the same of operands whose columns are all 16-byte aligned and not both along the reduction, which k_gemm_ring takes of others:
 # more than two 64 x 64 tiles per CU, strips of 33 to 63, one round of 32 x 32 blocks
 VEC_SHAPES = [(16388, 148, 160), (36, 9804, 204), (1652, 92, 224)]
@@ -513,10 +516,10 @@ VEC_SHAPES = [(16388, 148, 160), (36, 9804, 204), (1652, 92, 224)]
 
 # products that the host gives to k_gemm_split (tests/test_ring_plans.py): whole tiles, edges on both sides, a last stage of one
 # term and of all but one, two and more rounds of the CUs
-SPLIT_SHAPES = [(2048, 2048, 224), (1409, 1537, 705), (2049, 2047, 1001), (513, 4095, 703), (255, 16001, 200), (2048, 4095, 223), (3070, 2700, 400)]
+SPLIT_SHAPES = [(2040, 2047, 333), (2048, 2048, 300), (2041, 2046, 1060), (2048, 2048, 224), (1409, 1537, 705), (2049, 2047, 1001), (513, 4095, 703), (255, 16001, 200), (2048, 4095, 223), (3070, 2700, 400)]
 
 
-@pytest.mark.parametrize("m,n,k", RING_SHAPES + OTHER_SHAPES + VEC_SHAPES + SPLIT_SHAPES)
+@pytest.mark.parametrize("m,n,k", RING_SHAPES + OTHER_SHAPES + SLAB64_SHAPES + SLAB128_SHAPES + VEC_SHAPES + SPLIT_SHAPES)
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
 def test_products_on_tiles_that_move_back_inside(cm, rng, m, n, k, ta, tb):
     """The edges of k_gemm_ring, and of the kernels beside it: values beyond the operands (NaN here) never reach a result, and accumulating stores every

@@ -50,6 +50,9 @@ def test_the_products_of_the_other_kernels_are_not_on_ring_tiles(plans):
     assert [shape for shape in dot.OTHER_SHAPES if gemm_tile(plans, *shape)] == []
     assert [shape for shape in dot.VEC_SHAPES if gemm_tile(plans, *shape, vec=True) or not gemm_tile(plans, *shape)] == []
     assert [shape for shape in dot.RING_SHAPES if gemm_tile(plans, *shape, vec=True) != gemm_tile(plans, *shape)] == []
+    slabs = {64: dot.SLAB64_SHAPES, 128: dot.SLAB128_SHAPES}
+    assert {side: {plans.gemm_slab(*shape, CUS, vec) for shape in shapes for vec in (0, 1)} for side, shapes in slabs.items()} == {64: {64}, 128: {128}}
+    assert [shape for shape in dot.OTHER_SHAPES + dot.VEC_SHAPES + dot.RING_SHAPES for vec in (0, 1) if plans.gemm_split(*shape, CUS, vec)] == []
 
 
 def test_the_split_products_of_the_gpu_tests_are_k_gemm_split_s(plans):
