@@ -14,9 +14,11 @@ hipError_t dn_malloc(void** p, size_t bytes);
 
 // Grow-only device workspaces (slot 0: partials and scalar results; slot 1: conv patch matrix).
 void* dn_scratch(size_t bytes, int slot = 0);
+bool dn_scratch_holds(size_t bytes, int slot = 0);   // whether that much is there (launches nothing)
 
 // n 32-bit words that are zero between kernels (arrival counters); null when they cannot be had.
 unsigned* dn_zero_words(int n);
+bool dn_zero_words_hold(int n);
 // f is called when the last executable graph that this library made has been freed.
 void dn_set_no_graphs_hook(void (*f)());
 

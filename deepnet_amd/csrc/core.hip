@@ -118,6 +118,8 @@ void* dn_scratch(size_t bytes, int slot) {
   return g_scratch[slot];
 }
 
+bool dn_scratch_holds(size_t bytes, int slot) { return bytes <= g_scratch_bytes[slot]; }
+
 // ------------------------------------------------------------------ matrix memory
 // Matrices come from hipMalloc, one allocation each, as in the reference (cublasAlloc).
 // hipFree waits for the device, which stalls code that makes a temporary per step
@@ -192,6 +194,7 @@ unsigned* dn_zero_words(int n) {
   if (g_capturing) g_zero_words_recorded = true;
   return g_zero_words;
 }
+bool dn_zero_words_hold(int n) { return n <= g_zero_words_n; }
 
 // ------------------------------------------------------------------ kernels
 

@@ -941,19 +941,24 @@ static int rows_reduce_one(const float* M, int ld, int h, int w, const float* x,
 
 // The library's own workspace: arrival counters for 16384 row blocks (matrices with more rows
 // than that have no column slices), partials from the grow-only scratch.
+#define ROWS_COUNTERS 16384
 static int rows_workspace(int h, int w, RowsWorkspace* ws, int results = 1) {
-  const int kCounters = 16384;
   ws->partial = nullptr; ws->partial_floats = 0; ws->counters = nullptr; ws->num_counters = 0;
   const int splits = rows_one_splits(h, w);
   if (splits == 1) return 0;
-  unsigned* counters = dn_zero_words(kCounters);
+  unsigned* counters = dn_zero_words(ROWS_COUNTERS);
   if (!counters) return CUDA_ERROR;
   ws->partial = (float*)dn_scratch((size_t)results * splits * h * sizeof(float));
   if (!ws->partial) return CUDA_ERROR;
   ws->partial_floats = (size_t)results * splits * h;
   ws->counters = counters;
-  ws->num_counters = kCounters;
+  ws->num_counters = ROWS_COUNTERS;
   return 0;
+}
+// Whether rows_workspace would find it there.
+static bool rows_workspace_ready(int h, int w, int results) {
+  const int splits = rows_one_splits(h, w);
+  return splits == 1 || (dn_zero_words_hold(ROWS_COUNTERS) && dn_scratch_holds((size_t)results * splits * h * sizeof(float)));
 }
 
 template <int OP>
@@ -1338,17 +1343,19 @@ static inline bool spans_meet(const float* p, long long np, const float* q, long
 static bool reduction_hold(int kind, const float* M, int h, int w, float* y) {
   if (!dn_defer_enabled() || h <= 0 || w <= 0) return false;
   const int ny = kind < RED_ROW_SUM ? w : h;
-  const bool one = h >= 4 && rows_one_splits(h, w) > 0;
-  if (kind >= RED_ROW_SUM && !one) return false;           // (the two-stage kernels take their workspace when they run)
+  const bool rows = kind >= RED_ROW_SUM;
+  if (rows && !(h >= 4 && rows_one_splits(h, w) > 0)) return false;   // (the two-stage kernels take their workspace when they run)
   if (spans_meet(M, (long long)h * w, y, ny)) return false;
   bool joins = g_red.count > 0 && g_red.M == M && g_red.h == h && g_red.w == w && !g_red.y[kind];
   for (int k = 0; k < RED_KINDS && joins; ++k)
     if (g_red.y[k]) joins = !spans_meet(g_red.y[k], k < RED_ROW_SUM ? w : h, y, ny);
+  // The workspace that results along the rows take is there before the call returns; without it the call reports what it
+  // did.  (Making it launches what waits.)
+  if (rows && !rows_workspace_ready(h, w, 2)) joins = false;
   if (!joins) {
     dn_flush();                     // (what else is held back comes first)
-    // the workspace that the launch will take is there before the call returns; without it the call reports what it did
     RowsWorkspace ws;
-    if (one && rows_workspace(h, w, &ws, 2) != 0) return false;
+    if (rows && rows_workspace(h, w, &ws, 2) != 0) return false;
     g_red.M = M; g_red.h = h; g_red.w = w;
   }
   g_red.y[kind] = y;

@@ -6,6 +6,10 @@ the deferral switched off (each call its own launch) and on, and must leave the 
 matrix it touches and the same generator state; sequences that must NOT be folded (another
 matrix in between, a second bias, operands that change between the calls, reads, frees) are
 checked the same way."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -1025,3 +1029,37 @@ def test_sums_and_maxima_that_do_not_go_together(cm, rng):
     y.sum(axis=1, target=col)
     y.add_col_vec(col)                                           # reads what waits
     assert np.allclose(y.asarray(), b + b.astype(np.float64).sum(axis=1, keepdims=True), rtol=0, atol=48 * 32 * 2.0 ** -24)
+
+
+COLUMN_RESULTS = """
+import ctypes as ct, sys
+import numpy as np
+from deepnet_amd import cudamat as cm
+hip = ct.CDLL('libamdhip64.so')
+def free():
+    a, b = ct.c_size_t(), ct.c_size_t()
+    cm.cuda_sync_threads()
+    assert hip.hipMemGetInfo(ct.byref(a), ct.byref(b)) == 0
+    return a.value
+cm.cublas_init()
+x = cm.CUDAMatrix(np.ones((16448, 4096), dtype=np.float32, order='F'))
+col, row = cm.empty((16448, 1)), cm.empty((1, 4096))
+small, r3 = cm.CUDAMatrix(np.ones((3, 4096), dtype=np.float32, order='F')), cm.empty((1, 4096))
+small.sum(axis=0, target=r3); small.max(axis=0, target=r3); r3.asarray()      # (kernels are loaded)
+before = free()
+x.sum(axis=0, target=row); x.max(axis=0, target=r3)
+columns = before - free()
+assert row.asarray()[0, 5] == 16448 and r3.asarray()[0, 7] == 1
+x.sum(axis=1, target=col); x.max(axis=1, target=col)
+print(columns, before - free())
+"""
+
+
+def test_results_along_the_columns_take_no_workspace():
+    """In a process of its own (another one's workspace has grown): sums and maxima of columns leave the device memory as it
+    is, those of rows take their partial sums (16 slices of 16448 rows, two results: 2 MiB)."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, '-c', COLUMN_RESULTS], cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    columns, rows = map(int, r.stdout.split()[-2:])
+    assert columns == 0 and rows > 0
