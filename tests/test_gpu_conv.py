@@ -662,6 +662,56 @@ def test_infinities_on_the_bf16_matrix_cores(cm, cc, rng):
     assert 0 < (~ok).sum() < 2000 and np.linalg.norm(got[ok] - want[ok]) < 1e-5 * np.linalg.norm(want)
 
 
+# every tile of the bf16 matrix cores (tests/test_ring_plans.py), Outp whole and in 31 pieces
+NOT_FINITE = [('up', layer) for layer in SPLIT_LAYERS[:8]] + [('down', layer) for layer in SPLIT_LAYERS[8:18]] + \
+             [('outp', layer) for layer in SPLIT_LAYERS[18:]]
+NOT_FINITE_LOCAL = [('outp', SPLIT_LOCAL[0]), ('outp', SPLIT_LOCAL[1]), ('up', SPLIT_LOCAL[2]), ('outp', SPLIT_LOCAL[3])]
+
+
+@pytest.mark.parametrize("mode,layer", NOT_FINITE + [(mode, layer + ('local',)) for mode, layer in NOT_FINITE_LOCAL])
+def test_maps_that_are_not_finite_on_the_bf16_matrix_cores(cm, cc, rng, mode, layer):
+    """Infinities, NaN and numbers beyond 2^104 in a map (the tiles that meet them are computed again on the fp32 instructions): they
+    are where they belong, every other output is as near to 64 bits as fp32 sums are, whether its tile meets one or not."""
+    local = layer[-1] == 'local'
+    N, C, H, F, k, s, p, G = layer[:7] + (1,) if local else layer
+    Mx = co.n_modules(H, k, s, p)
+    M = Mx * Mx
+    x, y = _f(rng.standard_normal((N, C * H * H))), _f(rng.standard_normal((N, F * M)))
+    w = _f(0.1 * rng.standard_normal((F, (M if local else 1) * (C // G) * k * k)))
+    a = y if mode == 'down' else x
+    sites = M if mode == 'down' else H * H
+    at = lambda chan, site: min(chan, a.shape[1] // sites - 1) * sites + site          # of different colours or filters
+    a[7, at(0, sites // 2)] = np.inf
+    a[N - 1, at(1, sites // 3)] = -np.inf
+    a[N // 2, at(2, sites // 2 + 1)] = np.nan
+    a[3, at(3, 1)] = 3e31
+    if mode == 'up':
+        ref = lambda u, v: co.local_up(u, v, C, Mx, p, s) if local else co.conv_up(u, v, C, Mx, p, s, G)
+        ops, shape = (x, w), (N, F * M)
+        run = lambda u, v, t: cc.localUp(u, v, t, Mx, p, s, C) if local else cc.convUp(u, v, t, Mx, p, s, C, G)
+    elif mode == 'down':
+        ref = lambda u, v: co.conv_down(u, v, C, H, p, s, G)
+        ops, shape = (y, w), (N, C * H * H)
+        run = lambda u, v, t: cc.convDown(u, v, t, Mx, p, s, k, H, C, numGroups=G)
+    else:
+        ref = lambda u, v: co.local_outp(u, v, C, Mx, k, p, s) if local else co.conv_outp(u, v, C, Mx, k, p, s, G)
+        ops, shape = (x, y), w.shape
+        run = lambda u, v, t: cc.localOutp(u, v, t, Mx, p, k, s, C) if local else cc.convOutp(u, v, t, Mx, p, k, s, C, numGroups=G)
+    t = cm.CUDAMatrix(np.full(shape, 7.0, dtype=np.float32))
+    held = [cm.CUDAMatrix(o) for o in ops]
+    run(held[0], held[1], t)
+    got = t.asarray()
+    for h in held + [t]:
+        h.free_device_memory()
+    with np.errstate(invalid='ignore'):
+        want, bound = ref(*ops), ref(np.abs(ops[0]), np.abs(ops[1]))
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    ok = np.isfinite(want)
+    assert 0 < (~ok).sum() < 0.8 * ok.size and np.abs(want[ok]).max() > 1e28
+    assert _relerr(got[ok], want[ok], bound[ok] + 1e-6) < REL
+
+
 RING_LOCAL = [(128, 32, 6, 64, 3, 1, 1), (100, 20, 5, 48, 3, 1, 0), (67, 16, 6, 33, 3, 1, 1), (32, 36, 5, 16, 3, 2, 1),
               (45, 16, 7, 20, 5, 1, 2)]
 

@@ -99,6 +99,8 @@ def test_the_layers_of_the_gpu_tests_reach_every_tile_of_the_bf16_matrix_cores(p
     local = [{tile(mode, *layer, local=True) for mode in modes} - {None} for layer in conv.SPLIT_LOCAL]
     assert all(local) and (OUTP, False, 9) in set.union(*local)
     number = dict(up=UP, down=DOWN, outp=OUTP)
+    odd = {tile(number[mode], *layer) for mode, layer in conv.NOT_FINITE} | {tile(number[mode], *layer, local=True) for mode, layer in conv.NOT_FINITE_LOCAL}
+    assert odd == reached | {(OUTP, False, 9)}
     assert [layer for mode, layer in conv.FEW_SMALL_TILES if tile(number[mode], *layer)] == []
     assert [tile(number[mode], *layer, local=True) for mode, layer in conv.FEW_SMALL_TILES_LOCAL] == [None, None, (OUTP, False, 8)]
     moved = [layer for layer, passes in conv.OTHER_LAYERS.items() if any(tile(number[n], *layer) for n in passes.split())]
