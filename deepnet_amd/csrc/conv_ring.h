@@ -36,6 +36,7 @@ struct ConvRingArgs {
 template <int KIND, class Tile, int PER>
 struct ConvRingOperand : Tile {
   static_assert(Tile::KC == ((KIND >= 2 && KIND <= 4) || KIND == 7), "terms or rows in order of memory");
+  static_assert(Tile::REACH == 1 || KIND == 1 || KIND == 3 || KIND >= 5, "the table ends with the last stage");
   using Tile::NG;
   static constexpr int BK = Tile::BK;
   // an entry per group, else one per lane and stage
@@ -145,6 +146,10 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
   constexpr int EPL = Shape::EPL, LDS = Cfg::SPLIT ? Shape::LDS : 4 * Shape::LDS;
   static_assert(LDS == (Cfg::SPLIT ? conv_split_lds(BM, BN, BK) : conv_ring_lds(MODE, BM, BN, BK)) && LDS + RING_TABLE_BYTES <= RING_CU_LDS,
                 "as planned");
+  if constexpr (Cfg::SPLIT && SINGLE) {
+    constexpr int reach = OA::REACH > OB::REACH ? OA::REACH : OB::REACH;
+    static_assert(RING_AHEAD >= Shape::AHEAD + 1 + reach, "fetch() looks one stage ahead, and a lane's entry may lie reach - 1 stages behind that");
+  }
   __shared__ __attribute__((aligned(16))) char lds[LDS];
   extern __shared__ uint2 table[];
   const int tid = threadIdx.x;

@@ -50,8 +50,10 @@ static inline ConvRingTile conv_ring_cfg(int mode, int c) {
   if (c == 10 && mode != CONV_DOWN) f.bm = 0;
   return f;
 }
-// What a workgroup's LDS holds besides the two stages of its tile, which take 36 to 57 KB.  Two workgroups share a CU while
-// they take half of its 160 KB each; with a full table convUp on 32 x 16 and 16 x 32 tiles takes 82 KB and is alone.
+// What a workgroup's LDS holds besides the two stages of its tile, which take 36 to 57 KB in fp32.  Two workgroups share a CU
+// while they take half of its 160 KB each; with a full table convUp on 32 x 16 and 16 x 32 tiles takes 82 KB and is alone.  On the
+// bf16 matrix cores two stages take 48 (64 x 64) to 132 KB (128 x 48, 158 of the 160 with a full table): up to three workgroups of
+// 64 x 64 tiles share a CU while their tables are short, of the others one takes half of its registers or more and is alone.
 // The table also bounds the reduction of a convUp, with 8 bytes a term: 3328 terms on tiles over several modules, 3104 to
 // 2432 on those of one.  Longer ones (7 x 7 filters on 68 colours or more) stay on the other kernels.
 #define RING_TABLE_BYTES 26624
@@ -81,9 +83,9 @@ static inline int conv_ring_table(int mode, bool single, int bk, int stages) {  
   return ((stages < 1 ? 1 : stages) + (single ? RING_AHEAD : 0)) * conv_ring_entry(mode, single, bk);
 }
 
-// The tile (of the fp32 ones, or of those on the bf16 matrix cores) that is expected to be fastest, cfg < 0: none fits.  rows x cols outputs per period, `jobs` periods x groups x
-// chunks, K terms each, of which a tile has the share `used` on average; split_us: what adding up one more
-// partial output costs (Outp).
+// The tile (of the fp32 ones, or of those on the bf16 matrix cores) that is expected to be fastest, cfg < 0: none fits.
+// rows x cols outputs per period, `jobs` periods x groups x chunks, K terms each, of which a tile has the share `used` on
+// average; split_us: what adding up one more partial output costs (Outp).
 static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows, int cols, long long jobs, int K, double used,
                                           bool can_split, double split_us, int cus, bool bf16 = false) {
   ConvRingPlan best = {-1, 1, 0, false, 0.};

@@ -15,6 +15,7 @@ struct RingTile {
   static constexpr int BK = BK_;
   static constexpr bool KC = KC_;
   static constexpr int KPACK = KC ? 4 : 1;                 // consecutive terms of a lane's groups
+  static constexpr int REACH = 1;                          // stages that the lanes' first terms lie in
   static constexpr int NG = ROWS * BK / 4 / RING_THREADS;
   static_assert(NG * RING_THREADS * 4 == ROWS * BK, "whole groups per lane");
   static constexpr int PITCH = KC ? BK + 4 : ROWS + 4;

@@ -50,6 +50,8 @@ struct SplitTile {
   static constexpr int KPACK = KC ? 4 : NG;                // consecutive terms of a lane's groups
   static_assert(GROUPS % 64 == 0 && ROWS % 16 == 0 && BK % 32 == 0 && NT % (BK / 4) == 0, "whole wavefronts and blocks");
   static_assert(KC || ((NG == 2 || NG == 4) && ROWS % 32 == 0 && GROUPS / NG % 64 == 0), "whole packs of terms");
+  // stages that the lanes' first terms lie in: lanes that are left over have theirs behind the stage, and store nothing
+  static constexpr int REACH = KC ? 1 : 8 * ((NT - 1) / (8 * PACKS * (ROWS / 32))) / BK + 1;
   static constexpr int Q = ROWS % 64 == 0 ? 16 : 8;
   static constexpr int PLANE = BK * ROWS * 2, BYTES = 3 * PLANE;
   // group u of lane `tid`: its (first) term of the stage and its (first) row (beyond the stage for lanes that are left over)
@@ -146,6 +148,8 @@ struct SplitShape {
   static_assert(LDS >= 4 * BK * (BM + BN), "a stage in fp32");
   static constexpr int EPL = BM * BN / NT;                 // outputs per lane: e = tid + u * NT is (e % BM, e / BM)
   static_assert(EPL * NT == BM * BN, "whole tiles");
+
+  static constexpr int AHEAD = SETS - 1;                   // run() fetches stages up to nst + AHEAD
 
   struct Acc { ring_f32x4 main[TN][TM], small[TN][TM]; };
   struct Frags { split_bf16x8 a[TM], b[TN]; };             // of one plane
