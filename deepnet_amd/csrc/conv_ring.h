@@ -121,6 +121,9 @@ struct ConvRingOperand : Tile {
 //   3 -> 96 colours 11 x 11, stride 4, 224 x 224, 128 Up 260 -> 217 (128 x 96), Outp 237 -> 170 (96 x 128)
 //   32 -> 128 colours 3 x 3, 32 x 32, 128             Up 95 -> 68, Outp 91 -> 75
 //   64 -> 64 colours 5 x 5, 24 x 24, 128              Outp 128 -> 107 (64 x 128), Up and Down 124 and 118 -> 117 and 117: stay
+// Of random passes that they take, 400 took 0.84 times as long as before on one card, one of them more than 3 % longer (6 %);
+// 761 0.90 on one whose bf16 products take a sixth longer, 76 more than 3 % longer (22 % at most, 100 images, 72 -> 96 colours 5 x 5,
+// 7 x 7, Outp).  Margins for that card cost 2 % on the other.
 template <int TB, int BM_, int BN_, int BK_>
 struct ConvRingCfg {
   static constexpr int BM = BM_, BN = BN_, BK = BK_, THREADS = RING_THREADS, WAVES = 4;

@@ -8,7 +8,7 @@
 // its 4 wavefronts accumulates WM x WN blocks of 32 x 32.  Vector-shaped
 // products (a single row or column on either side, which is how sum(axis) and
 // add_sums arrive) go to the streaming matrix-vector kernels instead.  Large
-// products run on the bf16 matrix cores without loss (gemm_split.h), mid-sized
+// products run on the bf16 matrix cores, nearer to exact sums (gemm_split.h), mid-sized
 // ones on smaller tiles (gemm_ring.h).
 #include "common.h"
 #include "rowsum_jobs.h"

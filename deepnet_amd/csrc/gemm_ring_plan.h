@@ -110,7 +110,10 @@ static inline double split_us(int M, int N, int K, size_t a_bytes, size_t b_byte
 // Whether k_gemm_split is expected to be faster than `ring` or, where that is none, than k_gemm (fitted to the same
 // products).  Of the 462 it takes 99, which were 1.31 times as fast on average (4096 x 4096 x 4096 950 -> 670 us, 2048 x
 // 2048 x 2048 140 -> 90, 3904 x 800 x 1568 112 -> 70, 3278 x 3637 x 1110 279 -> 170); the best choice for each would have
-// gained 1 % more over all.  Strips of 129 to 191, whose second tile is mostly a repeat, have to win by more (169 x 54443 x
+// gained 1 % more over all.  Cards differ: of random products that it takes, 300 took 0.75 times as long as before on one (three
+// were more than 3 % slower, by 5 at most; the best choice for each 0.753 -> 0.753), 760 0.85 on one whose bf16 products take 18 %
+// longer (44, by 21 at most: 11456 x 268 x 2000 146 -> 177, 496 x 5720 x 208 17.9 -> 21.5; 0.851 -> 0.847).  Estimates that suit
+// the second card (1.37 us a stage) cost 3 % on the first and gain nothing on the second.  Strips of 129 to 191, whose second tile is mostly a repeat, have to win by more (169 x 54443 x
 // 552 117 -> 137).
 static inline bool gemm_split_wins(int M, int N, int K, bool beta, size_t a_bytes, size_t b_bytes, const RingPlan& ring, int cus) {
   auto tiles = [&](int side) { return (long long)((M + side - 1) / side) * ((N + side - 1) / side); };

@@ -5,12 +5,13 @@
 // Products that gemm_split_wins expects to be faster here (from about 160 tiles of 128 x 128 and 200 terms on): see split_tile.h for
 // the arithmetic.  8 wavefronts own a 128 x 128 tile of C, 64 x 32 outputs each; a stage is 32 terms, which are 96 MFMAs and
 // about 250 vector instructions (taking 8192 numbers apart) on each SIMD.  An MFMA leaves room for two of those and
-// every further one takes its four cycles, so the vector unit is as busy as the matrix cores; smaller tiles take more
+// every further one takes its four cycles: the matrix cores are busy for 58 % of the cycles and the issue of vector instructions
+// for 53, of which 15 are the MFMAs' own (4096 x 4096 x 4096, at a clock of 1.75 GHz).  Smaller tiles take more
 // numbers apart per product (128 x 64 tiles, two workgroups per CU, 2048 x 2048 x 2048: 111 us against 91), larger ones
 // do not fit the registers with two accumulators each (256 x 128, 4096 x 4096 x 4096: 690 us with 50 registers spilled,
 // against 670).  A stage takes 1.05 to 1.3 us, of which the MFMAs have 0.64.
-// Measured (us, operands from memory, before -> now): 4096 x 4096 x 4096 950 -> 670 (205 TFLOP/s of fp32 products), 2048 x 2048 x
-// 2048 140 -> 90, 3904 x 800 x 1568 112 -> 70, 1152 x 2208 x 256 21.4 -> 20.2.
+// Measured (us, operands from memory, before -> now): 4096 x 4096 x 4096 950 -> 670 to 705 (195 to 205 TFLOP/s of fp32 products; 770
+// to 880 on a card whose power limit leaves less), 2048 x 2048 x 2048 140 -> 90, 3904 x 800 x 1568 112 -> 70, 1152 x 2208 x 256 21.4 -> 20.2.
 // Edges, alignment and the numbering of the tiles as in k_gemm_ring.
 #define SPLIT_THREADS 512
 template <bool A_KC, bool B_KC>

@@ -1,18 +1,25 @@
-// fp32 products on the bf16 matrix cores without loss: the tile loop of the larger products (gemm_split.h) and
-// convolutions (conv_ring.h).
+// fp32 products on the bf16 matrix cores: the tile loop of the larger products (gemm_split.h) and convolutions (conv_ring.h).
 #pragma once
 #include "ring_tile.h"
 
 // Every operand is taken apart into three bf16 numbers h + m + l, each the nearest one to what is left: 8 + 8 + 8 bits of
-// mantissa, so the sum is the fp32 number itself.  A product a b is the six products hh, hm, mh, mm, hl, lh (the three
-// left out are below 2^-24 of it); hh has an accumulator of its own and the others, 2^-8 of it and less, share
-// another, which are added at the end.  Six v_mfma_f32_16x16x32_bf16 take 96 cycles where eight v_mfma_f32_16x16x4_f32 take
-// 256.  Against sums in 64 bits the results are nearer than those of the fp32 instructions, which round an accumulator for
+// mantissa, so the sum is the fp32 number itself.  A product a b is the six products hh, hm, mh, mm, hl, lh; ml, lm and ll are
+// left out, 2^-24 of it at most.  hh has an accumulator of its own and the others, 2^-8 of it and less, share another, which
+// are added at the end.  Six v_mfma_f32_16x16x32_bf16 take 96 cycles where eight v_mfma_f32_16x16x4_f32 take 256.
+// Against sums in 64 bits the results are nearer than those of the fp32 instructions, which round an accumulator for
 // every second term: the error is 0.3 to 0.4 times theirs for dense operands of 64 to 8192 terms, of both signs, of one
-// sign or rectified, 0.05 to 0.4 for samples of zeros and ones; from 0.65 to 1.0 at 64 terms of which few are not zero.
+// sign or rectified, 0.05 to 0.4 for samples of zeros and ones; from 0.65 to 1.0 at 64 terms of which few are not zero.  It is
+// larger where only one term of a sum is not zero and neither factor is short (0, 1, or 16 bits against 8, which are
+// exact): there they round once, by half an ulp at most and 0.2885 rms, and what is left out here makes it 0.954 and 0.297.  From
+// two terms on the rms error is the smaller one (ulp here / there: two terms 0.297 / 0.369, three 0.298 / 0.414, 705 2.01 / 3.12), the
+// largest up to four or so is not (two 1.7 / 1.25).  With ml and lm too, eight products, one term is as there (0.51, 0.2885)
+// and dense sums are no nearer, for 1.17 times the time (three products of a 4096 x 4096 layer 2081 -> 2432 us, convolutions of 96
+// -> 256 colours 1002 -> 1146): not done.
 // Numbers are scaled by 2^24 on the way in and results by 2^-48 on the way out: what is left of an fp32 number of any size,
 // denormals too, is then an ordinary bf16 number.  A tile whose sums are not all finite (an operand that is infinite,
-// not a number or beyond 2^104, a result beyond 2^80) is computed again on the fp32 instructions.
+// not a number or beyond 2^104, a result beyond 2^80) is computed again on the fp32 instructions, and takes 2.4 times as long as
+// on those alone (4096 x 4096 x 4096 with NaN in every tile 951 -> 2250 us, in one row 1057 -> 1080).  Loads ahead and unrolled
+// products there gave 5 to 7 % of it back and cost ordinary tiles 1 % (registers).
 #define SPLIT_IN 0x1p24f
 #define SPLIT_OUT 0x1p-48f
 

@@ -886,7 +886,8 @@ def _ew_call(cm, kind, x, y, t, vecs, s):
     calls[kind]()
 
 
-@pytest.mark.parametrize("h,w", [(1, 1), (3, 1), (1, 7), (64, 33), (65, 33), (130, 127), (1001, 37), (2052, 2049)])
+# (from 2^23 elements on calls without a common input do not wait for each other)
+@pytest.mark.parametrize("h,w", [(1, 1), (3, 1), (1, 7), (64, 33), (65, 33), (130, 127), (1001, 37), (2052, 2049), (2897, 2897)])
 @pytest.mark.parametrize("seed", range(4))
 def test_elementwise_calls_that_wait_keep_their_bits(cm, h, w, seed):
     """Random programs over few matrices (in place, reading what the call before wrote, through column views that overlap
