@@ -860,11 +860,14 @@ struct RowsWorkspace {
   int num_counters;
 };
 
+#define ROWS_COUNTERS 16384      // row blocks that the library's workspace counts
+
 // Number of column slices for the one-launch kernel: about one workgroup per CU, a slice
-// at least 256 columns wide.  0 when that would take more than ROWS_ONE_MAX_SPLITS slices
+// at least 256 columns wide, and one slice where there are more row blocks than counters.  0 when that would take more than ROWS_ONE_MAX_SPLITS slices
 // (few rows, very many columns): such shapes keep the two-stage kernels.
 static int rows_one_splits(int h, int w) {
   const int bx = (h + 63) / 64;
+  if (bx > ROWS_COUNTERS) return 1;
   const int cus = dn_num_cus();
   int splits = (cus + bx / 2) / bx;
   if (splits > w / 256) splits = w / 256;
@@ -941,7 +944,6 @@ static int rows_reduce_one(const float* M, int ld, int h, int w, const float* x,
 
 // The library's own workspace: arrival counters for 16384 row blocks (matrices with more rows
 // than that have no column slices), partials from the grow-only scratch.
-#define ROWS_COUNTERS 16384
 static int rows_workspace(int h, int w, RowsWorkspace* ws, int results = 1) {
   ws->partial = nullptr; ws->partial_floats = 0; ws->counters = nullptr; ws->num_counters = 0;
   const int splits = rows_one_splits(h, w);

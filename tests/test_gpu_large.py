@@ -53,6 +53,26 @@ def outer(cm):
         m.free_device_memory()
 
 
+def test_rows_of_more_blocks_than_the_workspace_counts(cm):
+    """16385 blocks of 64 rows: their sums and maxima (together, and each by itself) run in one slice of columns."""
+    h, w = 16384 * 64 + 64, 512
+    r = _f(np.arange(w).reshape(1, w) % 7 - 3)                    # (sums of whole numbers: exact)
+    a, R = cm.empty((h, w)), cm.CUDAMatrix(r)
+    a.assign(0.0)
+    a.add_row_vec(R)
+    results = [cm.empty((h, 1)) for _ in range(4)]
+    for t in results:
+        t.assign(np.nan)
+    a.sum(axis=1, target=results[0]); a.max(axis=1, target=results[1])
+    cm.cuda_sync_threads()
+    a.sum(axis=1, target=results[2]); cm.cuda_sync_threads()
+    a.max(axis=1, target=results[3])
+    for t, want in zip(results, (r.sum(), 3.0, r.sum(), 3.0)):
+        assert np.all(t.asarray() == want)
+    for m in results + [a, R]:
+        m.free_device_memory()
+
+
 def test_broadcasts_build_the_outer_product_exactly(cm, outer):
     a, v, r, V, R = outer
     for c, col in _cols(a).items():
