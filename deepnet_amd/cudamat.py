@@ -920,14 +920,17 @@ def set_deferred_epilogues(on):
     (the statistics of cudamat/examples/rbm_cudamat.py:73-86); an `add_dot` that stays alone takes the
     `add_sums` calls that follow it along in its launch (the gradients of a layer, deepnet/edge.py:236-242,
     layer.py:206-211), and `apply_softmax` waits for the `get_softmax_cross_entropy` and `apply_softmax_grad`
-    of its result (deepnet/softmax_layer.py:25-62).  On by default; returns the previous setting."""
+    of its result (deepnet/softmax_layer.py:25-62).  Elementwise and broadcast calls on matrices of as many elements wait for
+    each other and run as one pass, and so do `sum` and `max` along the axes of one matrix.  A call that waits is
+    launched by the next one that does not join it.  On by default; returns the previous setting."""
     return bool(_cudamat.set_deferred_epilogues(1 if on else 0))
 
 
 def launch_deferred():
     """Extension of this backend: queues the calls that are held back (see `set_deferred_epilogues`)
     and waits for nothing.  For a caller that records its own events on the NULL stream, or queues
-    other work behind the library's, and must have every call made so far in the stream."""
+    other work behind the library's, and must have every call made so far in the stream; or that turns to
+    other host work which the GPU should run beside."""
     _check(_cudamat.launch_deferred())
 
 

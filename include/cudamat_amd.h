@@ -5,7 +5,8 @@
  * code of the function it replaces in the reference's cudamat/cudamat.cu (cited
  * per group as file:line), so the reference's cudamat.py binds it unchanged
  * through ctypes.  All matrices are fp32, column-major, leading dimension
- * size[0], no padding.  Work is queued on the NULL HIP stream; only the calls
+ * size[0], no padding.  Work is queued on the NULL HIP stream, of many calls by
+ * the next one (see set_deferred_epilogues below); only the calls
  * that hand a value back to the host (copy_to_host, vdot, euclid_norm,
  * cuda_sync_threads) wait for the device.
  */
@@ -307,8 +308,14 @@ int get_softmax_cross_entropy(cudamat* mat, cudamat* labels, cudamat* target, fl
  * softmax / softmax_overwrite are held back too: get_softmax_cross_entropy and apply_softmax_grad (into another
  * matrix) of the result join it and the three run as softmax_ce_grad's launch (deepnet/softmax_layer.py:25-62).
  * set_deferred_epilogues(0) makes every call launch at once; returns the previous setting (default 1).
+ * Elementwise and broadcast calls (add_mult, mult_elementwise, add_elementwise, subtract_elementwise, divide_elementwise,
+ * mult_by_scalar, add_scalar, apply_sigmoid, apply_tanh, apply_exp, lower_bound_scalar,
+ * apply_rectified_linear_deriv, and those with a row or column vector) wait for more of them on as many elements that touch
+ * nothing the waiting ones write, or go on in place with the last one's target (up to eight, on up to four inputs; from
+ * 2^23 elements on only calls that share an input).  sum_by_axis and max_by_axis wait for each other on one matrix.
  * launch_deferred() queues what is held back now and waits for nothing: for a caller that records its own
- * events on the library's stream (the NULL stream) or queues other work behind the library's. ---- */
+ * events on the library's stream (the NULL stream), queues other work behind the library's, or does other host work
+ * that the GPU should run beside. ---- */
 int set_deferred_epilogues(int on);
 int launch_deferred(void);
 
