@@ -75,8 +75,9 @@ static inline RingPlan gemm_ring_plan(int M, int N, int K, size_t a_bytes, size_
 }
 
 // Whether k_gemm runs a product on 128 x 128 tiles (see gemm()), else on 64 x 64.  Since k_gemm_split has most of what these were
-// made for, strips are left: 33 to 191 rows or columns by more than 32768, and operands of 2 GiB and more.  Of those with 64 to
-// 127 they are still the faster ones (us, 128 x 128 / 64 x 64: 57467 x 105 x 2173 279 / 392, 119 x 61225 x 1591 278 / 324).
+// made for, strips are left: 33 to 191 rows or columns by more than 32768, and operands of 2 GiB and more.  Of 96 such strips those
+// of 64 to 127 are as fast on either on average, long reductions faster here (us, 128 x 128 / 64 x 64: 57467 x 105 x 2173 279 /
+// 392, 119 x 61225 x 1591 278 / 324); 33 to 63 would take 0.60 of the time on 64 x 64 tiles, 128 to 191 0.78.
 static inline bool gemm_slab_big(int M, int N, int K, bool beta, int cus) {
   auto tiles = [&](int side) { return (long long)((M + side - 1) / side) * ((N + side - 1) / side); };
   auto fill = [&](long long t) { return (double)t / (double)(((t + cus - 1) / cus) * cus); };

@@ -1064,3 +1064,63 @@ def test_results_along_the_columns_take_no_workspace():
     assert r.returncode == 0, r.stderr[-2000:]
     columns, rows = map(int, r.stdout.split()[-2:])
     assert columns == 0 and rows > 0
+
+
+# ---- the kinds of calls that wait, in any order
+
+def _mixed_sequence(cm, rng, pool, vecs, rows, params, n_ops):
+    M, V, R = (lambda l=l: l[rng.integers(len(l))] for l in (pool, vecs, rows))
+    scal = lambda: float(np.float32(rng.choice([0.0, 1.0, 0.5, 0.9, -0.01, 2.0])))
+    n, reads = pool[0].shape[1], []
+
+    def update():
+        w, wd, g = params[rng.integers(len(params))]
+        wd.mult(0.9); wd.add_mult(g); w.add_mult(wd, -0.01)
+        if rng.integers(2):
+            g.assign(0)
+
+    def look():
+        for q in rng.permutation(4)[:rng.integers(1, 5)]:
+            (a.sum if q < 2 else a.max)(axis=int(q % 2), target=V() if q % 2 else R())
+
+    def temporary():
+        t = cm.empty(a.shape)
+        a.add(b, target=t); t.sum(axis=0, target=R()); t.free_device_memory()
+
+    kinds = [look, look, update, update, temporary,
+             lambda: params[1][rng.integers(3)].add_sums(a, axis=1, mult=scal()), lambda: V().add_sums(a, axis=1),
+             lambda: cm.dot(pool.A.T, pool.B, target=a), lambda: a.add_dot(pool.A.T, pool.B, mult=scal()),
+             lambda: a.add_col_vec(V()), lambda: a.add_row_vec(R()), lambda: a.mult_by_col(V(), target=b), lambda: a.apply_sigmoid(target=b),
+             lambda: a.lower_bound(0), lambda: a.mult(b, target=c), lambda: a.add_mult(b, scal()), lambda: a.mult(scal()),
+             lambda: a.apply_rectified_linear_deriv(b), lambda: a.assign(b), lambda: a.apply_softmax(target=b), lambda: a.fill_with_rand(),
+             lambda: a.slice(0, 1).add_mult(V(), 0.5), lambda: a.slice(1, n).mult(0.5, target=(b if b is not a else c).slice(0, n - 1)) if c is not a else None,
+             lambda: V().mult(V(), target=V()), lambda: R().add(scal()), lambda: reads.append(_bits(R())), lambda: reads.append(_bits(a))]
+    hot = rng.integers(0, len(kinds), 10)                         # (every sequence favours some)
+    for _ in range(n_ops):
+        a, b, c = M(), M(), M()
+        kinds[hot[rng.integers(10)] if rng.random() < 0.7 else rng.integers(len(kinds))]()
+    return reads
+
+
+@pytest.mark.parametrize("shape", [(500, 100, 784), (33, 7, 20), (1024, 300, 64)], ids=lambda s: "%dx%dx%d" % s)
+@pytest.mark.parametrize("seed", range(8))
+def test_sums_maxima_updates_and_the_rest_keep_their_bits(cm, shape, seed):
+    m, n, k = shape
+    res = []
+    for deferred in (False, True):
+        cm.set_deferred_epilogues(deferred)
+        cm.CUDAMatrix.init_random(3 + seed)
+        rng = np.random.default_rng([seed, m])
+        g = lambda *d: cm.CUDAMatrix(_f(rng.standard_normal(d) * 0.5))
+        pool = _Pool(g(m, n) for _ in range(4))
+        pool.A, pool.B = g(k, m), g(k, n)
+        vecs, rows = [g(m, 1) for _ in range(3)], [g(1, n) for _ in range(3)]
+        params = [tuple(g(*d) for _ in range(3)) for d in ((m, n), (m, 1), (37, 10))]
+        reads = _mixed_sequence(cm, np.random.default_rng([seed, m, 9]), pool, vecs, rows, params, 60)
+        res.append([_bits(x) for x in list(pool) + vecs + rows + [x for t in params for x in t]] + reads)
+    cm.set_deferred_epilogues(True)
+    cm.CUDAMatrix.init_random(1)
+    assert len(res[0]) == len(res[1])
+    for i, (w, gt) in enumerate(zip(*res)):
+        nan = np.isnan(w.view(np.float32))                        # (of either sign)
+        assert np.array_equal(nan, np.isnan(gt.view(np.float32))) and np.array_equal(gt[~nan], w[~nan]), "result %d differs" % i
