@@ -33,12 +33,24 @@ hipStream_t dn_stream();
 // activation / sample calls that follow it run in the product's epilogue; dn_flush() launches what
 // is held back.  Called by everything that queues work, hands out workspaces, moves data or waits.
 void dn_flush();
+// Products that leave the held-back calls may share a launch (the open group, gemm.hip); dn_stream() and dn_flush() launch
+// it.  dn_flush_open() is dn_flush() without that: for calls whose product may still join.
+void dn_flush_open();
+void dn_close_group();
+void dn_set_group_open(bool on);
+void dn_set_group_hook(void (*f)());
+hipStream_t dn_stream_now();                // the stream, launching nothing
+void dn_group_allow(bool on);               // whether a product may go to the group instead of the stream
+bool dn_group_take_sums(const struct DnRowSumJob* jobs, int n);   // row sums that join the open group; false: launch them
+// whether dot() would run this product on k_gemm_ring
+bool dn_gemm_goes_ring(bool a_trans, bool b_trans, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float beta);
 void dn_set_pending(bool on);
 void dn_set_flush_hook(void (*f)());
 void dn_set_ext_flush_hook(void (*f)());   // the conv library's held-back calls
 void dn_set_ext_pending(bool on);
 void dn_flush_ext();
 bool dn_defer_enabled();                    // set_deferred_epilogues()
+bool dn_defer_enabled_at_all();             // ... also while the library issues the calls of a sequence itself
 void dn_refresh_pending();                  // recomputes whether anything is held back
 bool dn_softmax_held();                     // a softmax that waits for its loss and gradient (reduce.hip)
 void dn_softmax_flush();

@@ -305,7 +305,7 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
     }
   } else {
     float sum[EPL];
-    Shape::template run<false>(reinterpret_cast<float*>(lds), oa, ob, nst, 0, sum, [] {});
+    Shape::template run<false, false>(reinterpret_cast<float*>(lds), oa, ob, nst, 0, sum, [] {});
     const int em = m0 + tid % BM, en0 = n0 + tid / BM;
 #pragma unroll
     for (int u = 0; u < EPL; ++u) {

@@ -50,18 +50,36 @@ void dn_flush_ext() {
     if (g_ext_flush_hook) g_ext_flush_hook();
   }
 }
-void dn_flush() {
+// The open group (gemm.hip): products that have left the held-back calls, in call order, and share the next launch.  It is
+// older than anything that is held back, so everything that queues work closes it first.
+static bool g_group_open = false;
+static void (*g_group_hook)() = nullptr;
+void dn_set_group_hook(void (*f)()) { g_group_hook = f; }
+void dn_set_group_open(bool on) { g_group_open = on; }
+void dn_close_group() {
+  if (g_group_open) {
+    g_group_open = false;
+    if (g_group_hook) g_group_hook();
+  }
+}
+void dn_flush_open() {
   if (g_pending) {
     g_pending = false;
     if (g_flush_hook) g_flush_hook();
   }
   dn_flush_ext();
 }
+void dn_flush() {
+  dn_flush_open();
+  dn_close_group();
+}
 
 hipStream_t dn_stream() {
-  if (g_pending || g_ext_pending) dn_flush();
+  if (g_pending || g_ext_pending) dn_flush_open();
+  dn_close_group();
   return g_stream;
 }
+hipStream_t dn_stream_now() { return g_stream; }
 bool dn_capturing() { return g_capturing; }
 
 // ------------------------------------------------------------------ scratch

@@ -507,8 +507,10 @@ static int run_pending(rnd_struct* rnd, cudamat* sample) {
   refresh_pending();
   const bool saved = g_no_defer;
   g_no_defer = true;
+  dn_group_allow(true);
   const int e = dot_bias_act_impl(rnd, &p.a, &p.b, p.has_bias ? &p.bias : nullptr, &p.t, sample, p.act, p.has_gate ? &p.gate : nullptr,
                                   false, 0.f, p.has_mul ? &p.mul : nullptr);
+  dn_group_allow(false);
   g_no_defer = saved;
   return e;
 }
@@ -550,14 +552,20 @@ static int run_stats() {
   g_acc.active = false;
   g_nsums = 0;
   refresh_pending();
-  if (!p.active) return n > 0 ? dn_row_sum_jobs(jobs, n) : 0;
   const bool ta = p.a.is_trans != 0, tb = p.b.is_trans != 0;
-  if (p.paired)
-    return dn_gemm_pair_sums(ta, tb, p.m, p.n, p.k, p.alpha, p.a.data_device, p.a.size[0], p.b.data_device, p.b.size[0], p.beta,
-                             p.alpha2, p.a2.data_device, p.a2.size[0], p.b2.data_device, p.b2.size[0], p.t.data_device,
-                             p.t.size[0], jobs, n);
-  return dn_gemm_sums(ta, tb, p.m, p.n, p.k, p.alpha, p.a.data_device, p.a.size[0], p.b.data_device, p.b.size[0], p.beta,
-                      p.t.data_device, p.t.size[0], jobs, n);
+  dn_group_allow(true);
+  int e;
+  if (!p.active)
+    e = n == 0 || dn_group_take_sums(jobs, n) ? 0 : dn_row_sum_jobs(jobs, n);
+  else if (p.paired)
+    e = dn_gemm_pair_sums(ta, tb, p.m, p.n, p.k, p.alpha, p.a.data_device, p.a.size[0], p.b.data_device, p.b.size[0], p.beta,
+                          p.alpha2, p.a2.data_device, p.a2.size[0], p.b2.data_device, p.b2.size[0], p.t.data_device,
+                          p.t.size[0], jobs, n);
+  else
+    e = dn_gemm_sums(ta, tb, p.m, p.n, p.k, p.alpha, p.a.data_device, p.a.size[0], p.b.data_device, p.b.size[0], p.beta,
+                     p.t.data_device, p.t.size[0], jobs, n);
+  dn_group_allow(false);
+  return e;
 }
 
 // ---- the dropout mask: mask.fill_with_rand(); mask.greater_than(p); state.mult(mask)
@@ -864,8 +872,11 @@ bool dn_defer_dot(cudamat* mat1, cudamat* mat2, cudamat* target, float beta, flo
       g_acc.a2 = *mat1; g_acc.b2 = *mat2; g_acc.alpha2 = alpha;
       return true;
     }
-    dn_flush();
-    if (k > 128) return false;        // (pairs run as one launch only for short reductions)
+    dn_flush_open();                  // (a product that leaves may share this one's launch)
+    // pairs and sums run as one launch for short reductions, and on k_gemm_ring
+    if (k > 128 && !dn_gemm_goes_ring(mat1->is_trans != 0, mat2->is_trans != 0, m, n, k, mat1->data_device, mat1->size[0],
+                                      mat2->data_device, mat2->size[0], beta))
+      return false;
     g_acc.active = true;
     g_acc.paired = false;
     g_acc.a = *mat1; g_acc.b = *mat2; g_acc.t = *target;
@@ -875,7 +886,7 @@ bool dn_defer_dot(cudamat* mat1, cudamat* mat2, cudamat* target, float beta, flo
     return true;
   }
   if (alpha != 1.f || beta != 0.f) return false;
-  dn_flush();                         // at most one product is held back
+  dn_flush_open();                    // at most one product is held back; the one before may share this one's launch
   g_pend.active = true;
   g_pend.a = *mat1; g_pend.b = *mat2; g_pend.t = *target;
   g_pend.has_bias = false;
@@ -1042,6 +1053,7 @@ static inline bool pend_is(const cudamat* x) {
 static inline bool pend_open() { return g_pend.active && !g_no_defer; }
 
 bool dn_defer_enabled() { return g_defer_enabled && !g_no_defer; }
+bool dn_defer_enabled_at_all() { return g_defer_enabled; }
 
 extern "C" {
 
@@ -1081,7 +1093,9 @@ int apply_sigmoid(cudamat* mat, cudamat* target) {
 int apply_tanh(cudamat* mat, cudamat* target) {
   if (pend_open() && g_pend.act == 0 && !g_pend.has_mul && pend_is(mat) && pend_is(target)) {
     g_pend.act = 3;
-    return run_pending(nullptr, nullptr);
+    const int e = run_pending(nullptr, nullptr);
+    dn_close_group();
+    return e;
   }
   if (int e = check_unary(mat, target)) return e;
   return launch_ew<1>(mat->data_device, nullptr, target->data_device, dn_len(mat), FTanh{});
@@ -1095,7 +1109,9 @@ int apply_rectified_linear_deriv(cudamat* mat1, cudamat* mat2, cudamat* target) 
       !overlap(mat2->data_device, dn_len(mat2), target->data_device, dn_len(target))) {
     g_pend.gate = *mat2;
     g_pend.has_gate = true;
-    return run_pending(nullptr, nullptr);
+    const int e = run_pending(nullptr, nullptr);
+    dn_close_group();
+    return e;
   }
   if (int e = check_binary(mat1, mat2, target)) return e;
   return launch_ew<2>(mat1->data_device, mat2->data_device, target->data_device, dn_len(mat1), FReluDeriv{});

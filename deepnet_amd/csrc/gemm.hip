@@ -1152,8 +1152,150 @@ static void launch_gemm(bool a_kc, bool b_kc, dim3 grid, const float* A, int lda
 // the launch site that does so clears the count).
 static const RowSumJobs* g_side_jobs = nullptr;
 static int g_side_blocks = 0;
+static const DnRowSumJob* g_side_list = nullptr;
+static int g_side_count = 0;
 static inline bool side_jobs_fit(const GemmEpilogue& epi) {
   return g_side_blocks > 0 && g_side_jobs && !epi.bias && epi.act == GEMM_ACT_NONE && !epi.sample && !epi.gate && !epi.mul;
+}
+
+// ------------------------------------------------------------------ the open group
+// Products on k_gemm_ring that leave the held-back calls (elementwise.hip) go to the open group instead of the stream, and run
+// as one launch (k_gemm_group) when the next call comes that is no such product, or one that has to do with what they read
+// or write.  The group is older than everything that is held back and newer than all that is queued: dn_stream() launches it.
+struct GroupRange { const float* p; long long n; };
+static struct {
+  int n, nsums;
+  RingGroup G;
+  int cfg[RING_GROUP];
+  double us[RING_GROUP];                // of a tile
+  GroupRange reads[7 * RING_GROUP + 4], writes[RING_GROUP + 2];
+  int nr, nw;
+} g_group = {};
+static bool g_group_ok = false;         // (only where the caller goes on to close it, or to hold the next call back)
+void dn_group_allow(bool on) { g_group_ok = on && dn_defer_enabled_at_all(); }
+
+static bool group_meets(const GroupRange* a, int na, const GroupRange* b, int nb) {
+  for (int i = 0; i < na; ++i)
+    for (int j = 0; j < nb; ++j)
+      if (a[i].p < b[j].p + b[j].n && b[j].p < a[i].p + a[i].n) return true;
+  return false;
+}
+// Whether work with these ranges has nothing to do with what the group holds.
+static bool group_apart(const GroupRange* r, int nr, const GroupRange* w, int nw) {
+  return !group_meets(w, nw, g_group.reads, g_group.nr) && !group_meets(w, nw, g_group.writes, g_group.nw) &&
+         !group_meets(r, nr, g_group.writes, g_group.nw);
+}
+static void group_add_ranges(const GroupRange* r, int nr, const GroupRange* w, int nw) {
+  for (int i = 0; i < nr; ++i) g_group.reads[g_group.nr++] = r[i];
+  for (int i = 0; i < nw; ++i) g_group.writes[g_group.nw++] = w[i];
+}
+
+static void group_close() {
+  const int n = g_group.n, sums = g_group.nsums;
+  RingGroup G = g_group.G;
+  int cfg[RING_GROUP];
+  double us[RING_GROUP];
+  for (int i = 0; i < n; ++i) { cfg[i] = g_group.cfg[i]; us[i] = g_group.us[i]; }
+  g_group.n = g_group.nsums = g_group.nr = g_group.nw = 0;
+  G.sums_blocks = sums;
+  G.sums_end = (sums + 7) / 8 * 8;      // (a job starts on the first XCD)
+  if (n == 1 && sums == 0 && !G.job[0].second.A) {
+    ring_launch(cfg[0], (G.job[0].variant & 2) != 0, (G.job[0].variant & 1) != 0, G.job[0].g, G.job[0].epi);
+    return;
+  }
+  int c0 = cfg[0], c1 = cfg[0];         // (two different ones at most)
+  for (int i = 1; i < n; ++i) { c0 = cfg[i] < c0 ? cfg[i] : c0; c1 = cfg[i] > c1 ? cfg[i] : c1; }
+  if (c0 == c1) { if (c0 > 0) --c0; else ++c1; }
+  RingJob job[RING_GROUP];
+  int end = G.sums_end, order[RING_GROUP];
+  for (int i = 0; i < n; ++i) {
+    int at = i;
+    for (; at > 0 && us[order[at - 1]] < us[i]; --at) order[at] = order[at - 1];
+    order[at] = i;
+  }
+  for (int i = 0; i < n; ++i) {
+    const int o = order[i];
+    job[i] = G.job[o];
+    if (cfg[o] == c1) job[i].variant += 4;
+    const auto& f = g_ring_cfgs[cfg[o]];
+    job[i].g.gx = (job[i].g.M + f.bm - 1) / f.bm; job[i].g.gy = (job[i].g.N + f.bn - 1) / f.bn;
+    end += 8 * ((job[i].g.gx * job[i].g.gy + 7) / 8);
+    job[i].end = end;
+  }
+  for (int i = 0; i < n; ++i) G.job[i] = job[i];
+  ring_group_launch(c0, c1, G, end);
+}
+static const int g_group_registered = (dn_set_group_hook(group_close), 0);
+
+// Row sums that wait by themselves join the group's launch (the table has room for those of one launch).
+static bool group_take_table(const RowSumJobs& J, int blocks, const DnRowSumJob* jobs, int n) {
+  if (g_group.n == 0 || g_group.nsums > 0 || n > 4) return false;
+  GroupRange r[4], w[4];
+  for (int i = 0; i < n; ++i) {
+    r[i] = GroupRange{jobs[i].M, (long long)jobs[i].h * jobs[i].w};
+    w[i] = GroupRange{jobs[i].y, jobs[i].h};
+  }
+  if (!group_apart(r, n, w, n)) return false;
+  int nw = 1;                           // (two vectors at most)
+  for (int i = 1; i < n; ++i)
+    if (w[i].p != w[0].p) w[nw > 1 ? 1 : nw++] = w[i];
+  group_add_ranges(r, n, w, nw);
+  g_group.G.sums = J;
+  g_group.nsums = blocks;
+  return true;
+}
+bool dn_group_take_sums(const DnRowSumJob* jobs, int n) {
+  if (!g_group_ok || g_group.n == 0 || n <= 0) return false;
+  RowSumJobs J;
+  const int blocks = rows_sum_jobs_table(jobs, n, &J);
+  return blocks > 0 && group_take_table(J, blocks, jobs, n);
+}
+
+// The product `g` joins the open group, or opens one; false: it is to be launched.
+static bool group_take(const RingPlan& ring, bool a_kc, bool b_kc, const RingArgs& g, const GemmEpilogue& epi, const RingSecond& second) {
+  if (!g_group_ok || epi.sample) return false;
+  dn_flush_open();                      // (what is held back is older)
+  GroupRange r[7], w[1] = {{g.C, (long long)(g.N - 1) * g.ldc + g.M}};
+  int nr = 0;
+  r[nr++] = GroupRange{g.A, (long long)(g.a_bytes / 4)};
+  r[nr++] = GroupRange{g.B, (long long)(g.b_bytes / 4)};
+  if (second.A) {
+    r[nr++] = GroupRange{second.A, (long long)(second.a_bytes / 4)};
+    r[nr++] = GroupRange{second.B, (long long)(second.b_bytes / 4)};
+  }
+  if (epi.bias) r[nr++] = GroupRange{epi.bias, g.M};
+  if (epi.gate) r[nr++] = GroupRange{epi.gate, w[0].n};
+  if (epi.mul) r[nr++] = GroupRange{epi.mul, w[0].n};
+  // (up to four of them, on two kinds of tile)
+  int other = -1;
+  bool fits = g_group.n < RING_GROUP;
+  for (int i = 0; i < g_group.n; ++i)
+    if (g_group.cfg[i] != ring.cfg) {
+      fits = fits && (other < 0 || other == g_group.cfg[i]);
+      other = g_group.cfg[i];
+    }
+  if (!fits || !group_apart(r, nr, w, 1)) dn_close_group();
+  RingJob& J = g_group.G.job[g_group.n];
+  J.g = g; J.epi = epi; J.second = second; J.variant = 2 * (a_kc ? 1 : 0) + (b_kc ? 1 : 0);
+  g_group.cfg[g_group.n] = ring.cfg;
+  const auto& f = g_ring_cfgs[ring.cfg];
+  g_group.us[g_group.n++] = (second.A ? 2. : 1.) * f.stage * ((g.K + f.bk - 1) / f.bk);
+  group_add_ranges(r, nr, w, 1);
+  dn_set_group_open(true);
+  return true;
+}
+
+// The plan of a product that gemm() gives to k_gemm_ring; cfg < 0: another kernel.
+static RingPlan gemm_ring_route(bool a_kc, bool b_kc, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float beta) {
+  const int cus = dn_num_cus();
+  if (M <= 0 || N <= 0 || K <= BOX_K) return RingPlan{-1, 0.};
+  const bool vec = dn_aligned16(A) && lda % 4 == 0 && dn_aligned16(B) && ldb % 4 == 0 && !(a_kc && b_kc);
+  const size_t a_bytes = (size_t)lda * (a_kc ? M : K) * sizeof(float), b_bytes = (size_t)ldb * (b_kc ? N : K) * sizeof(float);
+  const RingPlan ring = gemm_ring_plan(M, N, K, a_bytes, b_bytes, cus, vec);
+  return gemm_split_wins(M, N, K, beta != 0.f, a_bytes, b_bytes, ring, cus) ? RingPlan{-1, 0.} : ring;
+}
+bool dn_gemm_goes_ring(bool a_trans, bool b_trans, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float beta) {
+  return gemm_ring_route(a_trans, !b_trans, M, N, K, A, lda, B, ldb, beta).cfg >= 0;
 }
 
 static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, const float* A, int lda, const float* B,
@@ -1235,6 +1377,12 @@ static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, co
     return dn_launch_status();
   }
   if (ring.cfg >= 0) {
+    if (group_take(ring, a_kc, b_kc, rargs, epi, RingSecond{})) {
+      if (g_side_blocks > 0 && group_take_table(*g_side_jobs, g_side_blocks, g_side_list, g_side_count)) g_side_blocks = 0;
+      if (fused) *fused = true;
+      return 0;
+    }
+    dn_stream();
     ring_launch(ring.cfg, a_kc, b_kc, rargs, epi);
     if (fused) *fused = true;
     if (sampled) *sampled = epi.sample != nullptr;
@@ -1366,13 +1514,16 @@ int dn_gemm_sums(bool a_trans, bool b_trans, int M, int N, int K, float alpha, c
   RowSumJobs J = {};
   const int jblocks = njobs > 0 ? rows_sum_jobs_table(jobs, njobs, &J) : 0;
   if (jblocks < 0) return ERROR_GENERIC;
-  dn_flush();                     // (no other product may be launched from inside this one's launch and take the sums)
+  dn_flush_open();                // (no other product may be launched from inside this one's launch and take the sums)
   g_side_jobs = &J;
   g_side_blocks = jblocks;
+  g_side_list = jobs;
+  g_side_count = njobs;
   const int e = gemm(a_trans, b_trans, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
   const bool taken = g_side_blocks == 0;
   g_side_jobs = nullptr;
-  g_side_blocks = 0;
+  g_side_list = nullptr;
+  g_side_blocks = g_side_count = 0;
   if (e) return e;
   return (taken || njobs <= 0) ? 0 : dn_row_sum_jobs(jobs, njobs);
 }
@@ -1435,6 +1586,17 @@ int dn_gemm_pair_sums(bool a_trans, bool b_trans, int M, int N, int K, float alp
 #undef GEMM_PAIR_SUMS
     }
     return dn_launch_status();
+  }
+  const RingPlan ring = g_group_ok ? gemm_ring_route(a_kc, b_kc, M, N, K, A, lda, B, ldb, beta) : RingPlan{-1, 0.};
+  if (ring.cfg >= 0 && gemm_ring_route(a_kc, b_kc, M, N, K, A2, lda2, B2, ldb2, 1.f).cfg == ring.cfg) {
+    const RingArgs g = {A, B, C, 4u * (unsigned)lda * (unsigned)(a_kc ? M : K), 4u * (unsigned)ldb * (unsigned)(b_kc ? N : K), lda, ldb, ldc, M, N, K, 0, 0,
+                        alpha, beta};
+    const RingSecond second = {A2, B2, 4u * (unsigned)lda2 * (unsigned)(a_kc ? M : K), 4u * (unsigned)ldb2 * (unsigned)(b_kc ? N : K), lda2, ldb2, alpha2};
+    const GemmEpilogue none = {nullptr, GEMM_ACT_NONE, nullptr, nullptr, nullptr, nullptr, 0u, nullptr, 0, 0.f, nullptr};
+    if (group_take(ring, a_kc, b_kc, g, none, second)) {
+      if (njobs > 0 && group_take_table(J, jblocks, jobs, njobs)) return 0;
+      return njobs > 0 ? dn_row_sum_jobs(jobs, njobs) : 0;
+    }
   }
   if (int e = gemm(a_trans, b_trans, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc)) return e;
   if (int e = gemm(a_trans, b_trans, M, N, K, alpha2, A2, lda2, B2, ldb2, 1.f, C, ldc)) return e;
@@ -1625,7 +1787,12 @@ int dot(cudamat* mat1, cudamat* mat2, cudamat* target, float beta, float alpha) 
     if (!tb) return dn_gemv_cols(B, ldb, k, n, A, C, alpha, beta);  // B is k x n
     return dn_gemv_rows(B, ldb, n, k, A, C, alpha, beta);           // B stored n x k
   }
-  return gemm(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+  // (with the products that wait for company, and not behind this call)
+  dn_group_allow(true);
+  const int e = gemm(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+  dn_group_allow(false);
+  dn_close_group();
+  return e ? e : dn_launch_status();
 }
 
 }  // extern "C"

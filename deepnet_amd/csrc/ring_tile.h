@@ -8,6 +8,18 @@
 typedef float ring_f32x16 __attribute__((ext_vector_type(16)));
 typedef float ring_f32x4 __attribute__((ext_vector_type(4)));
 
+// The lane's number.  OPAQUE: in a kernel that holds several tile loops, so that what each makes of it is not kept in registers
+// for all of them from the start (the eight loops of k_gemm_group<3, 4>: 109 -> 107 registers, of <1, 2> 128 -> 125).
+template <bool OPAQUE>
+__device__ __forceinline__ int ring_tid() {
+  unsigned t = threadIdx.x;
+  if (OPAQUE) {
+    asm volatile("" : "+v"(t));
+    __builtin_assume(t < RING_THREADS);
+  }
+  return (int)t;
+}
+
 // One operand of a stage in LDS: [row][BK + 4] when it is K-contiguous in memory (KC), [k][rows + 4] otherwise, both free
 // of bank conflicts for the order of terms that `frag` reads (pitch 4 mod 8).  A stage is NG 16-byte groups per lane.
 template <int ROWS, int BK_, bool KC_>
@@ -69,9 +81,9 @@ struct RingShape {
 
   // The tile's sums over nst >= 1 stages, lane by lane in sum[EPL].  kskip terms of the last stage are left out.
   // early(): called while the first loads are on their way.
-  template <bool SKIP, typename F>
+  template <bool SKIP, bool OPAQUE, typename F>
   __device__ __forceinline__ static void run(float* lds, OA& oa, OB& ob, int nst, int kskip, float (&sum)[EPL], F early) {
-    const int tid = threadIdx.x, lane = tid & 63, li = lane % TB, lk = lane / TB;
+    const int tid = ring_tid<OPAQUE>(), lane = tid & 63, li = lane % TB, lk = lane / TB;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wv % WM, wn = (wv / WM) % WN, ks = wv / (WM * WN);
     ring_f32x4 ra[RING_SETS][OA::NG], rb[RING_SETS][OB::NG];

@@ -294,12 +294,13 @@ int get_softmax_cross_entropy(cudamat* mat, cudamat* labels, cudamat* target, fl
  * (deepnet/parameter.py:80-106: w_delta *= momentum [; w_delta += l2 w] [; w_delta += l1 sign(w)] ;
  * w_delta += gradient ; w += -epsilon w_delta [; gradient = 0]) run as one pass when they spell it, and
  * updates that follow each other directly (up to eight, on arrays that do not overlap) as one launch.
- * A product with beta = 1 (add_dot, subtract_dot) of at most 128 terms waits for a second one of the
+ * A product with beta = 1 (add_dot, subtract_dot) of at most 128 terms, or one of mid-sized matrices, waits for a second one of the
  * same shape into the same target, and up to four add_sum_by_axis calls along the rows onto at most two
  * vectors wait for each other (the statistics of cudamat/examples/rbm_cudamat.py:73-86: six calls, two
  * launches; a product that stays alone takes the sums along in its own launch where its kernel can: a weight
  * gradient and the bias gradient of its layer, deepnet/edge.py:236-242, layer.py:206-211); same bits, call order
- * kept wherever two calls touch the same memory.  fill_with_rand is held
+ * kept wherever two calls touch the same memory.  Products of mid-sized matrices that have nothing to do with each other (up to
+ * four, sums beside them) share a launch.  fill_with_rand is held
  * back likewise: greater_than_scalar of that matrix in place and mult_elementwise of another matrix by it in
  * place (the dropout mask of deepnet/neuralnet.py:194-198) run with it as one pass, same draws and values.
  * Behind a held-back product with lower_bound_scalar(.., 0, ..) such a mask for the product's own target (at most

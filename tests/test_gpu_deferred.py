@@ -887,6 +887,60 @@ def _ew_call(cm, kind, x, y, t, vecs, s):
 
 
 # (from 2^23 elements on calls without a common input do not wait for each other)
+# sides of products on every tile of k_gemm_ring and on the kernels beside it (one of 128 terms at most is not on the ring)
+GROUP_SIDES = [[64, 130, 301, 700], [100, 200, 784, 1024], [129, 250, 1003, 1500], [16, 33, 520, 2100]]
+
+
+@pytest.mark.parametrize("sides", GROUP_SIDES, ids=lambda s: "-".join(map(str, s)))
+@pytest.mark.parametrize("seed", range(6))
+def test_products_that_share_a_launch_keep_their_bits(cm, sides, seed):
+    """Products in a row, independent ones and others (a target that the next reads or writes, an operand that the next writes, two
+    into one target), with biases, activations, gates, factors and row sums between them: the bits of one launch each."""
+    init = np.random.default_rng(99)
+    first = {(a, b, i): _f(0.1 * init.standard_normal((a, b))) for a in sides for b in sides for i in range(2)}
+    cols = {a: _f(init.standard_normal((a, 1))) for a in sides}
+
+    def run(deferred):
+        rng = np.random.default_rng(seed)
+        cm.set_deferred_epilogues(deferred)
+        mats = {k: cm.CUDAMatrix(v) for k, v in first.items()}
+        vecs = {k: cm.CUDAMatrix(v) for k, v in cols.items()}
+        pick = lambda a, b: (a, b, int(rng.integers(2)))
+        view = lambda key, trans: mats[key].T if trans else mats[key]
+        for _ in range(60):
+            m, n, k = (sides[int(i)] for i in rng.integers(0, len(sides), 3))
+            ta, tb, kind, tail = (int(rng.integers(x)) for x in (2, 2, 8, 5))
+            A, B, C = pick(k, m) if ta else pick(m, k), pick(n, k) if tb else pick(k, n), pick(m, n)
+            A2, gate, rows = pick(k, m) if ta else pick(m, k), pick(m, n), pick(m, n)
+            if C in (A, B, A2, gate):
+                continue                                     # (a product into one of its operands is no product)
+            T = mats[C]
+            if kind < 3:
+                cm.dot(view(A, ta), view(B, tb), target=T)
+                if tail == 1:
+                    T.add_col_vec(vecs[m]); T.apply_sigmoid()
+                elif tail == 2:
+                    T.apply_rectified_linear_deriv(mats[gate])
+                elif tail == 3:
+                    T.add_col_vec(vecs[m]); T.lower_bound(0)
+            elif kind < 6:
+                T.add_dot(view(A, ta), view(B, tb), mult=0.01)
+                if kind == 4:                                # ... and a second one into it
+                    T.add_dot(view(A2, ta), view(B, tb), mult=-0.01)
+                if tail < 3:
+                    vecs[m].add_sums(mats[rows], axis=1, mult=0.01)
+            elif kind == 6:
+                cm.dot(view(A, ta), view(B, tb), mult=0.5, target=T)
+            else:
+                mats[rows].mult(0.01)
+        out = [_bits(mats[k]) for k in sorted(mats)] + [_bits(vecs[k]) for k in sorted(vecs)]
+        cm.set_deferred_epilogues(True)
+        return out
+
+    for want, got in zip(run(False), run(True)):
+        assert np.array_equal(want, got)
+
+
 @pytest.mark.parametrize("h,w", [(1, 1), (3, 1), (1, 7), (64, 33), (65, 33), (130, 127), (1001, 37), (2052, 2049), (2897, 2897)])
 @pytest.mark.parametrize("seed", range(4))
 def test_elementwise_calls_that_wait_keep_their_bits(cm, h, w, seed):
