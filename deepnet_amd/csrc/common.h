@@ -39,9 +39,10 @@ void dn_flush_open();
 void dn_close_group();
 void dn_set_group_open(bool on);
 void dn_set_group_hook(void (*f)());
-hipStream_t dn_stream_now();                // the stream, launching nothing
 void dn_group_allow(bool on);               // whether a product may go to the group instead of the stream
 bool dn_group_take_sums(const struct DnRowSumJob* jobs, int n);   // row sums that join the open group; false: launch them
+// apply_rectified_linear_deriv(target, gate, target) of the target of a product of the open group joins it
+bool dn_group_take_gate(const float* target, const float* gate, int h, int w);
 // whether dot() would run this product on k_gemm_ring
 bool dn_gemm_goes_ring(bool a_trans, bool b_trans, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float beta);
 void dn_set_pending(bool on);

@@ -56,13 +56,17 @@ static bool g_group_open = false;
 static void (*g_group_hook)() = nullptr;
 void dn_set_group_hook(void (*f)()) { g_group_hook = f; }
 void dn_set_group_open(bool on) { g_group_open = on; }
+static bool g_closing = false;             // (its launches pass by what is held back, which is newer)
 void dn_close_group() {
   if (g_group_open) {
     g_group_open = false;
+    g_closing = true;
     if (g_group_hook) g_group_hook();
+    g_closing = false;
   }
 }
 void dn_flush_open() {
+  if (g_closing) return;
   if (g_pending) {
     g_pending = false;
     if (g_flush_hook) g_flush_hook();
@@ -75,11 +79,11 @@ void dn_flush() {
 }
 
 hipStream_t dn_stream() {
+  if (g_closing) return g_stream;
   if (g_pending || g_ext_pending) dn_flush_open();
   dn_close_group();
   return g_stream;
 }
-hipStream_t dn_stream_now() { return g_stream; }
 bool dn_capturing() { return g_capturing; }
 
 // ------------------------------------------------------------------ scratch

@@ -492,6 +492,7 @@ static bool g_no_defer = false;      // the library is issuing the calls of a se
 static bool g_defer_enabled = true;
 
 static void refresh_pending();      // tells the library whether anything is still held back
+static bool only_updates();
 static bool held_besides_updates();
 static inline bool pend_is(const cudamat* x);
 static inline bool pend_open();
@@ -830,7 +831,7 @@ static bool ew_hold(const EwCall& c) {
 }
 
 static bool g_flushing = false;
-// Launches the row sums that wait, and leaves the updates that wait (which have nothing to do with them).
+// Launches the row sums, or the updates, that wait, and nothing else (what else waits has nothing to do with them).
 static int run_sums_alone() {
   g_flushing = true;
   const int e = run_stats();
@@ -838,14 +839,21 @@ static int run_sums_alone() {
   dn_refresh_pending();
   return e;
 }
-static void flush_pending() {
+static int run_updates_alone() {
+  g_flushing = true;
+  const int e = run_batch();
+  g_flushing = false;
+  dn_refresh_pending();
+  return e;
+}
+static void flush_all(bool updates) {
   // (the launches below come back here through dn_stream(): what is still held back is launched by this
   // call, in order, not by theirs)
   if (g_flushing) return;
   g_flushing = true;
   if (g_ewn > 0) run_ew();                         // (nothing older waits with these)
   if (update_ready()) stash_ready(false);          // (a complete update joins the ones that wait)
-  if (batched_updates() > 0) run_batch();          // older than anything else that is held back
+  if (updates && batched_updates() > 0) run_batch();   // older than anything else that is held back
   if (g_pend.active) run_pending(nullptr, nullptr);
   if (queued_calls() > 0) run_queue(false);
   if (g_acc.active || g_nsums > 0) run_stats();
@@ -855,7 +863,28 @@ static void flush_pending() {
   g_flushing = false;
   refresh_pending();
 }
+static void flush_pending() { flush_all(true); }
+// Everything but the updates that wait, with which the rest has nothing to do; the open group stays open.
+static void flush_besides_updates() {
+  if (queued_calls() > 0 && !update_ready()) {     // (calls that may have to do with the updates)
+    dn_flush_open();
+    return;
+  }
+  flush_all(false);
+  dn_flush_ext();
+}
 static const int g_flush_registered = (dn_set_flush_hook(flush_pending), 0);
+
+// At most one product (or pair) is held back: launches what waits, or leaves it to the open group, whose launch the next
+// one may share.  Updates that have nothing to do with the product go on waiting: deepnet goes from the update of a layer's
+// parameters to the products of the one below (neuralnet.py:203-222, 300-312).
+static void flush_before_dot(const cudamat* mat1, const cudamat* mat2, const cudamat* target) {
+  if (update_ready()) stash_ready(false);
+  bool apart = true;
+  for (const cudamat* m : {mat1, mat2, target}) apart = apart && apart_from_updates(m->data_device, dn_len(m));
+  if (apart) flush_besides_updates();
+  else dn_flush_open();
+}
 
 bool dn_defer_dot(cudamat* mat1, cudamat* mat2, cudamat* target, float beta, float alpha, int m, int n, int k, int* err) {
   *err = 0;
@@ -868,11 +897,13 @@ bool dn_defer_dot(cudamat* mat1, cudamat* mat2, cudamat* target, float beta, flo
         (mat2->is_trans != 0) == (g_acc.b.is_trans != 0) &&
         !overlap(mat1->data_device, dn_len(mat1), target->data_device, dn_len(target)) &&
         !overlap(mat2->data_device, dn_len(mat2), target->data_device, dn_len(target)) && !g_acc.paired && g_nsums == 0) {
+      for (const cudamat* x : {mat1, mat2})
+        if (!apart_from_updates(x->data_device, dn_len(x))) *err = run_updates_alone();
       g_acc.paired = true;            // (stays held back: the sums of the same statistics may follow)
       g_acc.a2 = *mat1; g_acc.b2 = *mat2; g_acc.alpha2 = alpha;
       return true;
     }
-    dn_flush_open();                  // (a product that leaves may share this one's launch)
+    flush_before_dot(mat1, mat2, target);
     // pairs and sums run as one launch for short reductions, and on k_gemm_ring
     if (k > 128 && !dn_gemm_goes_ring(mat1->is_trans != 0, mat2->is_trans != 0, m, n, k, mat1->data_device, mat1->size[0],
                                       mat2->data_device, mat2->size[0], beta))
@@ -886,7 +917,7 @@ bool dn_defer_dot(cudamat* mat1, cudamat* mat2, cudamat* target, float beta, flo
     return true;
   }
   if (alpha != 1.f || beta != 0.f) return false;
-  dn_flush_open();                    // at most one product is held back; the one before may share this one's launch
+  flush_before_dot(mat1, mat2, target);
   g_pend.active = true;
   g_pend.a = *mat1; g_pend.b = *mat2; g_pend.t = *target;
   g_pend.has_bias = false;
@@ -989,9 +1020,10 @@ int mult_elementwise(cudamat* mat1, cudamat* mat2, cudamat* target) {
   if (pend_open() && g_pend.act == 0 && !g_pend.has_bias && !g_pend.has_gate && !g_pend.has_mul && g_drop.stage == 0 &&
       pend_is(mat1) && pend_is(target) && mat2->on_device && !mat2->is_trans && mat2->size[0] == target->size[0] &&
       mat2->size[1] == target->size[1] && !overlap(mat2->data_device, dn_len(mat2), target->data_device, dn_len(target))) {
+    const int e = apart_from_updates(mat2->data_device, dn_len(mat2)) ? 0 : run_updates_alone();
     g_pend.mul = *mat2;
     g_pend.has_mul = true;            // stays held back: the derivative of the activation may follow
-    return 0;
+    return e;
   }
   if (int e = check_binary(mat1, mat2, target)) return e;
   return launch_ew<2>(mat1->data_device, mat2->data_device, target->data_device, dn_len(mat1), FMul{});
@@ -1034,7 +1066,8 @@ bool dn_defer_row_sum(const float* M, float* y, int h, int w, float alpha, float
   // (us a step: 784-1024-1024-10 classifier, batch 128, 128 -> 120; 28 x 28 convnet, batch 100, 337 -> 332).
   if (!fits && update_ready()) *err = stash_ready(false);
   const bool apart = apart_from_updates(M, (long long)h * w) && apart_from_updates(y, h);
-  if (!apart || (!fits && held_besides_updates())) dn_flush();
+  if (!apart) dn_flush_open();
+  else if (!fits && held_besides_updates()) flush_besides_updates();
   else dn_flush_ext();
   g_sums[g_nsums++] = DnRowSumJob{M, y, h, w, alpha, beta, kind == 2 ? 1 : 0};
   dn_set_pending(true);
@@ -1073,9 +1106,10 @@ int launch_deferred(void) {
 int add_col_vec(cudamat* mat, cudamat* vec, cudamat* target) {
   if (pend_open() && !g_pend.has_bias && !g_pend.has_mul && g_pend.act == 0 && pend_is(mat) && pend_is(target) && vec->on_device &&
       !vec->is_trans && vec->size[0] == mat->size[0] && vec->size[1] == 1 && vec->data_device != mat->data_device) {
+    const int e = apart_from_updates(vec->data_device, dn_len(vec)) ? 0 : run_updates_alone();
     g_pend.bias = *vec;
     g_pend.has_bias = true;
-    return 0;
+    return e;
   }
   if (int e = check_colvec(mat, vec, target)) return e;
   return launch_bcast<true>(mat->data_device, vec->data_device, target->data_device, mat->size[0], mat->size[1], FAdd{});
@@ -1112,6 +1146,15 @@ int apply_rectified_linear_deriv(cudamat* mat1, cudamat* mat2, cudamat* target) 
     const int e = run_pending(nullptr, nullptr);
     dn_close_group();
     return e;
+  }
+  // ... or of one that has left for the open group, behind the layer's gradients and updates (neuralnet.py:203-222)
+  if (!g_no_defer && mat1->on_device && mat2->on_device && target->on_device && !mat1->is_trans && !mat2->is_trans && !target->is_trans &&
+      same_dims(mat1, mat2) && same_dims(mat1, target) && mat1->data_device == target->data_device && only_updates()) {
+    int e = update_ready() ? stash_ready(false) : 0;
+    if (queued_calls() == 0 && apart_from_updates(target->data_device, dn_len(target)) && apart_from_updates(mat2->data_device, dn_len(mat2)) &&
+        dn_group_take_gate(target->data_device, mat2->data_device, target->size[0], target->size[1]))
+      return e;
+    if (e) return e;
   }
   if (int e = check_binary(mat1, mat2, target)) return e;
   return launch_ew<2>(mat1->data_device, mat2->data_device, target->data_device, dn_len(mat1), FReluDeriv{});
@@ -1180,9 +1223,11 @@ static int batched_updates() { return g_ubn; }
 static bool held_besides_updates() {
   return g_pend.active || g_eqn > 0 || g_acc.active || g_nsums > 0 || g_drop.stage != 0 || g_ewn > 0 || dn_softmax_held() || dn_reductions_held();
 }
-static bool only_sums_and_updates() {
-  return !(g_pend.active || g_eqn > 0 || g_acc.active || g_drop.stage != 0 || g_ewn > 0 || dn_softmax_held() || dn_reductions_held());
+static bool only_sums_and_updates_or_queue() {
+  return !(g_pend.active || g_acc.active || g_drop.stage != 0 || g_ewn > 0 || dn_softmax_held() || dn_reductions_held());
 }
+static bool only_sums_and_updates() { return g_eqn == 0 && only_sums_and_updates_or_queue(); }
+static bool only_updates() { return only_sums_and_updates_or_queue() && g_nsums == 0; }
 // (the first n elements from p)
 static bool apart_from_updates(const float* p, long long n) {
   for (int i = 0; i < g_ubn; ++i)
@@ -1303,7 +1348,7 @@ int mult_by_scalar(cudamat* mat, float val, cudamat* target) {
       const int es = run_sums_alone();
       if (!e) e = es;
     }
-    if (held_besides_updates()) dn_flush();
+    if (held_besides_updates()) flush_besides_updates();
     if (e) return e;
     g_eq[0].kind = EQ_MULS; g_eq[0].dst = *mat; g_eq[0].src = *mat; g_eq[0].s = val;
     g_eqn = 1;

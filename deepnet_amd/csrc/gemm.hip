@@ -11,6 +11,7 @@
 // products run on the bf16 matrix cores, nearer to exact sums (gemm_split.h), mid-sized
 // ones on smaller tiles (gemm_ring.h).
 #include "common.h"
+#include <tuple>
 #include "rowsum_jobs.h"
 #include "rng.h"
 #include "wide_math.h"
@@ -1145,9 +1146,6 @@ static void launch_gemm(bool a_kc, bool b_kc, dim3 grid, const float* A, int lda
 #undef GEMM_GO
 }
 
-// Host-side dispatch shared with tests through dot().
-// epi: what to append to each output (bias / activation); *fused tells the caller whether
-// the launch could carry it (the split-K and empty-K paths cannot).
 // Sums along the rows that the next product may take along in its launch (dn_gemm_sums sets them;
 // the launch site that does so clears the count).
 static const RowSumJobs* g_side_jobs = nullptr;
@@ -1158,163 +1156,17 @@ static inline bool side_jobs_fit(const GemmEpilogue& epi) {
   return g_side_blocks > 0 && g_side_jobs && !epi.bias && epi.act == GEMM_ACT_NONE && !epi.sample && !epi.gate && !epi.mul;
 }
 
-// ------------------------------------------------------------------ the open group
-// Products on k_gemm_ring that leave the held-back calls (elementwise.hip) go to the open group instead of the stream, and run
-// as one launch (k_gemm_group) when the next call comes that is no such product, or one that has to do with what they read
-// or write.  The group is older than everything that is held back and newer than all that is queued: dn_stream() launches it.
-struct GroupRange { const float* p; long long n; };
-static struct {
-  int n, nsums;
-  RingGroup G;
-  int cfg[RING_GROUP];
-  double us[RING_GROUP];                // of a tile
-  GroupRange reads[7 * RING_GROUP + 4], writes[RING_GROUP + 2];
-  int nr, nw;
-} g_group = {};
-static bool g_group_ok = false;         // (only where the caller goes on to close it, or to hold the next call back)
-void dn_group_allow(bool on) { g_group_ok = on && dn_defer_enabled_at_all(); }
-
-static bool group_meets(const GroupRange* a, int na, const GroupRange* b, int nb) {
-  for (int i = 0; i < na; ++i)
-    for (int j = 0; j < nb; ++j)
-      if (a[i].p < b[j].p + b[j].n && b[j].p < a[i].p + a[i].n) return true;
-  return false;
-}
-// Whether work with these ranges has nothing to do with what the group holds.
-static bool group_apart(const GroupRange* r, int nr, const GroupRange* w, int nw) {
-  return !group_meets(w, nw, g_group.reads, g_group.nr) && !group_meets(w, nw, g_group.writes, g_group.nw) &&
-         !group_meets(r, nr, g_group.writes, g_group.nw);
-}
-static void group_add_ranges(const GroupRange* r, int nr, const GroupRange* w, int nw) {
-  for (int i = 0; i < nr; ++i) g_group.reads[g_group.nr++] = r[i];
-  for (int i = 0; i < nw; ++i) g_group.writes[g_group.nw++] = w[i];
-}
-
-static void group_close() {
-  const int n = g_group.n, sums = g_group.nsums;
-  RingGroup G = g_group.G;
-  int cfg[RING_GROUP];
-  double us[RING_GROUP];
-  for (int i = 0; i < n; ++i) { cfg[i] = g_group.cfg[i]; us[i] = g_group.us[i]; }
-  g_group.n = g_group.nsums = g_group.nr = g_group.nw = 0;
-  G.sums_blocks = sums;
-  G.sums_end = (sums + 7) / 8 * 8;      // (a job starts on the first XCD)
-  if (n == 1 && sums == 0 && !G.job[0].second.A) {
-    ring_launch(cfg[0], (G.job[0].variant & 2) != 0, (G.job[0].variant & 1) != 0, G.job[0].g, G.job[0].epi);
-    return;
-  }
-  int c0 = cfg[0], c1 = cfg[0];         // (two different ones at most)
-  for (int i = 1; i < n; ++i) { c0 = cfg[i] < c0 ? cfg[i] : c0; c1 = cfg[i] > c1 ? cfg[i] : c1; }
-  if (c0 == c1) { if (c0 > 0) --c0; else ++c1; }
-  RingJob job[RING_GROUP];
-  int end = G.sums_end, order[RING_GROUP];
-  for (int i = 0; i < n; ++i) {
-    int at = i;
-    for (; at > 0 && us[order[at - 1]] < us[i]; --at) order[at] = order[at - 1];
-    order[at] = i;
-  }
-  for (int i = 0; i < n; ++i) {
-    const int o = order[i];
-    job[i] = G.job[o];
-    if (cfg[o] == c1) job[i].variant += 4;
-    const auto& f = g_ring_cfgs[cfg[o]];
-    job[i].g.gx = (job[i].g.M + f.bm - 1) / f.bm; job[i].g.gy = (job[i].g.N + f.bn - 1) / f.bn;
-    end += 8 * ((job[i].g.gx * job[i].g.gy + 7) / 8);
-    job[i].end = end;
-  }
-  for (int i = 0; i < n; ++i) G.job[i] = job[i];
-  ring_group_launch(c0, c1, G, end);
-}
-static const int g_group_registered = (dn_set_group_hook(group_close), 0);
-
-// Row sums that wait by themselves join the group's launch (the table has room for those of one launch).
-static bool group_take_table(const RowSumJobs& J, int blocks, const DnRowSumJob* jobs, int n) {
-  if (g_group.n == 0 || g_group.nsums > 0 || n > 4) return false;
-  GroupRange r[4], w[4];
-  for (int i = 0; i < n; ++i) {
-    r[i] = GroupRange{jobs[i].M, (long long)jobs[i].h * jobs[i].w};
-    w[i] = GroupRange{jobs[i].y, jobs[i].h};
-  }
-  if (!group_apart(r, n, w, n)) return false;
-  int nw = 1;                           // (two vectors at most)
-  for (int i = 1; i < n; ++i)
-    if (w[i].p != w[0].p) w[nw > 1 ? 1 : nw++] = w[i];
-  group_add_ranges(r, n, w, nw);
-  g_group.G.sums = J;
-  g_group.nsums = blocks;
-  return true;
-}
-bool dn_group_take_sums(const DnRowSumJob* jobs, int n) {
-  if (!g_group_ok || g_group.n == 0 || n <= 0) return false;
-  RowSumJobs J;
-  const int blocks = rows_sum_jobs_table(jobs, n, &J);
-  return blocks > 0 && group_take_table(J, blocks, jobs, n);
-}
-
-// The product `g` joins the open group, or opens one; false: it is to be launched.
-static bool group_take(const RingPlan& ring, bool a_kc, bool b_kc, const RingArgs& g, const GemmEpilogue& epi, const RingSecond& second) {
-  if (!g_group_ok || epi.sample) return false;
-  dn_flush_open();                      // (what is held back is older)
-  GroupRange r[7], w[1] = {{g.C, (long long)(g.N - 1) * g.ldc + g.M}};
-  int nr = 0;
-  r[nr++] = GroupRange{g.A, (long long)(g.a_bytes / 4)};
-  r[nr++] = GroupRange{g.B, (long long)(g.b_bytes / 4)};
-  if (second.A) {
-    r[nr++] = GroupRange{second.A, (long long)(second.a_bytes / 4)};
-    r[nr++] = GroupRange{second.B, (long long)(second.b_bytes / 4)};
-  }
-  if (epi.bias) r[nr++] = GroupRange{epi.bias, g.M};
-  if (epi.gate) r[nr++] = GroupRange{epi.gate, w[0].n};
-  if (epi.mul) r[nr++] = GroupRange{epi.mul, w[0].n};
-  // (up to four of them, on two kinds of tile)
-  int other = -1;
-  bool fits = g_group.n < RING_GROUP;
-  for (int i = 0; i < g_group.n; ++i)
-    if (g_group.cfg[i] != ring.cfg) {
-      fits = fits && (other < 0 || other == g_group.cfg[i]);
-      other = g_group.cfg[i];
-    }
-  if (!fits || !group_apart(r, nr, w, 1)) dn_close_group();
-  RingJob& J = g_group.G.job[g_group.n];
-  J.g = g; J.epi = epi; J.second = second; J.variant = 2 * (a_kc ? 1 : 0) + (b_kc ? 1 : 0);
-  g_group.cfg[g_group.n] = ring.cfg;
-  const auto& f = g_ring_cfgs[ring.cfg];
-  g_group.us[g_group.n++] = (second.A ? 2. : 1.) * f.stage * ((g.K + f.bk - 1) / f.bk);
-  group_add_ranges(r, nr, w, 1);
-  dn_set_group_open(true);
-  return true;
-}
-
-// The plan of a product that gemm() gives to k_gemm_ring; cfg < 0: another kernel.
-static RingPlan gemm_ring_route(bool a_kc, bool b_kc, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float beta) {
+// ------------------------------------------------------------------ which kernel
+// K = 0; the whole reduction at once; bf16 matrix cores; ring of stages; blocks of 16 x 16 and of 32 x 32 over the wavefronts
+// of a workgroup; slabs (perhaps of a split reduction, summed by a second kernel)
+enum GemmKind { GEMM_EMPTY, GEMM_BOX, GEMM_SPLIT, GEMM_RING, GEMM_T16, GEMM_SMALL, GEMM_SLAB };
+struct GemmPlan { GemmKind kind; RingPlan ring; bool heavy; };
+static GemmPlan gemm_plan(bool a_kc, bool b_kc, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float beta) {
+  const RingPlan no_ring = {-1, 0.};
+  if (K <= 0) return GemmPlan{GEMM_EMPTY, no_ring, false};
   const int cus = dn_num_cus();
-  if (M <= 0 || N <= 0 || K <= BOX_K) return RingPlan{-1, 0.};
-  const bool vec = dn_aligned16(A) && lda % 4 == 0 && dn_aligned16(B) && ldb % 4 == 0 && !(a_kc && b_kc);
-  const size_t a_bytes = (size_t)lda * (a_kc ? M : K) * sizeof(float), b_bytes = (size_t)ldb * (b_kc ? N : K) * sizeof(float);
-  const RingPlan ring = gemm_ring_plan(M, N, K, a_bytes, b_bytes, cus, vec);
-  return gemm_split_wins(M, N, K, beta != 0.f, a_bytes, b_bytes, ring, cus) ? RingPlan{-1, 0.} : ring;
-}
-bool dn_gemm_goes_ring(bool a_trans, bool b_trans, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float beta) {
-  return gemm_ring_route(a_trans, !b_trans, M, N, K, A, lda, B, ldb, beta).cfg >= 0;
-}
-
-static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, const float* A, int lda, const float* B,
-                int ldb, float beta, float* C, int ldc, GemmEpilogue epi = GemmEpilogue{nullptr, GEMM_ACT_NONE, nullptr, nullptr, nullptr, nullptr, 0u, nullptr, 0, 0.f, nullptr},
-                bool* fused = nullptr, bool* sampled = nullptr) {
-  if (fused) *fused = false;
-  if (sampled) *sampled = false;
-  if (M <= 0 || N <= 0) return 0;
-  const int cus = dn_num_cus();
-  if (K <= 0) {
-    size_t total = (size_t)M * N;
-    unsigned blocks = (unsigned)((total + 255) / 256 < (size_t)cus * 8 ? (total + 255) / 256 : (size_t)cus * 8);
-    hipLaunchKernelGGL(k_scale, dim3(blocks), dim3(256), 0, dn_stream(), C, ldc, M, N, beta);
-    return dn_launch_status();
-  }
-  const bool a_kc = a_trans, b_kc = !b_trans;
   const bool a_vec = dn_aligned16(A) && (lda % 4 == 0);
   const bool b_vec = dn_aligned16(B) && (ldb % 4 == 0);
-
   // Tile choice: big tiles when they already fill the chip, else 64x64 tiles; when
   // even those cannot fill it, the 32x32-per-workgroup kernel that splits K over
   // its own wavefronts.
@@ -1338,6 +1190,254 @@ static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, co
     // against 8.7, 1280 x 1280 x 128 9.4 against 10.8; fewer than half a tile per CU and the
     // kernels that split K over wavefronts win, 640 x 640 x 128 4.6 us against 5.7; from about
     // 2.3 tiles per CU on the slab loop does, 1536 x 1536 x 64 8.4 us against 9.6)
+    return GemmPlan{GEMM_BOX, no_ring, heavy};
+  }
+  // Reductions of more than 128 terms: k_gemm_ring, unless another kernel is expected to be faster (gemm_ring_plan).
+  const size_t a_bytes = (size_t)lda * (a_kc ? M : K) * sizeof(float), b_bytes = (size_t)ldb * (b_kc ? N : K) * sizeof(float);
+  const RingPlan ring = K > BOX_K ? gemm_ring_plan(M, N, K, a_bytes, b_bytes, cus, a_vec && b_vec && !(a_kc && b_kc)) : no_ring;
+  if (gemm_split_wins(M, N, K, beta != 0.f, a_bytes, b_bytes, ring, cus)) return GemmPlan{GEMM_SPLIT, no_ring, heavy};   // (no product that draws a sample)
+  if (ring.cfg >= 0) return GemmPlan{GEMM_RING, ring, heavy};
+  // Two K-contiguous operands whose rows lie a multiple of 1 KiB apart: the 16 x 16 block kernel
+  // reads 16 such rows per load instruction and they meet in the same memory channels (measured
+  // 1024 x 128 x 1024 with both leading dimensions 1024: 9.2 us against 8.5 us on 32 x 32 blocks).
+  const bool kc_aliased = a_kc && b_kc && (lda % 256 == 0 || ldb % 256 == 0);
+  // With both operands K-contiguous a CU's time goes with the operand bytes it pulls through its L1:
+  // more 16 x 16 blocks than CUs then means a second round on some of them, and from K = 1024 on the
+  // 32 x 32 blocks below are faster (1536 x 64 x 4096: 30.3 us against 2048 x 64 x 4096 on them in 25.9).
+  const bool t16_second_round = a_kc && b_kc && tiles16 > cus && K >= 1024;
+  if (tiles64 < cus && off32 && !heavy && !t16_second_round &&
+      (tiles32 * 5 <= cus * 2 || (tiles32 * 2 <= cus && !kc_aliased))) {
+    // 32 x 32 blocks would leave half or more of the CUs idle: 16 x 16 blocks, K over 4 wavefronts
+    // (measured against 32 x 32 blocks: 500 x 100 x 784 4.4 us against 7.7, 1024 x 128 x 784 6.5 against
+    // 7.9, 1024 x 128 x 1024 with an M-contiguous first operand 7.2 against 8.8; against 8 wavefronts per
+    // block: 500 x 100 x 784 5.4 us against 6.0)
+    return GemmPlan{GEMM_T16, no_ring, heavy};
+  }
+  // 32 x 32 blocks, K over 8 wavefronts: a CU takes them two at a time in rounds of about 5 us per 512
+  // of K, so up to two rounds they beat one 64 x 64 tile per CU (512 x 1024 x 512: 10.2 us against
+  // 15.0, x 1024: 17.2 against 25.4) and from the third round on they do not (784 x 1000 x 200: 14.8 us
+  // against 9.0, x 1024: 37.6 against 25.9; 832 x 832 x 2048: 53.3 against 37.2). Two rounds of long
+  // reductions over operands that are both contiguous along the rows of the product lose to tiles with
+  // a split K (512 x 1024 x 2048: 39.2 us against 27.5).
+  const bool mn_both = !a_kc && !b_kc;
+  if (tiles32 <= 2ll * cus && !(mn_both && K >= 2048 && tiles32 > cus) && off32 && !heavy) return GemmPlan{GEMM_SMALL, no_ring, heavy};
+  return GemmPlan{GEMM_SLAB, no_ring, heavy};
+}
+bool dn_gemm_goes_ring(bool a_trans, bool b_trans, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float beta) {
+  return M > 0 && N > 0 && gemm_plan(a_trans, !b_trans, M, N, K, A, lda, B, ldb, beta).kind == GEMM_RING;
+}
+
+// ------------------------------------------------------------------ the open group
+// Products that leave the held-back calls (elementwise.hip) go to the open group instead of the stream, as far as one kernel
+// with an epilogue computes them in a few microseconds.  They are launched when the next call comes that is no such product,
+// or one that has to do with what they read or write: those on k_gemm_ring as one launch (k_gemm_group), row sums with one of
+// them.  The group is older than what is held back (but for parameter updates that have nothing to do with it) and newer than
+// all that is queued: dn_stream() launches it.  The derivative of a rectifier joins a product that waits here too.
+struct GroupRange { const float* p; long long n; };
+struct GroupJob {
+  GemmPlan plan;
+  bool a_kc, b_kc;
+  RingArgs g;
+  GemmEpilogue epi;
+  RingSecond second;
+  GroupRange reads[7];
+  int nr;
+};
+static struct {
+  int n, nsums;
+  GroupJob job[RING_GROUP];
+  DnRowSumJob sums[4];
+} g_group = {};
+static bool g_group_ok = false;         // (only where the caller goes on to close it, or to hold the next call back)
+void dn_group_allow(bool on) { g_group_ok = on && dn_defer_enabled_at_all(); }
+static const GemmEpilogue g_no_epilogue = {nullptr, GEMM_ACT_NONE, nullptr, nullptr, nullptr, nullptr, 0u, nullptr, 0, 0.f, nullptr};
+
+static inline bool ranges_meet(const GroupRange& a, const GroupRange& b) { return a.p < b.p + b.n && b.p < a.p + a.n; }
+static inline GroupRange group_target(const RingArgs& g) { return GroupRange{g.C, (long long)(g.N - 1) * g.ldc + g.M}; }
+// Whether the group, but for product `skip`, does not read or write (writes: only not write) a range.
+static bool group_apart(const GroupRange& r, bool writes_only, int skip = -1) {
+  for (int i = 0; i < g_group.n; ++i) {
+    if (i == skip) continue;
+    const GroupJob& J = g_group.job[i];
+    if (ranges_meet(r, group_target(J.g))) return false;
+    for (int k = 0; k < J.nr && !writes_only; ++k)
+      if (ranges_meet(r, J.reads[k])) return false;
+  }
+  for (int i = 0; i < g_group.nsums; ++i) {
+    const DnRowSumJob& s = g_group.sums[i];
+    if (ranges_meet(r, GroupRange{s.y, s.h}) || (!writes_only && ranges_meet(r, GroupRange{s.M, (long long)s.h * s.w}))) return false;
+  }
+  return true;
+}
+
+static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, const float* A, int lda, const float* B, int ldb, float beta,
+                float* C, int ldc, GemmEpilogue epi = g_no_epilogue, bool* fused = nullptr, bool* sampled = nullptr);
+
+// The products on the ring and the sums that go with them.
+static void group_launch_ring(const GroupJob* const* jobs, int n, const RowSumJobs& sums, int blocks) {
+  if (n == 1 && blocks == 0 && !jobs[0]->second.A) {
+    ring_launch(jobs[0]->plan.ring.cfg, jobs[0]->a_kc, jobs[0]->b_kc, jobs[0]->g, jobs[0]->epi);
+    return;
+  }
+  RingGroup G = {};
+  G.sums = sums;
+  G.sums_blocks = blocks;
+  G.sums_end = (blocks + 7) / 8 * 8;    // (a job starts on the first XCD)
+  int c0 = jobs[0]->plan.ring.cfg, c1 = c0;              // (two different ones at most)
+  const GroupJob* order[RING_GROUP];
+  auto us = [](const GroupJob* j) {                      // of a tile
+    const auto& f = g_ring_cfgs[j->plan.ring.cfg];
+    return (j->second.A ? 2. : 1.) * f.stage * ((j->g.K + f.bk - 1) / f.bk);
+  };
+  for (int i = 0; i < n; ++i) {
+    const int c = jobs[i]->plan.ring.cfg;
+    c0 = c < c0 ? c : c0; c1 = c > c1 ? c : c1;
+    int at = i;
+    for (; at > 0 && us(order[at - 1]) < us(jobs[i]); --at) order[at] = order[at - 1];
+    order[at] = jobs[i];
+  }
+  if (c0 == c1) { if (c0 > 0) --c0; else ++c1; }
+  int end = G.sums_end;
+  for (int i = 0; i < n; ++i) {
+    const GroupJob& o = *order[i];
+    RingJob& J = G.job[i];
+    J.g = o.g; J.epi = o.epi; J.second = o.second;
+    J.variant = (o.plan.ring.cfg == c1 ? 4 : 0) + (o.a_kc ? 2 : 0) + (o.b_kc ? 1 : 0);
+    const auto& f = g_ring_cfgs[o.plan.ring.cfg];
+    J.g.gx = (J.g.M + f.bm - 1) / f.bm; J.g.gy = (J.g.N + f.bn - 1) / f.bn;
+    end += 8 * ((J.g.gx * J.g.gy + 7) / 8);
+    J.end = end;
+  }
+  ring_group_launch(c0, c1, G, end);
+}
+
+static void group_close() {
+  const int n = g_group.n, nsums = g_group.nsums;
+  GroupJob job[RING_GROUP];
+  DnRowSumJob sums[4];
+  for (int i = 0; i < n; ++i) job[i] = g_group.job[i];
+  for (int i = 0; i < nsums; ++i) sums[i] = g_group.sums[i];
+  g_group.n = g_group.nsums = 0;
+  // (this may happen while another product, with sums of its own, is on its way)
+  const auto saved = std::make_tuple(g_group_ok, g_side_jobs, g_side_blocks, g_side_list, g_side_count);
+  g_group_ok = false;
+  RowSumJobs J = {};
+  int blocks = nsums > 0 ? rows_sum_jobs_table(sums, nsums, &J) : 0;
+  const GroupJob* ring[RING_GROUP];
+  int nring = 0;
+  for (int i = 0; i < n; ++i)
+    if (job[i].plan.kind == GEMM_RING) ring[nring++] = &job[i];
+  if (nring > 0) {
+    group_launch_ring(ring, nring, J, blocks);
+    blocks = 0;
+  }
+  for (int i = 0; i < n; ++i) {
+    const GroupJob& o = job[i];
+    if (o.plan.kind == GEMM_RING) continue;
+    g_side_jobs = &J;
+    g_side_blocks = blocks;
+    gemm(o.a_kc, !o.b_kc, o.g.M, o.g.N, o.g.K, o.g.alpha, o.g.A, o.g.lda, o.g.B, o.g.ldb, o.g.beta, o.g.C, o.g.ldc, o.epi);
+    blocks = g_side_blocks;             // (0 where the launch took them along)
+  }
+  if (blocks > 0) dn_row_sum_jobs(sums, nsums);
+  std::tie(g_group_ok, g_side_jobs, g_side_blocks, g_side_list, g_side_count) = saved;
+}
+static const int g_group_registered = (dn_set_group_hook(group_close), 0);
+
+// Row sums that wait by themselves join the group (it has room for those of one launch).
+static bool group_add_sums(const DnRowSumJob* jobs, int n) {
+  if (g_group.n == 0 || g_group.nsums > 0 || n <= 0 || n > 4) return false;
+  for (int i = 0; i < n; ++i)
+    if (!group_apart(GroupRange{jobs[i].M, (long long)jobs[i].h * jobs[i].w}, true) || !group_apart(GroupRange{jobs[i].y, jobs[i].h}, false))
+      return false;
+  for (int i = 0; i < n; ++i) g_group.sums[i] = jobs[i];
+  g_group.nsums = n;
+  return true;
+}
+bool dn_group_take_sums(const DnRowSumJob* jobs, int n) {
+  RowSumJobs J;
+  return g_group_ok && g_group.n > 0 && n > 0 && rows_sum_jobs_table(jobs, n, &J) > 0 && group_add_sums(jobs, n);
+}
+
+// The product joins the open group, or opens one; false: it is to be launched.
+static bool group_take(const GemmPlan& plan, bool a_kc, bool b_kc, const RingArgs& g, const GemmEpilogue& epi, const RingSecond& second) {
+  const bool ring = plan.kind == GEMM_RING;
+  if (!g_group_ok || epi.sample || !(ring || plan.kind == GEMM_BOX || plan.kind == GEMM_T16 || plan.kind == GEMM_SMALL)) return false;
+  dn_flush_open();                      // (what is held back is older)
+  GroupJob J;
+  J.plan = plan; J.a_kc = a_kc; J.b_kc = b_kc; J.g = g; J.epi = epi; J.second = second;
+  J.nr = 0;
+  const GroupRange target = group_target(g);
+  J.reads[J.nr++] = GroupRange{g.A, (long long)g.lda * (a_kc ? g.M : g.K)};
+  J.reads[J.nr++] = GroupRange{g.B, (long long)g.ldb * (b_kc ? g.N : g.K)};
+  if (second.A) {
+    J.reads[J.nr++] = GroupRange{second.A, (long long)second.lda * (a_kc ? g.M : g.K)};
+    J.reads[J.nr++] = GroupRange{second.B, (long long)second.ldb * (b_kc ? g.N : g.K)};
+  }
+  if (epi.bias) J.reads[J.nr++] = GroupRange{epi.bias, g.M};
+  if (epi.gate) J.reads[J.nr++] = GroupRange{epi.gate, target.n};
+  if (epi.mul) J.reads[J.nr++] = GroupRange{epi.mul, target.n};
+  // (up to four, those on the ring on two kinds of tile)
+  int other = -1;
+  bool fits = g_group.n < RING_GROUP && group_apart(target, false);
+  for (int k = 0; k < J.nr && fits; ++k) fits = group_apart(J.reads[k], true);
+  for (int i = 0; i < g_group.n && ring; ++i) {
+    const GemmPlan& p = g_group.job[i].plan;
+    if (p.kind == GEMM_RING && p.ring.cfg != plan.ring.cfg) {
+      fits = fits && (other < 0 || other == p.ring.cfg);
+      other = p.ring.cfg;
+    }
+  }
+  if (!fits) dn_close_group();
+  g_group.job[g_group.n++] = J;
+  dn_set_group_open(true);
+  return true;
+}
+
+bool dn_group_take_gate(const float* target, const float* gate, int h, int w) {
+  for (int i = 0; i < g_group.n; ++i) {
+    GroupJob& J = g_group.job[i];
+    if (J.g.C != target) continue;
+    const GroupRange t = group_target(J.g), r = {gate, t.n};
+    if (J.g.M != h || J.g.N != w || J.g.ldc != h || J.epi.bias || J.epi.act != GEMM_ACT_NONE || J.epi.gate || J.second.A || ranges_meet(r, t)) return false;
+    for (int k = 0; k < J.nr; ++k)
+      if (ranges_meet(t, J.reads[k])) return false;
+    if (!group_apart(r, true, i) || !group_apart(t, false, i)) return false;
+    J.epi.gate = gate;
+    J.reads[J.nr++] = r;
+    return true;
+  }
+  return false;
+}
+
+// Host-side dispatch shared with tests through dot().
+// epi: what to append to each output (bias / activation); *fused tells the caller whether
+// the launch could carry it (the split-K and empty-K paths cannot).
+static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, const float* A, int lda, const float* B, int ldb, float beta,
+                float* C, int ldc, GemmEpilogue epi, bool* fused, bool* sampled) {
+  if (fused) *fused = false;
+  if (sampled) *sampled = false;
+  if (M <= 0 || N <= 0) return 0;
+  const int cus = dn_num_cus();
+  const bool a_kc = a_trans, b_kc = !b_trans;
+  const GemmPlan plan = gemm_plan(a_kc, b_kc, M, N, K, A, lda, B, ldb, beta);
+  if (plan.kind == GEMM_EMPTY) {
+    size_t total = (size_t)M * N;
+    unsigned blocks = (unsigned)((total + 255) / 256 < (size_t)cus * 8 ? (total + 255) / 256 : (size_t)cus * 8);
+    hipLaunchKernelGGL(k_scale, dim3(blocks), dim3(256), 0, dn_stream(), C, ldc, M, N, beta);
+    return dn_launch_status();
+  }
+  const bool a_vec = dn_aligned16(A) && (lda % 4 == 0);
+  const bool b_vec = dn_aligned16(B) && (ldb % 4 == 0);
+  // (in 32 bits where the ring and the split kernel take them)
+  const RingArgs rargs = {A, B, C, (unsigned)((size_t)lda * (a_kc ? M : K) * sizeof(float)), (unsigned)((size_t)ldb * (b_kc ? N : K) * sizeof(float)),
+                          lda, ldb, ldc, M, N, K, 0, 0, alpha, beta};
+  if (group_take(plan, a_kc, b_kc, rargs, epi, RingSecond{})) {
+    if (g_side_blocks > 0 && group_add_sums(g_side_list, g_side_count)) g_side_blocks = 0;
+    if (fused) *fused = true;
+    return 0;
+  }
+  if (plan.kind == GEMM_BOX) {
     // 16-byte groups run along K for a K-contiguous operand (whole or unused when K % 4 == 0) and
     // along the rows for the other kind (rows % 4 == 0; the last group of an edge tile then starts
     // at rows - 4 or earlier)
@@ -1367,41 +1467,18 @@ static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, co
     if (fused) *fused = true;
     return dn_launch_status();
   }
-  // Reductions of more than 128 terms: k_gemm_ring, unless another kernel is expected to be faster (gemm_ring_plan).
-  const size_t a_bytes = (size_t)lda * (a_kc ? M : K) * sizeof(float), b_bytes = (size_t)ldb * (b_kc ? N : K) * sizeof(float);
-  const RingPlan ring = K > BOX_K ? gemm_ring_plan(M, N, K, a_bytes, b_bytes, cus, a_vec && b_vec && !(a_kc && b_kc)) : RingPlan{-1, 0.};
-  const RingArgs rargs = {A, B, C, (unsigned)a_bytes, (unsigned)b_bytes, lda, ldb, ldc, M, N, K, 0, 0, alpha, beta};
-  if (gemm_split_wins(M, N, K, beta != 0.f, a_bytes, b_bytes, ring, cus)) {   // (no product that draws a sample)
+  if (plan.kind == GEMM_SPLIT) {
     split_launch(a_kc, b_kc, rargs, epi);
     if (fused) *fused = true;
     return dn_launch_status();
   }
-  if (ring.cfg >= 0) {
-    if (group_take(ring, a_kc, b_kc, rargs, epi, RingSecond{})) {
-      if (g_side_blocks > 0 && group_take_table(*g_side_jobs, g_side_blocks, g_side_list, g_side_count)) g_side_blocks = 0;
-      if (fused) *fused = true;
-      return 0;
-    }
-    dn_stream();
-    ring_launch(ring.cfg, a_kc, b_kc, rargs, epi);
+  if (plan.kind == GEMM_RING) {
+    ring_launch(plan.ring.cfg, a_kc, b_kc, rargs, epi);
     if (fused) *fused = true;
     if (sampled) *sampled = epi.sample != nullptr;
     return dn_launch_status();
   }
-  // Two K-contiguous operands whose rows lie a multiple of 1 KiB apart: the 16 x 16 block kernel
-  // reads 16 such rows per load instruction and they meet in the same memory channels (measured
-  // 1024 x 128 x 1024 with both leading dimensions 1024: 9.2 us against 8.5 us on 32 x 32 blocks).
-  const bool kc_aliased = a_kc && b_kc && (lda % 256 == 0 || ldb % 256 == 0);
-  // With both operands K-contiguous a CU's time goes with the operand bytes it pulls through its L1:
-  // more 16 x 16 blocks than CUs then means a second round on some of them, and from K = 1024 on the
-  // 32 x 32 blocks below are faster (1536 x 64 x 4096: 30.3 us against 2048 x 64 x 4096 on them in 25.9).
-  const bool t16_second_round = a_kc && b_kc && tiles16 > cus && K >= 1024;
-  if (tiles64 < cus && off32 && !heavy && !t16_second_round &&
-      (tiles32 * 5 <= cus * 2 || (tiles32 * 2 <= cus && !kc_aliased))) {
-    // 32 x 32 blocks would leave half or more of the CUs idle: 16 x 16 blocks, K over 4 wavefronts
-    // (measured against 32 x 32 blocks: 500 x 100 x 784 4.4 us against 7.7, 1024 x 128 x 784 6.5 against
-    // 7.9, 1024 x 128 x 1024 with an M-contiguous first operand 7.2 against 8.8; against 8 wavefronts per
-    // block: 500 x 100 x 784 5.4 us against 6.0)
+  if (plan.kind == GEMM_T16) {
     dim3 grid((M + 15) / 16, (N + 15) / 16);
 #define GEMM_T16(AK, BK_)                                                                                  \
   hipLaunchKernelGGL((k_gemm_tile16<AK, BK_, 4>), grid, dim3(256), 0, dn_stream(), A, lda, B, ldb, C, ldc, M, N, K, \
@@ -1427,14 +1504,7 @@ static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, co
     if (sampled) *sampled = epi.sample != nullptr;
     return dn_launch_status();
   }
-  // 32 x 32 blocks, K over 8 wavefronts: a CU takes them two at a time in rounds of about 5 us per 512
-  // of K, so up to two rounds they beat one 64 x 64 tile per CU (512 x 1024 x 512: 10.2 us against
-  // 15.0, x 1024: 17.2 against 25.4) and from the third round on they do not (784 x 1000 x 200: 14.8 us
-  // against 9.0, x 1024: 37.6 against 25.9; 832 x 832 x 2048: 53.3 against 37.2). Two rounds of long
-  // reductions over operands that are both contiguous along the rows of the product lose to tiles with
-  // a split K (512 x 1024 x 2048: 39.2 us against 27.5).
-  const bool mn_both = !a_kc && !b_kc;
-  if (tiles32 <= 2ll * cus && !(mn_both && K >= 2048 && tiles32 > cus) && off32 && !heavy) {
+  if (plan.kind == GEMM_SMALL) {
     dim3 grid((M + 31) / 32, (N + 31) / 32);
 #define GEMM_SMALL(AK, BK_)                                                                                  \
   do {                                                                                                       \
@@ -1481,7 +1551,7 @@ static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, co
     // whole), and with 1.5 tiles per CU (1280 x 1280) it never does.
     // With four slices or more (tiles on two thirds of the CUs at most) it pays from K = 1024 on
     // (768 x 768 x 1024: 23.4 us against 25.9, x 1536: 29.9 against 36.3).
-    if ((K < 2048 && !(K >= 1024 && (heavy || want >= 4))) || tiles * 4 >= (long long)cus * 5) want = 1;
+    if ((K < 2048 && !(K >= 1024 && (plan.heavy || want >= 4))) || tiles * 4 >= (long long)cus * 5) want = 1;
     if (want > 1) splits = (int)want;
   }
   int kps = ((K + splits - 1) / splits + GEMM_BK - 1) / GEMM_BK * GEMM_BK;
@@ -1492,9 +1562,8 @@ static int gemm(bool a_trans, bool b_trans, int M, int N, int K, float alpha, co
     if (!partial) return CUDA_ERROR;
   }
   dim3 grid(gx, gy, splits);
-  const GemmEpilogue none = {nullptr, GEMM_ACT_NONE, nullptr, nullptr, nullptr, nullptr, 0u, nullptr, 0, 0.f, nullptr};
-  if (big) launch_gemm<2, 2>(a_kc, b_kc, grid, A, lda, B, ldb, C, ldc, M, N, K, kps, alpha, beta, partial, a_vec, b_vec, splits > 1 ? none : epi);
-  else launch_gemm<1, 1>(a_kc, b_kc, grid, A, lda, B, ldb, C, ldc, M, N, K, kps, alpha, beta, partial, a_vec, b_vec, splits > 1 ? none : epi);
+  if (big) launch_gemm<2, 2>(a_kc, b_kc, grid, A, lda, B, ldb, C, ldc, M, N, K, kps, alpha, beta, partial, a_vec, b_vec, splits > 1 ? g_no_epilogue : epi);
+  else launch_gemm<1, 1>(a_kc, b_kc, grid, A, lda, B, ldb, C, ldc, M, N, K, kps, alpha, beta, partial, a_vec, b_vec, splits > 1 ? g_no_epilogue : epi);
   if (fused) *fused = splits == 1;
   if (splits > 1) {
     size_t total = (size_t)M * N;
@@ -1528,24 +1597,9 @@ int dn_gemm_sums(bool a_trans, bool b_trans, int M, int N, int K, float alpha, c
   return (taken || njobs <= 0) ? 0 : dn_row_sum_jobs(jobs, njobs);
 }
 
-// Whether gemm() would hand this product to k_gemm_small<.., 4> (the conditions of its dispatch, in its order).
-static bool gemm_goes_small4(bool a_kc, bool b_kc, int M, int N, int K, int lda, int ldb) {
-  if (M <= 0 || N <= 0 || K <= 0 || K > 128) return false;
-  const int cus = dn_num_cus();
-  const long long tiles64 = (long long)((M + 63) / 64) * ((N + 63) / 64);
-  const bool off32 = (size_t)lda * (a_kc ? M : K) < (1u << 30) && (size_t)ldb * (b_kc ? N : K) < (1u << 30);
-  const long long tiles32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
-  const long long tiles16 = (long long)((M + 15) / 16) * ((N + 15) / 16);
-  const double per_1024 = tiles16 <= cus ? 4.0 : tiles32 <= cus ? 6.2 : 15.5;
-  const bool heavy = 12.0 + 1.5e-8 * (double)M * (double)N * (double)K < per_1024 * (double)K / 1024.0;
-  if (K <= BOX_K && tiles64 >= cus / 2 && tiles64 <= 2 * cus) return false;            // k_gemm_box
-  const bool kc_aliased = a_kc && b_kc && (lda % 256 == 0 || ldb % 256 == 0);
-  const bool t16_second_round = a_kc && b_kc && tiles16 > cus && K >= 1024;
-  if (tiles64 < cus && off32 && !heavy && !t16_second_round &&
-      (tiles32 * 5 <= cus * 2 || (tiles32 * 2 <= cus && !kc_aliased)))
-    return false;                                                                      // k_gemm_tile16
-  const bool mn_both = !a_kc && !b_kc;
-  return tiles32 <= 2ll * cus && !(mn_both && K >= 2048 && tiles32 > cus) && off32 && !heavy;
+// Whether gemm() would hand this product to k_gemm_small<.., 4>.
+static bool gemm_goes_small4(bool a_kc, bool b_kc, int M, int N, int K, const float* A, int lda, const float* B, int ldb) {
+  return M > 0 && N > 0 && K > 0 && K <= 128 && gemm_plan(a_kc, b_kc, M, N, K, A, lda, B, ldb, 1.f).kind == GEMM_SMALL;
 }
 
 // C = beta*C + alpha*op(A)*op(B), then C = C + alpha2*op(A2)*op(B2) (the second pair of operands has the
@@ -1558,7 +1612,7 @@ int dn_gemm_pair_sums(bool a_trans, bool b_trans, int M, int N, int K, float alp
   RowSumJobs J = {};
   const int jblocks = njobs > 0 ? rows_sum_jobs_table(jobs, njobs, &J) : 0;
   if (jblocks < 0) return ERROR_GENERIC;
-  if (gemm_goes_small4(a_kc, b_kc, M, N, K, lda, ldb) && gemm_goes_small4(a_kc, b_kc, M, N, K, lda2, ldb2)) {
+  if (gemm_goes_small4(a_kc, b_kc, M, N, K, A, lda, B, ldb) && gemm_goes_small4(a_kc, b_kc, M, N, K, A2, lda2, B2, ldb2)) {
     GemmPairArgs g;
     g.A = A; g.B = B; g.A2 = A2; g.B2 = B2; g.C = C;
     g.lda = lda; g.ldb = ldb; g.lda2 = lda2; g.ldb2 = ldb2; g.ldc = ldc; g.M = M; g.N = N; g.K = K;
@@ -1587,16 +1641,13 @@ int dn_gemm_pair_sums(bool a_trans, bool b_trans, int M, int N, int K, float alp
     }
     return dn_launch_status();
   }
-  const RingPlan ring = g_group_ok ? gemm_ring_route(a_kc, b_kc, M, N, K, A, lda, B, ldb, beta) : RingPlan{-1, 0.};
-  if (ring.cfg >= 0 && gemm_ring_route(a_kc, b_kc, M, N, K, A2, lda2, B2, ldb2, 1.f).cfg == ring.cfg) {
+  const GemmPlan plan = gemm_plan(a_kc, b_kc, M, N, K, A, lda, B, ldb, beta), plan2 = gemm_plan(a_kc, b_kc, M, N, K, A2, lda2, B2, ldb2, 1.f);
+  if (plan.kind == GEMM_RING && plan2.kind == GEMM_RING && plan.ring.cfg == plan2.ring.cfg) {
     const RingArgs g = {A, B, C, 4u * (unsigned)lda * (unsigned)(a_kc ? M : K), 4u * (unsigned)ldb * (unsigned)(b_kc ? N : K), lda, ldb, ldc, M, N, K, 0, 0,
                         alpha, beta};
     const RingSecond second = {A2, B2, 4u * (unsigned)lda2 * (unsigned)(a_kc ? M : K), 4u * (unsigned)ldb2 * (unsigned)(b_kc ? N : K), lda2, ldb2, alpha2};
-    const GemmEpilogue none = {nullptr, GEMM_ACT_NONE, nullptr, nullptr, nullptr, nullptr, 0u, nullptr, 0, 0.f, nullptr};
-    if (group_take(ring, a_kc, b_kc, g, none, second)) {
-      if (njobs > 0 && group_take_table(J, jblocks, jobs, njobs)) return 0;
-      return njobs > 0 ? dn_row_sum_jobs(jobs, njobs) : 0;
-    }
+    if (group_take(plan, a_kc, b_kc, g, g_no_epilogue, second))
+      return njobs == 0 || group_add_sums(jobs, njobs) ? 0 : dn_row_sum_jobs(jobs, njobs);
   }
   if (int e = gemm(a_trans, b_trans, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc)) return e;
   if (int e = gemm(a_trans, b_trans, M, N, K, alpha2, A2, lda2, B2, ldb2, 1.f, C, ldc)) return e;
@@ -1731,7 +1782,7 @@ int cd_update(cudamat* W, cudamat* bv, cudamat* bh, cudamat* v, cudamat* h, cuda
   // Batches of up to 128: the two products and the four sums of the reference's spelling as they
   // are, in one launch (k_gemm_small_pair_sums: the bits of the six calls, and faster than the
   // augmented product below: 784 x 500, batch 100: 8 us against 11 under the tracer)
-  if (gemm_goes_small4(false, false, nv, nh, B, nv, nh) &&
+  if (gemm_goes_small4(false, false, nv, nh, B, v->data_device, nv, h->data_device, nh) &&
       (!bv || (dn_row_sum_job_ok(v->data_device, nv, B) && dn_row_sum_job_ok(v2->data_device, nv, B))) &&
       (!bh || (dn_row_sum_job_ok(h->data_device, nh, B) && dn_row_sum_job_ok(h2->data_device, nh, B)))) {
     DnRowSumJob jobs[4];

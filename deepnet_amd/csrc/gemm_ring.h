@@ -153,7 +153,7 @@ template <int TB, int BM, int BN, int BK>
 static void ring_launch_cfg(bool a_kc, bool b_kc, RingArgs g, const GemmEpilogue& epi) {
   g.gx = (g.M + BM - 1) / BM; g.gy = (g.N + BN - 1) / BN;
   const dim3 grid((unsigned)(8 * ((g.gx * g.gy + 7) / 8)));
-#define RING_GO(AK, BK_) hipLaunchKernelGGL((k_gemm_ring<TB, BM, BN, BK, AK, BK_>), grid, dim3(RING_THREADS), 0, dn_stream_now(), g, epi)
+#define RING_GO(AK, BK_) hipLaunchKernelGGL((k_gemm_ring<TB, BM, BN, BK, AK, BK_>), grid, dim3(RING_THREADS), 0, dn_stream(), g, epi)
   if (a_kc && b_kc) RING_GO(true, true);
   else if (a_kc) RING_GO(true, false);
   else if (b_kc) RING_GO(false, true);
@@ -220,7 +220,7 @@ static void ring_group_launch(int c0, int c1, const RingGroup& G, int blocks) {
       const int v = G.job[j].variant;                                                                                        \
       room(v < 4 ? ring_lds_bytes<A>((v & 2) != 0, (v & 1) != 0) : ring_lds_bytes<B>((v & 2) != 0, (v & 1) != 0));           \
     }                                                                                                                        \
-    hipLaunchKernelGGL((k_gemm_group<A, B>), dim3((unsigned)blocks), dim3(RING_THREADS), (unsigned)lds, dn_stream_now(), G); \
+    hipLaunchKernelGGL((k_gemm_group<A, B>), dim3((unsigned)blocks), dim3(RING_THREADS), (unsigned)lds, dn_stream(), G); \
     return;                                                                                                                  \
   }
   RING_GROUP_GO(0, 1) RING_GROUP_GO(0, 2) RING_GROUP_GO(0, 3) RING_GROUP_GO(0, 4) RING_GROUP_GO(0, 5)
