@@ -2654,7 +2654,7 @@ static void conv_outp_filters(cudamat* images, cudamat* hidActs, cudamat* target
 static ConvRingArgs ring_args(const ConvArgs& a) {
   ConvRingArgs p = {};
   p.N = a.N; p.H = a.H; p.HH = a.HH; p.Mx = a.Mx; p.M = a.M; p.k = a.k; p.kk2 = a.kk2; p.s = a.s; p.pad0 = a.pad0;
-  p.Cg = a.Cg; p.Fg = a.Fg; p.F = a.F; p.G = a.G; p.local = a.local; p.out = a.out;
+  p.Cg = a.Cg; p.Fg = a.Fg; p.Fg4 = (a.Fg + 3) / 4 * 4; p.F = a.F; p.G = a.G; p.local = a.local; p.out = a.out;
   p.m_count = a.m_count; p.splits = 1; p.periods = 1;
   return p;
 }
@@ -2674,7 +2674,7 @@ static bool conv_rows_ring(const ConvArgs& a, int mode, const char* where) {
   const ConvRingPlan plan = conv_rows_choice(a, mode, ring_maps16(a), dn_aligned16(a.flt), dn_num_cus());
   if (plan.cfg < 0) return false;
   const bool single = plan.single;
-  const int sites = up ? a.M : a.HH, cols = up ? a.Fg : a.Cg, K = a.kk2 * (up ? a.Cg : a.Fg);
+  const int sites = up ? a.M : a.HH, cols = up ? a.Fg : a.Cg, K = a.kk2 * (up ? a.Cg : (a.Fg + 3) / 4 * 4);
   const long long bank = (long long)a.Cg * a.kk2 * (a.local ? a.M : 1);
   ConvRingArgs p = ring_args(a);
   p.a = up ? a.img : a.hid; p.b = a.flt;
@@ -2684,6 +2684,27 @@ static bool conv_rows_ring(const ConvArgs& a, int mode, const char* where) {
   p.ldc = (long long)a.N * sites;
   if (up) { if (single) conv_ring_launch<CONV_UP, true>(plan, p); else conv_ring_launch<CONV_UP, false>(plan, p); }
   else { if (single) conv_ring_launch<CONV_DOWN, true>(plan, p); else conv_ring_launch<CONV_DOWN, false>(plan, p); }
+  return ring_done(where);
+}
+
+// Down on tiles of one pixel or block of pixels (conv_pixels_choice); false: not a pass for them.
+static bool conv_pixels_ring(const ConvArgs& a, const char* where) {
+  const ConvRingPlan plan = conv_pixels_choice(a, ring_maps16(a), dn_aligned16(a.flt), dn_num_cus());
+  if (plan.cfg < 0) return false;
+  const int b = plan.blocks > 0 ? plan.blocks : 1, taps = b - 1 + (a.k + a.s - 1) / a.s;
+  const bool flat = plan.blocks < 0;
+  ConvRingArgs p = ring_args(a);
+  p.a = a.hid; p.b = a.flt;
+  p.a_bytes = (unsigned)((long long)a.N * a.M * a.F * 4);
+  p.b_bytes = (unsigned)((long long)a.F * a.Cg * a.kk2 * 4);
+  p.block = plan.blocks > 0 ? b * a.s : 1;
+  p.lines = plan.blocks > 0 ? (a.H - a.pad0 - 1) / p.block + 1 : a.H;
+  p.rows = flat ? a.HH * a.N : a.N; p.cols = a.Cg * p.block * p.block; p.periods = flat ? 1 : p.lines * p.lines; p.gz = a.G;
+  p.K = (flat ? a.kk2 : taps * taps) * p.Fg4;
+  p.ldc = (long long)a.N * a.HH;
+  if (plan.blocks > 0) conv_ring_launch<CONV_DOWNM, true>(plan, p);
+  else if (flat) conv_ring_launch<CONV_DOWN, false>(plan, p);
+  else conv_ring_launch<CONV_DOWN, true>(plan, p);
   return ring_done(where);
 }
 
@@ -2747,6 +2768,7 @@ void convDown(cudamat* hidActs, cudamat* filters, cudamat* targets, int imgSize,
   ConvArgs a;
   if (!conv_down_args(hidActs, filters, targets, imgSize, paddingStart, moduleStride, numImgColors, numGroups, "convDown", false, a)) return;
   if (conv_rows_ring(a, CONV_DOWN, "convDown")) return;
+  if (conv_pixels_ring(a, "convDown")) return;
   PaddedBatch pb(hidActs, targets, nullptr);
   if (pb.on) {
     pb.fill(0, hidActs);

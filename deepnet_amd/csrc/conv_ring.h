@@ -6,21 +6,25 @@
 // A term of the reduction, as the workgroup keeps it in LDS for its reduction (one entry per term for Up, per four
 // for Down and Outp): the byte offset that it adds to a lane's, and which filter rows (bits 0-14) and columns (15-29)
 // have to be inside (Up, Down: `mask` of the entry has to be part of the lane's) or are inside (Outp: the other way
-// round).  RING_FAR stands in no lane's mask: such a term reads as zero.
+// round).  RING_FAR stands in no lane's mask: such a term reads as zero.  Of filters that are no multiple of four, the last
+// entry of a tap (RING_LAST in its mask) moves back to the last four, and leaves out those that the entry before has.
 #define RING_FAR 0x80000000u
+#define RING_LAST 0x40000000u
+static_assert(2 * RING_MAX_SIDE <= 30, "masks below RING_LAST");
 static_assert(RING_AHEAD >= RING_SETS + 3, "fetch() looks one stage ahead, the loop RING_SETS + 2");
 
 struct ConvRingArgs {
   const float* a; const float* b;
   float* out;
   unsigned a_bytes, b_bytes;
-  int N, H, HH, Mx, M, k, kk2, s, pad0, Cg, Fg, F, G;
+  int N, H, HH, Mx, M, k, kk2, s, pad0, Cg, Fg, Fg4, F, G;          // Fg4: filters of a group in whole fours
   int local;                    // one filter bank per module
   int rows, cols;               // of one period: a tile lies inside one (one module or pixel, or everything)
   int periods, gx, gy, gz;      // tiles per period down the rows, across; Up / Down: groups; Outp: chunks x splits x groups
   int K;                        // Outp: terms of a chunk
+  int block, lines;             // DownM: side of a block of pixels, blocks per side of a map
   int m_count, splits, split_stages;
-  FastDiv dN, dMx, dk, dkk2, dH, dFg, dgx, dgy, dper, dsplits, dG;
+  FastDiv dN, dMx, dk, dkk2, dH, dFg4, dgx, dgy, dper, dsplits, dG, ds, dblock, dblock2, dlines;
   long long ldc, out_stride;    // of a column; Outp: of a (chunk, split)
 };
 
@@ -33,21 +37,23 @@ struct ConvRingArgs {
 //   On tiles of one module or pixel every entry is an offset into each operand, or RING_FAR behind the last term:
 //      5, 6: A (x of an entry) and B (y) of Up and A of Down
 //      7: B of Down
+//      9: A of DownM (its mask: RING_LAST where the lane's term of a tap's last entry is taken by the one before)
+//      8: B of DownM: rows are (colour, row and column of a pixel in its block), which have a tap for some entries (tab1: masks as above)
 template <int KIND, class Tile, int PER>
 struct ConvRingOperand : Tile {
-  static_assert(Tile::KC == ((KIND >= 2 && KIND <= 4) || KIND == 7), "terms or rows in order of memory");
+  static_assert(Tile::KC == ((KIND >= 2 && KIND <= 4) || KIND == 7 || KIND == 8), "terms or rows in order of memory");
   static_assert(Tile::REACH == 1 || KIND == 1 || KIND == 3 || KIND >= 5, "the table ends with the last stage");
   using Tile::NG;
   static constexpr int BK = Tile::BK;
   // an entry per group, else one per lane and stage
-  static constexpr bool ENT = (KIND == 0 || KIND == 5 || KIND == 6) && !(Tile::KPACK >= NG && NG <= PER);
+  static constexpr bool ENT = (KIND == 0 || KIND == 5 || KIND == 6 || KIND == 9) && !(Tile::KPACK >= NG && NG <= PER);
   static constexpr bool LOOKS = KIND != 1 && KIND != 3;
   __amdgpu_buffer_rsrc_t rsrc;
   unsigned off[NG], mask[NG];
   unsigned step;                                                          // KIND 1
   int left;                                                               // KIND 3: terms behind the lane's first one
   const uint2* tab;                                                       // KIND 0, 4 .. 7
-  const unsigned* tab1;                                                   // KIND 2
+  const unsigned* tab1;                                                   // KIND 2, 8, 9
   uint2 ent[ENT ? NG : 1];
   __device__ __forceinline__ void look(int t, int nst) {
     const int at = (t < nst ? t : nst - 1) * (BK / PER);
@@ -66,6 +72,17 @@ struct ConvRingOperand : Tile {
       }
     }
     if (KIND == 7) ent[0].x = tab[free + Tile::group_k(threadIdx.x, 0) / PER].y;
+    if (KIND == 9) {
+#pragma unroll
+      for (int u = 0; u < (ENT ? NG : 1); ++u) {
+        const int e = free + Tile::group_k(threadIdx.x, u) / PER;
+        ent[u] = make_uint2(tab[e].x, tab1[e]);
+      }
+    }
+    if (KIND == 8) {
+      const int e = free + Tile::group_k(threadIdx.x, 0) / PER;
+      ent[0] = make_uint2(tab[e].y, tab1[e]);
+    }
   }
   __device__ __forceinline__ void fetch(int t, int nst, ring_f32x4 (&r)[NG]) {
     const unsigned behind = (unsigned)(nst - 1 - t) & RING_FAR;           // a stage behind the last one goes nowhere
@@ -83,6 +100,10 @@ struct ConvRingOperand : Tile {
         o = (off[u] + ent[0].x) | behind;
       } else if (KIND == 3) {
         o = t * BK < left ? off[u] + (unsigned)(t * BK * 4) : RING_FAR;
+      } else if (KIND == 8) {
+        o = (mask[u] & ent[0].y) == ent[0].y ? off[u] + ent[0].x : RING_FAR;
+      } else if (KIND == 9) {
+        o = mask[u] & ent[ENT ? u : 0].y ? RING_FAR : off[u] + ent[ENT ? u : 0].x;
       } else if (KIND >= 5) {
         o = off[u] + ent[ENT ? u : 0].x;
       } else {
@@ -95,6 +116,23 @@ struct ConvRingOperand : Tile {
   }
 };
 
+// An output of Down by itself, (y, x) counted from the padding's edge: where a module that is not finite reaches a block but not
+// this pixel, whose tap in the product is a zero.
+__device__ __forceinline__ float conv_down_one(const ConvRingArgs& p, int g, int c, int y, int x, int n) {
+  float acc = 0.f;
+  const int top = (int)fd_div((uint32_t)y, p.ds), right = (int)fd_div((uint32_t)x, p.ds);
+#pragma unroll 1
+  for (int my = top < p.Mx - 1 ? top : p.Mx - 1; my >= 0 && y - my * p.s < p.k; --my)
+#pragma unroll 1
+    for (int mx = right < p.Mx - 1 ? right : p.Mx - 1; mx >= 0 && x - mx * p.s < p.k; --mx) {
+      const float* h = p.a + (size_t)p.N * ((size_t)p.M * (g * p.Fg) + my * p.Mx + mx) + n;
+      const float* w = p.b + (size_t)p.F * ((c * p.k + y - my * p.s) * p.k + x - mx * p.s) + g * p.Fg;
+#pragma unroll 1
+      for (int f = 0; f < p.Fg; ++f) acc += h[(size_t)p.N * p.M * f] * w[f];
+    }
+  return acc;
+}
+
 // A convolution pass as a product on the tile loop of ring_tile.h (see there and k_gemm_ring): layers on small and
 // mid-sized maps, locally connected layers, and batches that are no multiple of 16, in one launch each.  What bounded
 // these on k_conv_mfma: one or two workgroups of four wavefronts per CU that wait for every slab, reductions split over
@@ -105,6 +143,16 @@ struct ConvRingOperand : Tile {
 // instructions per group and stage.  Tiles of one module or pixel (SINGLE: locally connected layers, batches that are no
 // multiple of 4 or that the tile divides) need no masks and leave out the taps beyond the edge.
 // convOutp splits its reduction over workgroups and is summed by k_conv_outp_finish*.
+// convDown onto few colours (DownM) fills a tile's columns with the pixels of a block beside the colours: k + (b - 1) s rows of taps
+// a line where a pixel has k / s, for b s times as many columns; strided layers take tiles of one pixel or one block too, which
+// have the taps that exist and no others.  What these took before: a product of all taps and a gather of its outputs
+// (a patch matrix, 5 passes over the maps), phases of 128 images, copies of batches and filters to whole groups, or one lane per output.
+// Measured, us, operands in the caches, before -> now:
+//   96 -> 112 colours 7 x 7, stride 2, 10 x 10, batch 128   131 -> 17      1 -> 64 of 11 x 11, stride 2, 223 x 223, 100    2044 -> 506
+//   84 -> 148 of 5 x 5, stride 2, 11 x 11, 100    120 -> 36                3 -> 32 of 5 x 5, 18 x 18, 100     21 -> 11
+//   24 -> 93 of 7 x 7, 31 x 31, 151 (whole fours of filters)    645 -> 339
+// Of 210 random layers that they take, one was 4 % slower than before, none by more; half are twice as fast.  (3 -> 96 of 11 x 11,
+// stride 4, 224 x 224, 128, as fast either way, stays on phases of 128 images.)
 // Measured, us Up / Down / Outp, operands from memory, before -> now (with the copies and sums):
 //   64 -> 64 colours 5 x 5, 13 x 13, batch 100      70 / 62 / 65 -> 46 / 45 / 39      (22 each at 157 TFLOP/s)
 //   64 -> 64 colours 3 x 3, 17 x 17, batch 100      69 / 57 / 55 -> 27 / 27 / 32      (14)
@@ -142,8 +190,8 @@ struct ConvSplitCfg {
 template <int MODE, bool SINGLE, class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRingArgs p) {
   constexpr int PER = MODE == CONV_UP ? 1 : 4, BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, THREADS = Cfg::THREADS;
-  using OA = ConvRingOperand<MODE == CONV_OUTP ? 3 : SINGLE ? 5 : 0, typename Cfg::template Tile<BM, MODE == CONV_OUTP>, PER>;
-  using OB = ConvRingOperand<MODE == CONV_UP ? (SINGLE ? 6 : 1) : MODE == CONV_DOWN ? (SINGLE ? 7 : 2) : 4,
+  using OA = ConvRingOperand<MODE == CONV_OUTP ? 3 : MODE == CONV_DOWNM ? 9 : SINGLE ? 5 : 0, typename Cfg::template Tile<BM, MODE == CONV_OUTP>, PER>;
+  using OB = ConvRingOperand<MODE == CONV_UP ? (SINGLE ? 6 : 1) : MODE == CONV_DOWN ? (SINGLE ? 7 : 2) : MODE == CONV_DOWNM ? 8 : 4,
                              typename Cfg::template Tile<BN, MODE != CONV_UP>, PER>;
   using Shape = typename Cfg::template Shape<OA, OB>;
   constexpr int EPL = Shape::EPL, LDS = Cfg::SPLIT ? Shape::LDS : 4 * Shape::LDS;
@@ -168,58 +216,90 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
   const int bx = t - rest * p.gx, z = div(rest, p.dper), per = rest - z * p.periods;
   // a tile over the edge moves back inside; the outputs it shares with its neighbour are that one's to store
   const int m_lo = bx * BM, n_lo = by * BN;
-  const int m0 = m_lo + BM <= p.rows ? m_lo : p.rows - BM, n0 = n_lo + BN <= p.cols ? n_lo : p.cols - BN;
+  const int m0 = m_lo + BM <= p.rows ? m_lo : p.rows - BM, n0 = n_lo + BN <= p.cols || p.cols < BN ? n_lo : p.cols - BN;
 
   OA oa; OB ob;
   int nst, g = z;
   float* out = p.out;
   if constexpr (SINGLE) {
-    // One module or pixel: taps that leave the image, or reach no module, are left out.  The others are rows ky0 ..
-    // ky0 + ny - 1 and columns kx0 .. kx0 + nx - 1 of the filter.
-    const int line = div(per, MODE == CONV_UP ? p.dMx : p.dH), at = per - line * (MODE == CONV_UP ? Mx : H);
-    const int y = MODE == CONV_UP ? line * p.s + p.pad0 : line - p.pad0, x = MODE == CONV_UP ? at * p.s + p.pad0 : at - p.pad0;
-    auto range = [&](int v, int* first) {
-      const int lo = MODE == CONV_UP ? -v : v - Mx + 1, hi = MODE == CONV_UP ? H - v : v + 1;
-      *first = lo > 0 ? lo : 0;
-      return (hi < k ? hi : k) - *first;
+    // One module or pixel: taps that leave the image, or reach no module, are left out.  Up: the others are rows ky0 ..
+    // ky0 + ny - 1 and columns kx0 .. kx0 + nx - 1 of the filter.  Down: modules my0, my0 - 1 .. my0 - ny + 1 (of a line) have the
+    // pixel at rows ky0, ky0 + s ..; a block of pixels: the tap of its first pixel there, which may lie outside the filter.
+    constexpr bool UP = MODE == CONV_UP, MERGED = MODE == CONV_DOWNM;
+    const int s = p.s, blocks = MERGED ? div(p.block, p.ds) : 1;
+    const int line = div(per, UP ? p.dMx : MERGED ? p.dlines : p.dH), at = per - line * (UP ? Mx : MERGED ? p.lines : H);
+    const int y = UP ? line * s + p.pad0 : MERGED ? line * p.block : line - p.pad0, x = UP ? at * s + p.pad0 : MERGED ? at * p.block : at - p.pad0;
+    auto range = [&](int v, int* first, int* m_first) {
+      if (UP) {
+        *first = -v > 0 ? -v : 0;
+        return (H - v < k ? H - v : k) - *first;
+      }
+      const int top = div(v, p.ds) + blocks - 1, m = top < Mx - 1 ? top : Mx - 1, reach = MERGED ? k + s * (blocks - 1) : k;
+      *m_first = m;
+      *first = v - s * m;                                               // (from -s (blocks - 1) on)
+      const int n = *first < k ? div(reach - 1 - (*first + s * (blocks - 1)), p.ds) + 1 : 0;
+      return n < m + 1 ? n : m + 1;
     };
-    int ky0, kx0;
-    int ny = range(y, &ky0), nx = range(x, &kx0);
+    int ky0, kx0, my0 = 0, mx0 = 0;
+    int ny = range(y, &ky0, &my0), nx = range(x, &kx0, &mx0);
     if (ny <= 0 || nx <= 0) { ny = 0; nx = 1; }
-    const int area = ny * nx, K = area * (MODE == CONV_UP ? p.Cg : p.Fg);
+    const int area = ny * nx, K = area * (UP ? p.Cg : p.Fg4);
     nst = K > BK ? (K + BK - 1) / BK : 1;
+    unsigned* tab1 = reinterpret_cast<unsigned*>(table + (nst + RING_AHEAD) * (BK / PER));
     // exact for dividends below 2^12 and divisors up to RING_MAX_SIDE^2
     const unsigned inv_nx = 65536u / (unsigned)nx + 1u, inv_area = (1u << 20) / (unsigned)(area > 0 ? area : 1) + 1u;
     const unsigned Nu = (unsigned)N, Fu = (unsigned)p.F;
     for (int e = tid; e < (nst + RING_AHEAD) * (BK / PER); e += THREADS) {
       uint2 t2 = make_uint2(RING_FAR, RING_FAR);
+      unsigned need = 0u;
       if (PER * e < K) {
-        const int c = MODE == CONV_UP ? (int)((unsigned)e * inv_area >> 20) : 0;
-        const int tap = MODE == CONV_UP ? e - c * area : div(4 * e, p.dFg), f = MODE == CONV_UP ? 0 : 4 * e - tap * p.Fg;
-        const int ty = (int)((unsigned)tap * inv_nx >> 16), ky = ky0 + ty, kx = kx0 + tap - ty * nx;
-        if (MODE == CONV_UP) {
-          const int bank = p.local ? per : 0;
+        const int c = UP ? (int)((unsigned)e * inv_area >> 20) : 0;
+        const int tap = UP ? e - c * area : div(4 * e, p.dFg4);
+        const int ty = (int)((unsigned)tap * inv_nx >> 16), tx = tap - ty * nx;
+        if (UP) {
+          const int bank = p.local ? per : 0, ky = ky0 + ty, kx = kx0 + tx;
           t2.x = 4u * Nu * (unsigned)((g * p.Cg + c) * p.HH + (y + ky) * H + x + kx);
           t2.y = 4u * Fu * (unsigned)((bank * p.Cg + c) * p.kk2 + ky * k + kx);
         } else {
-          const int m = (y - ky) * Mx + x - kx;
+          const int m = (my0 - ty) * Mx + mx0 - tx, ky = ky0 + s * ty, kx = kx0 + s * tx;
+          int f = 4 * e - tap * p.Fg4;
+          if (MERGED && f + 4 > p.Fg) { f = p.Fg - 4; need = RING_LAST; }
           t2.x = 4u * Nu * (unsigned)(p.M * (g * p.Fg + f) + m);
           t2.y = 4u * ((unsigned)f + Fu * (unsigned)(ky * k + kx + p.Cg * p.kk2 * (p.local ? m : 0)));
+          // (the first pixel's row and column, from -s (blocks - 1) on, in steps of s; a lane's mask says with which its own has a tap)
+          if (MERGED) need |= 1u << (div(ky + s * (blocks - 1), p.ds)) | 1u << (RING_MAX_SIDE + div(kx + s * (blocks - 1), p.ds));
         }
       }
       table[e] = t2;
+      if (MERGED) tab1[e] = need;
     }
     oa.tab = ob.tab = table;
     const int n = m0 + OA::group_row(tid, 0);
 #pragma unroll
-    for (int u = 0; u < OA::NG; ++u) oa.off[u] = 4u * (unsigned)(n + (PER == 4 ? N * p.M * (OA::group_k(tid, u) % 4) : 0));
+    for (int u = 0; u < OA::NG; ++u) {
+      oa.off[u] = 4u * (unsigned)(n + (PER == 4 ? N * p.M * (OA::group_k(tid, u) % 4) : 0));
+      if (MERGED) oa.mask[u] = OA::group_k(tid, u) % 4 < p.Fg4 - p.Fg ? RING_LAST : 0u;
+    }
 #pragma unroll
     for (int u = 0; u < OB::NG; ++u) {
       const int col = n0 + OB::group_row(tid, u);
-      ob.off[u] = 4u * (unsigned)(g * p.Fg + (MODE == CONV_UP ? col : p.F * p.kk2 * col));
+      if (MERGED) {
+        const int c = div(col, p.dblock2), q = col - c * p.block * p.block, py = div(q, p.dblock), px = q - py * p.block;
+        ob.off[u] = 4u * (unsigned)(g * p.Fg + p.F * (c * p.kk2 + py * k + px));
+        // rows 0 <= first + py < k of the filter, first = s (t - blocks + 1), as bits t
+        auto taps = [&](int q0) {
+          const int back = s * (blocks - 1) - q0;                       // first + q0 = s t - back
+          return ring_bits(back > 0 ? div(back + s - 1, p.ds) : 0, back + k > 0 ? div(back + k - 1, p.ds) + 1 : 0);
+        };
+        ob.mask[u] = col < p.cols ? taps(py) | taps(px) << RING_MAX_SIDE | RING_LAST : 0u;
+      } else {
+        ob.off[u] = 4u * (unsigned)(g * p.Fg + (MODE == CONV_UP ? col : p.F * p.kk2 * col));
+      }
     }
+    if (MERGED) oa.tab1 = ob.tab1 = tab1;
     ob.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p.b, 0, (int)p.b_bytes, 0x00020000);
-    out += (long long)g * p.cols * p.ldc + (long long)per * p.rows;
+    if (MERGED) out += (long long)g * p.Cg * p.HH * N;
+    else out += (long long)g * p.cols * p.ldc + (long long)per * p.rows;
   } else if constexpr (MODE == CONV_UP) {
     const int K = p.Cg * p.kk2;
     nst = (K + BK - 1) / BK;
@@ -244,13 +324,14 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
       ob.off[u] = 4u * (unsigned)(OB::group_k(tid, u) * p.F + g * p.Fg + n0 + OB::group_row(tid, u));
     out += (long long)g * p.Fg * p.ldc;
   } else if constexpr (MODE == CONV_DOWN) {
-    const int K = p.kk2 * p.Fg;
+    const int K = p.kk2 * p.Fg4;
     nst = (K + BK - 1) / BK;
     unsigned* tab1 = reinterpret_cast<unsigned*>(table + nst * (BK / 4));
     for (int e = tid; e < nst * (BK / 4); e += THREADS) {
-      const int tap = div(4 * e, p.dFg), f = 4 * e - tap * p.Fg, ky = div(tap, p.dk), kx = tap - ky * k;
+      const int tap = div(4 * e, p.dFg4), f0 = 4 * e - tap * p.Fg4, f = f0 + 4 > p.Fg ? p.Fg - 4 : f0, ky = div(tap, p.dk), kx = tap - ky * k;
       const bool in = 4 * e < K;
-      table[e] = make_uint2(4u * (unsigned)N * (unsigned)(p.M * f - ky * Mx - kx), in ? 1u << ky | 1u << (RING_MAX_SIDE + kx) : RING_FAR);
+      table[e] = make_uint2(4u * (unsigned)N * (unsigned)(p.M * f - ky * Mx - kx),
+                            in ? 1u << ky | 1u << (RING_MAX_SIDE + kx) | (f < f0 ? RING_LAST : 0u) : RING_FAR);
       tab1[e] = in ? 4u * (unsigned)(f + p.F * tap) : RING_FAR;
     }
     const int r = m0 + OA::group_row(tid, 0);
@@ -258,7 +339,8 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
 #pragma unroll
     for (int u = 0; u < OA::NG; ++u) {
       oa.off[u] = 4u * (unsigned)(n + N * (y * Mx + x + p.M * (g * p.Fg + OA::group_k(tid, u) % 4)));
-      oa.mask[u] = ring_bits(y - Mx + 1, y + 1 < k ? y + 1 : k) | ring_bits(x - Mx + 1, x + 1 < k ? x + 1 : k) << RING_MAX_SIDE;
+      oa.mask[u] = ring_bits(y - Mx + 1, y + 1 < k ? y + 1 : k) | ring_bits(x - Mx + 1, x + 1 < k ? x + 1 : k) << RING_MAX_SIDE |
+                   (OA::group_k(tid, u) % 4 < p.Fg4 - p.Fg ? 0u : RING_LAST);
     }
     oa.tab = table;
     ob.tab1 = tab1;
@@ -296,22 +378,34 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
   oa.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, (int)p.a_bytes, 0x00020000);
   __syncthreads();
 
+  // output (em, en) of the tile: at column en, or (DownM) at the pixel that it stands for, which may lie outside the map
+  auto store = [&](int em, int en, float v) {
+    if (em < m_lo || en < n_lo || en >= p.cols) return;
+    if constexpr (MODE == CONV_DOWNM) {
+      const int line = div(per, p.dlines), at = per - line * p.lines;
+      const int c = div(en, p.dblock2), q = en - c * p.block * p.block, py = div(q, p.dblock), px = q - py * p.block;
+      const int y = line * p.block + py + p.pad0, x = at * p.block + px + p.pad0;
+      if ((unsigned)y < (unsigned)H && (unsigned)x < (unsigned)H) {
+        if (!(__builtin_fabsf(v) < __builtin_inff())) v = conv_down_one(p, g, c, y - p.pad0, x - p.pad0, em);
+        out[(long long)(c * p.HH + y * H + x) * N + em] = v;
+      }
+    } else {
+      out[(long long)en * p.ldc + em] = v;
+    }
+  };
   if constexpr (Cfg::SPLIT) {
     Shape::template run<false>(lds, oa, ob, nst, 0, [] {});
 #pragma unroll
     for (int u = 0; u < EPL; ++u) {
-      const int e = tid + THREADS * u, em = m0 + e % BM, en = n0 + e / BM;
-      if (em >= m_lo && en >= n_lo) out[(long long)en * p.ldc + em] = Shape::sum(lds, tid, u);
+      const int e = tid + THREADS * u;
+      store(m0 + e % BM, n0 + e / BM, Shape::sum(lds, tid, u));
     }
   } else {
     float sum[EPL];
     Shape::template run<false, false>(reinterpret_cast<float*>(lds), oa, ob, nst, 0, sum, [] {});
     const int em = m0 + tid % BM, en0 = n0 + tid / BM;
 #pragma unroll
-    for (int u = 0; u < EPL; ++u) {
-      const int en = en0 + u * (THREADS / BM);
-      if (em >= m_lo && en >= n_lo) out[(long long)en * p.ldc + em] = sum[u];
-    }
+    for (int u = 0; u < EPL; ++u) store(em, en0 + u * (THREADS / BM), sum[u]);
   }
 }
 
@@ -323,8 +417,9 @@ static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
   const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)));
   const int stages = MODE == CONV_OUTP ? plan.split_stages : (p.K + f.bk - 1) / f.bk;
   p.dN = make_fastdiv(p.N); p.dMx = make_fastdiv(p.Mx); p.dk = make_fastdiv(p.k); p.dkk2 = make_fastdiv(p.kk2); p.dH = make_fastdiv(p.H);
-  p.dFg = make_fastdiv(p.Fg); p.dgx = make_fastdiv(p.gx); p.dgy = make_fastdiv(p.gy); p.dper = make_fastdiv(p.periods);
-  p.dsplits = make_fastdiv(p.splits); p.dG = make_fastdiv(p.G);
+  p.dFg4 = make_fastdiv(p.Fg4); p.dgx = make_fastdiv(p.gx); p.dgy = make_fastdiv(p.gy); p.dper = make_fastdiv(p.periods);
+  p.dsplits = make_fastdiv(p.splits); p.dG = make_fastdiv(p.G); p.ds = make_fastdiv(p.s);
+  p.dblock = make_fastdiv(p.block); p.dblock2 = make_fastdiv(p.block * p.block); p.dlines = make_fastdiv(p.lines);
   const size_t tab = (size_t)conv_ring_table(MODE, SINGLE, f.bk, stages);
 #define CONV_RING(...) hipLaunchKernelGGL((k_conv_ring<MODE, SINGLE, __VA_ARGS__>), grid, dim3(__VA_ARGS__::THREADS), tab, dn_stream(), p)
   switch (plan.cfg) {
@@ -338,7 +433,7 @@ static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
     case 7: if constexpr (MODE == CONV_OUTP) CONV_RING(ConvSplitCfg<96, 128, 32, 2, 4, 1, 2, 2>); else CONV_RING(ConvSplitCfg<128, 96, 32, 4, 2, 1, 2, 2>); break;
     case 8: if constexpr (MODE == CONV_OUTP) CONV_RING(ConvSplitCfg<64, 128, 32, 2, 4, 1, 2, 2>); else CONV_RING(ConvSplitCfg<128, 64, 32, 4, 2, 1, 2, 2>); break;
     case 9: CONV_RING(ConvSplitCfg<64, 64, 32, 2, 2, 1, 2, 3>); break;
-    default: if constexpr (MODE == CONV_DOWN) CONV_RING(ConvSplitCfg<128, 48, 64, 4, 1, 2, 2, 2>); break;
+    default: if constexpr (MODE == CONV_DOWN || MODE == CONV_DOWNM) CONV_RING(ConvSplitCfg<128, 48, 64, 4, 1, 2, 2, 2>); break;
   }
 #undef CONV_RING
 }

@@ -2,8 +2,8 @@
 // itself).  Args: ConvArgs or anything with its sizes.
 #pragma once
 
-// CONV_DOWNM: convDown for strided layers with few colours, all stride*stride pixel
-// phases merged into the columns of one product (uniform-row kernels only).
+// CONV_DOWNM: convDown of few colours, the pixels of a block (of the stride's side, on ring tiles of a multiple of it)
+// merged into the columns of one product (uniform-row kernels and ring tiles of one block each).
 enum { CONV_UP = 0, CONV_DOWN = 1, CONV_OUTP = 2, CONV_DOWNM = 3 };
 
 #define RING_MAX_SIDE 15   // filter rows and columns that a mask has room for
@@ -47,7 +47,7 @@ static const ConvRingTile g_conv_ring_cfgs[CONV_CFGS] = {
 static inline ConvRingTile conv_ring_cfg(int mode, int c) {
   ConvRingTile f = g_conv_ring_cfgs[c];
   if (mode == CONV_OUTP && (c == 7 || c == 8)) { f.bm = f.bn; f.bn = 128; }
-  if (c == 10 && mode != CONV_DOWN) f.bm = 0;
+  if (c == 10 && mode != CONV_DOWN && mode != CONV_DOWNM) f.bm = 0;
   return f;
 }
 // What a workgroup's LDS holds besides the two stages of its tile, which take 36 to 57 KB in fp32.  Two workgroups share a CU
@@ -74,10 +74,10 @@ static inline int conv_tile_lds(int mode, int c) {
   return c < CONV_RING_CFGS ? conv_ring_lds(mode, f.bm, f.bn, f.bk) : conv_split_lds(f.bm, f.bn, f.bk);
 }
 
-struct ConvRingPlan { int cfg, splits, split_stages; bool single; double us; };
+struct ConvRingPlan { int cfg, splits, split_stages; bool single; double us; int blocks; };   // blocks: conv_pixels_plan's
 
 static inline int conv_ring_entry(int mode, bool single, int bk) {      // table bytes per stage
-  return mode == CONV_UP ? 8 * bk : mode == CONV_DOWN && !single ? 3 * bk : 2 * bk;
+  return mode == CONV_UP ? 8 * bk : mode == CONV_DOWNM || (mode == CONV_DOWN && !single) ? 3 * bk : 2 * bk;
 }
 static inline int conv_ring_table(int mode, bool single, int bk, int stages) {      // table bytes of a workgroup
   return ((stages < 1 ? 1 : stages) + (single ? RING_AHEAD : 0)) * conv_ring_entry(mode, single, bk);
@@ -87,11 +87,11 @@ static inline int conv_ring_table(int mode, bool single, int bk, int stages) {  
 // rows x cols outputs per period, `jobs` periods x groups x chunks, K terms each, of which a tile has the share `used` on
 // average; split_us: what adding up one more partial output costs (Outp).
 static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows, int cols, long long jobs, int K, double used,
-                                          bool can_split, double split_us, int cus, bool bf16 = false) {
+                                          bool can_split, double split_us, int cus, bool bf16 = false, bool uneven = false) {
   ConvRingPlan best = {-1, 1, 0, false, 0.};
   for (int c = bf16 ? CONV_RING_CFGS : 0; c < (bf16 ? CONV_CFGS : CONV_RING_CFGS); ++c) {
     const ConvRingTile f = conv_ring_cfg(mode, c);
-    if (f.bm == 0 || rows < f.bm || cols < f.bn) continue;
+    if (f.bm == 0 || rows < f.bm || (cols < f.bn && mode != CONV_DOWNM)) continue;   // (of DownM columns may be missing)
     const long long tiles = (rows + f.bm - 1) / f.bm * ((cols + f.bn - 1) / f.bn) * jobs;
     const int nst = (K + f.bk - 1) / f.bk;
     const int most = RING_TABLE_BYTES / conv_ring_entry(mode, single, f.bk) - (single ? RING_AHEAD : 0);
@@ -109,9 +109,9 @@ static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows,
       // alone on its CU a workgroup shows its waits (122 -> 126 colours of 5 x 5 on 16 filters, 24 x 24, batch 100: 66 -> 77 us)
       if (rounds > 1. && c < CONV_RING_CFGS && 2 * (conv_tile_lds(mode, c) + conv_ring_table(mode, single, f.bk, per)) > RING_CU_LDS) rounds *= 1.16;
       double share = used;
+      // where there are few rounds, the tiles in the middle of a map, which have all taps, end the last one
+      if (c >= CONV_RING_CFGS || uneven) share += (1. - used) / (rounds > 1. ? rounds : 1.);
       if (c >= CONV_RING_CFGS) {
-        // these have few rounds, and the tiles in the middle of a map, which have all taps, end the last one
-        share += (1. - used) / (rounds > 1. ? rounds : 1.);
         // Few of the smallest per CU show their waits.  Measured on two cards, against the fp32 tiles: convUp and convDown take
         // 1.10 and 1.08 times as long with one, 1.02 and 0.97 with two, 0.84 and 0.80 with more; Outp, of short reductions,
         // 1.05 and 1.01 with one or two, 0.95 and 0.90 with three or four, 0.88 and 0.83 with more.
@@ -119,7 +119,7 @@ static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows,
         rounds *= 1.08;                               // (what the estimates miss: they are to win by that much)
       }
       const double us = 3. + rounds * (share * per * f.stage + f.tile) + (real > 1 ? 2.5 + real * split_us : 0.);
-      if (best.cfg < 0 || us < best.us) best = {c, real, per, single, us};
+      if (best.cfg < 0 || us < best.us) best = {c, real, per, single, us, 0};
     }
   }
   return best;
@@ -215,7 +215,7 @@ static inline double ring_crowd(const Args& a) {
   return all > 0. ? most / all : 1.;
 }
 
-static inline ConvRingPlan conv_no_ring() { return {-1, 1, 0, false, 0.}; }
+static inline ConvRingPlan conv_no_ring() { return {-1, 1, 0, false, 0., 0}; }
 
 // Up and Down: tiles over any run of (module | pixel, image) groups, which needs batches of whole groups of four, or of
 // one module or pixel each, which leave out taps beyond the edge and need no masks.  cfg < 0: none fits.
@@ -251,6 +251,75 @@ static inline ConvRingPlan conv_rows_choice(const Args& a, int mode, bool maps16
   const ConvRingPlan ring = conv_rows_plan(a, mode, maps16, filters16, cus), split = conv_rows_best(a, mode, cus, true);
   const double other = ring.cfg >= 0 ? ring.us : conv_other_us(a, mode, mode == CONV_UP ? a.M : a.HH, maps16, filters16, cus);
   return split.cfg >= 0 && split.us < other ? split : ring;
+}
+
+// Down of strided layers, of few colours, or of filters that are no multiple of four: on tiles of one pixel (blocks = 0), or
+// (DownM) of one block of `blocks` x `blocks` strides of pixels, whose pixels are columns beside the colours: a tile's terms are
+// the modules that reach it, of which a pixel of a block has a tap with some only.  blocks < 0: on tiles over any run of (pixel,
+// image) groups, of stride 1.  The last entry of a tap may repeat filters where entries have masks (RING_LAST): not of one pixel.
+template <class Args>
+static inline ConvRingPlan conv_pixels_plan(const Args& a, int blocks, int cus, bool bf16) {
+  const int b = blocks > 0 ? blocks : 1, side = blocks > 0 ? b * a.s : 1, taps = b - 1 + (a.k + a.s - 1) / a.s, Fg4 = (a.Fg + 3) / 4 * 4;
+  const long long cols = (long long)a.Cg * side * side;
+  if (a.local || !ring_ok(a, (long long)a.Cg * a.kk2) || a.Fg < 4 || taps > RING_MAX_SIDE) return conv_no_ring();
+  if (blocks < 0) {
+    if (a.s != 1 || a.N % 4 != 0) return conv_no_ring();
+    ConvRingPlan plan = conv_ring_plan(CONV_DOWN, false, (long long)a.HH * a.N, a.Cg, a.G, a.kk2 * Fg4, 1., false, 0., cus, bf16);
+    plan.blocks = blocks;
+    return plan;
+  }
+  if ((blocks == 0 && a.Fg != Fg4) || cols > 2048) return conv_no_ring();
+  const int lines = blocks > 0 ? (a.H - a.pad0 - 1) / side + 1 : a.H;
+  long long have = 0;                                                    // modules of a line that the taps of its pixels reach
+  for (int i = 0; i < lines; ++i) {
+    const int v = blocks > 0 ? i * b : (i - a.pad0) / a.s;               // the last module but b - 1 that reaches the first pixel
+    const int top = v + b - 1 < a.Mx - 1 ? v + b - 1 : a.Mx - 1, low = v + b - taps > 0 ? v + b - taps : 0;
+    if (top >= low) have += top - low + 1;
+  }
+  const double one = (double)have / ((double)lines * taps);
+  ConvRingPlan plan = conv_ring_plan(blocks > 0 ? CONV_DOWNM : CONV_DOWN, true, a.N, (int)cols, (long long)lines * lines * a.G, taps * taps * Fg4,
+                                     one * one, false, 0., cus, bf16, true);
+  plan.blocks = blocks;
+  return plan;
+}
+
+// What Down takes on the other kernels, in us (of layers on these tiles).
+template <class Args>
+static inline double conv_pixels_other_us(const Args& a, bool maps16, bool filters16, int cus) {
+  const double any = conv_other_us(a, CONV_DOWN, a.HH, maps16, filters16, cus);
+  if (a.s == 1)      // (k_conv_down_px: pixels in registers)
+    return a.Cg <= 4 && (a.k == 3 || a.k == 5) && a.Fg % 8 == 0 && a.Fg <= 128 ? 0.7 * any : any;
+  const int Np = padded_batch(a.N), Fp = padded_filters(a.F, a.G), Fg = Fp / a.G;
+  if (Np % 16 != 0 || Fg % 16 != 0 || !((Np != a.N || maps16) && filters16)) return any;      // (one lane per output)
+  const double maps = 1e-9 * 8. * Np * ((double)a.M * a.F + (double)a.HH * a.C), hid = 1e-9 * 8. * Np * a.M * Fp;   // GB of a copy
+  const double copies = (Np != a.N ? 5. + maps / 5e-3 : 0.) + (Fp != a.F ? 5. + hid / 5e-3 : 0.);
+  if (a.Cg > 16) {   // a pixel has every s-th tap of a row and column
+    const double flops = 2e-9 * Np * a.HH * ((a.Cg + 31) / 32 * 32) * a.G * a.kk2 * Fg / (a.s * a.s);
+    return 9. + flops / 85. * 1e3 + copies;
+  }
+  if (Np % 128 == 0) {   // pixels of a block as columns
+    const int taps = (a.k + a.s - 1) / a.s, cols = a.Cg * a.s * a.s;
+    const double lines = (a.H - 1 - a.pad0) / a.s + 1;
+    return 9. + 2e-9 * Np * lines * lines * ((cols + 15) / 16 * 16) * a.G * taps * taps * Fg / (cols <= 16 ? 75. : 110.) * 1e3 + copies;
+  }
+  // the patch matrix, written by a product and read by a gather
+  const double patch = 1e-9 * 8. * Np * a.M * a.Cg * a.kk2 * a.G;
+  return 9. + (2e-9 * Np * a.M * Fp * a.Cg * a.kk2 / 105. + patch / 5.) * 1e3 + copies;
+}
+
+// The fastest of these tiles, on the bf16 matrix cores or not; cfg < 0: none fits, or another kernel is expected to be faster.
+// (0.87: of layers whose estimates are as near as that, measured, half lose, by 20 % at most: 3 -> 208 colours of 7 x 7, stride 4, 200 x
+// 200, batch 80, 190 -> 237 us; 1 -> 48 of 7 x 7, 26 x 26, 80, 14.6 -> 18.1.)
+template <class Args>
+static inline ConvRingPlan conv_pixels_choice(const Args& a, bool maps16, bool filters16, int cus) {
+  ConvRingPlan best = conv_no_ring();
+  if (a.s == 1 && a.Cg > 16 && a.Fg % 4 == 0) return best;
+  for (int blocks = -1; blocks <= 4; blocks = blocks > 0 ? 2 * blocks : blocks + 1)
+    for (int bf16 = 0; bf16 < 2; ++bf16) {
+      const ConvRingPlan plan = conv_pixels_plan(a, blocks, cus, bf16 != 0);
+      if (plan.cfg >= 0 && (best.cfg < 0 || plan.us < best.us)) best = plan;
+    }
+  return best.cfg >= 0 && best.us < 0.87 * conv_pixels_other_us(a, maps16, filters16, cus) ? best : conv_no_ring();
 }
 
 // Outp of `a`, whose batch the ring takes in whole groups of four images: others are copied with up to three images of zeros.

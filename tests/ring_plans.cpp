@@ -45,4 +45,18 @@ void conv_tile(int mode, int N, int C, int H, int F, int k, int Mx, int s, int p
   out[4] = p.us;
 }
 
+// convDown of strided layers, few colours or filters that are no whole fours: out = {tile number or -1, side of a block in strides, 0 a
+// pixel or -1 any run, stages of the table, LDS bytes of a workgroup}
+void conv_pixels_tile(int N, int C, int H, int F, int k, int Mx, int s, int pad0, int G, int cus, double* out) {
+  const Sizes a = {N, C, C / G, H, H * H, F, F / G, k, k * k, Mx, Mx * Mx, s, pad0, G, 0, Mx * Mx, 1};
+  const ConvRingPlan p = conv_pixels_choice(a, N % 4 == 0, true, cus);
+  out[0] = p.cfg; out[1] = p.blocks;
+  if (p.cfg < 0) return;
+  const int mode = p.blocks > 0 ? CONV_DOWNM : CONV_DOWN, b = p.blocks > 0 ? p.blocks : 1, taps = b - 1 + (k + s - 1) / s;
+  const ConvRingTile f = conv_ring_cfg(mode, p.cfg);
+  const int terms = (p.blocks < 0 ? k * k : taps * taps) * ((a.Fg + 3) / 4 * 4), stages = (terms + f.bk - 1) / f.bk;
+  out[2] = stages;
+  out[3] = conv_tile_lds(mode, p.cfg) + conv_ring_table(mode, p.blocks >= 0, f.bk, stages);
+}
+
 }  // extern "C"

@@ -844,3 +844,58 @@ def test_locally_connected_layers_on_the_other_kernels(cm, cc, rng, N, C, H, F, 
             assert _relerr(got, f(a, b, c), f(np.abs(a), np.abs(b), np.abs(c)) + 1e-6) < REL
     for m in (X, W, Y, up, down, outp):
         m.free_device_memory()
+
+
+# convDown on tiles of a pixel or of a block of pixels (tests/test_ring_plans.py: every kind, on fp32 and bf16 tiles)
+PIXEL_LAYERS = [  # N, C, H, F, k, stride, padding, groups
+    (100, 16, 10, 256, 7, 2, 0, 1), (128, 24, 6, 128, 5, 2, 2, 1), (65, 72, 11, 16, 3, 2, 0, 1), (100, 84, 11, 148, 5, 2, 2, 1),
+    (47, 3, 17, 32, 5, 1, 2, 1), (33, 1, 13, 18, 7, 1, 3, 1), (100, 1, 16, 112, 3, 1, 0, 1), (128, 1, 26, 16, 3, 1, 0, 1),
+    (100, 20, 8, 32, 7, 1, 0, 2), (100, 28, 6, 64, 5, 1, 2, 2), (17, 1, 9, 5, 4, 3, 1, 1), (100, 3, 19, 256, 7, 2, 0, 1),
+    (128, 3, 29, 45, 11, 4, 5, 1), (36, 2, 12, 7, 3, 3, 0, 1), (100, 96, 7, 23, 7, 1, 0, 1), (176, 72, 6, 11, 3, 1, 1, 1),
+    (100, 68, 7, 25, 5, 1, 0, 1), (240, 16, 7, 17, 7, 1, 3, 1), (64, 56, 14, 65, 5, 1, 0, 1), (128, 24, 14, 93, 5, 1, 2, 1),
+    (144, 44, 16, 34, 3, 2, 1, 2), (151, 40, 14, 80, 5, 2, 2, 1), (128, 3, 58, 96, 11, 4, 0, 1), (100, 96, 14, 5, 3, 1, 0, 1),
+    (256, 32, 18, 5, 5, 2, 2, 1), (100, 96, 7, 16, 3, 3, 0, 1), (47, 16, 17, 5, 3, 2, 1, 1), (200, 96, 10, 32, 4, 4, 2, 1), (256, 48, 9, 16, 4, 4, 2, 1),
+    (100, 60, 9, 26, 3, 1, 1, 2), (64, 56, 7, 5, 3, 1, 0, 1)]
+
+
+@pytest.mark.parametrize("finite", [True, False])
+@pytest.mark.parametrize("N,C,H,F,k,s,p,G", PIXEL_LAYERS)
+def test_gradients_on_tiles_of_pixels(cm, cc, rng, N, C, H, F, k, s, p, G, finite):
+    """Every pixel has the modules that reach it and no others: where some are not finite, neither are just those pixels."""
+    Mx = co.n_modules(H, k, s, p)
+    y, w = _f(rng.standard_normal((N, F * Mx * Mx))), _f(0.1 * rng.standard_normal((F, C // G * k * k)))
+    if not finite:
+        y[0, Mx * Mx // 2] = np.inf
+        y[N - 1, (F - 1) * Mx * Mx] = np.nan
+        y[N // 2, -1] = -np.inf
+    Y, W, T = cm.CUDAMatrix(y), cm.CUDAMatrix(w), cm.CUDAMatrix(np.full((N, C * H * H), 7.0, dtype=np.float32))
+    cc.convDown(Y, W, T, Mx, p, s, k, H, C, numGroups=G)
+    got = T.asarray()
+    for m in (Y, W, T):
+        m.free_device_memory()
+    with np.errstate(invalid='ignore'):
+        want, bound = co.conv_down(y, w, C, H, p, s, G), co.conv_down(np.abs(y), np.abs(w), C, H, p, s, G)
+    if finite:
+        assert _relerr(got, want, bound + 1e-6) < REL
+        return
+    ok = co.conv_down(np.isfinite(y) == 0, np.ones_like(w), C, H, p, s, G) == 0
+    assert ok.any() and (~ok).any() and not np.isfinite(got[~ok]).any()
+    assert np.max(np.abs(got[ok] - want[ok]) / (bound[ok] + 1e-6)) < REL
+
+
+# the same layers on the kernels beside ring tiles, which filters of 16 x 16 are too large for: phases merged into 16 to 128 columns, the
+# patch matrix, uniform rows and 128- and 256-row tiles
+SIXTEEN = [(128, c, 18, 16, 16, 4, 0, 1) for c in (1, 2, 3, 4, 6, 8)] + [(32, 3, 18, 16, 16, 2, 0, 1), (17, 2, 17, 5, 16, 1, 0, 1)] + \
+          [(128, c, 17, 16, 16, 1, 0, 1) for c in (20, 40, 60, 100)] + [(32, c, 17, 16, 16, 1, 0, 1) for c in (20, 40, 70, 100)] + \
+          [(1024, 20, 18, 16, 16, 2, 0, 1)]
+
+
+@pytest.mark.parametrize("N,C,H,F,k,s,p,G", SIXTEEN)
+def test_gradients_of_filters_too_large_for_ring_tiles(cm, cc, rng, N, C, H, F, k, s, p, G):
+    Mx = co.n_modules(H, k, s, p)
+    y, w = _f(rng.standard_normal((N, F * Mx * Mx))), _f(0.1 * rng.standard_normal((F, C // G * k * k)))
+    Y, W, T = cm.CUDAMatrix(y), cm.CUDAMatrix(w), cm.CUDAMatrix(np.full((N, C * H * H), np.nan, dtype=np.float32))
+    cc.convDown(Y, W, T, Mx, p, s, k, H, C, numGroups=G)
+    assert _relerr(T.asarray(), co.conv_down(y, w, C, H, p, s, G), co.conv_down(np.abs(y), np.abs(w), C, H, p, s, G) + 1e-6) < REL
+    for m in (Y, W, T):
+        m.free_device_memory()

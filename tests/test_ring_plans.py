@@ -177,3 +177,32 @@ def test_long_strips_of_33_to_63_are_not_on_ring_tiles(plans):
         assert gemm_tile(plans, m, n, k) is None
     for m, n, k in ((19399, 49, 252), (57, 17393, 163), (26761, 64, 168), (32, 26761, 168)):
         assert gemm_tile(plans, m, n, k) is not None
+
+
+def pixels_tile(plans, N, C, H, F, k, s, p, G=1):
+    out = (ct.c_double * 4)()
+    plans.conv_pixels_tile(N, C, H, F, k, co.n_modules(H, k, s, p), s, -p, G, CUS, out)
+    return tuple(int(v) for v in out) if out[0] >= 0 else None
+
+
+def test_gradients_of_the_gpu_tests_reach_every_kind_of_pixel_tile(plans):
+    got = [pixels_tile(plans, *layer) for layer in conv.PIXEL_LAYERS]
+    assert None not in got and {t[1] for t in got} == {-1, 0, 1, 2, 4}
+    assert {t[0] >= 6 for t in got if t[1] == -1} == {t[0] >= 6 for t in got if t[1] > 0} == {False, True}
+    for tile, blocks, stages, lds in got:
+        assert lds <= 160 << 10 and stages >= 1
+    assert [layer for layer in conv.PIXEL_LAYERS if conv_tile(plans, DOWN, *layer)] == []
+    for layer in conv.SIXTEEN:
+        assert pixels_tile(plans, *layer) is None and conv_tile(plans, DOWN, *layer) is None
+
+
+def test_tables_of_pixel_tiles_fit(plans):
+    import random
+    rng, taken = random.Random(5), 0
+    for _ in range(3000):
+        k = rng.randint(1, 16)
+        H, s, p = rng.randint(k, 60), rng.randint(1, min(k, 5)), rng.choice([0, k // 2])
+        t = pixels_tile(plans, rng.randint(1, 260), rng.randint(1, 130), H, rng.randint(1, 260), k, s, p)
+        taken += t is not None
+        assert t is None or (t[3] <= 160 << 10 and k <= 15)
+    assert taken > 800
