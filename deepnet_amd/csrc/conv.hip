@@ -45,6 +45,7 @@
 #include "conv_ring_plan.h"
 #include <math.h>
 #include <stdio.h>
+#include <string.h>
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -2654,7 +2655,7 @@ static void conv_outp_filters(cudamat* images, cudamat* hidActs, cudamat* target
 static ConvRingArgs ring_args(const ConvArgs& a) {
   ConvRingArgs p = {};
   p.N = a.N; p.H = a.H; p.HH = a.HH; p.Mx = a.Mx; p.M = a.M; p.k = a.k; p.kk2 = a.kk2; p.s = a.s; p.pad0 = a.pad0;
-  p.Cg = a.Cg; p.Fg = a.Fg; p.Fg4 = (a.Fg + 3) / 4 * 4; p.F = a.F; p.G = a.G; p.local = a.local; p.out = a.out;
+  p.Cg = a.Cg; p.Fg = a.Fg; p.F = a.F; p.G = a.G; p.local = a.local; p.out = a.out;
   p.m_count = a.m_count; p.splits = 1; p.periods = 1;
   return p;
 }
@@ -2668,11 +2669,50 @@ static bool ring_maps16(const ConvArgs& a) {
   return dn_aligned16(a.img ? a.img : a.hid) && dn_aligned16(a.hid) && dn_aligned16(a.out);
 }
 
+// Down on tiles of one pixel or block of pixels (conv_pixels_plan).
+static bool conv_pixels_ring(const ConvArgs& a, const ConvRingPlan& plan, const char* where) {
+  const int b = plan.blocks > 0 ? plan.blocks : 1, taps = b - 1 + (a.k + a.s - 1) / a.s;
+  const bool flat = plan.blocks < 0;
+  ConvRingArgs p = ring_args(a);
+  p.a = a.hid; p.b = a.flt;
+  p.a_bytes = (unsigned)((long long)a.N * a.M * a.F * 4);
+  p.b_bytes = (unsigned)((long long)a.F * a.Cg * a.kk2 * 4);
+  p.block = plan.blocks > 0 ? b * a.s : 1;
+  p.lines = plan.blocks > 0 ? (a.H - a.pad0 - 1) / p.block + 1 : a.H;
+  p.rows = flat ? a.HH * a.N : a.N; p.cols = a.Cg * p.block * p.block; p.periods = flat ? 1 : p.lines * p.lines; p.gz = a.G;
+  p.K = (flat ? a.kk2 : taps * taps) * p.Fg4();
+  p.ldc = (long long)a.N * a.HH;
+  if (plan.blocks > 0) conv_ring_launch<CONV_DOWNM, true>(plan, p);
+  else if (flat) conv_ring_launch<CONV_DOWN, false>(plan, p);
+  else conv_ring_launch<CONV_DOWNS, true>(plan, p);
+  return ring_done(where);
+}
+
+// The choice for a layer (it depends on its sizes and alignment only), kept for the next call: it prices some hundred plans, which is
+// several microseconds of the host's, as long as the shortest passes take.
+static const ConvChoice& conv_chosen(const ConvArgs& a, int mode) {
+  struct Entry { int key[14]; bool used; ConvChoice choice; };
+  static Entry cache[128];
+  const int key[14] = {mode, a.N, a.C, a.H, a.F, a.k, a.Mx, a.s, a.pad0, a.G, a.local, a.m_count, a.chunks,
+                       (ring_maps16(a) ? 2 : 0) + (dn_aligned16(a.flt) ? 1 : 0)};
+  unsigned h = 0;
+  for (int v : key) h = h * 0x9e3779b1u + (unsigned)v;
+  Entry& e = cache[(h >> 16) % 128];
+  if (!e.used || memcmp(e.key, key, sizeof key) != 0) {
+    e.choice = conv_choice(a, mode, ring_maps16(a), dn_aligned16(a.flt), dn_num_cus());
+    memcpy(e.key, key, sizeof key);
+    e.used = true;
+  }
+  return e.choice;
+}
+
 // Up and Down on ring tiles; false: not a pass for them.
 static bool conv_rows_ring(const ConvArgs& a, int mode, const char* where) {
   const bool up = mode == CONV_UP;
-  const ConvRingPlan plan = conv_rows_choice(a, mode, ring_maps16(a), dn_aligned16(a.flt), dn_num_cus());
+  const ConvChoice& choice = conv_chosen(a, mode);
+  const ConvRingPlan& plan = choice.plan;
   if (plan.cfg < 0) return false;
+  if (choice.pixels) return conv_pixels_ring(a, plan, where);
   const bool single = plan.single;
   const int sites = up ? a.M : a.HH, cols = up ? a.Fg : a.Cg, K = a.kk2 * (up ? a.Cg : (a.Fg + 3) / 4 * 4);
   const long long bank = (long long)a.Cg * a.kk2 * (a.local ? a.M : 1);
@@ -2687,27 +2727,6 @@ static bool conv_rows_ring(const ConvArgs& a, int mode, const char* where) {
   return ring_done(where);
 }
 
-// Down on tiles of one pixel or block of pixels (conv_pixels_choice); false: not a pass for them.
-static bool conv_pixels_ring(const ConvArgs& a, const char* where) {
-  const ConvRingPlan plan = conv_pixels_choice(a, ring_maps16(a), dn_aligned16(a.flt), dn_num_cus());
-  if (plan.cfg < 0) return false;
-  const int b = plan.blocks > 0 ? plan.blocks : 1, taps = b - 1 + (a.k + a.s - 1) / a.s;
-  const bool flat = plan.blocks < 0;
-  ConvRingArgs p = ring_args(a);
-  p.a = a.hid; p.b = a.flt;
-  p.a_bytes = (unsigned)((long long)a.N * a.M * a.F * 4);
-  p.b_bytes = (unsigned)((long long)a.F * a.Cg * a.kk2 * 4);
-  p.block = plan.blocks > 0 ? b * a.s : 1;
-  p.lines = plan.blocks > 0 ? (a.H - a.pad0 - 1) / p.block + 1 : a.H;
-  p.rows = flat ? a.HH * a.N : a.N; p.cols = a.Cg * p.block * p.block; p.periods = flat ? 1 : p.lines * p.lines; p.gz = a.G;
-  p.K = (flat ? a.kk2 : taps * taps) * p.Fg4;
-  p.ldc = (long long)a.N * a.HH;
-  if (plan.blocks > 0) conv_ring_launch<CONV_DOWNM, true>(plan, p);
-  else if (flat) conv_ring_launch<CONV_DOWN, false>(plan, p);
-  else conv_ring_launch<CONV_DOWN, true>(plan, p);
-  return ring_done(where);
-}
-
 static void launch_outp_finish(const ConvArgs& a) {
   const int total = a.F * a.Cg * a.kk2;
   if (a.splits >= 64 && a.chunks == 1) hipLaunchKernelGGL(k_conv_outp_finish_wide, dim3((total + 63) / 64), dim3(1024), 0, dn_stream(), a);
@@ -2716,7 +2735,7 @@ static void launch_outp_finish(const ConvArgs& a) {
 }
 
 static bool conv_outp_ring(const ConvArgs& a0, cudamat* images, cudamat* hidActs, const char* where) {
-  const ConvRingPlan plan = conv_outp_choice(a0, ring_maps16(a0), dn_aligned16(a0.flt), dn_num_cus());
+  const ConvRingPlan& plan = conv_chosen(a0, CONV_OUTP).plan;
   if (plan.cfg < 0) return false;
   ConvArgs a = a0;
   const int N4 = (a.N + 3) / 4 * 4, cols = a.Cg * a.kk2, K = a.m_count * N4;
@@ -2768,7 +2787,6 @@ void convDown(cudamat* hidActs, cudamat* filters, cudamat* targets, int imgSize,
   ConvArgs a;
   if (!conv_down_args(hidActs, filters, targets, imgSize, paddingStart, moduleStride, numImgColors, numGroups, "convDown", false, a)) return;
   if (conv_rows_ring(a, CONV_DOWN, "convDown")) return;
-  if (conv_pixels_ring(a, "convDown")) return;
   PaddedBatch pb(hidActs, targets, nullptr);
   if (pb.on) {
     pb.fill(0, hidActs);

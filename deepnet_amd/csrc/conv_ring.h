@@ -17,14 +17,22 @@ struct ConvRingArgs {
   const float* a; const float* b;
   float* out;
   unsigned a_bytes, b_bytes;
-  int N, H, HH, Mx, M, k, kk2, s, pad0, Cg, Fg, Fg4, F, G;          // Fg4: filters of a group in whole fours
+  int N, H, HH, Mx, M, k, kk2, s, pad0, Cg, Fg, F, G;
   int local;                    // one filter bank per module
   int rows, cols;               // of one period: a tile lies inside one (one module or pixel, or everything)
   int periods, gx, gy, gz;      // tiles per period down the rows, across; Up / Down: groups; Outp: chunks x splits x groups
   int K;                        // Outp: terms of a chunk
-  int block, lines;             // DownM: side of a block of pixels, blocks per side of a map
-  int m_count, splits, split_stages;
-  FastDiv dN, dMx, dk, dkk2, dH, dFg4, dgx, dgy, dper, dsplits, dG, ds, dblock, dblock2, dlines;
+  // (what only Outp has, and only DownM: side of a block of pixels, blocks per side of a map.  64 bytes more of arguments are 0.15 us
+  // a launch)
+  union { int m_count, block; };
+  union { int splits, lines; };
+  int split_stages;
+  FastDiv dN, dH, dFg4, dgx, dgy, dper, dG;
+  union { FastDiv dsplits, ds; };                                        // Outp; Down
+  union { FastDiv dMx, dlines; };                                        // all others; DownM
+  union { FastDiv dk, dblock; };
+  union { FastDiv dkk2, dblock2; };
+  __host__ __device__ int Fg4() const { return (Fg + 3) & ~3; }          // filters of a group in whole fours
   long long ldc, out_stride;    // of a column; Outp: of a (chunk, split)
 };
 
@@ -151,6 +159,8 @@ __device__ __forceinline__ float conv_down_one(const ConvRingArgs& p, int g, int
 //   96 -> 112 colours 7 x 7, stride 2, 10 x 10, batch 128   131 -> 17      1 -> 64 of 11 x 11, stride 2, 223 x 223, 100    2044 -> 506
 //   84 -> 148 of 5 x 5, stride 2, 11 x 11, 100    120 -> 36                3 -> 32 of 5 x 5, 18 x 18, 100     21 -> 11
 //   24 -> 93 of 7 x 7, 31 x 31, 151 (whole fours of filters)    645 -> 339
+// Filters, colours, images or taps that are fewer than any tile has (13 filters, 9 taps) run on tiles larger than them as well: 60 ->
+// 13 colours 7 x 7, 11 x 11, 100 61 -> 23 us Up, 54 -> 21 Outp (before: a copy to 16 filters, or one lane per output).
 // Of 210 random layers that they take, one was 4 % slower than before, none by more; half are twice as fast.  (3 -> 96 of 11 x 11,
 // stride 4, 224 x 224, 128, as fast either way, stays on phases of 128 images.)
 // Measured, us Up / Down / Outp, operands from memory, before -> now (with the copies and sums):
@@ -191,7 +201,7 @@ template <int MODE, bool SINGLE, class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRingArgs p) {
   constexpr int PER = MODE == CONV_UP ? 1 : 4, BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, THREADS = Cfg::THREADS;
   using OA = ConvRingOperand<MODE == CONV_OUTP ? 3 : MODE == CONV_DOWNM ? 9 : SINGLE ? 5 : 0, typename Cfg::template Tile<BM, MODE == CONV_OUTP>, PER>;
-  using OB = ConvRingOperand<MODE == CONV_UP ? (SINGLE ? 6 : 1) : MODE == CONV_DOWN ? (SINGLE ? 7 : 2) : MODE == CONV_DOWNM ? 8 : 4,
+  using OB = ConvRingOperand<MODE == CONV_UP ? (SINGLE ? 6 : 1) : MODE == CONV_DOWN ? (SINGLE ? 7 : 2) : MODE == CONV_DOWNS ? 7 : MODE == CONV_DOWNM ? 8 : 4,
                              typename Cfg::template Tile<BN, MODE != CONV_UP>, PER>;
   using Shape = typename Cfg::template Shape<OA, OB>;
   constexpr int EPL = Shape::EPL, LDS = Cfg::SPLIT ? Shape::LDS : 4 * Shape::LDS;
@@ -214,9 +224,12 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
   const int by = t - rest * p.gy;
   t = rest; rest = div(t, p.dgx);
   const int bx = t - rest * p.gx, z = div(rest, p.dper), per = rest - z * p.periods;
-  // a tile over the edge moves back inside; the outputs it shares with its neighbour are that one's to store
+  // a tile over the edge moves back inside; the outputs it shares with its neighbour are that one's to store (of a tile larger than
+  // all there is, rows and columns behind the last are computed from what stands there, or zeros, and not stored)
   const int m_lo = bx * BM, n_lo = by * BN;
-  const int m0 = m_lo + BM <= p.rows ? m_lo : p.rows - BM, n0 = n_lo + BN <= p.cols || p.cols < BN ? n_lo : p.cols - BN;
+  constexpr bool LOOSE = conv_may_be_loose(MODE, Cfg::SPLIT);
+  const int m0 = m_lo + BM <= p.rows || (LOOSE && p.rows < BM) ? m_lo : p.rows - BM;
+  const int n0 = n_lo + BN <= p.cols || (LOOSE && p.cols < BN) ? n_lo : p.cols - BN;
 
   OA oa; OB ob;
   int nst, g = z;
@@ -225,14 +238,19 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
     // One module or pixel: taps that leave the image, or reach no module, are left out.  Up: the others are rows ky0 ..
     // ky0 + ny - 1 and columns kx0 .. kx0 + nx - 1 of the filter.  Down: modules my0, my0 - 1 .. my0 - ny + 1 (of a line) have the
     // pixel at rows ky0, ky0 + s ..; a block of pixels: the tap of its first pixel there, which may lie outside the filter.
-    constexpr bool UP = MODE == CONV_UP, MERGED = MODE == CONV_DOWNM;
-    const int s = p.s, blocks = MERGED ? div(p.block, p.ds) : 1;
+    constexpr bool UP = MODE == CONV_UP, MERGED = MODE == CONV_DOWNM, ONE = MODE == CONV_DOWN;      // ONE: of stride 1
+    const int s = ONE ? 1 : p.s, blocks = MERGED ? div(p.block, p.ds) : 1;
     const int line = div(per, UP ? p.dMx : MERGED ? p.dlines : p.dH), at = per - line * (UP ? Mx : MERGED ? p.lines : H);
     const int y = UP ? line * s + p.pad0 : MERGED ? line * p.block : line - p.pad0, x = UP ? at * s + p.pad0 : MERGED ? at * p.block : at - p.pad0;
     auto range = [&](int v, int* first, int* m_first) {
       if (UP) {
         *first = -v > 0 ? -v : 0;
         return (H - v < k ? H - v : k) - *first;
+      }
+      if (ONE) {
+        *first = v - Mx + 1 > 0 ? v - Mx + 1 : 0;
+        *m_first = v - *first;
+        return (v + 1 < k ? v + 1 : k) - *first;
       }
       const int top = div(v, p.ds) + blocks - 1, m = top < Mx - 1 ? top : Mx - 1, reach = MERGED ? k + s * (blocks - 1) : k;
       *m_first = m;
@@ -243,7 +261,7 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
     int ky0, kx0, my0 = 0, mx0 = 0;
     int ny = range(y, &ky0, &my0), nx = range(x, &kx0, &mx0);
     if (ny <= 0 || nx <= 0) { ny = 0; nx = 1; }
-    const int area = ny * nx, K = area * (UP ? p.Cg : p.Fg4);
+    const int area = ny * nx, K = area * (UP ? p.Cg : p.Fg4());
     nst = K > BK ? (K + BK - 1) / BK : 1;
     unsigned* tab1 = reinterpret_cast<unsigned*>(table + (nst + RING_AHEAD) * (BK / PER));
     // exact for dividends below 2^12 and divisors up to RING_MAX_SIDE^2
@@ -261,8 +279,8 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
           t2.x = 4u * Nu * (unsigned)((g * p.Cg + c) * p.HH + (y + ky) * H + x + kx);
           t2.y = 4u * Fu * (unsigned)((bank * p.Cg + c) * p.kk2 + ky * k + kx);
         } else {
-          const int m = (my0 - ty) * Mx + mx0 - tx, ky = ky0 + s * ty, kx = kx0 + s * tx;
-          int f = 4 * e - tap * p.Fg4;
+          const int ky = ky0 + s * ty, kx = kx0 + s * tx, m = ONE ? (y - ky) * Mx + x - kx : (my0 - ty) * Mx + mx0 - tx;
+          int f = 4 * e - tap * p.Fg4();
           if (MERGED && f + 4 > p.Fg) { f = p.Fg - 4; need = RING_LAST; }
           t2.x = 4u * Nu * (unsigned)(p.M * (g * p.Fg + f) + m);
           t2.y = 4u * ((unsigned)f + Fu * (unsigned)(ky * k + kx + p.Cg * p.kk2 * (p.local ? m : 0)));
@@ -278,7 +296,7 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
 #pragma unroll
     for (int u = 0; u < OA::NG; ++u) {
       oa.off[u] = 4u * (unsigned)(n + (PER == 4 ? N * p.M * (OA::group_k(tid, u) % 4) : 0));
-      if (MERGED) oa.mask[u] = OA::group_k(tid, u) % 4 < p.Fg4 - p.Fg ? RING_LAST : 0u;
+      if (MERGED) oa.mask[u] = OA::group_k(tid, u) % 4 < p.Fg4() - p.Fg ? RING_LAST : 0u;
     }
 #pragma unroll
     for (int u = 0; u < OB::NG; ++u) {
@@ -324,11 +342,11 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
       ob.off[u] = 4u * (unsigned)(OB::group_k(tid, u) * p.F + g * p.Fg + n0 + OB::group_row(tid, u));
     out += (long long)g * p.Fg * p.ldc;
   } else if constexpr (MODE == CONV_DOWN) {
-    const int K = p.kk2 * p.Fg4;
+    const int K = p.kk2 * p.Fg4();
     nst = (K + BK - 1) / BK;
     unsigned* tab1 = reinterpret_cast<unsigned*>(table + nst * (BK / 4));
     for (int e = tid; e < nst * (BK / 4); e += THREADS) {
-      const int tap = div(4 * e, p.dFg4), f0 = 4 * e - tap * p.Fg4, f = f0 + 4 > p.Fg ? p.Fg - 4 : f0, ky = div(tap, p.dk), kx = tap - ky * k;
+      const int tap = div(4 * e, p.dFg4), f0 = 4 * e - tap * p.Fg4(), f = f0 + 4 > p.Fg ? p.Fg - 4 : f0, ky = div(tap, p.dk), kx = tap - ky * k;
       const bool in = 4 * e < K;
       table[e] = make_uint2(4u * (unsigned)N * (unsigned)(p.M * f - ky * Mx - kx),
                             in ? 1u << ky | 1u << (RING_MAX_SIDE + kx) | (f < f0 ? RING_LAST : 0u) : RING_FAR);
@@ -340,7 +358,7 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
     for (int u = 0; u < OA::NG; ++u) {
       oa.off[u] = 4u * (unsigned)(n + N * (y * Mx + x + p.M * (g * p.Fg + OA::group_k(tid, u) % 4)));
       oa.mask[u] = ring_bits(y - Mx + 1, y + 1 < k ? y + 1 : k) | ring_bits(x - Mx + 1, x + 1 < k ? x + 1 : k) << RING_MAX_SIDE |
-                   (OA::group_k(tid, u) % 4 < p.Fg4 - p.Fg ? 0u : RING_LAST);
+                   (OA::group_k(tid, u) % 4 < p.Fg4() - p.Fg ? 0u : RING_LAST);
     }
     oa.tab = table;
     ob.tab1 = tab1;
@@ -379,8 +397,9 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
   __syncthreads();
 
   // output (em, en) of the tile: at column en, or (DownM) at the pixel that it stands for, which may lie outside the map
-  auto store = [&](int em, int en, float v) {
-    if (em < m_lo || en < n_lo || en >= p.cols) return;
+  const unsigned ms = (unsigned)((m0 + BM < p.rows ? m0 + BM : p.rows) - m_lo), ns = (unsigned)((n0 + BN < p.cols ? n0 + BN : p.cols) - n_lo);
+  auto store = [&](int em, int en, float v) __attribute__((always_inline)) {
+    if (LOOSE ? (unsigned)(em - m_lo) >= ms || (unsigned)(en - n_lo) >= ns : em < m_lo || en < n_lo) return;
     if constexpr (MODE == CONV_DOWNM) {
       const int line = div(per, p.dlines), at = per - line * p.lines;
       const int c = div(en, p.dblock2), q = en - c * p.block * p.block, py = div(q, p.dblock), px = q - py * p.block;
@@ -416,10 +435,12 @@ static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
   const long long tiles = (long long)p.periods * p.gx * p.gy * p.gz;
   const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)));
   const int stages = MODE == CONV_OUTP ? plan.split_stages : (p.K + f.bk - 1) / f.bk;
-  p.dN = make_fastdiv(p.N); p.dMx = make_fastdiv(p.Mx); p.dk = make_fastdiv(p.k); p.dkk2 = make_fastdiv(p.kk2); p.dH = make_fastdiv(p.H);
-  p.dFg4 = make_fastdiv(p.Fg4); p.dgx = make_fastdiv(p.gx); p.dgy = make_fastdiv(p.gy); p.dper = make_fastdiv(p.periods);
-  p.dsplits = make_fastdiv(p.splits); p.dG = make_fastdiv(p.G); p.ds = make_fastdiv(p.s);
-  p.dblock = make_fastdiv(p.block); p.dblock2 = make_fastdiv(p.block * p.block); p.dlines = make_fastdiv(p.lines);
+  p.dN = make_fastdiv(p.N); p.dH = make_fastdiv(p.H); p.dFg4 = make_fastdiv(p.Fg4()); p.dG = make_fastdiv(p.G);
+  p.dgx = make_fastdiv(p.gx); p.dgy = make_fastdiv(p.gy); p.dper = make_fastdiv(p.periods);
+  p.dsplits = make_fastdiv(MODE == CONV_OUTP ? p.splits : p.s);
+  p.dMx = make_fastdiv(MODE == CONV_DOWNM ? p.lines : p.Mx);
+  p.dk = make_fastdiv(MODE == CONV_DOWNM ? p.block : p.k);
+  p.dkk2 = make_fastdiv(MODE == CONV_DOWNM ? p.block * p.block : p.kk2);
   const size_t tab = (size_t)conv_ring_table(MODE, SINGLE, f.bk, stages);
 #define CONV_RING(...) hipLaunchKernelGGL((k_conv_ring<MODE, SINGLE, __VA_ARGS__>), grid, dim3(__VA_ARGS__::THREADS), tab, dn_stream(), p)
   switch (plan.cfg) {
@@ -433,7 +454,7 @@ static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
     case 7: if constexpr (MODE == CONV_OUTP) CONV_RING(ConvSplitCfg<96, 128, 32, 2, 4, 1, 2, 2>); else CONV_RING(ConvSplitCfg<128, 96, 32, 4, 2, 1, 2, 2>); break;
     case 8: if constexpr (MODE == CONV_OUTP) CONV_RING(ConvSplitCfg<64, 128, 32, 2, 4, 1, 2, 2>); else CONV_RING(ConvSplitCfg<128, 64, 32, 4, 2, 1, 2, 2>); break;
     case 9: CONV_RING(ConvSplitCfg<64, 64, 32, 2, 2, 1, 2, 3>); break;
-    default: if constexpr (MODE == CONV_DOWN || MODE == CONV_DOWNM) CONV_RING(ConvSplitCfg<128, 48, 64, 4, 1, 2, 2, 2>); break;
+    default: if constexpr (MODE == CONV_DOWN || MODE == CONV_DOWNS || MODE == CONV_DOWNM) CONV_RING(ConvSplitCfg<128, 48, 64, 4, 1, 2, 2, 2>); break;
   }
 #undef CONV_RING
 }

@@ -4,7 +4,8 @@
 
 // CONV_DOWNM: convDown of few colours, the pixels of a block (of the stride's side, on ring tiles of a multiple of it)
 // merged into the columns of one product (uniform-row kernels and ring tiles of one block each).
-enum { CONV_UP = 0, CONV_DOWN = 1, CONV_OUTP = 2, CONV_DOWNM = 3 };
+// CONV_DOWNS: convDown of any stride on ring tiles of one pixel (CONV_DOWN there: of stride 1).
+enum { CONV_UP = 0, CONV_DOWN = 1, CONV_OUTP = 2, CONV_DOWNM = 3, CONV_DOWNS = 4 };
 
 #define RING_MAX_SIDE 15   // filter rows and columns that a mask has room for
 #define RING_AHEAD 7       // stages that the table of a tile of one module or pixel reaches beyond its last one
@@ -47,7 +48,7 @@ static const ConvRingTile g_conv_ring_cfgs[CONV_CFGS] = {
 static inline ConvRingTile conv_ring_cfg(int mode, int c) {
   ConvRingTile f = g_conv_ring_cfgs[c];
   if (mode == CONV_OUTP && (c == 7 || c == 8)) { f.bm = f.bn; f.bn = 128; }
-  if (c == 10 && mode != CONV_DOWN && mode != CONV_DOWNM) f.bm = 0;
+  if (c == 10 && (mode == CONV_UP || mode == CONV_OUTP)) f.bm = 0;
   return f;
 }
 // What a workgroup's LDS holds besides the two stages of its tile, which take 36 to 57 KB in fp32.  Two workgroups share a CU
@@ -83,15 +84,18 @@ static inline int conv_ring_table(int mode, bool single, int bk, int stages) {  
   return ((stages < 1 ? 1 : stages) + (single ? RING_AHEAD : 0)) * conv_ring_entry(mode, single, bk);
 }
 
+// Whether a tile may be larger than all of a period (see k_conv_ring).
+static constexpr bool conv_may_be_loose(int mode, bool bf16) { return !bf16 || mode == CONV_DOWNM; }
+
 // The tile (of the fp32 ones, or of those on the bf16 matrix cores) that is expected to be fastest, cfg < 0: none fits.
 // rows x cols outputs per period, `jobs` periods x groups x chunks, K terms each, of which a tile has the share `used` on
-// average; split_us: what adding up one more partial output costs (Outp).
+// average; split_us: what adding up one more partial output costs (Outp).  loose: tiles may be larger than all of a period.
 static inline ConvRingPlan conv_ring_plan(int mode, bool single, long long rows, int cols, long long jobs, int K, double used,
-                                          bool can_split, double split_us, int cus, bool bf16 = false, bool uneven = false) {
+                                          bool can_split, double split_us, int cus, bool bf16 = false, bool uneven = false, bool loose = false) {
   ConvRingPlan best = {-1, 1, 0, false, 0.};
   for (int c = bf16 ? CONV_RING_CFGS : 0; c < (bf16 ? CONV_CFGS : CONV_RING_CFGS); ++c) {
     const ConvRingTile f = conv_ring_cfg(mode, c);
-    if (f.bm == 0 || rows < f.bm || (cols < f.bn && mode != CONV_DOWNM)) continue;   // (of DownM columns may be missing)
+    if (f.bm == 0 || ((rows < f.bm || cols < f.bn) && !(loose && conv_may_be_loose(mode, c >= CONV_RING_CFGS)))) continue;
     const long long tiles = (rows + f.bm - 1) / f.bm * ((cols + f.bn - 1) / f.bn) * jobs;
     const int nst = (K + f.bk - 1) / f.bk;
     const int most = RING_TABLE_BYTES / conv_ring_entry(mode, single, f.bk) - (single ? RING_AHEAD : 0);
@@ -220,15 +224,15 @@ static inline ConvRingPlan conv_no_ring() { return {-1, 1, 0, false, 0., 0}; }
 // Up and Down: tiles over any run of (module | pixel, image) groups, which needs batches of whole groups of four, or of
 // one module or pixel each, which leave out taps beyond the edge and need no masks.  cfg < 0: none fits.
 template <class Args>
-static inline ConvRingPlan conv_rows_best(const Args& a, int mode, int cus, bool bf16) {
+static inline ConvRingPlan conv_rows_best(const Args& a, int mode, int cus, bool bf16, bool loose = false) {
   const bool up = mode == CONV_UP;
   if (!ring_ok(a, (long long)a.Cg * a.kk2 * (a.local ? a.M : 1)) || (!up && (a.s != 1 || a.Fg % 4 != 0)))
     return conv_no_ring();                                               // (Down: an entry is four filters of a tap)
   const int sites = up ? a.M : a.HH, cols = up ? a.Fg : a.Cg, K = a.kk2 * (up ? a.Cg : a.Fg);
   if (bf16 && K < 9) return conv_no_ring();                              // (a stage of 32 terms is mostly empty)
-  ConvRingPlan plan = conv_ring_plan(mode, true, a.N, cols, (long long)sites * a.G, K, ring_used(a, mode), false, 0., cus, bf16);
+  ConvRingPlan plan = conv_ring_plan(mode, true, a.N, cols, (long long)sites * a.G, K, ring_used(a, mode), false, 0., cus, bf16, false, loose);
   if (!a.local && a.N % 4 == 0) {
-    const ConvRingPlan flat = conv_ring_plan(mode, false, (long long)sites * a.N, cols, a.G, K, 1., false, 0., cus, bf16);
+    const ConvRingPlan flat = conv_ring_plan(mode, false, (long long)sites * a.N, cols, a.G, K, 1., false, 0., cus, bf16, false, loose);
     if (flat.cfg >= 0 && (plan.cfg < 0 || flat.us < plan.us)) plan = flat;
   }
   return plan;
@@ -264,7 +268,7 @@ static inline ConvRingPlan conv_pixels_plan(const Args& a, int blocks, int cus, 
   if (a.local || !ring_ok(a, (long long)a.Cg * a.kk2) || a.Fg < 4 || taps > RING_MAX_SIDE) return conv_no_ring();
   if (blocks < 0) {
     if (a.s != 1 || a.N % 4 != 0) return conv_no_ring();
-    ConvRingPlan plan = conv_ring_plan(CONV_DOWN, false, (long long)a.HH * a.N, a.Cg, a.G, a.kk2 * Fg4, 1., false, 0., cus, bf16);
+    ConvRingPlan plan = conv_ring_plan(CONV_DOWN, false, (long long)a.HH * a.N, a.Cg, a.G, a.kk2 * Fg4, 1., false, 0., cus, bf16, false, true);
     plan.blocks = blocks;
     return plan;
   }
@@ -278,7 +282,7 @@ static inline ConvRingPlan conv_pixels_plan(const Args& a, int blocks, int cus, 
   }
   const double one = (double)have / ((double)lines * taps);
   ConvRingPlan plan = conv_ring_plan(blocks > 0 ? CONV_DOWNM : CONV_DOWN, true, a.N, (int)cols, (long long)lines * lines * a.G, taps * taps * Fg4,
-                                     one * one, false, 0., cus, bf16, true);
+                                     one * one, false, 0., cus, bf16, true, true);
   plan.blocks = blocks;
   return plan;
 }
@@ -324,13 +328,13 @@ static inline ConvRingPlan conv_pixels_choice(const Args& a, bool maps16, bool f
 
 // Outp of `a`, whose batch the ring takes in whole groups of four images: others are copied with up to three images of zeros.
 template <class Args>
-static inline ConvRingPlan conv_outp_best(const Args& a, int cus, bool bf16) {
+static inline ConvRingPlan conv_outp_best(const Args& a, int cus, bool bf16, bool loose = false) {
   Args r = a;
   r.N = (a.N + 3) / 4 * 4;
   const int cols = a.Cg * a.kk2;
   if (!ring_ok(r, (long long)cols * a.chunks) || a.chunks > 32767) return conv_no_ring();
   ConvRingPlan plan = conv_ring_plan(CONV_OUTP, false, a.Fg, cols, (long long)a.G * a.chunks, a.m_count * r.N, 1., true,
-                                     2e-6 * a.chunks * a.F * cols, cus, bf16);
+                                     2e-6 * a.chunks * a.F * cols, cus, bf16, false, loose);
   const double maps = 1e-9 * 8. * r.N * ((double)a.M * a.F + (double)a.HH * a.C);
   // (1.12: what a layer's sums over many splits take beyond the plan's estimate)
   plan.us = 1.12 * plan.us + (r.N != a.N ? 5. + maps / 5e-3 : 0.);
@@ -346,4 +350,31 @@ static inline ConvRingPlan conv_outp_choice(const Args& a, bool maps16, bool fil
   const ConvRingPlan ring = conv_outp_plan(a, maps16, filters16, cus), split = conv_outp_best(a, cus, true);
   const double other = ring.cfg >= 0 ? ring.us : conv_other_us(a, CONV_OUTP, a.M, maps16, filters16, cus);
   return split.cfg >= 0 && split.us < other ? split : ring;
+}
+
+// What a pass runs on, where its tile may be larger than all the filters, colours or taps there are (conv_ring_plan: loose): the choice
+// of the tiles that are not, unless such a one is expected to be faster.
+template <class Args>
+static inline ConvRingPlan conv_loose_choice(const Args& a, int mode, bool maps16, bool filters16, int cus) {
+  const ConvRingPlan tight = mode == CONV_OUTP ? conv_outp_choice(a, maps16, filters16, cus) : conv_rows_choice(a, mode, maps16, filters16, cus);
+  const double other = tight.cfg >= 0 ? tight.us : conv_other_us(a, mode, mode == CONV_DOWN ? a.HH : a.M, maps16, filters16, cus);
+  ConvRingPlan best = tight;
+  double us = 0.87 * other;
+  for (int bf16 = 0; bf16 < 2; ++bf16) {
+    const ConvRingPlan plan = mode == CONV_OUTP ? conv_outp_best(a, cus, bf16 != 0, true) : conv_rows_best(a, mode, cus, bf16 != 0, true);
+    if (plan.cfg >= 0 && plan.us < us) { best = plan; us = plan.us; }
+  }
+  return best;
+}
+
+// What a pass runs on: `pixels` says that `plan` is conv_pixels_plan's.  cfg < 0: another kernel.
+struct ConvChoice { ConvRingPlan plan; bool pixels; };
+template <class Args>
+static inline ConvChoice conv_choice(const Args& a, int mode, bool maps16, bool filters16, int cus) {
+  const ConvRingPlan rows = conv_loose_choice(a, mode, maps16, filters16, cus);
+  if (mode == CONV_DOWN) {
+    const ConvRingPlan pixels = conv_pixels_choice(a, maps16, filters16, cus);
+    if (pixels.cfg >= 0 && (rows.cfg < 0 || pixels.us < rows.us)) return {pixels, true};
+  }
+  return {rows, false};
 }

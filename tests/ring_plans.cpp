@@ -45,6 +45,16 @@ void conv_tile(int mode, int N, int C, int H, int F, int k, int Mx, int s, int p
   out[4] = p.us;
 }
 
+// Whether a pass runs on a tile that is larger than all its rows or columns (of one module or pixel, where the tile lies in one).
+int conv_tile_is_loose(int mode, int N, int C, int H, int F, int k, int Mx, int s, int pad0, int G, int cus) {
+  const Sizes a = {N, C, C / G, H, H * H, F, F / G, k, k * k, Mx, Mx * Mx, s, pad0, G, 0, Mx * Mx, 1};
+  const ConvChoice c = conv_choice(a, mode, N % 4 == 0, true, cus);
+  if (c.plan.cfg < 0 || c.pixels) return 0;
+  const ConvRingTile f = conv_ring_cfg(mode, c.plan.cfg);
+  const int cols = mode == CONV_UP ? a.Fg : mode == CONV_DOWN ? a.Cg : a.Cg * a.kk2;
+  return (mode == CONV_OUTP ? a.Fg : c.plan.single ? N : 1 << 30) < f.bm || cols < f.bn;
+}
+
 // convDown of strided layers, few colours or filters that are no whole fours: out = {tile number or -1, side of a block in strides, 0 a
 // pixel or -1 any run, stages of the table, LDS bytes of a workgroup}
 void conv_pixels_tile(int N, int C, int H, int F, int k, int Mx, int s, int pad0, int G, int cus, double* out) {

@@ -899,3 +899,14 @@ def test_gradients_of_filters_too_large_for_ring_tiles(cm, cc, rng, N, C, H, F, 
     assert _relerr(T.asarray(), co.conv_down(y, w, C, H, p, s, G), co.conv_down(np.abs(y), np.abs(w), C, H, p, s, G) + 1e-6) < REL
     for m in (Y, W, T):
         m.free_device_memory()
+
+
+# tiles that are larger than all the filters, colours, images or taps there are (tests/test_ring_plans.py)
+LOOSE_LAYERS = {(100, 60, 11, 13, 7, 1, 3, 1): "up outp", (2, 3, 6, 16, 3, 1, 1, 1): "up",
+                (101, 44, 9, 11, 3, 1, 0, 1): "up outp", (35, 1, 21, 240, 3, 1, 1, 1): "up outp", (7, 5, 9, 6, 4, 2, 1, 1): "up",
+                (100, 24, 9, 14, 3, 1, 1, 2): "up outp", (251, 1, 20, 50, 3, 1, 0, 1): "up outp"}
+
+
+@pytest.mark.parametrize("N,C,H,F,k,s,p,G", list(LOOSE_LAYERS))
+def test_three_conv_passes_on_tiles_larger_than_their_layer(cm, cc, rng, N, C, H, F, k, s, p, G):
+    test_three_conv_passes(cm, cc, rng, N, C, H, F, k, s, p, G)

@@ -206,3 +206,10 @@ def test_tables_of_pixel_tiles_fit(plans):
         taken += t is not None
         assert t is None or (t[3] <= 160 << 10 and k <= 15)
     assert taken > 800
+
+
+def test_the_loose_layers_of_the_gpu_tests_are_loose(plans):
+    for layer, passes in conv.LOOSE_LAYERS.items():
+        N, C, H, F, k, s, p, G = layer
+        got = [n for n, mode in (('up', UP), ('outp', OUTP)) if plans.conv_tile_is_loose(mode, N, C, H, F, k, co.n_modules(H, k, s, p), s, -p, G, CUS)]
+        assert got == passes.split(), layer
