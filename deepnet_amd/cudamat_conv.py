@@ -13,7 +13,7 @@ import ctypes as ct
 import math
 import os
 
-from .cudamat import CUDAMatException, cudamat
+from .cudamat import CUDAMatException, _fast_calls, cudamat
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(_HERE, 'libcudamat_conv.so')
@@ -45,6 +45,7 @@ for _n, _args in _SIGNATURES.items():
     _fn = getattr(_ConvNet, _n)
     _fn.restype = None
     _fn.argtypes = _args
+_fast_calls(_ConvNet, {_n: (None, _args) for _n, _args in _SIGNATURES.items()})
 _ConvNet.conv_last_error.restype = ct.c_char_p
 _ConvNet.conv_last_error.argtypes = []
 

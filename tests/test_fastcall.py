@@ -1,0 +1,64 @@
+"""The callables of csrc/fastcall.c in the place of ctypes functions: every kind of argument arrives as ctypes hands it over, and what they
+do not take goes to ctypes (CPU only: the functions that are called are ctypes callbacks)."""
+import ctypes as ct
+
+import numpy as np
+import pytest
+
+from deepnet_amd import cudamat as cm
+from deepnet_amd import cudamat_conv as cc
+
+fastcall = pytest.importorskip('deepnet_amd._fastcall')
+KIND = {'P': ct.c_void_p, 'i': ct.c_int, 'f': ct.c_float}
+
+
+def pair(kinds):
+    """A fast callable and the ctypes function beside it, both of a callback that notes its arguments."""
+    seen = []
+    kind = kinds.lstrip('v')
+    proto = ct.CFUNCTYPE(None if kinds.startswith('v') else ct.c_int, *[KIND[k] for k in kind])
+
+    def note(*args):
+        seen.append(args)
+        return None if kinds.startswith('v') else len(seen)
+    slow = proto(note)
+    return fastcall.Function(ct.cast(slow, ct.c_void_p).value, kinds, (ct.POINTER(cm.cudamat),), slow), slow, seen
+
+
+SIGNATURES = sorted({('' if res is not None else 'v') + ''.join(dict(zip((cm._M, cm._f, cm._i, cm._u), 'Pfii'))[a] for a in args)
+                     for lib, table in ((cm._cudamat, cm._SIGNATURES), (cc._ConvNet, {n: (None, a) for n, a in cc._SIGNATURES.items()}))
+                     for name, (res, args) in table.items() if isinstance(getattr(lib, name), fastcall.Function)})
+
+
+@pytest.mark.parametrize("kinds", SIGNATURES)
+def test_arguments_arrive_in_their_places(kinds):
+    fast, slow, seen = pair(kinds)
+    mats = [cm.cudamat() for _ in kinds]
+    value = dict(P=lambda j: ct.pointer(mats[j]), i=lambda j: -7 * j - 3, f=lambda j: 0.1 * j + 1e-3)
+    args = [value[k](j) for j, k in enumerate(kinds.lstrip('v'))]
+    assert fast(*args) in (0, 1)
+    slow(*args)
+    assert seen[0] == seen[1] and len(seen[0]) == len(args)
+
+
+def test_other_arguments_go_to_ctypes():
+    fast, slow, seen = pair('PPif')
+    mat = cm.cudamat()
+    p = ct.pointer(mat)
+    for args in ((None, p, 3, 1.5), (ct.byref(mat), p, 3, 1.5), (p, ct.addressof(mat), 3, 2), (p, p, np.int64(4), np.float64(0.5)),
+                 (p, p, True, 1.0), (p, p, 2 ** 32 + 5, 1.0), (ct.pointer(cm.rnd_struct()), p, ct.c_int(3), ct.c_float(1.5))):
+        del seen[:]
+        outcome = []
+        for f in (fast, slow):
+            try:
+                f(*args)
+                outcome.append(None)
+            except (TypeError, ct.ArgumentError) as e:
+                outcome.append(type(e))
+        assert outcome[0] == outcome[1] and len(seen) in (0, 2) and seen[:1] == seen[1:], args
+    for bad in ((p, p, 3), (p, p, 'x', 1.0), (p, 2.5, 3, 1.0)):
+        with pytest.raises((TypeError, ct.ArgumentError)):
+            fast(*bad)
+    assert fast.argtypes == slow.argtypes and cm._cudamat.dot.argtypes == cm._SIGNATURES['dot'][1]
+    with pytest.raises(KeyError):
+        fastcall.Function(1, 'ffff', (), slow)
