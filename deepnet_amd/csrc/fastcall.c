@@ -2,7 +2,7 @@
  * call (1.0 us a call against 0.27; a step of a 784-1024-1024-10 classifier makes 66).  Function(address, kinds, types, slow) is called
  * like the ctypes function `slow`, whose kinds of arguments are given as text: P a pointer object of one of `types` or None, i a whole
  * number, f a float; other arguments, and signatures that are not in the table below, go to `slow`.  The interpreter's lock is
- * released during the call, as by ctypes.  kinds starting with v: a function without a result. */
+ * released during the call, as by ctypes.  kinds starting with v: a function without a result, which is None here too. */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <stddef.h>
@@ -58,7 +58,7 @@ typedef struct {
   void* fn;
   Call call;
   const char* kinds;
-  int n;
+  int n, is_void;
   PyTypeObject* types[MAX_TYPES];
   PyObject* slow;
 } Function;
@@ -96,6 +96,7 @@ static PyObject* function_call(PyObject* callable, PyObject* const* args, size_t
     Py_BEGIN_ALLOW_THREADS
     res = self->call(self->fn, a);
     Py_END_ALLOW_THREADS
+    if (self->is_void) Py_RETURN_NONE;
     return PyLong_FromLong(res);
   }
 slow:
@@ -116,7 +117,8 @@ static PyObject* function_new(PyTypeObject* type, PyObject* args, PyObject* kw) 
   self->vectorcall = function_call;
   self->fn = (void*)(uintptr_t)address;
   self->call = g_calls[s];
-  self->kinds = g_kinds[s] + (kinds[0] == 'v');
+  self->is_void = kinds[0] == 'v';
+  self->kinds = g_kinds[s] + self->is_void;
   self->n = (int)strlen(self->kinds);
   for (Py_ssize_t t = 0; t < PyTuple_GET_SIZE(types) && t < MAX_TYPES; ++t) {
     PyObject* o = PyTuple_GET_ITEM(types, t);
