@@ -2689,10 +2689,10 @@ static bool conv_pixels_ring(const ConvArgs& a, const ConvRingPlan& plan, const 
 }
 
 // The choice for a layer (it depends on its sizes and alignment only), kept for the next call: it prices some hundred plans, which is
-// several microseconds of the host's, as long as the shortest passes take.
+// several microseconds of the host's, as long as the shortest passes take.  One table a thread: ctypes gives up the interpreter's lock.
 static const ConvChoice& conv_chosen(const ConvArgs& a, int mode) {
   struct Entry { int key[14]; bool used; ConvChoice choice; };
-  static Entry cache[128];
+  static thread_local Entry cache[128];
   const int key[14] = {mode, a.N, a.C, a.H, a.F, a.k, a.Mx, a.s, a.pad0, a.G, a.local, a.m_count, a.chunks,
                        (ring_maps16(a) ? 2 : 0) + (dn_aligned16(a.flt) ? 1 : 0)};
   unsigned h = 0;
