@@ -5,14 +5,22 @@ import ctypes as ct
 import numpy as np
 import pytest
 
-from deepnet_amd import cudamat as cm
-from deepnet_amd import cudamat_conv as cc
-
-fastcall = pytest.importorskip('deepnet_amd._fastcall')
 KIND = {'P': ct.c_void_p, 'i': ct.c_int, 'f': ct.c_float}
 
 
-def pair(kinds):
+# (imported by the tests: a process that loads these libraries before torch, which other files import, has two HIP runtimes)
+@pytest.fixture
+def cm():
+    from deepnet_amd import cudamat
+    return cudamat
+
+
+@pytest.fixture
+def fastcall():
+    return pytest.importorskip('deepnet_amd._fastcall')
+
+
+def pair(cm, fastcall, kinds):
     """A fast callable and the ctypes function beside it, both of a callback that notes its arguments."""
     seen = []
     kind = kinds.lstrip('v')
@@ -25,24 +33,25 @@ def pair(kinds):
     return fastcall.Function(ct.cast(slow, ct.c_void_p).value, kinds, (ct.POINTER(cm.cudamat),), slow), slow, seen
 
 
-SIGNATURES = sorted({('' if res is not None else 'v') + ''.join(dict(zip((cm._M, cm._f, cm._i, cm._u), 'Pfii'))[a] for a in args)
-                     for lib, table in ((cm._cudamat, cm._SIGNATURES), (cc._ConvNet, {n: (None, a) for n, a in cc._SIGNATURES.items()}))
-                     for name, (res, args) in table.items() if isinstance(getattr(lib, name), fastcall.Function)})
+def test_arguments_arrive_in_their_places(cm, fastcall):
+    from deepnet_amd import cudamat_conv as cc
+    letters = {cm._M: 'P', cm._f: 'f', cm._i: 'i', cm._u: 'i'}
+    tables = ((cm._cudamat, cm._SIGNATURES), (cc._ConvNet, {n: (None, a) for n, a in cc._SIGNATURES.items()}))
+    signatures = {('' if res is not None else 'v') + ''.join(letters[a] for a in args) for lib, table in tables
+                  for name, (res, args) in table.items() if isinstance(getattr(lib, name), fastcall.Function)}
+    assert len(signatures) > 10
+    for kinds in sorted(signatures):
+        fast, slow, seen = pair(cm, fastcall, kinds)
+        mats = [cm.cudamat() for _ in kinds]
+        value = dict(P=lambda j: ct.pointer(mats[j]), i=lambda j: -7 * j - 3, f=lambda j: 0.1 * j + 1e-3)
+        args = [value[k](j) for j, k in enumerate(kinds.lstrip('v'))]
+        first, second = fast(*args), slow(*args)
+        assert (first, second) == ((None, None) if kinds.startswith('v') else (1, 2)), kinds
+        assert seen[0] == seen[1] and len(seen[0]) == len(args), kinds
 
 
-@pytest.mark.parametrize("kinds", SIGNATURES)
-def test_arguments_arrive_in_their_places(kinds):
-    fast, slow, seen = pair(kinds)
-    mats = [cm.cudamat() for _ in kinds]
-    value = dict(P=lambda j: ct.pointer(mats[j]), i=lambda j: -7 * j - 3, f=lambda j: 0.1 * j + 1e-3)
-    args = [value[k](j) for j, k in enumerate(kinds.lstrip('v'))]
-    first, second = fast(*args), slow(*args)
-    assert (first, second) == ((None, None) if kinds.startswith('v') else (1, 2))
-    assert seen[0] == seen[1] and len(seen[0]) == len(args)
-
-
-def test_other_arguments_go_to_ctypes():
-    fast, slow, seen = pair('PPif')
+def test_other_arguments_go_to_ctypes(cm, fastcall):
+    fast, slow, seen = pair(cm, fastcall, 'PPif')
     mat = cm.cudamat()
     p = ct.pointer(mat)
     for args in ((None, p, 3, 1.5), (ct.byref(mat), p, 3, 1.5), (p, ct.addressof(mat), 3, 2), (p, p, np.int64(4), np.float64(0.5)),
