@@ -2683,6 +2683,7 @@ static bool conv_pixels_ring(const ConvArgs& a, const ConvRingPlan& plan, const 
   p.K = (flat ? a.kk2 : taps * taps) * p.Fg4();
   p.ldc = (long long)a.N * a.HH;
   if (plan.blocks > 0) conv_ring_launch<CONV_DOWNM, true>(plan, p);
+  else if (flat && a.Fg % 4 != 0) conv_ring_launch<CONV_DOWNO, false>(plan, p);
   else if (flat) conv_ring_launch<CONV_DOWN, false>(plan, p);
   else conv_ring_launch<CONV_DOWNS, true>(plan, p);
   return ring_done(where);

@@ -124,8 +124,9 @@ struct ConvRingOperand : Tile {
   }
 };
 
-// An output of Down by itself, (y, x) counted from the padding's edge: where a module that is not finite reaches a block but not
-// this pixel, whose tap in the product is a zero.
+// An output of Down by itself, (y, x) counted from the padding's edge, where the product has terms that this sum has not, with a
+// zero for one factor: modules that reach a block but not this pixel (DownM), filters that a tap's last entry repeats (DownM, DownO).
+// Where the other factor is not finite, neither is the product's output, whatever this sum is.
 __device__ __forceinline__ float conv_down_one(const ConvRingArgs& p, int g, int c, int y, int x, int n) {
   float acc = 0.f;
   const int top = (int)fd_div((uint32_t)y, p.ds), right = (int)fd_div((uint32_t)x, p.ds);
@@ -201,7 +202,7 @@ template <int MODE, bool SINGLE, class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRingArgs p) {
   constexpr int PER = MODE == CONV_UP ? 1 : 4, BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, THREADS = Cfg::THREADS;
   using OA = ConvRingOperand<MODE == CONV_OUTP ? 3 : MODE == CONV_DOWNM ? 9 : SINGLE ? 5 : 0, typename Cfg::template Tile<BM, MODE == CONV_OUTP>, PER>;
-  using OB = ConvRingOperand<MODE == CONV_UP ? (SINGLE ? 6 : 1) : MODE == CONV_DOWN ? (SINGLE ? 7 : 2) : MODE == CONV_DOWNS ? 7 : MODE == CONV_DOWNM ? 8 : 4,
+  using OB = ConvRingOperand<MODE == CONV_UP ? (SINGLE ? 6 : 1) : MODE == CONV_OUTP ? 4 : MODE == CONV_DOWNM ? 8 : SINGLE ? 7 : 2,
                              typename Cfg::template Tile<BN, MODE != CONV_UP>, PER>;
   using Shape = typename Cfg::template Shape<OA, OB>;
   constexpr int EPL = Shape::EPL, LDS = Cfg::SPLIT ? Shape::LDS : 4 * Shape::LDS;
@@ -341,12 +342,13 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
     for (int u = 0; u < OB::NG; ++u)
       ob.off[u] = 4u * (unsigned)(OB::group_k(tid, u) * p.F + g * p.Fg + n0 + OB::group_row(tid, u));
     out += (long long)g * p.Fg * p.ldc;
-  } else if constexpr (MODE == CONV_DOWN) {
-    const int K = p.kk2 * p.Fg4();
+  } else if constexpr (MODE == CONV_DOWN || MODE == CONV_DOWNO) {
+    constexpr bool ODD = MODE == CONV_DOWNO;
+    const int Fg4 = ODD ? p.Fg4() : p.Fg, K = p.kk2 * Fg4;
     nst = (K + BK - 1) / BK;
     unsigned* tab1 = reinterpret_cast<unsigned*>(table + nst * (BK / 4));
     for (int e = tid; e < nst * (BK / 4); e += THREADS) {
-      const int tap = div(4 * e, p.dFg4), f0 = 4 * e - tap * p.Fg4(), f = f0 + 4 > p.Fg ? p.Fg - 4 : f0, ky = div(tap, p.dk), kx = tap - ky * k;
+      const int tap = div(4 * e, p.dFg4), f0 = 4 * e - tap * Fg4, f = ODD && f0 + 4 > p.Fg ? p.Fg - 4 : f0, ky = div(tap, p.dk), kx = tap - ky * k;
       const bool in = 4 * e < K;
       table[e] = make_uint2(4u * (unsigned)N * (unsigned)(p.M * f - ky * Mx - kx),
                             in ? 1u << ky | 1u << (RING_MAX_SIDE + kx) | (f < f0 ? RING_LAST : 0u) : RING_FAR);
@@ -357,8 +359,8 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
 #pragma unroll
     for (int u = 0; u < OA::NG; ++u) {
       oa.off[u] = 4u * (unsigned)(n + N * (y * Mx + x + p.M * (g * p.Fg + OA::group_k(tid, u) % 4)));
-      oa.mask[u] = ring_bits(y - Mx + 1, y + 1 < k ? y + 1 : k) | ring_bits(x - Mx + 1, x + 1 < k ? x + 1 : k) << RING_MAX_SIDE |
-                   (OA::group_k(tid, u) % 4 < p.Fg4() - p.Fg ? 0u : RING_LAST);
+      oa.mask[u] = ring_bits(y - Mx + 1, y + 1 < k ? y + 1 : k) | ring_bits(x - Mx + 1, x + 1 < k ? x + 1 : k) << RING_MAX_SIDE;
+      if (ODD && OA::group_k(tid, u) % 4 >= Fg4 - p.Fg) oa.mask[u] |= RING_LAST;
     }
     oa.tab = table;
     ob.tab1 = tab1;
@@ -398,19 +400,25 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
 
   // output (em, en) of the tile: at column en, or (DownM) at the pixel that it stands for, which may lie outside the map
   const unsigned ms = (unsigned)((m0 + BM < p.rows ? m0 + BM : p.rows) - m_lo), ns = (unsigned)((n0 + BN < p.cols ? n0 + BN : p.cols) - n_lo);
-  auto store = [&](int em, int en, float v) __attribute__((always_inline)) {
-    if (LOOSE ? (unsigned)(em - m_lo) >= ms || (unsigned)(en - n_lo) >= ns : em < m_lo || en < n_lo) return;
+  auto place = [&](int em, int en, long long* at) __attribute__((always_inline)) {
+    if (LOOSE ? (unsigned)(em - m_lo) >= ms || (unsigned)(en - n_lo) >= ns : em < m_lo || en < n_lo) return false;
     if constexpr (MODE == CONV_DOWNM) {
-      const int line = div(per, p.dlines), at = per - line * p.lines;
+      const int line = div(per, p.dlines), col = per - line * p.lines;
       const int c = div(en, p.dblock2), q = en - c * p.block * p.block, py = div(q, p.dblock), px = q - py * p.block;
-      const int y = line * p.block + py + p.pad0, x = at * p.block + px + p.pad0;
-      if ((unsigned)y < (unsigned)H && (unsigned)x < (unsigned)H) {
-        if (!(__builtin_fabsf(v) < __builtin_inff())) v = conv_down_one(p, g, c, y - p.pad0, x - p.pad0, em);
-        out[(long long)(c * p.HH + y * H + x) * N + em] = v;
-      }
-    } else {
-      out[(long long)en * p.ldc + em] = v;
+      const int y = line * p.block + py + p.pad0, x = col * p.block + px + p.pad0;
+      *at = (long long)(c * p.HH + y * H + x) * N + em;
+      return (unsigned)y < (unsigned)H && (unsigned)x < (unsigned)H;
     }
+    *at = (long long)en * p.ldc + em;
+    return true;
+  };
+  constexpr bool AGAIN = MODE == CONV_DOWNM || MODE == CONV_DOWNO;        // see conv_down_one
+  bool again = false;
+  auto store = [&](int em, int en, float v) __attribute__((always_inline)) {
+    long long at;
+    if (!place(em, en, &at)) return;
+    if (AGAIN) again |= !(__builtin_fabsf(v) < __builtin_inff());
+    out[at] = v;
   };
   if constexpr (Cfg::SPLIT) {
     Shape::template run<false>(lds, oa, ob, nst, 0, [] {});
@@ -425,6 +433,17 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
     const int em = m0 + tid % BM, en0 = n0 + tid / BM;
 #pragma unroll
     for (int u = 0; u < EPL; ++u) store(em, en0 + u * (THREADS / BM), sum[u]);
+  }
+  if (AGAIN && again) {
+#pragma unroll 1
+    for (int u = 0; u < EPL; ++u) {
+      const int e = tid + THREADS * u, em = m0 + e % BM;
+      long long at;
+      if (!place(em, n0 + e / BM, &at) || __builtin_fabsf(out[at]) < __builtin_inff()) continue;
+      // [colour][pixel][image], of a group's first colour on (ring_ok: 31 bits)
+      const int row = (int)at / N, c = row / p.HH, pix = row - c * p.HH, y = pix / H, x = pix - y * H;
+      out[at] = conv_down_one(p, g, c, y - p.pad0, x - p.pad0, (int)at - row * N);
+    }
   }
 }
 

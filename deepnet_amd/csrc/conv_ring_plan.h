@@ -5,7 +5,8 @@
 // CONV_DOWNM: convDown of few colours, the pixels of a block (of the stride's side, on ring tiles of a multiple of it)
 // merged into the columns of one product (uniform-row kernels and ring tiles of one block each).
 // CONV_DOWNS: convDown of any stride on ring tiles of one pixel (CONV_DOWN there: of stride 1).
-enum { CONV_UP = 0, CONV_DOWN = 1, CONV_OUTP = 2, CONV_DOWNM = 3, CONV_DOWNS = 4 };
+// CONV_DOWNO: convDown of filters that are no whole fours, on ring tiles over any run of pixels.
+enum { CONV_UP = 0, CONV_DOWN = 1, CONV_OUTP = 2, CONV_DOWNM = 3, CONV_DOWNS = 4, CONV_DOWNO = 5 };
 
 #define RING_MAX_SIDE 15   // filter rows and columns that a mask has room for
 #define RING_AHEAD 7       // stages that the table of a tile of one module or pixel reaches beyond its last one
@@ -78,7 +79,7 @@ static inline int conv_tile_lds(int mode, int c) {
 struct ConvRingPlan { int cfg, splits, split_stages; bool single; double us; int blocks; };   // blocks: conv_pixels_plan's
 
 static inline int conv_ring_entry(int mode, bool single, int bk) {      // table bytes per stage
-  return mode == CONV_UP ? 8 * bk : mode == CONV_DOWNM || (mode == CONV_DOWN && !single) ? 3 * bk : 2 * bk;
+  return mode == CONV_UP ? 8 * bk : mode == CONV_DOWNM || mode == CONV_DOWNO || (mode == CONV_DOWN && !single) ? 3 * bk : 2 * bk;
 }
 static inline int conv_ring_table(int mode, bool single, int bk, int stages) {      // table bytes of a workgroup
   return ((stages < 1 ? 1 : stages) + (single ? RING_AHEAD : 0)) * conv_ring_entry(mode, single, bk);

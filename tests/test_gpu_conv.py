@@ -883,6 +883,26 @@ def test_gradients_on_tiles_of_pixels(cm, cc, rng, N, C, H, F, k, s, p, G, finit
     assert np.max(np.abs(got[ok] - want[ok]) / (bound[ok] + 1e-6)) < REL
 
 
+# (the last entry of a tap repeats filters, whose weights are then multiplied by zeros)
+@pytest.mark.parametrize("N,C,H,F,k,s,p,G", [layer for layer in PIXEL_LAYERS if layer[3] // layer[7] % 4])
+def test_gradients_through_infinite_weights_of_odd_filter_counts(cm, cc, rng, N, C, H, F, k, s, p, G):
+    """One infinite weight of a group's last filters per colour: the pixels that it reaches are infinite, of the gradient's sign, and no others."""
+    Mx, Fg, Cg = co.n_modules(H, k, s, p), F // G, C // G
+    y, w = _f(rng.standard_normal((N, F * Mx * Mx))), _f(0.1 * rng.standard_normal((F, Cg * k * k)))
+    for c in range(0, Cg, 2 if Cg > 1 else 1):
+        w[c % G * Fg + Fg - 1 - c // 2 % min(Fg, 5), c * k * k + 7 * c % (k * k)] = np.inf if c % 4 else -np.inf
+    Y, W, T = cm.CUDAMatrix(y), cm.CUDAMatrix(w), cm.CUDAMatrix(np.full((N, C * H * H), 7.0, dtype=np.float32))
+    cc.convDown(Y, W, T, Mx, p, s, k, H, C, numGroups=G)
+    got = T.asarray()
+    for m in (Y, W, T):
+        m.free_device_memory()
+    want = co.conv_down(y, w, C, H, p, s, G)
+    ok = np.isfinite(want)
+    assert np.isinf(want).any() and not np.isnan(want).any() and np.array_equal(np.where(ok, 0, got), np.where(ok, 0, want))
+    bound = co.conv_down(np.abs(y), np.abs(np.where(np.isfinite(w), w, 0)), C, H, p, s, G)
+    assert np.max(np.abs(got[ok] - want[ok]) / (bound[ok] + 1e-6), initial=0.) < REL
+
+
 # the same layers on the kernels beside ring tiles, which filters of 16 x 16 are too large for: phases merged into 16 to 128 columns, the
 # patch matrix, uniform rows and 128- and 256-row tiles
 SIXTEEN = [(128, c, 18, 16, 16, 4, 0, 1) for c in (1, 2, 3, 4, 6, 8)] + [(32, 3, 18, 16, 16, 2, 0, 1), (17, 2, 17, 5, 16, 1, 0, 1)] + \
