@@ -473,7 +473,7 @@ static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
     case 7: if constexpr (MODE == CONV_OUTP) CONV_RING(ConvSplitCfg<96, 128, 32, 2, 4, 1, 2, 2>); else CONV_RING(ConvSplitCfg<128, 96, 32, 4, 2, 1, 2, 2>); break;
     case 8: if constexpr (MODE == CONV_OUTP) CONV_RING(ConvSplitCfg<64, 128, 32, 2, 4, 1, 2, 2>); else CONV_RING(ConvSplitCfg<128, 64, 32, 4, 2, 1, 2, 2>); break;
     case 9: CONV_RING(ConvSplitCfg<64, 64, 32, 2, 2, 1, 2, 3>); break;
-    default: if constexpr (MODE == CONV_DOWN || MODE == CONV_DOWNS || MODE == CONV_DOWNM) CONV_RING(ConvSplitCfg<128, 48, 64, 4, 1, 2, 2, 2>); break;
+    default: if constexpr (conv_ring_cfg(MODE, 10).bm != 0) CONV_RING(ConvSplitCfg<128, 48, 64, 4, 1, 2, 2, 2>); break;
   }
 #undef CONV_RING
 }

@@ -40,13 +40,13 @@ static inline int padded_filters(int F, int numGroups) {
 struct ConvRingTile { int bm, bn, bk; double stage, tile; };
 #define CONV_RING_CFGS 6                 // the fp32 tiles
 #define CONV_CFGS 11
-static const ConvRingTile g_conv_ring_cfgs[CONV_CFGS] = {
+static constexpr ConvRingTile g_conv_ring_cfgs[CONV_CFGS] = {
     {64, 64, 32, 0.545, 1.45}, {64, 32, 64, 0.574, 1.46}, {32, 64, 64, 0.58, 1.45},
     {32, 32, 64, 0.322, 1.0}, {32, 16, 128, 0.372, 1.2}, {16, 32, 128, 0.372, 1.17},
     // on the bf16 matrix cores (split_tile.h), fitted to 280 passes (of 1161 others they miss by 5 to 8 % rms, tile by tile)
     {128, 128, 32, 1.12, 5.}, {128, 96, 32, 1.08, 4.5}, {128, 64, 32, 0.8, 3.5}, {64, 64, 32, 0.53, 1.}, {128, 48, 64, 1.2, 4.}};
 // (of Outp the rows are the filters, and there is no tile of 48)
-static inline ConvRingTile conv_ring_cfg(int mode, int c) {
+static constexpr ConvRingTile conv_ring_cfg(int mode, int c) {
   ConvRingTile f = g_conv_ring_cfgs[c];
   if (mode == CONV_OUTP && (c == 7 || c == 8)) { f.bm = f.bn; f.bn = 128; }
   if (c == 10 && (mode == CONV_UP || mode == CONV_OUTP)) f.bm = 0;

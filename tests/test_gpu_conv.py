@@ -855,7 +855,7 @@ PIXEL_LAYERS = [  # N, C, H, F, k, stride, padding, groups
     (100, 68, 7, 25, 5, 1, 0, 1), (240, 16, 7, 17, 7, 1, 3, 1), (64, 56, 14, 65, 5, 1, 0, 1), (128, 24, 14, 93, 5, 1, 2, 1),
     (144, 44, 16, 34, 3, 2, 1, 2), (151, 40, 14, 80, 5, 2, 2, 1), (128, 3, 58, 96, 11, 4, 0, 1), (100, 96, 14, 5, 3, 1, 0, 1),
     (256, 32, 18, 5, 5, 2, 2, 1), (100, 96, 7, 16, 3, 3, 0, 1), (47, 16, 17, 5, 3, 2, 1, 1), (200, 96, 10, 32, 4, 4, 2, 1), (256, 48, 9, 16, 4, 4, 2, 1),
-    (100, 60, 9, 26, 3, 1, 1, 2), (64, 56, 7, 5, 3, 1, 0, 1)]
+    (100, 60, 9, 26, 3, 1, 1, 2), (64, 56, 7, 5, 3, 1, 0, 1), (100, 48, 14, 9, 6, 1, 3, 1)]
 
 
 @pytest.mark.parametrize("finite", [True, False])

@@ -189,6 +189,8 @@ def test_gradients_of_the_gpu_tests_reach_every_kind_of_pixel_tile(plans):
     got = [pixels_tile(plans, *layer) for layer in conv.PIXEL_LAYERS]
     assert None not in got and {t[1] for t in got} == {-1, 0, 1, 2, 4}
     assert {t[0] >= 6 for t in got if t[1] == -1} == {t[0] >= 6 for t in got if t[1] > 0} == {False, True}
+    odd = {t[0] for layer, t in zip(conv.PIXEL_LAYERS, got) if t[1] == -1 and layer[3] // layer[7] % 4}
+    assert {0, 1, 3, 4, 7, 10} <= odd                    # (an instance of its own)
     for tile, blocks, stages, lds in got:
         assert lds <= 160 << 10 and stages >= 1
     assert [layer for layer in conv.PIXEL_LAYERS if conv_tile(plans, DOWN, *layer)] == []
