@@ -262,7 +262,7 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
     int ky0, kx0, my0 = 0, mx0 = 0;
     int ny = range(y, &ky0, &my0), nx = range(x, &kx0, &mx0);
     if (ny <= 0 || nx <= 0) { ny = 0; nx = 1; }
-    const int area = ny * nx, K = area * (UP ? p.Cg : p.Fg4());
+    const int Fg4 = MERGED ? p.Fg4() : p.Fg, area = ny * nx, K = area * (UP ? p.Cg : Fg4);
     nst = K > BK ? (K + BK - 1) / BK : 1;
     unsigned* tab1 = reinterpret_cast<unsigned*>(table + (nst + RING_AHEAD) * (BK / PER));
     // exact for dividends below 2^12 and divisors up to RING_MAX_SIDE^2
@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
           t2.y = 4u * Fu * (unsigned)((bank * p.Cg + c) * p.kk2 + ky * k + kx);
         } else {
           const int ky = ky0 + s * ty, kx = kx0 + s * tx, m = ONE ? (y - ky) * Mx + x - kx : (my0 - ty) * Mx + mx0 - tx;
-          int f = 4 * e - tap * p.Fg4();
+          int f = 4 * e - tap * Fg4;
           if (MERGED && f + 4 > p.Fg) { f = p.Fg - 4; need = RING_LAST; }
           t2.x = 4u * Nu * (unsigned)(p.M * (g * p.Fg + f) + m);
           t2.y = 4u * ((unsigned)f + Fu * (unsigned)(ky * k + kx + p.Cg * p.kk2 * (p.local ? m : 0)));
@@ -297,7 +297,7 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
 #pragma unroll
     for (int u = 0; u < OA::NG; ++u) {
       oa.off[u] = 4u * (unsigned)(n + (PER == 4 ? N * p.M * (OA::group_k(tid, u) % 4) : 0));
-      if (MERGED) oa.mask[u] = OA::group_k(tid, u) % 4 < p.Fg4() - p.Fg ? RING_LAST : 0u;
+      if (MERGED) oa.mask[u] = OA::group_k(tid, u) % 4 < Fg4 - p.Fg ? RING_LAST : 0u;
     }
 #pragma unroll
     for (int u = 0; u < OB::NG; ++u) {

@@ -223,6 +223,12 @@ struct SplitShape {
     multiply(f1, f1, acc.small);                  \
   } while (0)
     int s = 0;
+    // The code ahead of it decides where the loop falls in the 32 bytes that a fetch of instructions takes, and on 128 x 48 tiles that
+    // is up to 3 % of the time: convDown of 96 -> 256 colours 5 x 5, 2 groups, 27 x 27, batch 128 takes 399 us with the loop's head 8 bytes
+    // behind a multiple of 32, 402 with 16 or 20, 407 to 411 elsewhere; 84 -> 256 of 9 x 9, stride 2, 15 x 15, 128 233 and 239.  So the
+    // place is fixed, 8 bytes in front of the head (4 more where offsets have masks, which make no difference there).  Other tiles
+    // differ by 0.5 %.
+    if (BN == 48 && U + 1 < nst) asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0");
     for (; s + U + 1 < nst; s += U) {
 #pragma unroll
       for (int q = 0; q < U; ++q) {
