@@ -55,6 +55,15 @@ int conv_tile_is_loose(int mode, int N, int C, int H, int F, int k, int Mx, int 
   return (mode == CONV_OUTP ? a.Fg : c.plan.single ? N : 1 << 30) < f.bm || cols < f.bn;
 }
 
+// What a pass runs on: out = {tile number or -1, one module or pixel per tile, from conv_pixels_plan, us, us on the other kernels, how much
+// longer the busiest XCD takes}
+void conv_route(int mode, int N, int C, int H, int F, int k, int Mx, int s, int pad0, int G, int cus, double* out) {
+  const Sizes a = {N, C, C / G, H, H * H, F, F / G, k, k * k, Mx, Mx * Mx, s, pad0, G, 0, Mx * Mx, 1};
+  const ConvChoice c = conv_choice(a, mode, N % 4 == 0, true, cus);
+  out[0] = c.plan.cfg; out[1] = c.plan.single; out[2] = c.pixels; out[3] = c.plan.us;
+  out[4] = conv_other_us(a, mode, mode == CONV_DOWN ? a.HH : a.M, N % 4 == 0, true, cus); out[5] = ring_crowd(a);
+}
+
 // convDown of strided layers, few colours or filters that are no whole fours: out = {tile number or -1, side of a block in strides, 0 a
 // pixel or -1 any run, stages of the table, LDS bytes of a workgroup}
 void conv_pixels_tile(int N, int C, int H, int F, int k, int Mx, int s, int pad0, int G, int cus, double* out) {

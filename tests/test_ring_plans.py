@@ -215,3 +215,31 @@ def test_the_loose_layers_of_the_gpu_tests_are_loose(plans):
         N, C, H, F, k, s, p, G = layer
         got = [n for n, mode in (('up', UP), ('outp', OUTP)) if plans.conv_tile_is_loose(mode, N, C, H, F, k, co.n_modules(H, k, s, p), s, -p, G, CUS)]
         assert got == passes.split(), layer
+
+
+def test_the_busiest_xcd_counts_for_every_tile_of_few_colours(plans):
+    """convDown of at most 16 colours on tiles of one pixel is expected to be faster than the patch form on the busiest XCD too, also where
+    the tile is larger than the layer; among random layers are some that only that refuses."""
+    import random
+    rng, taken, refused, out = random.Random(6), 0, 0, (ct.c_double * 6)()
+    for _ in range(4000):
+        N, C, k, F = rng.randint(16, 260), rng.randint(4, 16), rng.randint(1, 11), 4 * rng.randint(2, 64)
+        H, p = rng.randint(k, 40), rng.choice([0, k // 2])
+        plans.conv_route(DOWN, N, C, H, F, k, co.n_modules(H, k, 1, p), 1, -p, 1, CUS, out)
+        tile, single, pixels, us, other, crowd = out
+        if tile >= 0 and single and not pixels:
+            assert us * crowd <= other + 6 * (crowd - 1)
+            taken += 1
+        refused += tile < 0 and crowd > 1.2
+    assert taken > 200 and refused > 50
+
+
+# convDown, us: on the other kernels / on the tiles that coarser estimates took it to
+SLOWER_ON_TILES = [(173, 13, 15, 244, 7, 1, 0, 1), (205, 8, 12, 236, 5, 1, 0, 1), (146, 13, 20, 220, 6, 1, 0, 1)]       # 86 / 142, 46 / 70, 132 / 172
+
+
+def test_layers_that_tiles_made_slower_are_on_the_other_kernels(plans):
+    out = (ct.c_double * 6)()
+    for N, C, H, F, k, s, p, G in SLOWER_ON_TILES:
+        plans.conv_route(DOWN, N, C, H, F, k, co.n_modules(H, k, s, p), s, -p, G, CUS, out)
+        assert out[0] < 0, (N, C, H, F, k, s, p, G)
