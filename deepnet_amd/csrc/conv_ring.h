@@ -162,8 +162,8 @@ __device__ __forceinline__ float conv_down_one(const ConvRingArgs& p, int g, int
 //   24 -> 93 of 7 x 7, 31 x 31, 151 (whole fours of filters)    645 -> 339
 // Filters, colours, images or taps that are fewer than any tile has (13 filters, 9 taps) run on tiles larger than them as well: 60 ->
 // 13 colours 7 x 7, 11 x 11, 100 61 -> 23 us Up, 54 -> 21 Outp (before: a copy to 16 filters, or one lane per output).
-// Of 210 random layers that they take, one was 4 % slower than before, none by more; half are twice as fast.  (3 -> 96 of 11 x 11,
-// stride 4, 224 x 224, 128, as fast either way, stays on phases of 128 images.)
+// Of the random layers that these tiles take about one in forty is more than 4 % slower than before (see conv_pixels_choice); half are
+// nearly twice as fast.  (3 -> 96 of 11 x 11, stride 4, 224 x 224, 128, as fast either way, stays on phases of 128 images.)
 // Measured, us Up / Down / Outp, operands from memory, before -> now (with the copies and sums):
 //   64 -> 64 colours 5 x 5, 13 x 13, batch 100      70 / 62 / 65 -> 46 / 45 / 39      (22 each at 157 TFLOP/s)
 //   64 -> 64 colours 3 x 3, 17 x 17, batch 100      69 / 57 / 55 -> 27 / 27 / 32      (14)

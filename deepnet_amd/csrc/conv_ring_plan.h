@@ -262,6 +262,10 @@ static inline ConvRingPlan conv_rows_choice(const Args& a, int mode, bool maps16
   return split.cfg >= 0 && split.us < other ? split : ring;
 }
 
+// Strided layers of many colours, whose Down is a product for each of the stride^2 phases of pixels on the other kernels.
+template <class Args>
+static inline bool conv_phases(const Args& a) { return a.s > 1 && a.Cg > 16; }
+
 // Down of strided layers, of few colours, or of filters that are no multiple of four: on tiles of one pixel (blocks = 0), or
 // (DownM) of one block of `blocks` x `blocks` strides of pixels, whose pixels are columns beside the colours: a tile's terms are
 // the modules that reach it, of which a pixel of a block has a tap with some only.  blocks < 0: on tiles over any run of (pixel,
@@ -288,6 +292,7 @@ static inline ConvRingPlan conv_pixels_plan(const Args& a, int blocks, int cus, 
   const double one = (double)have / ((double)lines * taps);
   ConvRingPlan plan = conv_ring_plan(blocks > 0 ? CONV_DOWNM : CONV_DOWN, true, a.N, (int)cols, (long long)lines * lines * a.G, taps * taps * Fg4,
                                      one * one, false, 0., cus, bf16, true, true);
+  if (blocks > 0 && conv_phases(a)) plan.us = 3. + 1.2 * (plan.us - 3.);
   plan.blocks = blocks;
   return plan;
 }
@@ -302,9 +307,13 @@ static inline double conv_pixels_other_us(const Args& a, bool maps16, bool filte
   if (Np % 16 != 0 || Fg % 16 != 0 || !((Np != a.N || maps16) && filters16)) return any;      // (one lane per output)
   const double maps = 1e-9 * 8. * Np * ((double)a.M * a.F + (double)a.HH * a.C), hid = 1e-9 * 8. * Np * a.M * Fp;   // GB of a copy
   const double copies = (Np != a.N ? 5. + maps / 5e-3 : 0.) + (Fp != a.F ? 5. + hid / 5e-3 : 0.);
-  if (a.Cg > 16) {   // a pixel has every s-th tap of a row and column
-    const double flops = 2e-9 * Np * a.HH * ((a.Cg + 31) / 32 * 32) * a.G * a.kk2 * Fg / (a.s * a.s);
-    return 9. + flops / 85. * 1e3 + copies;
+  if (conv_phases(a)) {   // a pixel has every s-th tap of a row and column
+    // (uniform rows: as in conv_other_us; fewer tiles than CUs: as long as one tile takes, 24 ns a term and 32 columns)
+    const bool uniform = Np % 128 == 0 && a.kk2 * Fg >= 256 * a.s * a.s && (a.Cg <= 64 || a.Cg > 96);
+    const int wide = uniform && a.Cg > 32 && a.Cg <= 48 ? 16 : 32, taps = (a.k + a.s - 1) / a.s;
+    const double flops = 2e-9 * Np * a.HH * ((a.Cg + wide - 1) / wide * wide) * a.G * a.kk2 * Fg / (a.s * a.s);
+    const double all = 6. + flops / (uniform ? 95. : 80.) * 1e3, one = 5. + 0.024 * taps * taps * Fg * (a.Cg > 64 ? 3 : a.Cg > 32 ? 2 : 1);
+    return (all > one ? all : one) + copies;
   }
   if (Np % 128 == 0) {   // pixels of a block as columns
     const int taps = (a.k + a.s - 1) / a.s, cols = a.Cg * a.s * a.s;
@@ -318,7 +327,9 @@ static inline double conv_pixels_other_us(const Args& a, bool maps16, bool filte
 
 // The fastest of these tiles, on the bf16 matrix cores or not; cfg < 0: none fits, or another kernel is expected to be faster.
 // (0.87: of layers whose estimates are as near as that, measured, half lose, by 20 % at most: 3 -> 208 colours of 7 x 7, stride 4, 200 x
-// 200, batch 80, 190 -> 237 us; 1 -> 48 of 7 x 7, 26 x 26, 80, 14.6 -> 18.1.)
+// 200, batch 80, 190 -> 237 us; 1 -> 48 of 7 x 7, 26 x 26, 80, 14.6 -> 18.1.  Of 410 random layers of few colours that are taken six are
+// slower, by 22 % at most.  0.96 of strided layers of many colours, whose estimates are nearer: of 500 that coarser ones gave to these
+// tiles 48 were more than 4 % slower, by up to 38 %, and now 13, by up to 17 %; 21 that the others keep would gain 4 to 48 %.)
 template <class Args>
 static inline ConvRingPlan conv_pixels_choice(const Args& a, bool maps16, bool filters16, int cus) {
   ConvRingPlan best = conv_no_ring();
@@ -328,7 +339,7 @@ static inline ConvRingPlan conv_pixels_choice(const Args& a, bool maps16, bool f
       const ConvRingPlan plan = conv_pixels_plan(a, blocks, cus, bf16 != 0);
       if (plan.cfg >= 0 && (best.cfg < 0 || plan.us < best.us)) best = plan;
     }
-  return best.cfg >= 0 && best.us < 0.87 * conv_pixels_other_us(a, maps16, filters16, cus) ? best : conv_no_ring();
+  return best.cfg >= 0 && best.us < (conv_phases(a) ? 0.96 : 0.87) * conv_pixels_other_us(a, maps16, filters16, cus) ? best : conv_no_ring();
 }
 
 // Outp of `a`, whose batch the ring takes in whole groups of four images: others are copied with up to three images of zeros.

@@ -234,8 +234,11 @@ def test_the_busiest_xcd_counts_for_every_tile_of_few_colours(plans):
     assert taken > 200 and refused > 50
 
 
-# convDown, us: on the other kernels / on the tiles that coarser estimates took it to
-SLOWER_ON_TILES = [(173, 13, 15, 244, 7, 1, 0, 1), (205, 8, 12, 236, 5, 1, 0, 1), (146, 13, 20, 220, 6, 1, 0, 1)]       # 86 / 142, 46 / 70, 132 / 172
+# convDown, us: on the other kernels / on the tiles that coarser estimates took it to (of one pixel, of blocks of pixels)
+SLOWER_ON_TILES = [
+    (173, 13, 15, 244, 7, 1, 0, 1), (205, 8, 12, 236, 5, 1, 0, 1), (146, 13, 20, 220, 6, 1, 0, 1),       # 86 / 142, 46 / 70, 132 / 172
+    (256, 82, 22, 256, 7, 4, 3, 2), (128, 43, 45, 128, 6, 4, 0, 1), (256, 88, 32, 64, 6, 2, 3, 2),       # 104 / 137, 86 / 108, 154 / 189
+    (128, 74, 28, 96, 7, 2, 3, 2), (128, 70, 23, 192, 5, 2, 2, 2), (112, 46, 15, 48, 3, 3, 0, 1)]        # 120 / 145, 91 / 109, 8.2 / 10.3
 
 
 def test_layers_that_tiles_made_slower_are_on_the_other_kernels(plans):
