@@ -1071,8 +1071,9 @@ bool dn_defer_row_sum(const float* M, float* y, int h, int w, float alpha, float
   else dn_flush_ext();
   g_sums[g_nsums++] = DnRowSumJob{M, y, h, w, alpha, beta, kind == 2 ? 1 : 0};
   dn_set_pending(true);
-  if (g_nsums == 4) {
+  if (g_nsums == 4) {               // (nothing more can join, and no call is held back that would close the group)
     const int e = run_stats();
+    dn_close_group();
     if (!*err) *err = e;
   }
   return true;

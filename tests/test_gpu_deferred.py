@@ -778,6 +778,29 @@ def test_launch_deferred_queues_what_is_held_back(cm, rng):
     cm.launch_deferred()                      # nothing held back: no effect
 
 
+@pytest.mark.parametrize("shape", [(1003, 700, 250), (784, 500, 100)], ids=lambda s: "%dx%dx%d" % s)
+def test_the_statistics_of_a_step_are_queued_with_its_last_sum(cm, shape):
+    """With two products and four sums nothing more can join: they are on their way when the last call returns (mid-sized products, of
+    more than 128 terms, share a launch with others, smaller ones do not)."""
+    import ctypes as ct
+    hip = ct.CDLL('libamdhip64.so')
+    hip.hipMemcpy.argtypes = [ct.c_void_p, ct.c_void_p, ct.c_size_t, ct.c_int]
+    res = []
+    for deferred in (False, True):
+        cm.set_deferred_epilogues(deferred)
+        o = _Stat(cm, shape, 13)
+        stat_cd(cm, o)
+        out = []
+        for m in (o.W, o.bv, o.bh):
+            got = np.empty(m.shape, dtype=np.float32, order='F')
+            assert hip.hipMemcpy(got.ctypes.data, ct.cast(m.p_mat.contents.data_device, ct.c_void_p), got.nbytes, 2) == 0
+            out.append(got.view(np.uint32))
+        res.append(out)
+    cm.set_deferred_epilogues(True)
+    for w, g in zip(*res):
+        assert np.array_equal(g, w)
+
+
 # ---- random call sequences: whatever is held back, every matrix ends with the bits of the separate launches
 
 def _random_sequence(cm, rng_ops, pool, vecs, rows, n_ops):
