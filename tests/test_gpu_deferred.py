@@ -695,6 +695,117 @@ def upd_sum_then_read(cm, P):
     return P[0][0].asarray().view(np.uint32).copy()
 
 
+# Products that updates wait behind, and their late operands.  X, Y, Z: 300 x 300, updates (X[0], X[1], X[2]); b: 300 x 1; A, B, T, U:
+# products of 300 terms (k_gemm_ring); late_*: the operand comes when the product waits, or has left for the products that share a launch
+
+def late_bias_of_an_update(cm, o):
+    for i in range(3):
+        _upd(*o.b, reset=i != 2); cm.dot(o.A, o.B, target=o.T); o.T.add_col_vec(o.b[i]); o.T.apply_sigmoid(); o.U.add(o.T)
+
+
+def late_bias_beside_an_update(cm, o):
+    _upd(*o.X); cm.dot(o.A, o.B, target=o.T); o.T.add_col_vec(o.b[0]); o.T.lower_bound(0); _upd(*o.b)
+
+
+def late_factor_of_an_update(cm, o):
+    for i in range(3):
+        _upd(*o.X, reset=i != 2); cm.dot(o.A, o.B, target=o.T); o.T.mult(o.X[i]); o.T.apply_rectified_linear_deriv(o.Y[0]); o.U.add(o.T)
+
+
+def late_factor_and_gate_of_updates(cm, o):
+    _upd(*o.X); _upd(*o.Y, reset=False); cm.dot(o.A, o.B, target=o.T); o.T.mult(o.X[0]); o.T.apply_rectified_linear_deriv(o.Y[0])
+
+
+def late_gate_of_an_update(cm, o):
+    for i in range(3):
+        _upd(*o.X, reset=i != 2); cm.dot(o.A, o.B, target=o.T); o.T.apply_rectified_linear_deriv(o.X[i]); o.U.add(o.T)
+
+
+def late_second_product_of_an_update(cm, o):
+    for i in range(3):
+        _upd(*o.X, reset=i != 2); o.T.add_dot(o.A, o.B, mult=0.1); o.T.add_dot(o.X[i], o.B, mult=-0.1)
+        _upd(*o.X, reset=i != 2); o.T.add_dot(o.A, o.B, mult=0.1); o.T.add_dot(o.A, o.X[i], mult=-0.1); o.b[2].add_sums(o.T, axis=1, mult=0.01)
+
+
+def late_gate_behind_updates(cm, o):
+    # the layer's order of deepnet: input gradient, weight gradient, its update, the sums and update of the biases, the gate
+    cm.dot(o.A, o.B, target=o.T); o.X[2].add_dot(o.A, o.Y[0]); _upd(*o.X); o.b[2].add_sums(o.A, axis=1); _upd(*o.b)
+    o.T.apply_rectified_linear_deriv(o.Y[0]); o.U.add(o.T)
+
+
+def late_gate_that_an_update_writes(cm, o):
+    for i in range(3):
+        cm.dot(o.A, o.B, target=o.T); _upd(*o.X, reset=i != 2); o.T.apply_rectified_linear_deriv(o.X[i]); o.U.add(o.T)
+
+
+def late_gate_that_a_grouped_product_writes(cm, o):
+    cm.dot(o.A, o.B, target=o.T); o.Y[2].add_dot(o.A, o.B, mult=-0.1); _upd(*o.X); o.T.apply_rectified_linear_deriv(o.Y[2])
+
+
+def late_gate_that_a_grouped_sum_writes(cm, o):
+    cm.dot(o.A, o.B, target=o.T); o.col.add_sums(o.A, axis=1, mult=0.1); _upd(*o.X); o.T.apply_rectified_linear_deriv(o.over_col)
+
+
+def late_gate_of_a_target_that_a_grouped_product_reads(cm, o):
+    cm.dot(o.A, o.B, target=o.T); o.Y[2].add_dot(o.T, o.B, mult=0.1); _upd(*o.X); o.T.apply_rectified_linear_deriv(o.Y[0])
+
+
+def late_gate_of_a_target_that_a_grouped_sum_reads(cm, o):
+    cm.dot(o.A, o.B, target=o.T); o.b[2].add_sums(o.T, axis=1, mult=0.1); _upd(*o.X); o.T.apply_rectified_linear_deriv(o.Y[0])
+
+
+def late_gate_of_an_update_of_the_target(cm, o):
+    cm.dot(o.A, o.B, target=o.T); _upd(o.X[0], o.X[1], o.T); o.T.apply_rectified_linear_deriv(o.Y[0])
+    cm.dot(o.A, o.B, target=o.X[0]); _upd(*o.X); o.X[0].apply_rectified_linear_deriv(o.Y[0])
+
+
+def late_gate_of_an_accumulating_product(cm, o):
+    o.T.add_dot(o.A, o.B, mult=0.1); _upd(*o.X); o.T.apply_rectified_linear_deriv(o.Y[0])
+    o.T.add_dot(o.A, o.B, mult=0.1); o.T.add_dot(o.A, o.Y[1], mult=0.1); _upd(*o.X); o.T.apply_rectified_linear_deriv(o.Y[0])
+
+
+def late_gate_twice_and_into_another_target(cm, o):
+    cm.dot(o.A, o.B, target=o.T); _upd(*o.X); o.T.apply_rectified_linear_deriv(o.Y[0]); o.T.apply_rectified_linear_deriv(o.Y[1])
+    cm.dot(o.A, o.B, target=o.T); _upd(*o.X); o.T.apply_rectified_linear_deriv(o.Y[0], target=o.U)
+
+
+def late_gate_behind_an_unfinished_update(cm, o):
+    cm.dot(o.A, o.B, target=o.T); o.X[1].mult(0.9); o.X[1].add_mult(o.X[2]); o.T.apply_rectified_linear_deriv(o.X[1])
+    cm.dot(o.A, o.B, target=o.T); o.Y[0].mult(0.9); o.T.apply_rectified_linear_deriv(o.Y[0])
+
+
+LATE = [f for n, f in sorted(globals().items()) if n.startswith('late_')]
+
+
+class _Late:
+    def __init__(self, cm, seed, side):
+        rng = np.random.default_rng(seed)
+        g = lambda *d: cm.CUDAMatrix(_f(rng.standard_normal(d)))
+        n = side
+        self.X, self.Y, self.b = ([g(*d) for _ in range(3)] for d in ((n, n), (n, n), (n, 1)))
+        self.A, self.B, self.T, self.U, self.over_col = (g(n, n) for _ in range(5))
+        self.col = self.over_col.slice(n - 1, n)              # (its last column)
+
+    def all(self):
+        return self.X + self.Y + self.b + [self.A, self.B, self.T, self.U, self.over_col]
+
+
+@pytest.mark.parametrize("seq", LATE, ids=lambda f: f.__name__)
+@pytest.mark.parametrize("side", [300, 60, 640])
+def test_late_operands_of_products_keep_the_order_of_calls(cm, seq, side):
+    """(60: on the kernels of 16 x 16 blocks; 640: another tile)"""
+    res = []
+    for deferred in (False, True):
+        cm.set_deferred_epilogues(deferred)
+        o = _Late(cm, 31, side)
+        for _ in range(2):
+            seq(cm, o)
+        res.append([_bits(x) for x in o.all()])
+    cm.set_deferred_epilogues(True)
+    for i, (w, g) in enumerate(zip(*res)):
+        assert np.array_equal(g, w), "matrix %d differs" % i
+
+
 UPDS = [upd_sums_between, upd_sums_of_what_waits, upd_sums_into_what_waits, upd_sums_that_join_and_do_not, upd_sum_then_read, upd_six_in_a_row, upd_without_resets, upd_mixed_decays_and_resets, upd_eleven, upd_tied, upd_gradient_is_another_delta,
         upd_then_scale_that_is_no_update, upd_then_read, upd_interleaved_with_a_product, upd_reset_of_another_gradient]
 
@@ -909,7 +1020,6 @@ def _ew_call(cm, kind, x, y, t, vecs, s):
     calls[kind]()
 
 
-# (from 2^23 elements on calls without a common input do not wait for each other)
 # sides of products on every tile of k_gemm_ring and on the kernels beside it (one of 128 terms at most is not on the ring)
 GROUP_SIDES = [[64, 130, 301, 700], [100, 200, 784, 1024], [129, 250, 1003, 1500], [16, 33, 520, 2100]]
 
@@ -935,7 +1045,7 @@ def test_products_that_share_a_launch_keep_their_bits(cm, sides, seed):
             ta, tb, kind, tail = (int(rng.integers(x)) for x in (2, 2, 8, 5))
             A, B, C = pick(k, m) if ta else pick(m, k), pick(n, k) if tb else pick(k, n), pick(m, n)
             A2, gate, rows = pick(k, m) if ta else pick(m, k), pick(m, n), pick(m, n)
-            if C in (A, B, A2, gate):
+            if kind < 7 and (C in (A, B) or (kind == 4 and C == A2) or (kind < 3 and tail == 2 and C == gate)):
                 continue                                     # (a product into one of its operands is no product)
             T = mats[C]
             if kind < 3:
@@ -964,6 +1074,7 @@ def test_products_that_share_a_launch_keep_their_bits(cm, sides, seed):
         assert np.array_equal(want, got)
 
 
+# (from 2^23 elements on calls without a common input do not wait for each other)
 @pytest.mark.parametrize("h,w", [(1, 1), (3, 1), (1, 7), (64, 33), (65, 33), (130, 127), (1001, 37), (2052, 2049), (2897, 2897)])
 @pytest.mark.parametrize("seed", range(4))
 def test_elementwise_calls_that_wait_keep_their_bits(cm, h, w, seed):
