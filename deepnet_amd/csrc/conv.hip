@@ -2689,19 +2689,19 @@ static bool conv_pixels_ring(const ConvArgs& a, const ConvRingPlan& plan, const 
   return ring_done(where);
 }
 
-// The choice for a layer (it depends on its sizes and alignment only), kept for the next call: it prices some hundred plans, which is
-// several microseconds of the host's, as long as the shortest passes take.  One table a thread: ctypes gives up the interpreter's lock.
+// The choice for a layer (see conv_key), kept for the next call: it prices some hundred plans, which is several microseconds of the
+// host's, as long as the shortest passes take.  One table a thread: ctypes gives up the interpreter's lock.
 static const ConvChoice& conv_chosen(const ConvArgs& a, int mode) {
-  struct Entry { int key[14]; bool used; ConvChoice choice; };
+  struct Entry { ConvKey key; bool used; ConvChoice choice; };
   static thread_local Entry cache[128];
-  const int key[14] = {mode, a.N, a.C, a.H, a.F, a.k, a.Mx, a.s, a.pad0, a.G, a.local, a.m_count, a.chunks,
-                       (ring_maps16(a) ? 2 : 0) + (dn_aligned16(a.flt) ? 1 : 0)};
+  const bool maps16 = ring_maps16(a), filters16 = dn_aligned16(a.flt);
+  const ConvKey key = conv_key(a, mode, maps16, filters16, dn_num_cus());
   unsigned h = 0;
-  for (int v : key) h = h * 0x9e3779b1u + (unsigned)v;
+  for (int v : key.v) h = h * 0x9e3779b1u + (unsigned)v;
   Entry& e = cache[(h >> 16) % 128];
-  if (!e.used || memcmp(e.key, key, sizeof key) != 0) {
-    e.choice = conv_choice(a, mode, ring_maps16(a), dn_aligned16(a.flt), dn_num_cus());
-    memcpy(e.key, key, sizeof key);
+  if (!e.used || memcmp(&e.key, &key, sizeof key) != 0) {
+    e.choice = conv_choice(a, mode, maps16, filters16, dn_num_cus());
+    e.key = key;
     e.used = true;
   }
   return e.choice;

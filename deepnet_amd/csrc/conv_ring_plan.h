@@ -399,3 +399,10 @@ static inline ConvChoice conv_choice(const Args& a, int mode, bool maps16, bool 
   }
   return {rows, false};
 }
+
+// All that conv_choice depends on.
+struct ConvKey { int v[15]; };
+template <class Args>
+static inline ConvKey conv_key(const Args& a, int mode, bool maps16, bool filters16, int cus) {
+  return {{mode, a.N, a.C, a.H, a.F, a.k, a.Mx, a.s, a.pad0, a.G, a.local, a.m_count, a.chunks, (maps16 ? 2 : 0) + (filters16 ? 1 : 0), cus}};
+}

@@ -64,6 +64,15 @@ void conv_route(int mode, int N, int C, int H, int F, int k, int Mx, int s, int 
   out[4] = conv_other_us(a, mode, mode == CONV_DOWN ? a.HH : a.M, N % 4 == 0, true, cus); out[5] = ring_crowd(a);
 }
 
+// What a layer's choice is kept by; in: mode, the sizes from N to chunks but for those that follow from others, both alignments, CUs.
+int conv_key_of(const int* in, int* out) {
+  const Sizes a = {in[1], in[2], in[2] / in[9], in[3], in[3] * in[3], in[4], in[4] / in[9], in[5], in[5] * in[5], in[6], in[6] * in[6], in[7], in[8],
+                   in[9], in[10], in[11], in[12]};
+  const ConvKey key = conv_key(a, in[0], in[13] != 0, in[14] != 0, in[15]);
+  for (int v : key.v) *out++ = v;
+  return sizeof key / sizeof(int);
+}
+
 // convDown of strided layers, few colours or filters that are no whole fours: out = {tile number or -1, side of a block in strides, 0 a
 // pixel or -1 any run, stages of the table, LDS bytes of a workgroup}
 void conv_pixels_tile(int N, int C, int H, int F, int k, int Mx, int s, int pad0, int G, int cus, double* out) {

@@ -246,3 +246,14 @@ def test_layers_that_tiles_made_slower_are_on_the_other_kernels(plans):
     for N, C, H, F, k, s, p, G in SLOWER_ON_TILES:
         plans.conv_route(DOWN, N, C, H, F, k, co.n_modules(H, k, s, p), s, -p, G, CUS, out)
         assert out[0] < 0, (N, C, H, F, k, s, p, G)
+
+
+def test_the_choice_of_a_layer_is_kept_by_all_that_it_depends_on(plans):
+    layer = [DOWN, 128, 24, 14, 96, 5, 10, 1, 0, 2, 0, 100, 1, 1, 1, CUS]
+
+    def key(values):
+        out = (ct.c_int * 32)()
+        return list(out[:plans.conv_key_of((ct.c_int * 16)(*values), out)])
+    for i, other in enumerate([UP, 100, 48, 16, 64, 3, 12, 2, -2, 1, 1, 50, 2, 0, 0, 304]):
+        assert other != layer[i] and key(layer) != key(layer[:i] + [other] + layer[i + 1:]), i
+    assert key(layer) == key(list(layer))
