@@ -1,6 +1,7 @@
 """The callables of csrc/fastcall.c in the place of ctypes functions: every kind of argument arrives as ctypes hands it over, and what they
 do not take goes to ctypes (CPU only: the functions that are called are ctypes callbacks)."""
 import ctypes as ct
+import sysconfig
 
 import numpy as np
 import pytest
@@ -71,3 +72,8 @@ def test_other_arguments_go_to_ctypes(cm, fastcall):
     assert fast.argtypes == slow.argtypes and cm._cudamat.dot.argtypes == cm._SIGNATURES['dot'][1]
     with pytest.raises(KeyError):
         fastcall.Function(1, 'ffff', (), slow)
+
+
+def test_the_module_is_named_for_its_interpreter(fastcall):
+    """(another version of Python does not find it, and takes ctypes)"""
+    assert fastcall.__file__.endswith('/_fastcall' + sysconfig.get_config_var('EXT_SUFFIX'))
