@@ -137,12 +137,19 @@ static void function_dealloc(PyObject* o) {
   Py_TYPE(o)->tp_free(o);
 }
 
-/* restype, argtypes and the like are those of the ctypes function */
+/* restype, argtypes and the like are those of the ctypes function, which is also what ctypes takes as an argument (cast) */
 static PyObject* function_getattro(PyObject* o, PyObject* name) {
+  PyObject* slow = ((Function*)o)->slow;
   PyObject* res = PyObject_GenericGetAttr(o, name);
   if (res || !PyErr_ExceptionMatches(PyExc_AttributeError)) return res;
   PyErr_Clear();
-  return PyObject_GetAttr(((Function*)o)->slow, name);
+  if (PyUnicode_CompareWithASCIIString(name, "_as_parameter_") == 0) { Py_INCREF(slow); return slow; }
+  return PyObject_GetAttr(slow, name);
+}
+/* ... and once a program has set one, the calls go there */
+static int function_setattro(PyObject* o, PyObject* name, PyObject* value) {
+  ((Function*)o)->n = -1;
+  return value ? PyObject_SetAttr(((Function*)o)->slow, name, value) : PyObject_DelAttr(((Function*)o)->slow, name);
 }
 
 static PyTypeObject FunctionType = {
@@ -152,6 +159,7 @@ static PyTypeObject FunctionType = {
     .tp_vectorcall_offset = offsetof(Function, vectorcall),
     .tp_call = PyVectorcall_Call,
     .tp_getattro = function_getattro,
+    .tp_setattro = function_setattro,
     .tp_new = function_new,
     .tp_dealloc = function_dealloc,
 };

@@ -77,3 +77,16 @@ def test_other_arguments_go_to_ctypes(cm, fastcall):
 def test_the_module_is_named_for_its_interpreter(fastcall):
     """(another version of Python does not find it, and takes ctypes)"""
     assert fastcall.__file__.endswith('/_fastcall' + sysconfig.get_config_var('EXT_SUFFIX'))
+
+
+def test_what_ctypes_functions_take_besides_calls(cm, fastcall):
+    fast, slow, seen = pair(cm, fastcall, 'Pf')
+    assert ct.cast(fast, ct.c_void_p).value == ct.cast(slow, ct.c_void_p).value
+    assert fast(None, 1.5) == 1 and fast(None, 1.5) == 2
+    fast.errcheck = lambda result, func, args: result + 100          # (what is set, counts from the next call on)
+    assert fast(None, 2.5) == 103 and slow(None, 2.5) == 104 and fast.errcheck is slow.errcheck
+    assert [s[1] for s in seen] == [1.5, 1.5, 2.5, 2.5]
+    del fast.errcheck
+    assert fast(None, 2.5) == 5
+    with pytest.raises(TypeError):
+        fast.argtypes = 3
