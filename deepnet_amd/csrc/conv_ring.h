@@ -22,16 +22,18 @@ struct ConvRingArgs {
   int rows, cols;               // of one period: a tile lies inside one (one module or pixel, or everything)
   int periods, gx, gy, gz;      // tiles per period down the rows, across; Up / Down: groups; Outp: chunks x splits x groups
   int K;                        // Outp: terms of a chunk
-  // (what only Outp has, and only DownM: side of a block of pixels, blocks per side of a map.  64 bytes more of arguments are 0.15 us
-  // a launch)
+  // (What only Outp has, and only DownM: side of a block of pixels, blocks per side of a map.  64 bytes more of arguments are 0.15 us
+  // a launch, and so is a line of 64 that a pass reads for one of them only: what every tile needs of the divisors lies next to ldc.)
   union { int m_count, block; };
   union { int splits, lines; };
   int split_stages;
-  FastDiv dN, dH, dFg4, dgx, dgy, dper, dG;
-  union { FastDiv dsplits, ds; };                                        // Outp; Down
+  FastDiv dN;
   union { FastDiv dMx, dlines; };                                        // all others; DownM
   union { FastDiv dk, dblock; };
   union { FastDiv dkk2, dblock2; };
+  FastDiv dH, dFg4, dgx, dgy, dper;
+  union { FastDiv dsplits, ds; };                                        // Outp; Down
+  FastDiv dG;
   __host__ __device__ int Fg4() const { return (Fg + 3) & ~3; }          // filters of a group in whole fours
   long long ldc, out_stride;    // of a column; Outp: of a (chunk, split)
 };
@@ -198,7 +200,9 @@ struct ConvSplitCfg {
   template <int ROWS, bool KC> using Tile = SplitTile<ROWS, BK, KC, THREADS>;
   template <class OA, class OB> using Shape = SplitShape<BM, BN, BK, WM, WN, KS, SETS, OA, OB>;
 };
-template <int MODE, bool SINGLE, class Cfg>
+// LOOSE: of a tile that may be larger than all rows or columns there are.  (Instances of their own: with the bounds that it needs
+// convUp of the locally connected layer above takes 8.80 us instead of 8.70.)
+template <int MODE, bool SINGLE, bool LOOSE, class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRingArgs p) {
   constexpr int PER = MODE == CONV_UP ? 1 : 4, BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, THREADS = Cfg::THREADS;
   using OA = ConvRingOperand<MODE == CONV_OUTP ? 3 : MODE == CONV_DOWNM ? 9 : SINGLE ? 5 : 0, typename Cfg::template Tile<BM, MODE == CONV_OUTP>, PER>;
@@ -228,7 +232,6 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
   // a tile over the edge moves back inside; the outputs it shares with its neighbour are that one's to store (of a tile larger than
   // all there is, rows and columns behind the last are computed from what stands there, or zeros, and not stored)
   const int m_lo = bx * BM, n_lo = by * BN;
-  constexpr bool LOOSE = conv_may_be_loose(MODE, Cfg::SPLIT);
   const int m0 = m_lo + BM <= p.rows || (LOOSE && p.rows < BM) ? m_lo : p.rows - BM;
   const int n0 = n_lo + BN <= p.cols || (LOOSE && p.cols < BN) ? n_lo : p.cols - BN;
 
@@ -447,6 +450,20 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES) k_conv_ring(ConvRing
   }
 }
 
+// (of these modes there is no instance without LOOSE: their layers are of few colours, odd or strided, and mostly small)
+static constexpr bool conv_always_loose(int mode) { return mode == CONV_DOWNM || mode == CONV_DOWNS || mode == CONV_DOWNO; }
+template <int MODE, bool SINGLE, class Cfg>
+static void conv_ring_go(const ConvRingArgs& p, dim3 grid, size_t tab) {
+  constexpr bool may = conv_may_be_loose(MODE, Cfg::SPLIT), always = may && conv_always_loose(MODE);
+  if constexpr (may) {
+    if (always || p.rows < Cfg::BM || p.cols < Cfg::BN) {
+      hipLaunchKernelGGL((k_conv_ring<MODE, SINGLE, true, Cfg>), grid, dim3(Cfg::THREADS), tab, dn_stream(), p);
+      return;
+    }
+  }
+  if constexpr (!always) hipLaunchKernelGGL((k_conv_ring<MODE, SINGLE, false, Cfg>), grid, dim3(Cfg::THREADS), tab, dn_stream(), p);
+}
+
 template <int MODE, bool SINGLE>
 static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
   const ConvRingTile f = conv_ring_cfg(MODE, plan.cfg);
@@ -461,7 +478,7 @@ static void conv_ring_launch(const ConvRingPlan& plan, ConvRingArgs p) {
   p.dk = make_fastdiv(MODE == CONV_DOWNM ? p.block : p.k);
   p.dkk2 = make_fastdiv(MODE == CONV_DOWNM ? p.block * p.block : p.kk2);
   const size_t tab = (size_t)conv_ring_table(MODE, SINGLE, f.bk, stages);
-#define CONV_RING(...) hipLaunchKernelGGL((k_conv_ring<MODE, SINGLE, __VA_ARGS__>), grid, dim3(__VA_ARGS__::THREADS), tab, dn_stream(), p)
+#define CONV_RING(...) conv_ring_go<MODE, SINGLE, __VA_ARGS__>(p, grid, tab)
   switch (plan.cfg) {
     case 0: CONV_RING(ConvRingCfg<32, 64, 64, 32>); break;
     case 1: CONV_RING(ConvRingCfg<32, 64, 32, 64>); break;
