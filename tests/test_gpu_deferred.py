@@ -912,6 +912,38 @@ def test_the_statistics_of_a_step_are_queued_with_its_last_sum(cm, shape):
         assert np.array_equal(g, w)
 
 
+def _launches(cm, run):
+    """Kernels that the calls of run() queue (recorded on a stream of the test's own)."""
+    import ctypes as ct
+    hip = ct.CDLL('libamdhip64.so')
+    stream, graph, nodes = ct.c_void_p(), ct.c_void_p(), ct.c_size_t()
+    run()
+    cm.cuda_sync_threads()
+    assert hip.hipStreamCreateWithFlags(ct.byref(stream), 1) == 0
+    assert hip.hipStreamBeginCapture(stream, 1) == 0
+    cm._cudamat.graph_set_stream(stream, 1)
+    run()
+    cm.launch_deferred()
+    cm._cudamat.graph_set_stream(None, 0)
+    assert hip.hipStreamEndCapture(stream, ct.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, ct.byref(nodes)) == 0
+    assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(stream) == 0
+    return nodes.value
+
+
+@pytest.mark.parametrize("inputs,outputs,batch", [(279, 681, 103), (734, 123, 116), (107, 531, 124)])
+def test_sums_go_with_their_product_where_others_wait(cm, inputs, outputs, batch):
+    """A gradient of at most 128 terms takes the sums of its layer along: also behind products that wait to share a launch and read or write
+    what the sums do, or have sums of their own."""
+    g = lambda *d: cm.CUDAMatrix(_f(0.1 * np.random.default_rng(d[0]).standard_normal(d)))
+    W, X, Y, D, DX, G, G2, b, b2 = (g(inputs, outputs), g(inputs, batch), g(outputs, batch), g(outputs, batch), g(inputs, batch), g(inputs, outputs),
+                                    g(inputs, outputs), g(outputs, 1), g(outputs, 1))
+    # (at most as many as the gradients and the other products)
+    assert _launches(cm, lambda: (G.add_dot(X, D.T), b.add_sums(D, axis=1))) == 1
+    assert _launches(cm, lambda: (cm.dot(W.T, X, target=Y), Y.add_col_vec(b), cm.dot(W, D, target=DX), G.add_dot(X, D.T), b.add_sums(D, axis=1))) <= 3
+    assert _launches(cm, lambda: (G.add_dot(X, D.T), b.add_sums(D, axis=1), G2.add_dot(X, D.T), b2.add_sums(D, axis=1))) <= 2
+
+
 # ---- random call sequences: whatever is held back, every matrix ends with the bits of the separate launches
 
 def _random_sequence(cm, rng_ops, pool, vecs, rows, n_ops):
